@@ -30,12 +30,15 @@
 // State lives in LDS for rows up to the LDS capacity (15 bytes per position: an 8-byte record,
 // product and gate of the position's pair, and the two queues), and in a global scratch area
 // (L2-resident, 32-bit links) for longer rows that cannot be cut into chunks.
+#include "bpe_automaton.hpp"
 #include "common.hpp"
 
 #include <stdlib.h>
 #include <string.h>
 #include <atomic>
 #include <mutex>
+#include <new>
+#include <type_traits>
 #include <unordered_map>
 #include <vector>
 
@@ -50,6 +53,13 @@ struct dnatok_bpe_table {
     int32_t *out_remap;          // [n_symbols] or nullptr
     uint32_t *ltab;              // the compact form of the table that fits LDS (kLdsTabWords words), or nullptr
     uint32_t lmul1, lmul2;       // its two multipliers
+    // the vocabulary as an automaton (bpe_automaton.hpp); auto_states = 0: it has none
+    uint32_t auto_states, auto_letters;
+    int auto_wide;               // transitions as 32-bit entries in global memory instead of 16-bit ones in LDS
+    void *auto_next;
+    uint8_t *auto_len;
+    uint16_t *auto_sym;
+    int32_t *auto_id;
     void *first;                 // dnatok::FirstPairs on the device, or nullptr (more bytes with rules than classes)
     // dnatok_bpe_encode_padded: the tree of atomics that carries a call's longest row
     // (dnatok::publish_max), one per stream that encodes with this table (calls on one stream are
@@ -1955,6 +1965,12 @@ __global__ __launch_bounds__(256) void bpe_gather_wave_kernel(
     }
 }
 
+}  // namespace dnatok
+
+#include "bpe_automaton_kernel.hpp"
+
+namespace dnatok {
+
 // Whole-row kernel for rows above the LDS capacity that could not be chunked: one workgroup per
 // row, state in global scratch (26 bytes / base).
 template <int NT>
@@ -2139,6 +2155,27 @@ extern "C" int dnatok_bpe_table_create(const int32_t *byte_to_id_h, const int32_
         }
     }
 
+    // the automaton, where the table has one (a table that does not is encoded by the merge engine)
+    BpeAutomaton fa;
+    bool wide = false;
+#ifndef DNATOK_BPE_PHASE_CYCLES                      // (that build measures the merge engine)
+    if (monotone) {
+        std::vector<uint8_t> in_effect(n_merges);
+        for (int32_t i = 0; i < n_merges; ++i)
+            in_effect[i] = last_entry[((uint32_t)pair_a_h[i] << 16) | (uint32_t)pair_b_h[i]] == i;
+        try {
+            if (!build_bpe_automaton(byte_to_id_h, pair_a_h, pair_b_h, new_id_h, in_effect.data(), n_merges, n_symbols, &fa))
+                fa = BpeAutomaton{};
+        } catch (const std::bad_alloc &) {
+            fa = BpeAutomaton{};
+        }
+        wide = fa.n_states > kAutoNarrowStates;
+    }
+#endif
+    // its arrays as the kernels read them: one more state for a byte that is no letter, whose
+    // successors are the row start's, and behind the states the symbols of the bytes
+    const size_t auto_n = fa.n_states ? (size_t)fa.n_states + 1 : 0;
+
     auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
     const size_t o_tab = 0;
     const size_t o_b2s = up(o_tab + (size_t)slots * sizeof(uint4));
@@ -2146,13 +2183,33 @@ extern "C" int dnatok_bpe_table_create(const int32_t *byte_to_id_h, const int32_
     const size_t o_first = up(o_remap + (out_remap_h ? (size_t)n_symbols * 4 : 0));
     const size_t o_ltab = up(o_first + sizeof(FirstPairs));
     const size_t o_trees = up(o_ltab + ltab.size() * 4);
-    const size_t total = up(o_trees + (size_t)kMaxTreeSlots * kTreeWords * 8) + 256;
+    const size_t o_anext = up(o_trees + (size_t)kMaxTreeSlots * kTreeWords * 8);
+    const size_t o_alen = up(o_anext + auto_n * 4 * (wide ? 4 : 2));
+    const size_t o_asym = up(o_alen + auto_n);
+    const size_t o_aid = up(o_asym + (auto_n ? auto_n + 256 : 0) * 2);
+    const size_t total = up(o_aid + (auto_n && out_remap_h ? auto_n + 256 : 0) * 4) + 256;
     std::vector<uint8_t> host(total, 0);             // (the trees start as zeros)
     memcpy(&host[o_tab], tab.data(), (size_t)slots * sizeof(uint4));
     memcpy(&host[o_b2s], b2s.data(), 512);
     if (out_remap_h) memcpy(&host[o_remap], out_remap_h, (size_t)n_symbols * 4);
     if (!ltab.empty()) memcpy(&host[o_ltab], ltab.data(), ltab.size() * 4);
     memcpy(&host[o_first], &first, sizeof(FirstPairs));
+    if (auto_n) {
+        uint16_t *const sym = reinterpret_cast<uint16_t *>(&host[o_asym]);
+        for (size_t i = 0; i + 1 < auto_n; ++i) {
+            host[o_alen + i] = fa.len[i];
+            sym[i] = fa.sym[i];
+        }
+        host[o_alen + auto_n - 1] = 1;
+        for (int v = 0; v < 256; ++v) sym[auto_n + v] = b2s[v];
+        for (size_t i = 0; i < 4 * auto_n; ++i) {
+            const uint32_t to = fa.next[i < 4 * (size_t)fa.n_states ? i : i - 4 * (size_t)fa.n_states];
+            if (wide) reinterpret_cast<uint32_t *>(&host[o_anext])[i] = (to * 4) << 8 | fa.len[to];
+            else reinterpret_cast<uint16_t *>(&host[o_anext])[i] = (uint16_t)(to * 4);
+        }
+        if (out_remap_h)
+            for (size_t i = 0; i < auto_n + 256; ++i) reinterpret_cast<int32_t *>(&host[o_aid])[i] = out_remap_h[sym[i]];
+    }
     void *blob = nullptr;
     hipError_t e = hipMalloc(&blob, total);
     if (e == hipSuccess) e = hipMemcpy(blob, host.data(), total, hipMemcpyHostToDevice);
@@ -2172,6 +2229,11 @@ extern "C" int dnatok_bpe_table_create(const int32_t *byte_to_id_h, const int32_
     t->lmul1 = lmul1; t->lmul2 = lmul2;
     t->first = have_first ? (void *)(b + o_first) : nullptr;
     t->max_trees = (unsigned long long *)(b + o_trees);
+    t->auto_states = fa.n_states; t->auto_letters = fa.letters; t->auto_wide = wide ? 1 : 0;
+    t->auto_next = b + o_anext;
+    t->auto_len = b + o_alen;
+    t->auto_sym = (uint16_t *)(b + o_asym);
+    t->auto_id = out_remap_h ? (int32_t *)(b + o_aid) : nullptr;
     *out = t;
     return DNATOK_OK;
 }
@@ -2316,6 +2378,82 @@ int launch_lds_ltab(const BpeArgs &a, const uint8_t *bytes, const int64_t *offse
     return DNATOK_OK;
 }
 
+// The work list of rows that are cut into chunks, or are dealt by length.
+int launch_plan(int chunking, const int64_t *offsets, const BpePlan &p, int64_t n_rows, hipStream_t s)
+{
+    const int expand_here = chunking >> 1;
+    if (n_rows >= kPlanTiledFrom) {
+        const int tiles = (int)((n_rows + kPlanTile - 1) / kPlanTile);
+        bpe_plan_kernel<1><<<tiles, 1024, 0, s>>>(offsets, n_rows, chunking & 1, 0, p);
+        DNATOK_HIP_TRY(hipGetLastError());
+        bpe_plan_kernel<2><<<tiles, 1024, 0, s>>>(offsets, n_rows, chunking & 1, 0, p);
+    } else {
+        bpe_plan_kernel<0><<<1, 1024, 0, s>>>(offsets, n_rows, chunking & 1, expand_here, p);
+    }
+    DNATOK_HIP_TRY(hipGetLastError());
+    if ((chunking & 1) && !expand_here) {
+        bpe_expand_kernel<<<(int)((n_rows + 255) / 256), 256, 0, s>>>(offsets, n_rows, p);
+        DNATOK_HIP_TRY(hipGetLastError());
+    }
+    return DNATOK_OK;
+}
+
+template <bool WIDE, int P, bool CHUNKS, bool CHARS, bool PADDED>
+int launch_auto_as(const dnatok_bpe_t *t, const BpeArgs &a, AutoArgs aa, const uint8_t *bytes, const int64_t *offsets,
+                   const BpePlan &p, int64_t n_rows, int64_t items, int32_t *tok_tmp, int32_t *lengths, hipStream_t s)
+{
+    const size_t lds = AutoLds<WIDE, P>::bytes(t->auto_states);
+    auto kern = bpe_auto_kernel<WIDE, P, CHUNKS, CHARS, PADDED>;
+    // (once per kernel form; two threads that both find it unset both set it, to the same value)
+    static std::atomic<bool> attr_set{false};
+    if (!attr_set.load(std::memory_order_acquire)) {
+        DNATOK_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           (int)(WIDE ? lds : AutoLds<WIDE, P>::bytes(kAutoNarrowStates))));
+        attr_set.store(true, std::memory_order_release);
+    }
+    // (narrow: the workgroups of the largest table, which are those of any)
+    static const int64_t resident =
+        resident_workgroups(kern, 64 * kAutoWaves, AutoLds<WIDE, P>::bytes(WIDE ? 0 : kAutoNarrowStates), 1);
+    int64_t grid = items < resident ? items : resident;
+    if (a.max_tree && grid > kTreeRows) grid = kTreeRows;
+    if (grid < 1) grid = 1;
+    kern<<<(int)grid, 64 * kAutoWaves, lds, s>>>(a, aa, bytes, offsets, p, (int32_t)n_rows, tok_tmp, lengths);
+    DNATOK_HIP_TRY(hipGetLastError());
+    return DNATOK_OK;
+}
+
+// The automaton over the batch: rows of at most p.ext bytes whole, longer ones in the chunks of the work list.
+template <bool WIDE>
+int run_auto(const dnatok_bpe_t *t, const BpeArgs &a, int chunking, const uint8_t *bytes, const int64_t *offsets,
+             const BpePlan &p, int64_t n_rows, int64_t max_len, int64_t total, int32_t *tok_tmp, int32_t *lengths, hipStream_t s)
+{
+    AutoArgs aa{t->auto_next, t->auto_len, t->auto_sym, t->auto_id, t->auto_states, t->auto_letters, 64, 1, -1, total};
+    if (chunking & 1) {
+        const int rc = launch_plan(chunking, offsets, p, n_rows, s);
+        if (rc) return rc;
+        if (a.char_ids) return launch_auto_as<WIDE, 32, true, true, false>(t, a, aa, bytes, offsets, p, n_rows, p.max_items, tok_tmp, lengths, s);
+        return launch_auto_as<WIDE, 32, true, false, false>(t, a, aa, bytes, offsets, p, n_rows, p.max_items, tok_tmp, lengths, s);
+    }
+    // Regions of 32 bytes, of 16 when the batch is so small that its waves find a place at once either way
+    // (a lane's walk is then half as long, and twice the lanes share it).
+    const int64_t len = max_len < 1 ? 1 : max_len;
+    const int64_t lanes16 = (len + 15) / 16;
+    const bool small = len <= 1024 && (n_rows + 64 / lanes16 - 1) / (64 / lanes16) <= 256 * kAutoWaves;
+    aa.lanes = (int32_t)(small ? lanes16 : (len + 31) / 32);
+    aa.rows = 64 / aa.lanes;
+    const int64_t groups = (n_rows + aa.rows - 1) / aa.rows;
+    aa.n_groups = (int32_t)groups;
+    if (small) {
+        if (a.pad_ids) return launch_auto_as<WIDE, 16, false, false, true>(t, a, aa, bytes, offsets, p, n_rows, groups, tok_tmp, lengths, s);
+        if (a.char_ids) return launch_auto_as<WIDE, 16, false, true, false>(t, a, aa, bytes, offsets, p, n_rows, groups, tok_tmp, lengths, s);
+        return launch_auto_as<WIDE, 16, false, false, false>(t, a, aa, bytes, offsets, p, n_rows, groups, tok_tmp, lengths, s);
+    }
+    if (a.pad_ids) return launch_auto_as<WIDE, 32, false, false, true>(t, a, aa, bytes, offsets, p, n_rows, groups, tok_tmp, lengths, s);
+    if (a.char_ids) return launch_auto_as<WIDE, 32, false, true, false>(t, a, aa, bytes, offsets, p, n_rows, groups, tok_tmp, lengths, s);
+    return launch_auto_as<WIDE, 32, false, false, false>(t, a, aa, bytes, offsets, p, n_rows, groups, tok_tmp, lengths, s);
+}
+
 // The work list (plan) is needed when rows are cut into chunks or left to the whole-row kernel,
 // and when there are more rows than resident teams: rows then are dealt through the list's
 // counter, since rows take different times and a fixed share per team ends in a long tail
@@ -2341,20 +2479,8 @@ int run_lds_part(bool long_rows, int chunking, bool force_plan, const BpeArgs &a
             bpe_plan_in_order_kernel<<<1, 64, 0, s>>>((int32_t)n_rows, p);
             DNATOK_HIP_TRY(hipGetLastError());
         } else {
-            const int expand_here = chunking >> 1;
-            if (n_rows >= kPlanTiledFrom) {
-                const int tiles = (int)((n_rows + kPlanTile - 1) / kPlanTile);
-                bpe_plan_kernel<1><<<tiles, 1024, 0, s>>>(offsets, n_rows, chunking & 1, 0, p);
-                DNATOK_HIP_TRY(hipGetLastError());
-                bpe_plan_kernel<2><<<tiles, 1024, 0, s>>>(offsets, n_rows, chunking & 1, 0, p);
-            } else {
-                bpe_plan_kernel<0><<<1, 1024, 0, s>>>(offsets, n_rows, chunking & 1, expand_here, p);
-            }
-            DNATOK_HIP_TRY(hipGetLastError());
-            if ((chunking & 1) && !expand_here) {
-                bpe_expand_kernel<<<(int)((n_rows + 255) / 256), 256, 0, s>>>(offsets, n_rows, p);
-                DNATOK_HIP_TRY(hipGetLastError());
-            }
+            const int rc = launch_plan(chunking, offsets, p, n_rows, s);
+            if (rc) return rc;
         }
         if (chunking & 1) {
             if (a.char_ids) return launch_lds_as<NT, TEAMS, CAP, true, true>(a, bytes, offsets, p, n_rows, tok_tmp, lengths, s);
@@ -2424,14 +2550,20 @@ static int bpe_encode_launch(const dnatok_bpe_t *t, const uint8_t *bytes, const 
     // get a launch of their own.  The two launches cannot both carry the longest row up the one
     // tree: it is taken from the lengths afterwards.
     const bool split = work_len > 512 && n_rows >= 1024 && total / n_rows <= 384 && p.ext / 4 <= 512;
-    int32_t *const longest_after = split && a.max_tree ? a.longest : nullptr;
-    if (split) {
+    // The automaton takes what it can: every row of at most 2,048 bytes, and chunks of the shipped sizes.
+    // (The switches of the tests and measurements select the merge engine, whose they are.)
+    const bool automaton = t->auto_states != 0 && a.placement == 0 && p.ext <= 2048 && (p.ext & 1) == 0 && (!long_rows || chunking) &&
+                           t->chunk_core.load(std::memory_order_relaxed) == 0;
+    int32_t *const longest_after = split && a.max_tree && !automaton ? a.longest : nullptr;
+    if (split && !automaton) {
         a.in_order = 0;
         a.max_tree = nullptr;
     }
     // short rows: a wave per row, four rows to a workgroup (a 256-thread team would leave most of
     // its lanes without a position, and a row's time is its rounds, not its length)
-    if (work_len <= 256)         rc = run_lds<64, 4, 256>(long_rows, chunking, split, a, bytes, offsets, p, n_rows, tok_tmp, lengths, s);
+    if (automaton)               rc = t->auto_wide ? run_auto<true>(t, a, chunking, bytes, offsets, p, n_rows, max_len, total, tok_tmp, lengths, s)
+                                                   : run_auto<false>(t, a, chunking, bytes, offsets, p, n_rows, max_len, total, tok_tmp, lengths, s);
+    else if (work_len <= 256)    rc = run_lds<64, 4, 256>(long_rows, chunking, split, a, bytes, offsets, p, n_rows, tok_tmp, lengths, s);
     else if (work_len <= 384)    rc = run_lds<64, 4, 384>(long_rows, chunking, split, a, bytes, offsets, p, n_rows, tok_tmp, lengths, s);
     else if (work_len <= 512)    rc = run_lds<64, 4, 512>(long_rows, chunking, split, a, bytes, offsets, p, n_rows, tok_tmp, lengths, s);
     else if (work_len <= 1024)   rc = run_lds<256, 1, 1024>(long_rows, chunking, split, a, bytes, offsets, p, n_rows, tok_tmp, lengths, s);

@@ -1111,6 +1111,38 @@ def test_bpe_many_short_rows_a_wave_each(bpe, longest):
             np.testing.assert_array_equal(tok[b.offsets[i]:b.offsets[i] + lengths[i]], e, err_msg=f"row {i}")
 
 
+@pytest.mark.parametrize("count", [7, 6000])
+@pytest.mark.parametrize("longest", [1, 16, 17, 32, 33, 511, 1024, 1025, 2047, 2048, 2049])
+def test_bpe_automaton_at_the_edges_of_regions(bpe, longest, count):
+    """Rows whose lengths end at, before and behind the edges of a lane's region (16 bytes in a small
+    batch, 32 in a large one) and of the lanes a row has, few and many rows to a wave, with tandem
+    repeats that no two lanes agree in and bytes that are no letters: the oracle's tokens, and the same
+    as the merge engine's (which a set chunk geometry selects)."""
+    which, enc, bo = bpe
+    say(f"bpe{which} regions, longest {longest}, {count} rows")
+    rng = random.Random(longest * 10 + count)
+    count = min(count, 2_000_000 // longest)
+    def row(n):
+        kind = rng.randrange(4)
+        if kind == 0:
+            unit = "".join(rng.choices("ACGT", k=rng.randint(1, 6)))
+            return (unit * (n // len(unit) + 1))[:n]
+        weights = [24, 24, 24, 24, 4 if kind == 1 else 0]
+        return "".join(rng.choices("ACGTN", weights=weights, k=n))
+    seqs = [row(max(0, longest - rng.choice([0, 0, 1, 15, 16, 17, longest // 2, longest]))) for _ in range(count)]
+    seqs[0] = row(longest)
+    b = util.batch_from_strings(seqs)
+    got = bpe_rows(enc, b)
+    for i, (r, e) in enumerate(zip(got, bo.encode_batch(b.data, b.offsets))):
+        np.testing.assert_array_equal(r, e, err_msg=f"row {i}")
+    enc.set_chunk_geometry(1792, 128)
+    try:
+        for i, (r, e) in enumerate(zip(got, bpe_rows(enc, b))):
+            np.testing.assert_array_equal(r, e, err_msg=f"row {i}, merge engine")
+    finally:
+        enc.set_chunk_geometry(0, 0)
+
+
 @pytest.mark.parametrize("long_ones", ["up to 1 KB", "up to 2 KB", "cut into chunks"])
 def test_bpe_mostly_short_rows_with_some_long_ones(bpe, long_ones):
     """A batch of mostly short rows with a few long ones among them is split between two launches (the
