@@ -21,13 +21,19 @@
 //
 // What bounds it: the forward walk is a chain of dependent reads, one per byte and lane, so the
 // transition table has to be near.  Narrow form: 16-bit transitions and the token lengths in LDS,
-// staged once per workgroup, one workgroup of eight waves per CU (8,972 states: 81 KB, and 8 KB per
-// wave for states and tokens).  Wide form: 32-bit entries {state, token length} in global memory
+// staged once per workgroup, one workgroup of up to sixteen waves per CU (8,972 states: 81 KB, and 5 KB
+// per wave for states and tokens).  Wide form: 32-bit entries {state, token length} in global memory
 // (L2: 164,729 states are 2.6 MB), the waves' share of LDS alone.
 //
-// Per call, the merge engine -> the automaton: 1,024 rows of 1 KB 29.4 -> 14.7 us, 16,384 of them 236.5 ->
-// 54.7 us, 100,000 reads of 100 - 300 bp (int64 rows) 349 -> 123 us, 4,096 ragged reads of 12 Mbp 253.5 ->
-// 124.9 us (all with the vocabulary of 4,096), 32 rows of 100 kbp (32,000) 143.8 -> 96.2 us.
+// Every phase is a chain of dependent reads, so what a launch takes is the number of waves in flight.
+// Sixteen share the table instead of eight since a wave's tokens leave through a window of one per four
+// bytes (more than that are written lane by lane) and a chunk's go where the states were: 16,384 rows of
+// 1 KB 54.7 -> 29.2 us, 100,000 reads 123 -> 57 us.  (That includes the walk into the next region four bytes
+// at a time, comparing the last of the four, and the padded rows of a wave written as one run of cells.)
+//
+// Per call, the merge engine -> the automaton: 1,024 rows of 1 KB 29.4 -> 11.7 us, 16,384 of them 236.5 ->
+// 29.2 us, 100,000 reads of 100 - 300 bp (int64 rows) 349 -> 57 us, 4,096 ragged reads of 12 Mbp 253.5 ->
+// 83.9 us (all with the vocabulary of 4,096), 32 rows of 100 kbp (32,000) 143.8 -> 74.3 us.
 #pragma once
 
 namespace dnatok {
@@ -36,30 +42,47 @@ struct AutoArgs {
     const void *next;            // narrow: uint16 [4 * (n_states + 1)], entry = 4 * state; wide: uint32, entry = 4 * state << 8 | length
     const uint8_t *len;          // [n_states + 1] (narrow)
     const uint16_t *sym;         // [n_states + 1 + 256] token of a state; behind the states: symbol of a byte
-    const int32_t *id;           // the same through the table's out_remap (null: no remap)
+    const int32_t *id;           // the same through the table's out_remap
     uint32_t other;              // the state behind a byte that is no letter; its successors are the row start's
     uint32_t letters;            // the letters by code (bits 1 and 2 of the byte)
     int32_t lanes, rows;         // lanes per row, rows per wave (lanes * rows <= 64)
-    int32_t n_groups;            // (whole rows, none listed) n_rows / rows, rounded up; -1: items from the work list, a wave each
+    int32_t n_groups;            // whole rows: n_rows / rows, rounded up (chunks: the work list says)
+    int32_t window;              // tokens a wave has room for on their way out
     int64_t total;               // bytes of the batch
 };
 
-constexpr int kAutoWaves = 8;
-constexpr uint32_t kAutoNoToken = 0xFFFFu;
-constexpr uint32_t kAutoNarrowStates = 10400;    // the most the narrow form has LDS for, beside eight waves with regions of 32 bytes
+// Waves of a workgroup, which has a CU to itself: as many as the LDS holds, at most sixteen (four per SIMD).
+constexpr int kAutoMaxWaves = 16;
+constexpr uint32_t kAutoNarrowStates = 10400;    // the most the narrow form has LDS for, beside the waves' share
+constexpr size_t kAutoLdsBytes = 163840 - 1152;  // what a workgroup may take: the CU's, less the static arrays (1,088 bytes)
 
 typedef uint32_t auto_u32_a1 __attribute__((aligned(1), may_alias));
 typedef uint32_t auto_u32x4_a1 __attribute__((ext_vector_type(4), aligned(1), may_alias));
+typedef int32_t auto_i32x4 __attribute__((ext_vector_type(4)));
 
 template <bool WIDE, int P>
 struct AutoLds {
     typedef typename std::conditional<WIDE, uint32_t, uint16_t>::type Entry;
-    static constexpr size_t wave_bytes = 2 * 64 * P * sizeof(Entry);       // states, and tokens on their way out
+    static constexpr size_t state_bytes = 64 * P * sizeof(Entry);
+    static constexpr int least_window = 16 * P;                            // a token per four bytes
     static size_t table_bytes(uint32_t n_states)
     {
         return WIDE ? 0 : ((((size_t)n_states + 1) * 8 + 15) & ~(size_t)15) + ((((size_t)n_states + 1) + 15) & ~(size_t)15);
     }
-    static size_t bytes(uint32_t n_states) { return table_bytes(n_states) + kAutoWaves * wave_bytes; }
+    static int waves(uint32_t n_states)
+    {
+        const size_t w = (kAutoLdsBytes - table_bytes(n_states)) / (state_bytes + least_window * sizeof(Entry));
+        return w > (size_t)kAutoMaxWaves ? kAutoMaxWaves : (int)w;
+    }
+    static int window(uint32_t n_states)
+    {
+        const size_t w = ((kAutoLdsBytes - table_bytes(n_states)) / waves(n_states) - state_bytes) / sizeof(Entry) & ~(size_t)7;
+        return w > (size_t)(64 * P) ? 64 * P : (int)w;
+    }
+    static size_t bytes(uint32_t n_states)
+    {
+        return table_bytes(n_states) + waves(n_states) * (state_bytes + window(n_states) * sizeof(Entry));
+    }
 };
 
 // Between two phases of a wave's work on its LDS: what a lane wrote before is what the others read after.
@@ -89,64 +112,63 @@ __device__ __forceinline__ uint32_t letter_codes16(const auto_u32x4_a1 w, uint32
     return codes;
 }
 
-// Cells [0, stride) of `rows` neighbouring rows of the padded output, whose tokens lie in `staged`
-// (row r's from r * cap on).  ELEM: bytes of an id.
-template <int ELEM, typename Entry>
-__device__ __forceinline__ void auto_put_rows(const Entry *staged, int cap, const int32_t *counts, int rows, int64_t row0,
-                                              int64_t stride, bool pad_left, int32_t pad_id, const uint16_t *sym, const int32_t *id,
-                                              const int32_t *remap2, void *ids, uint8_t *mask, int lane)
+// One id, in the padded output's own integer width.
+__device__ __forceinline__ void auto_put(void *ids, int elem, int64_t at, int32_t v)
 {
-    typedef typename std::conditional<ELEM == 8, int64_t, typename std::conditional<ELEM == 4, int32_t,
-            typename std::conditional<ELEM == 2, int16_t, uint8_t>::type>::type>::type Out;
-    Out *const out0 = reinterpret_cast<Out *>(ids);
-    // four cells to a lane where the rows start on such a boundary
-    const bool four = (stride & 3) == 0 && ((uintptr_t)ids & (4 * ELEM < 16 ? 4 * ELEM - 1 : 15)) == 0 &&
-                      ((uintptr_t)mask & 3) == 0;
-    auto cell = [&](int c, int shift, int kept, const Entry *st) -> int32_t {
-        const int t = c - shift;
-        if (t < 0 || t >= kept) return pad_id;
-        const uint32_t v = st[t];
-        int32_t x = id ? id[v] : (int32_t)sym[v];
-        if (remap2) x = remap2[x];
-        return x;
-    };
-    for (int r = 0; r < rows; ++r) {
-        const int n = counts[r];
-        if (n < 0) continue;                               // (behind the batch's last row)
-        const int kept = n < stride ? n : (int)stride;
-        const int shift = pad_left ? (int)stride - kept : 0;
-        const Entry *const st = staged + r * cap;
-        Out *const out = out0 + (row0 + r) * stride;
-        uint8_t *const mk = mask ? mask + (row0 + r) * stride : nullptr;
-        if (four) {
-            for (int c = 4 * lane; c < (int)stride; c += 256) {
-                int32_t v[4];
-                uint32_t live = 0;
+    if (elem == 4) reinterpret_cast<int32_t *>(ids)[at] = v;
+    else if (elem == 8) reinterpret_cast<int64_t *>(ids)[at] = (int64_t)v;
+    else if (elem == 2) reinterpret_cast<int16_t *>(ids)[at] = (int16_t)v;
+    else reinterpret_cast<uint8_t *>(ids)[at] = (uint8_t)v;
+}
+
+// The rows [row0, row0 + rows) of the padded output, whose tokens lie in `staged`: row r's n_tok tokens
+// from `base` on, both known to lane r * G.  The rows are taken as one run of cells, four to a lane
+// (they start on such a boundary).
+template <int ELEM, typename Entry>
+__device__ __forceinline__ void auto_put_rows(const BpeArgs &a, const int32_t *id, const Entry *staged, int base, int n_tok,
+                                              int G, int rows, int64_t row0, int lane)
+{
+    const int stride = (int)a.pad_stride, quads = stride >> 2;
+    const int64_t n_steps = ((int64_t)rows * quads + 63) >> 6;
+    int r = 0, c = lane;
+    for (int64_t step = 0; step < n_steps; ++step, c += 64) {
+        while (c >= quads && r < rows) { c -= quads; ++r; }
+        const int from = (r < rows ? r : 0) * G;
+        const int n = __shfl(n_tok, from), b = __shfl(base, from);
+        if (r < rows) {
+            const int kept = n < stride ? n : stride;
+            const int shift = a.pad_left ? stride - kept : 0;
+            const Entry *const st = staged + b;
+            int32_t v[4];
+            uint32_t live = 0;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    v[q] = cell(c + q, shift, kept, st);
-                    live |= (c + q >= shift && c + q < shift + kept ? 1u : 0u) << (8 * q);
-                }
-                if (ELEM == 4) {
-                    *reinterpret_cast<int4 *>(out + c) = int4{v[0], v[1], v[2], v[3]};
-                } else if (ELEM == 8) {
-                    longlong2 *const o = reinterpret_cast<longlong2 *>(out + c);
-                    o[0] = longlong2{v[0], v[1]};
-                    o[1] = longlong2{v[2], v[3]};
-                } else if (ELEM == 2) {
-                    *reinterpret_cast<uint2 *>(out + c) = uint2{((uint32_t)v[0] & 0xFFFFu) | ((uint32_t)v[1] << 16),
-                                                               ((uint32_t)v[2] & 0xFFFFu) | ((uint32_t)v[3] << 16)};
-                } else {
-                    *reinterpret_cast<uint32_t *>(out + c) = ((uint32_t)v[0] & 0xFFu) | (((uint32_t)v[1] & 0xFFu) << 8) |
-                                                             (((uint32_t)v[2] & 0xFFu) << 16) | ((uint32_t)v[3] << 24);
-                }
-                if (mk) *reinterpret_cast<uint32_t *>(mk + c) = live;
+            for (int q = 0; q < 4; ++q) {
+                const int t = 4 * c + q - shift;
+                const bool token = t >= 0 && t < kept;
+                v[q] = a.pad_id;
+                if (token) v[q] = id[st[t]];
+                live |= (token ? 1u : 0u) << (8 * q);
             }
-        } else {
-            for (int c = lane; c < (int)stride; c += 64) {
-                out[c] = (Out)cell(c, shift, kept, st);
-                if (mk) mk[c] = c >= shift && c < shift + kept ? 1 : 0;
+            if (a.pad_remap) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (live >> (8 * q) & 1u) v[q] = a.pad_remap[v[q]];
             }
+            const int64_t at = (row0 + r) * stride + 4 * c;
+            if (ELEM == 4) {
+                *reinterpret_cast<auto_i32x4 *>(reinterpret_cast<int32_t *>(a.pad_ids) + at) = auto_i32x4{v[0], v[1], v[2], v[3]};
+            } else if (ELEM == 8) {
+                auto_i32x4 *const o = reinterpret_cast<auto_i32x4 *>(reinterpret_cast<int64_t *>(a.pad_ids) + at);
+                o[0] = auto_i32x4{v[0], v[0] >> 31, v[1], v[1] >> 31};
+                o[1] = auto_i32x4{v[2], v[2] >> 31, v[3], v[3] >> 31};
+            } else if (ELEM == 2) {
+                *reinterpret_cast<uint2 *>(reinterpret_cast<int16_t *>(a.pad_ids) + at) =
+                    uint2{((uint32_t)v[0] & 0xFFFFu) | ((uint32_t)v[1] << 16), ((uint32_t)v[2] & 0xFFFFu) | ((uint32_t)v[3] << 16)};
+            } else {
+                *reinterpret_cast<uint32_t *>(reinterpret_cast<uint8_t *>(a.pad_ids) + at) =
+                    ((uint32_t)v[0] & 0xFFu) | (((uint32_t)v[1] & 0xFFu) << 8) | (((uint32_t)v[2] & 0xFFu) << 16) | ((uint32_t)v[3] << 24);
+            }
+            if (a.pad_mask) *reinterpret_cast<uint32_t *>(a.pad_mask + at) = live;
         }
     }
 }
@@ -155,37 +177,38 @@ __device__ __forceinline__ void auto_put_rows(const Entry *staged, int cap, cons
 // list (chunks of long rows, then the rows that are one item), a wave each.  CHARS: with the
 // single-character ids.
 template <bool WIDE, int P, bool CHUNKS, bool CHARS, bool PADDED>
-__global__ __launch_bounds__(64 * kAutoWaves) void bpe_auto_kernel(
+__global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
     BpeArgs a, AutoArgs t, const uint8_t *__restrict__ bytes, const int64_t *__restrict__ offsets,
     BpePlan p, int32_t n_rows, int32_t *__restrict__ tok_tmp, int32_t *__restrict__ lengths)
 {
     typedef typename AutoLds<WIDE, P>::Entry Entry;
     static_assert(P == 16 || P == 32, "a region's token starts are the bits of one word");
+    static_assert(!CHUNKS || P == 32, "a chunk of 2,048 bytes is a wave");
     extern __shared__ __align__(16) uint8_t smem[];
-    __shared__ int32_t s_count[kAutoWaves][64];
-    __shared__ int32_t s_longest[kAutoWaves];
+    __shared__ int32_t s_longest[PADDED ? kAutoMaxWaves : 1];
     __shared__ int32_t s_lut[CHARS ? 256 : 1];
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int n_waves = (int)blockDim.x >> 6;
     const uint32_t n_entries = 4 * (t.other + 1);
-    size_t table_bytes = 0;
+    uint32_t table_bytes = 0;
     if (!WIDE) {
         // the transition table and the token lengths, 16 bytes per thread and step
         const uint32_t tab16 = (n_entries * 2 + 15) / 16, len16 = (t.other + 1 + 15) / 16;
         const uint4 *const src = reinterpret_cast<const uint4 *>(t.next);
         uint4 *const dst = reinterpret_cast<uint4 *>(smem);
-        for (uint32_t i = threadIdx.x; i < tab16; i += 64 * kAutoWaves) dst[i] = src[i];
+        for (uint32_t i = threadIdx.x; i < tab16; i += blockDim.x) dst[i] = src[i];
         const uint4 *const src_len = reinterpret_cast<const uint4 *>(t.len);
-        for (uint32_t i = threadIdx.x; i < len16; i += 64 * kAutoWaves) dst[tab16 + i] = src_len[i];
-        table_bytes = 16 * ((size_t)tab16 + len16);
+        for (uint32_t i = threadIdx.x; i < len16; i += blockDim.x) dst[tab16 + i] = src_len[i];
+        table_bytes = 16 * (tab16 + len16);
     }
     if (CHARS)
-        for (int i = threadIdx.x; i < 256; i += 64 * kAutoWaves) s_lut[i] = a.char_lut[i];
+        for (int i = threadIdx.x; i < 256; i += blockDim.x) s_lut[i] = a.char_lut[i];
     const uint16_t *const table = reinterpret_cast<const uint16_t *>(smem);
     const uint8_t *const len_of = smem + (size_t)((n_entries * 2 + 15) / 16) * 16;
     const uint32_t *const far_table = reinterpret_cast<const uint32_t *>(t.next);
-    Entry *const state = reinterpret_cast<Entry *>(smem + table_bytes + (size_t)wv * AutoLds<WIDE, P>::wave_bytes);   // [P][64]
-    Entry *const staged = state + 64 * P;
+    Entry *const state = reinterpret_cast<Entry *>(smem + table_bytes) + (size_t)wv * (64 * P + t.window);   // [P][64]
+    Entry *const staged = state + 64 * P;                                                                    // [t.window]
     const Entry other = WIDE ? (Entry)((t.other * 4) << 8 | 1u) : (Entry)(t.other * 4);
     __syncthreads();
 
@@ -209,7 +232,7 @@ __global__ __launch_bounds__(64 * kAutoWaves) void bpe_auto_kernel(
     const int32_t n_single0 = CHUNKS ? p.counts[4] : 0, n_single1 = CHUNKS ? p.counts[5] : 0;
     int32_t longest = 0;
     // (neighbouring items go to different CUs, so that a small batch spreads over the chip)
-    for (int64_t item64 = (int64_t)wv * gridDim.x + blockIdx.x; item64 < n_items; item64 += (int64_t)gridDim.x * kAutoWaves) {
+    for (int64_t item64 = (int64_t)wv * gridDim.x + blockIdx.x; item64 < n_items; item64 += (int64_t)gridDim.x * n_waves) {
         const int32_t item = (int32_t)item64;
         int32_t row = 0, k = 0, nc = 1;
         bool have = true;
@@ -248,7 +271,7 @@ __global__ __launch_bounds__(64 * kAutoWaves) void bpe_auto_kernel(
 
         // the region's bytes as codes; cnt: how many of its P positions the row has
         const int cnt = n - s < 0 ? 0 : (n - s < P ? n - s : P);
-        uint32_t codes[P / 16], foreign[P / 16];
+        uint32_t codes[P / 16], flags = 0;
 #pragma unroll
         for (int q = 0; q < P / 16; ++q) {
             auto_u32x4_a1 w = {0, 0, 0, 0};
@@ -265,12 +288,11 @@ __global__ __launch_bounds__(64 * kAutoWaves) void bpe_auto_kernel(
                         w[i] = (uint32_t)b[4 * i] | ((uint32_t)b[4 * i + 1] << 8) | ((uint32_t)b[4 * i + 2] << 16) | ((uint32_t)b[4 * i + 3] << 24);
                 }
             }
-            codes[q] = letter_codes16(w, t.letters, foreign[q]);
-            const int here = cnt - 16 * q;                           // (the flags of positions the row does not have are dropped)
-            foreign[q] &= here >= 16 ? 0xFFFFu : (here <= 0 ? 0u : (1u << here) - 1u);
+            uint32_t foreign;
+            codes[q] = letter_codes16(w, t.letters, foreign);
+            flags |= foreign << (16 * q);
         }
-        uint32_t flags = foreign[0];
-        if (P == 32) flags |= foreign[P / 16 - 1] << 16;
+        flags &= cnt >= 32 ? ~0u : (1u << cnt) - 1u;                 // (of the positions the row has)
         const bool any_foreign = __ballot(flags != 0) != 0;
 
         // forward over the own region
@@ -289,31 +311,38 @@ __global__ __launch_bounds__(64 * kAutoWaves) void bpe_auto_kernel(
                 state[i * 64 + lane] = e;
             }
         }
-        // and on into the regions to the right until the states are the same
+        // and on into the regions to the right until the states are the same, four bytes at a time: once
+        // equal they stay equal, so the last of the four tells, and writing equal ones again does no
+        // harm (nor does a state behind the row's end, which nothing reads)
         bool going = cnt == P;
         for (int ahead = 1;; ++ahead) {
             const int from = (lane + ahead) & 63;
-            uint32_t c2[P / 16], f2 = 0;
-#pragma unroll
-            for (int q = 0; q < P / 16; ++q) c2[q] = (uint32_t)__shfl((int)codes[q], from);
+            uint32_t word = 0, next_word = 0, f2 = 0;
+            word = (uint32_t)__shfl((int)codes[0], from);
+            if (P == 32) next_word = (uint32_t)__shfl((int)codes[P / 16 - 1], from);
             if (any_foreign) f2 = (uint32_t)__shfl((int)flags, from);
             const int cnt2 = __shfl(cnt, from);
-            int limit = going && j + ahead < G ? cnt2 : 0;
-            going = limit > 0;
+            going = going && j + ahead < G && cnt2 > 0;
             if (!__ballot(going)) break;
             wave_phase();
-            for (int i = 0; i < P; ++i) {
-                if (i < limit) {
-                    const uint32_t word = (P == 32 && i >= 16) ? c2[P / 16 - 1] : c2[0];
-                    e = step(e, (word >> (2 * (i & 15))) & 3u);
-                    if (any_foreign && (f2 >> i & 1u)) e = other;
+            for (int i = 0; i < P; i += 4) {
+                if (going) {
                     Entry *const at = state + i * 64 + lane + ahead;
-                    if (*at == e) { going = false; limit = 0; } else { *at = e; }
+                    const Entry there = at[3 * 64];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        e = step(e, (word >> (2 * q)) & 3u);
+                        if (any_foreign && (f2 >> q & 1u)) e = other;
+                        at[q * 64] = e;
+                    }
+                    going = e != there;
                 }
-                if ((i & 3) == 3 && !__ballot(i + 1 < limit)) break;
+                if (!__ballot(going)) break;
+                word >>= 8;
+                f2 >>= 4;
+                if (P == 32 && i == 12) word = next_word;
             }
         }
-
         wave_phase();
 
         // backward: token starts of the region as bits, first from the region's own end
@@ -377,42 +406,35 @@ __global__ __launch_bounds__(64 * kAutoWaves) void bpe_auto_kernel(
             if (!__ballot(moved)) break;
         }
 
-        // every token's number within its row
+        // every token's number among the wave's
         const uint32_t mine = (uint32_t)__builtin_popcount(starts);
         const uint32_t inc = wave_inclusive_sum_u32(mine);
         const uint32_t before_row = (uint32_t)__shfl((int)inc, lane0 > 0 ? lane0 - 1 : 0);
         const uint32_t base = lane0 > 0 ? before_row : 0u;
         const uint32_t row_last = (uint32_t)__shfl((int)inc, lane0 + G - 1 < 64 ? lane0 + G - 1 : 63);
         const uint32_t n_tok = row_last - base;
-
-        // tokens on their way out: state numbers (behind the states: the byte, where it is no letter)
         const bool chunk = CHUNKS && nc > 1;
-        if (chunk) {
-            // by the position they start at
-            uint4 *const clear = reinterpret_cast<uint4 *>(staged);
-#pragma unroll
-            for (int i = 0; i < (int)(64 * P * sizeof(Entry) / 16 / 64); ++i) clear[i * 64 + lane] = uint4{~0u, ~0u, ~0u, ~0u};
-            wave_phase();
-        }
-        {
+
+        // the region's tokens, last one first: f(number of the token's state -- behind the states: the byte,
+        // where it is no letter --, position of its first byte in the region)
+        auto each_token = [&](auto f) {
             uint32_t left = starts;
             int end = right_end;
-            int at = r * cap + (int)(inc - base);
             while (left) {
                 const int b = 31 - __builtin_clz(left);
                 left ^= 1u << b;
-                const Entry st = state_at(end - 1);
-                uint32_t v = number_of(st);
+                uint32_t v = number_of(state_at(end - 1));
                 if (any_foreign && v == t.other) v = t.other + 1 + src[end - 1];
                 end = s + b;
-                if (chunk) staged[end] = (Entry)v;
-                else staged[--at] = (Entry)v;
+                f(v, b);
             }
-        }
-        wave_phase();
+        };
 
         if (chunk) {
-            // the symbol at every start, kNone elsewhere, and how many start where no neighbour reaches
+            // The state's number (wide: the symbol) at every start, kNone elsewhere, and how many start
+            // where no neighbour reaches.  A token's number goes to the place of its first byte, whose state
+            // no token needs (it is inside one, unless the token is that byte alone).
+            each_token([&](uint32_t v, int b) { state[b * 64 + lane] = (Entry)v; });
             int64_t mid_lo = k > 0 ? (int64_t)k * p.core + p.overlap : 0;
             if (mid_lo > len) mid_lo = len;
             const int64_t mid_hi = k + 1 < nc ? (int64_t)(k + 1) * p.core - p.overlap : len;
@@ -422,46 +444,71 @@ __global__ __launch_bounds__(64 * kAutoWaves) void bpe_auto_kernel(
             if (hi < 32) in_mid &= hi <= 0 ? 0u : ~0u >> (32 - hi);
             const uint32_t live = wave_inclusive_sum_u32((uint32_t)__builtin_popcount(in_mid));
             if (lane == 63) p.cnt[4 * (size_t)item] = (int32_t)live;
-            uint16_t *const raw = p.chunk_sym + (size_t)item * p.ext;
-            for (int i = lane * 2; i < n; i += 128) {
-                const uint32_t v0 = staged[i], v1 = staged[i + 1];
-                const uint32_t y0 = (Entry)v0 == (Entry)~(Entry)0 ? kAutoNoToken : (uint32_t)t.sym[v0];
-                const uint32_t y1 = (Entry)v1 == (Entry)~(Entry)0 ? kAutoNoToken : (uint32_t)t.sym[v1];
-                if (i + 1 < n) {
-                    if ((p.ext & 1) == 0) {
-                        *reinterpret_cast<uint32_t *>(raw + i) = y0 | (y1 << 16);
-                    } else {
-                        raw[i] = (uint16_t)y0;
-                        raw[i + 1] = (uint16_t)y1;
+            uint16_t *const raw = p.chunk_sym + (size_t)item * p.ext + s;
+#pragma unroll
+            for (int i = 0; i < P; i += 8) {
+                uint32_t y[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    y[q] = kNone;
+                    if (starts >> (i + q) & 1u) {
+                        const uint32_t v = state[(i + q) * 64 + lane];
+                        y[q] = WIDE ? (uint32_t)t.sym[v] : v;
                     }
-                } else {
-                    raw[i] = (uint16_t)y0;
                 }
+                if (i < cnt)                               // (a slot is whole vectors: what lies behind the chunk's end is kNone)
+                    *reinterpret_cast<uint4 *>(raw + i) = uint4{y[0] | y[1] << 16, y[2] | y[3] << 16, y[4] | y[5] << 16, y[6] | y[7] << 16};
             }
         } else {
             if (j == 0 && have) {
-                const int32_t count = too_long ? -1 : (int32_t)n_tok;
-                lengths[row] = count;
-                longest = count > longest ? count : longest;
+                lengths[row] = too_long ? -1 : (int32_t)n_tok;
+                longest = (int32_t)n_tok > longest ? (int32_t)n_tok : longest;
+            }
+            // through LDS, where the wave's tokens fit its window (a token per four bytes always does)
+            const bool fits = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63) <= (uint32_t)t.window;
+            if (fits) {
+                uint32_t at = inc;
+                each_token([&](uint32_t v, int) { staged[--at] = (Entry)v; });
+                wave_phase();
             }
             if (PADDED) {
-                if (j == 0 && r < R) s_count[wv][r] = have ? (int32_t)n_tok : -1;
-                wave_phase();
                 const int64_t row0 = (int64_t)item * R;
-                if (a.pad_elem == 4)
-                    auto_put_rows<4>(staged, cap, s_count[wv], R, row0, a.pad_stride, a.pad_left, a.pad_id, t.sym, t.id, a.pad_remap, a.pad_ids, a.pad_mask, lane);
-                else if (a.pad_elem == 8)
-                    auto_put_rows<8>(staged, cap, s_count[wv], R, row0, a.pad_stride, a.pad_left, a.pad_id, t.sym, t.id, a.pad_remap, a.pad_ids, a.pad_mask, lane);
-                else if (a.pad_elem == 2)
-                    auto_put_rows<2>(staged, cap, s_count[wv], R, row0, a.pad_stride, a.pad_left, a.pad_id, t.sym, t.id, a.pad_remap, a.pad_ids, a.pad_mask, lane);
-                else
-                    auto_put_rows<1>(staged, cap, s_count[wv], R, row0, a.pad_stride, a.pad_left, a.pad_id, t.sym, t.id, a.pad_remap, a.pad_ids, a.pad_mask, lane);
+                const int rows = n_rows - row0 < R ? (int)(n_rows - row0) : R;
+                const int elem = a.pad_elem;
+                if (fits && (a.pad_stride & 3) == 0 && ((uintptr_t)a.pad_ids & (elem >= 4 ? 15 : 4 * elem - 1)) == 0 &&
+                    ((uintptr_t)a.pad_mask & 3) == 0) {
+                    if (elem == 4) auto_put_rows<4>(a, t.id, staged, (int)base, (int)n_tok, G, rows, row0, lane);
+                    else if (elem == 8) auto_put_rows<8>(a, t.id, staged, (int)base, (int)n_tok, G, rows, row0, lane);
+                    else if (elem == 2) auto_put_rows<2>(a, t.id, staged, (int)base, (int)n_tok, G, rows, row0, lane);
+                    else auto_put_rows<1>(a, t.id, staged, (int)base, (int)n_tok, G, rows, row0, lane);
+                } else {
+                    // cell by cell: the lanes their own tokens, the row's lanes its padding and mask
+                    const int64_t stride = a.pad_stride, at0 = (int64_t)row * stride;
+                    const int kept = (int64_t)n_tok < stride ? (int)n_tok : (int)stride;
+                    const int64_t shift = a.pad_left ? stride - kept : 0;
+                    int at = (int)(inc - base);
+                    each_token([&](uint32_t v, int) {
+                        --at;
+                        if (at < kept) {
+                            const int32_t x = t.id[v];
+                            auto_put(a.pad_ids, elem, at0 + shift + at, a.pad_remap ? a.pad_remap[x] : x);
+                        }
+                    });
+                    if (have) {
+                        for (int64_t c = j; c < stride; c += G) {
+                            const bool token = c >= shift && c < shift + kept;
+                            if (!token) auto_put(a.pad_ids, elem, at0 + c, a.pad_id);
+                            if (a.pad_mask) a.pad_mask[at0 + c] = token ? 1 : 0;
+                        }
+                    }
+                }
             } else {
-                // the row's own lanes write its run
                 int32_t *const out = tok_tmp + start;
-                for (uint32_t c = j; c < n_tok && have; c += G) {
-                    const uint32_t v = staged[r * cap + c];
-                    out[c] = t.id ? t.id[v] : (int32_t)t.sym[v];
+                if (fits) {                                // the row's own lanes write its run
+                    for (uint32_t c = j; c < n_tok; c += G) out[c] = t.id[staged[base + c]];
+                } else {
+                    uint32_t at = inc - base;
+                    each_token([&](uint32_t v, int) { out[--at] = t.id[v]; });
                 }
             }
         }
@@ -477,9 +524,8 @@ __global__ __launch_bounds__(64 * kAutoWaves) void bpe_auto_kernel(
             for (int64_t g = (g0 & ~(int64_t)3) + 4 * j; g < g1; g += 4 * G) {
                 if (quads && g >= g0 && g + 4 <= g1) {
                     const uint32_t w = *reinterpret_cast<const auto_u32_a1 *>(bytes + g);
-                    typedef int32_t ivec4 __attribute__((ext_vector_type(4)));
-                    const ivec4 v = {s_lut[w & 255u], s_lut[w >> 8 & 255u], s_lut[w >> 16 & 255u], s_lut[w >> 24]};
-                    __builtin_nontemporal_store(v, reinterpret_cast<ivec4 *>(a.char_ids + g));
+                    const auto_i32x4 v = {s_lut[w & 255u], s_lut[w >> 8 & 255u], s_lut[w >> 16 & 255u], s_lut[w >> 24]};
+                    __builtin_nontemporal_store(v, reinterpret_cast<auto_i32x4 *>(a.char_ids + g));
                     if (a.char_mask) __builtin_nontemporal_store(0x01010101u, reinterpret_cast<uint32_t *>(a.char_mask + g));
                 } else {
                     for (int q = 0; q < 4; ++q)
@@ -498,8 +544,7 @@ __global__ __launch_bounds__(64 * kAutoWaves) void bpe_auto_kernel(
         __syncthreads();
         if (threadIdx.x == 0) {
             int32_t all = 0;
-#pragma unroll
-            for (int q = 0; q < kAutoWaves; ++q) all = s_longest[q] > all ? s_longest[q] : all;
+            for (int q = 0; q < n_waves; ++q) all = s_longest[q] > all ? s_longest[q] : all;
             publish_max(a.max_tree, (unsigned)all, a.longest);
         }
     }

@@ -2187,7 +2187,7 @@ extern "C" int dnatok_bpe_table_create(const int32_t *byte_to_id_h, const int32_
     const size_t o_alen = up(o_anext + auto_n * 4 * (wide ? 4 : 2));
     const size_t o_asym = up(o_alen + auto_n);
     const size_t o_aid = up(o_asym + (auto_n ? auto_n + 256 : 0) * 2);
-    const size_t total = up(o_aid + (auto_n && out_remap_h ? auto_n + 256 : 0) * 4) + 256;
+    const size_t total = up(o_aid + (auto_n ? auto_n + 256 : 0) * 4) + 256;
     std::vector<uint8_t> host(total, 0);             // (the trees start as zeros)
     memcpy(&host[o_tab], tab.data(), (size_t)slots * sizeof(uint4));
     memcpy(&host[o_b2s], b2s.data(), 512);
@@ -2207,8 +2207,8 @@ extern "C" int dnatok_bpe_table_create(const int32_t *byte_to_id_h, const int32_
             if (wide) reinterpret_cast<uint32_t *>(&host[o_anext])[i] = (to * 4) << 8 | fa.len[to];
             else reinterpret_cast<uint16_t *>(&host[o_anext])[i] = (uint16_t)(to * 4);
         }
-        if (out_remap_h)
-            for (size_t i = 0; i < auto_n + 256; ++i) reinterpret_cast<int32_t *>(&host[o_aid])[i] = out_remap_h[sym[i]];
+        for (size_t i = 0; i < auto_n + 256; ++i)
+            reinterpret_cast<int32_t *>(&host[o_aid])[i] = out_remap_h ? out_remap_h[sym[i]] : (int32_t)sym[i];
     }
     void *blob = nullptr;
     hipError_t e = hipMalloc(&blob, total);
@@ -2233,7 +2233,7 @@ extern "C" int dnatok_bpe_table_create(const int32_t *byte_to_id_h, const int32_
     t->auto_next = b + o_anext;
     t->auto_len = b + o_alen;
     t->auto_sym = (uint16_t *)(b + o_asym);
-    t->auto_id = out_remap_h ? (int32_t *)(b + o_aid) : nullptr;
+    t->auto_id = (int32_t *)(b + o_aid);
     *out = t;
     return DNATOK_OK;
 }
@@ -2402,23 +2402,22 @@ template <bool WIDE, int P, bool CHUNKS, bool CHARS, bool PADDED>
 int launch_auto_as(const dnatok_bpe_t *t, const BpeArgs &a, AutoArgs aa, const uint8_t *bytes, const int64_t *offsets,
                    const BpePlan &p, int64_t n_rows, int64_t items, int32_t *tok_tmp, int32_t *lengths, hipStream_t s)
 {
-    const size_t lds = AutoLds<WIDE, P>::bytes(t->auto_states);
+    typedef AutoLds<WIDE, P> Lds;
     auto kern = bpe_auto_kernel<WIDE, P, CHUNKS, CHARS, PADDED>;
     // (once per kernel form; two threads that both find it unset both set it, to the same value)
     static std::atomic<bool> attr_set{false};
     if (!attr_set.load(std::memory_order_acquire)) {
         DNATOK_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)(WIDE ? lds : AutoLds<WIDE, P>::bytes(kAutoNarrowStates))));
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)kAutoLdsBytes));
         attr_set.store(true, std::memory_order_release);
     }
-    // (narrow: the workgroups of the largest table, which are those of any)
-    static const int64_t resident =
-        resident_workgroups(kern, 64 * kAutoWaves, AutoLds<WIDE, P>::bytes(WIDE ? 0 : kAutoNarrowStates), 1);
+    const int waves = Lds::waves(t->auto_states);
+    aa.window = Lds::window(t->auto_states);
+    static const int64_t resident = resident_workgroups(kern, 64 * kAutoMaxWaves, kAutoLdsBytes, 1);
     int64_t grid = items < resident ? items : resident;
     if (a.max_tree && grid > kTreeRows) grid = kTreeRows;
     if (grid < 1) grid = 1;
-    kern<<<(int)grid, 64 * kAutoWaves, lds, s>>>(a, aa, bytes, offsets, p, (int32_t)n_rows, tok_tmp, lengths);
+    kern<<<(int)grid, 64 * waves, Lds::bytes(t->auto_states), s>>>(a, aa, bytes, offsets, p, (int32_t)n_rows, tok_tmp, lengths);
     DNATOK_HIP_TRY(hipGetLastError());
     return DNATOK_OK;
 }
@@ -2428,7 +2427,7 @@ template <bool WIDE>
 int run_auto(const dnatok_bpe_t *t, const BpeArgs &a, int chunking, const uint8_t *bytes, const int64_t *offsets,
              const BpePlan &p, int64_t n_rows, int64_t max_len, int64_t total, int32_t *tok_tmp, int32_t *lengths, hipStream_t s)
 {
-    AutoArgs aa{t->auto_next, t->auto_len, t->auto_sym, t->auto_id, t->auto_states, t->auto_letters, 64, 1, -1, total};
+    AutoArgs aa{t->auto_next, t->auto_len, t->auto_sym, t->auto_id, t->auto_states, t->auto_letters, 64, 1, 0, 0, total};
     if (chunking & 1) {
         const int rc = launch_plan(chunking, offsets, p, n_rows, s);
         if (rc) return rc;
@@ -2439,7 +2438,7 @@ int run_auto(const dnatok_bpe_t *t, const BpeArgs &a, int chunking, const uint8_
     // (a lane's walk is then half as long, and twice the lanes share it).
     const int64_t len = max_len < 1 ? 1 : max_len;
     const int64_t lanes16 = (len + 15) / 16;
-    const bool small = len <= 1024 && (n_rows + 64 / lanes16 - 1) / (64 / lanes16) <= 256 * kAutoWaves;
+    const bool small = len <= 1024 && (n_rows + 64 / lanes16 - 1) / (64 / lanes16) <= 256 * kAutoMaxWaves;
     aa.lanes = (int32_t)(small ? lanes16 : (len + 31) / 32);
     aa.rows = 64 / aa.lanes;
     const int64_t groups = (n_rows + aa.rows - 1) / aa.rows;
@@ -2552,7 +2551,7 @@ static int bpe_encode_launch(const dnatok_bpe_t *t, const uint8_t *bytes, const 
     const bool split = work_len > 512 && n_rows >= 1024 && total / n_rows <= 384 && p.ext / 4 <= 512;
     // The automaton takes what it can: every row of at most 2,048 bytes, and chunks of the shipped sizes.
     // (The switches of the tests and measurements select the merge engine, whose they are.)
-    const bool automaton = t->auto_states != 0 && a.placement == 0 && p.ext <= 2048 && (p.ext & 1) == 0 && (!long_rows || chunking) &&
+    const bool automaton = t->auto_states != 0 && a.placement == 0 && p.ext <= 2048 && p.ext % 8 == 0 && (!long_rows || chunking) &&
                            t->chunk_core.load(std::memory_order_relaxed) == 0;
     int32_t *const longest_after = split && a.max_tree && !automaton ? a.longest : nullptr;
     if (split && !automaton) {
@@ -2574,6 +2573,9 @@ static int bpe_encode_launch(const dnatok_bpe_t *t, const uint8_t *bytes, const 
     if (rc) return rc;
     if (long_rows) {
         if (chunking) {
+            // (the narrow automaton hands back the numbers of states instead of symbols)
+            BpeArgs ga = a;
+            if (automaton && !t->auto_wide) ga.out_remap = t->auto_id;
             int64_t g = p.max_mc < 4096 ? p.max_mc : 4096;
             if (2 * p.overlap <= kSeamMaskSpan) {                          // a wave per seam, the search on ballots
                 int64_t gs = (p.max_mc + 3) / 4;
@@ -2588,11 +2590,11 @@ static int bpe_encode_launch(const dnatok_bpe_t *t, const uint8_t *bytes, const 
             if (p.max_mc >= kSeamWaveFrom) {
                 int64_t gs = (p.max_mc + 3) / 4;
                 if (p.ext <= kGatherExt && p.ext % 8 == 0)
-                    bpe_gather_wave_kernel<<<(int)(gs > 4096 ? 4096 : gs), 256, 0, s>>>(a, offsets, p, tok_tmp, lengths);
+                    bpe_gather_wave_kernel<<<(int)(gs > 4096 ? 4096 : gs), 256, 0, s>>>(ga, offsets, p, tok_tmp, lengths);
                 else
-                    bpe_gather_kernel<64><<<(int)(gs > 4096 ? 4096 : gs), 256, 0, s>>>(a, offsets, p, tok_tmp, lengths);
+                    bpe_gather_kernel<64><<<(int)(gs > 4096 ? 4096 : gs), 256, 0, s>>>(ga, offsets, p, tok_tmp, lengths);
             } else {
-                bpe_gather_kernel<256><<<(int)(g < 1 ? 1 : g), 256, 0, s>>>(a, offsets, p, tok_tmp, lengths);
+                bpe_gather_kernel<256><<<(int)(g < 1 ? 1 : g), 256, 0, s>>>(ga, offsets, p, tok_tmp, lengths);
             }
             DNATOK_HIP_TRY(hipGetLastError());
         }
