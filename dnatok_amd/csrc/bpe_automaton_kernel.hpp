@@ -23,7 +23,9 @@
 // transition table has to be near.  Narrow form: 16-bit transitions and the token lengths in LDS,
 // staged once per workgroup, one workgroup of up to sixteen waves per CU (8,972 states: 81 KB, and 5 KB
 // per wave for states and tokens).  Wide form: 32-bit entries {state, token length} in global memory
-// (L2: 164,729 states are 2.6 MB), the waves' share of LDS alone.
+// (L2: 164,729 states are 2.6 MB).  (With the transitions of the first 4,992 states, where every second
+// step is, in LDS as well, the walk over the own region went from 10.7 to 7.8 us, staging them took the 3 us
+// back, and the walk into the next region, a few lanes inside tandem repeats, stayed at 16 us.)
 //
 // Every phase is a chain of dependent reads, so what a launch takes is the number of waves in flight.
 // Sixteen share the table instead of eight since a wave's tokens leave through a window of one per four
@@ -48,6 +50,8 @@ struct AutoArgs {
     int32_t lanes, rows;         // lanes per row, rows per wave (lanes * rows <= 64)
     int32_t n_groups;            // whole rows: n_rows / rows, rounded up (chunks: the work list says)
     int32_t window;              // tokens a wave has room for on their way out
+    int32_t list_here;           // (chunks) the kernel makes the work list itself: at most kAutoListRows rows
+    int32_t *zero;               // (chunks) a word to be cleared for the kernels behind this one, or null
     int64_t total;               // bytes of the batch
 };
 
@@ -84,6 +88,11 @@ struct AutoLds {
         return table_bytes(n_states) + waves(n_states) * (state_bytes + window(n_states) * sizeof(Entry));
     }
 };
+
+// Up to this many rows a wave finds its item among the rows itself (their lengths are one load per 64
+// rows, beside each other) instead of in a list that a launch in front has made: 5 us per call, as long
+// as anything that a batch of a few rows waits for.
+constexpr int kAutoListRows = 256;
 
 // Between two phases of a wave's work on its LDS: what a lane wrote before is what the others read after.
 __device__ __forceinline__ void wave_phase()
@@ -227,16 +236,74 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
     const int s = j * P;                                   // first byte of the region
     const int lane0 = lane - j;                            // the row's first lane
     const int cap = G * P;
-    const int32_t n_items = CHUNKS ? p.counts[0] : t.n_groups;
-    const int32_t n_mc = CHUNKS ? p.counts[1] : 0;
-    const int32_t n_single0 = CHUNKS ? p.counts[4] : 0, n_single1 = CHUNKS ? p.counts[5] : 0;
+    // (list_here) chunk slots and single rows up to and including row 64 q + lane
+    constexpr int kListWords = CHUNKS ? kAutoListRows / 64 : 1;
+    int32_t slots_to[kListWords], singles_to[kListWords];
+    int32_t n_items = t.n_groups, n_mc = 0, n_single0 = 0, n_single1 = 0;
+    if (CHUNKS && t.list_here) {
+        int64_t from[kListWords], to[kListWords];
+#pragma unroll
+        for (int q = 0; q < kListWords; ++q) {
+            const int row = 64 * q + lane;
+            from[q] = to[q] = 0;
+            if (row < n_rows) { from[q] = offsets[row]; to[q] = offsets[row + 1]; }
+        }
+        int32_t n_singles = 0;
+#pragma unroll
+        for (int q = 0; q < kListWords; ++q) {
+            const int64_t len = to[q] - from[q];
+            const bool here = 64 * q + lane < n_rows, cut = here && len > p.ext;
+            const uint32_t inc = wave_inclusive_sum_u32(cut ? (uint32_t)((len + p.core - 1) / p.core) : 0u);
+            const uint64_t single = __ballot(here && !cut);
+            slots_to[q] = n_mc + (int32_t)inc;
+            singles_to[q] = n_singles + (int32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(single >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)single, 0u)) +
+                            (int32_t)(single >> lane & 1u);
+            n_mc = __builtin_amdgcn_readlane(slots_to[q], 63);
+            n_singles += (int32_t)__builtin_popcountll(single);
+        }
+        n_items = n_mc + n_singles;
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            p.counts[0] = n_items;
+            p.counts[1] = n_mc;
+            p.counts[2] = 0;
+            p.counts[3] = 0;
+        }
+    } else if (CHUNKS) {
+        n_items = p.counts[0];
+        n_mc = p.counts[1];
+        n_single0 = p.counts[4];
+        n_single1 = p.counts[5];
+    }
+    if (CHUNKS && t.zero && blockIdx.x == 0 && threadIdx.x == 0) *t.zero = 0;
     int32_t longest = 0;
     // (neighbouring items go to different CUs, so that a small batch spreads over the chip)
     for (int64_t item64 = (int64_t)wv * gridDim.x + blockIdx.x; item64 < n_items; item64 += (int64_t)gridDim.x * n_waves) {
         const int32_t item = (int32_t)item64;
         int32_t row = 0, k = 0, nc = 1;
         bool have = true;
-        if (CHUNKS) {
+        if (CHUNKS && t.list_here) {
+            // the first row whose slots (or single rows) reach beyond the item
+            const bool cut = item < n_mc;
+            const int32_t want = cut ? item : item - n_mc;
+            int32_t before = 0, upto = 0;
+            row = -1;
+#pragma unroll
+            for (int q = 0; q < kListWords; ++q) {
+                const int32_t mine = cut ? slots_to[q] : singles_to[q];
+                const uint64_t beyond = __ballot(mine > want);
+                if (row < 0 && beyond) {
+                    const int at = __builtin_ctzll(beyond);
+                    row = 64 * q + at;
+                    upto = __builtin_amdgcn_readlane(mine, at);
+                    if (at > 0) before = __builtin_amdgcn_readlane(mine, at - 1);
+                }
+                if (row < 0) before = __builtin_amdgcn_readlane(mine, 63);
+            }
+            if (cut) {
+                k = item - before;
+                nc = upto - before;
+            }
+        } else if (CHUNKS) {
             if (item < n_mc) {
                 const int4 rc = p.rec[item];
                 row = rc.x; k = rc.y; nc = rc.z;
@@ -260,6 +327,10 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
         const int64_t start = offsets[row];
         const int64_t len = offsets[row + 1] - start;
         int64_t e0 = 0, e1 = len;
+        if (CHUNKS && t.list_here && nc > 1 && lane == 0) {
+            p.rec[item] = make_int4(row, k, nc, (int)len);
+            if (k == 0) p.row_fail[row] = 0;
+        }
         if (CHUNKS && nc > 1) {
             e0 = (int64_t)k * p.core - p.overlap < 0 ? 0 : (int64_t)k * p.core - p.overlap;
             e1 = (int64_t)(k + 1) * p.core + p.overlap;
@@ -416,17 +487,38 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
         const bool chunk = CHUNKS && nc > 1;
 
         // the region's tokens, last one first: f(number of the token's state -- behind the states: the byte,
-        // where it is no letter --, position of its first byte in the region)
+        // where it is no letter --, position of its first byte in the region).  Four at a time: their
+        // states are read together.
         auto each_token = [&](auto f) {
             uint32_t left = starts;
             int end = right_end;
             while (left) {
-                const int b = 31 - __builtin_clz(left);
-                left ^= 1u << b;
-                uint32_t v = number_of(state_at(end - 1));
-                if (any_foreign && v == t.other) v = t.other + 1 + src[end - 1];
-                end = s + b;
-                f(v, b);
+                int b[4], last[4];
+                bool is[4];
+                uint32_t v[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    is[q] = left != 0;
+                    b[q] = is[q] ? 31 - __builtin_clz(left) : 0;
+                    last[q] = is[q] ? end - 1 : s;
+                    left &= ~(1u << b[q]);
+                    end = s + b[q];
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q) v[q] = number_of(state_at(last[q]));
+                if (any_foreign) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        if (is[q] && v[q] == t.other) v[q] = t.other + 1 + src[last[q]];
+                }
+                if (WIDE && chunk) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        if (is[q]) v[q] = t.sym[v[q]];
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (is[q]) f(v[q], b[q]);
             }
         };
 
@@ -453,7 +545,7 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
                     y[q] = kNone;
                     if (starts >> (i + q) & 1u) {
                         const uint32_t v = state[(i + q) * 64 + lane];
-                        y[q] = WIDE ? (uint32_t)t.sym[v] : v;
+                        y[q] = v;
                     }
                 }
                 if (i < cnt)                               // (a slot is whole vectors: what lies behind the chunk's end is kNone)
@@ -472,8 +564,8 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
                 wave_phase();
             }
             if (PADDED) {
-                const int64_t row0 = (int64_t)item * R;
-                const int rows = n_rows - row0 < R ? (int)(n_rows - row0) : R;
+                const int64_t row0 = CHUNKS ? (int64_t)row : (int64_t)item * R;
+                const int rows = CHUNKS ? 1 : (n_rows - row0 < R ? (int)(n_rows - row0) : R);
                 const int elem = a.pad_elem;
                 if (fits && (a.pad_stride & 3) == 0 && ((uintptr_t)a.pad_ids & (elem >= 4 ? 15 : 4 * elem - 1)) == 0 &&
                     ((uintptr_t)a.pad_mask & 3) == 0) {
@@ -538,7 +630,7 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
         }
         wave_phase();                                      // the wave's part of LDS is rewritten by its next item
     }
-    if (PADDED && a.max_tree) {
+    if (PADDED && !CHUNKS && a.max_tree) {
         const uint32_t m = wave_max_u32((uint32_t)longest);
         if (lane == 0) s_longest[wv] = (int32_t)m;
         __syncthreads();
@@ -547,6 +639,157 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
             for (int q = 0; q < n_waves; ++q) all = s_longest[q] > all ? s_longest[q] : all;
             publish_max(a.max_tree, (unsigned)all, a.longest);
         }
+    }
+}
+
+// The rows behind the seam kernel: the chunks' tokens put together, a wave per chunk (the chunk is held as in
+// bpe_gather_wave_kernel), and the rows that have no seam redone whole.  The two are independent, so they
+// share a launch: the first n_slabs workgroups take the rows to be redone (nearly always none), the others
+// the chunks.  PADDED: a row goes straight to its cells of a.pad_ids, its padding shared out among its
+// chunks; then this launch stands for three (gather, whole rows, padding: 32 rows of 100 kbp, 6.5 + 4.5 +
+// 5.3 us).  count_longest: *a.longest (cleared by the kernel in front) becomes the longest row.
+template <bool PADDED>
+__global__ __launch_bounds__(1024) void bpe_auto_join_kernel(
+    BpeArgs a, const int32_t *__restrict__ id, const uint8_t *__restrict__ bytes, const int64_t *__restrict__ offsets, int64_t n_rows,
+    int64_t max_len, BpePlan p, int count_longest, int32_t *__restrict__ tok_tmp, int32_t *__restrict__ lengths)
+{
+    __shared__ __align__(16) uint16_t compact_s[16][kGatherExt];
+    const int lane = threadIdx.x & 63;
+    if ((int)blockIdx.x < p.n_slabs) {
+        if (PADDED && count_longest && blockIdx.x == 0 && threadIdx.x < 64) {      // the rows that were no chunks
+            int32_t most = 0;
+            for (int64_t row = lane; row < n_rows; row += 64)
+                if (offsets[row + 1] - offsets[row] <= p.ext && lengths[row] > most) most = lengths[row];
+            const uint32_t m = wave_max_u32((uint32_t)most);
+            if (lane == 0) atomicMax(a.longest, (int32_t)m);
+        }
+        if (p.counts[3] == 0) return;
+        uint8_t *const lds = reinterpret_cast<uint8_t *>(compact_s);
+        uint32_t *const red = reinterpret_cast<uint32_t *>(lds);
+        uint16_t *const b2s = reinterpret_cast<uint16_t *>(lds + 512);
+        uint8_t *const D = lds + 1024;
+        for (int i = threadIdx.x; i < 256; i += 1024) b2s[i] = a.byte_to_sym[i];
+        __syncthreads();
+        uint8_t *const slab = p.slabs + (size_t)blockIdx.x * p.slab_bytes;
+        const PairTable pt{a.tab, a.shift, a.mul1, a.mul2};
+        for (int64_t row = blockIdx.x; row < n_rows; row += p.n_slabs) {
+            const int64_t start = offsets[row];
+            const int64_t len = offsets[row + 1] - start;
+            if (len <= p.ext || !p.row_fail[row]) continue;
+            if (len > max_len) {                           // longer than the caller declared: no room in the slab
+                if (threadIdx.x == 0) lengths[row] = -1;
+            } else {
+                const size_t n = ((size_t)len + 7) & ~(size_t)7;
+                PosRec<uint32_t> *const P = reinterpret_cast<PosRec<uint32_t> *>(slab);
+                uint32_t *const PG = reinterpret_cast<uint32_t *>(P + n);
+                uint32_t *const Q = PG + n;
+                uint32_t *const C = Q + n / 2;
+                bpe_row<1024, uint32_t, 0>(pt, b2s, a.out_remap, bytes + start, (int)len, P, PG, Q, C, D, red, threadIdx.x,
+                                           tok_tmp + start, lengths + row);
+            }
+            __syncthreads();
+            if (PADDED) {
+                // the row's own workgroup has just written its run and its length
+                const int32_t n_tok = __hip_atomic_load(lengths + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const int64_t stride = a.pad_stride, at0 = row * stride;
+                const int64_t kept = n_tok < 0 ? 0 : (n_tok < stride ? n_tok : stride), shift = a.pad_left ? stride - kept : 0;
+                for (int64_t c = threadIdx.x; c < stride; c += 1024) {
+                    const bool token = c >= shift && c < shift + kept;
+                    int32_t v = a.pad_id;
+                    if (token) {
+                        v = __hip_atomic_load(tok_tmp + start + (c - shift), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        if (a.pad_remap) v = a.pad_remap[v];
+                    }
+                    auto_put(a.pad_ids, a.pad_elem, at0 + c, v);
+                    if (a.pad_mask) a.pad_mask[at0 + c] = token ? 1 : 0;
+                }
+                if (count_longest && threadIdx.x == 0) atomicMax(a.longest, n_tok);
+                __syncthreads();
+            }
+        }
+        return;
+    }
+    const int wv = threadIdx.x >> 6;
+    uint16_t *const compact = compact_s[wv];
+    const int32_t n_mc = p.counts[1];
+    const int64_t n_waves = ((int64_t)gridDim.x - p.n_slabs) * 16;
+    for (int64_t m64 = (int64_t)wv * (gridDim.x - p.n_slabs) + (blockIdx.x - p.n_slabs); m64 < n_mc; m64 += n_waves) {
+        const int32_t m = (int32_t)m64;
+        // first trip: the chunk's symbols and its record
+        const uint4 *const src = reinterpret_cast<const uint4 *>(p.chunk_sym + (size_t)m * p.ext);
+        uint4 g[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            g[q] = lane * 32 + q * 8 < p.ext ? src[lane * 4 + q] : uint4{~0u, ~0u, ~0u, ~0u};
+        const int4 rc = p.rec[m];
+        const int32_t row = rc.x, k = rc.y, nc = rc.z;
+        const int64_t len = rc.w;
+        const int64_t e0 = (int64_t)k * p.core - p.overlap < 0 ? 0 : (int64_t)k * p.core - p.overlap;
+        // second trip: the seams, the row's state and place, the chunks' counts
+        const int32_t seam_l = k > 0 ? p.seam[m - 1] : 0;
+        const int32_t seam_r = k + 1 < nc ? p.seam[m] : 0;
+        const int32_t failed = p.row_fail[row];
+        const int64_t row_at = offsets[row];
+        uint32_t before = 0, behind = 0;
+        for (int32_t j = lane; j < (PADDED ? nc : k); j += 64) {
+            const int4 part = *reinterpret_cast<const int4 *>(p.cnt + 4 * (size_t)(m - k + j));   // {unshared, after left seam, before right seam, -}
+            const uint32_t c = (uint32_t)(part.x + (j > 0 ? part.y : 0) + (j + 1 < nc ? part.z : 0));
+            if (j < k) before += c; else behind += c;
+        }
+        if (failed) continue;                              // (the same for the whole wave)
+        const uint32_t base = (uint32_t)__builtin_amdgcn_readlane((int)wave_inclusive_sum_u32(before), 63);
+        const int64_t lo = k > 0 ? (int64_t)seam_l : 0, hi = k + 1 < nc ? (int64_t)seam_r : len;
+        // which of the lane's positions lie in [lo, hi) and start a token
+        const int64_t p0 = e0 + lane * 32;
+        uint32_t in_span = ~0u;
+        if (lo > p0) in_span = lo - p0 >= 32 ? 0u : (~0u << (uint32_t)(lo - p0));
+        if (hi < p0 + 32) in_span &= hi <= p0 ? 0u : (~0u >> (uint32_t)(p0 + 32 - hi));
+        const uint32_t w[16] = {g[0].x, g[0].y, g[0].z, g[0].w, g[1].x, g[1].y, g[1].z, g[1].w,
+                                g[2].x, g[2].y, g[2].z, g[2].w, g[3].x, g[3].y, g[3].z, g[3].w};
+        uint32_t live = 0;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            live |= ((w[q] & 0xFFFFu) != kNone ? 1u : 0u) << (2 * q);
+            live |= ((w[q] >> 16) != kNone ? 1u : 0u) << (2 * q + 1);
+        }
+        live &= in_span;
+        const uint32_t mine = (uint32_t)__builtin_popcount(live);
+        const uint32_t inc = wave_inclusive_sum_u32(mine);
+        const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
+        uint32_t at = inc - mine;
+#pragma unroll
+        for (int q = 0; q < 32; ++q) {
+            if (live >> q & 1u) compact[at++] = (uint16_t)(q & 1 ? w[q >> 1] >> 16 : w[q >> 1] & 0xFFFFu);
+        }
+        wave_phase();
+        if (!PADDED) {
+            int32_t *const out = tok_tmp + row_at + base;
+#pragma unroll 4
+            for (uint32_t t = lane; t < total; t += 64) out[t] = id ? id[compact[t]] : (int32_t)compact[t];
+            if (lane == 0 && k + 1 == nc) lengths[row] = (int32_t)(base + total);
+        } else {
+            const uint32_t n_tok = base + (uint32_t)__builtin_amdgcn_readlane((int)wave_inclusive_sum_u32(behind), 63);
+            const int64_t stride = a.pad_stride, at0 = (int64_t)row * stride;
+            const int64_t kept = (int64_t)n_tok < stride ? (int64_t)n_tok : stride, shift = a.pad_left ? stride - kept : 0;
+            const int64_t put = kept - (int64_t)base < (int64_t)total ? kept - (int64_t)base : (int64_t)total;
+            for (int64_t t = lane; t < put; t += 64) {
+                int32_t v = id ? id[compact[t]] : (int32_t)compact[t];
+                if (a.pad_remap) v = a.pad_remap[v];
+                auto_put(a.pad_ids, a.pad_elem, at0 + shift + base + t, v);
+                if (a.pad_mask) a.pad_mask[at0 + shift + base + t] = 1;
+            }
+            // the chunk's share of the padding
+            const int64_t pads = stride - kept, pad0 = a.pad_left ? 0 : kept;
+            for (int64_t c = pads * k / nc + lane; c < pads * (k + 1) / nc; c += 64) {
+                auto_put(a.pad_ids, a.pad_elem, at0 + pad0 + c, a.pad_id);
+                if (a.pad_mask) a.pad_mask[at0 + pad0 + c] = 0;
+            }
+            if (lane == 0 && k + 1 == nc) {
+                lengths[row] = (int32_t)n_tok;
+                if (count_longest) atomicMax(a.longest, (int32_t)n_tok);
+            }
+        }
+        wave_phase();                                      // the wave's part of LDS is rewritten by its next chunk
     }
 }
 

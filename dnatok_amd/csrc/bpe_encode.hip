@@ -116,7 +116,8 @@ struct BpeArgs {
     // shortest rows, 2 that class alone (a batch of mostly short rows with a few long ones is split
     // between a launch with 256-thread teams and one with teams of one wave)
     int32_t part;
-    // host side only: where the merge table is kept (dnatok_bpe_table_set_placement)
+    // host side only: whether the automaton encodes a padded batch (decided once per call); where the merge table is kept (dnatok_bpe_table_set_placement)
+    int32_t by_automaton;
     int32_t placement;
 };
 
@@ -2427,10 +2428,17 @@ template <bool WIDE>
 int run_auto(const dnatok_bpe_t *t, const BpeArgs &a, int chunking, const uint8_t *bytes, const int64_t *offsets,
              const BpePlan &p, int64_t n_rows, int64_t max_len, int64_t total, int32_t *tok_tmp, int32_t *lengths, hipStream_t s)
 {
-    AutoArgs aa{t->auto_next, t->auto_len, t->auto_sym, t->auto_id, t->auto_states, t->auto_letters, 64, 1, 0, 0, total};
+    AutoArgs aa{t->auto_next, t->auto_len, t->auto_sym, t->auto_id, t->auto_states, t->auto_letters, 64, 1, 0, 0, 0, nullptr, total};
     if (chunking & 1) {
-        const int rc = launch_plan(chunking, offsets, p, n_rows, s);
-        if (rc) return rc;
+        aa.list_here = n_rows <= kAutoListRows ? 1 : 0;
+        if (!aa.list_here) {
+            const int rc = launch_plan(chunking, offsets, p, n_rows, s);
+            if (rc) return rc;
+        }
+        if (a.pad_ids) {
+            aa.zero = a.longest;                     // (see the join kernel)
+            return launch_auto_as<WIDE, 32, true, false, true>(t, a, aa, bytes, offsets, p, n_rows, p.max_items, tok_tmp, lengths, s);
+        }
         if (a.char_ids) return launch_auto_as<WIDE, 32, true, true, false>(t, a, aa, bytes, offsets, p, n_rows, p.max_items, tok_tmp, lengths, s);
         return launch_auto_as<WIDE, 32, true, false, false>(t, a, aa, bytes, offsets, p, n_rows, p.max_items, tok_tmp, lengths, s);
     }
@@ -2516,6 +2524,14 @@ int run_lds(bool long_rows, int chunking, bool split, const BpeArgs &a_in, const
 
 }  // namespace
 
+// The automaton takes what it can: every row of at most 2,048 bytes, and chunks of the shipped sizes.
+// (The switches of the tests and measurements select the merge engine, whose they are.)
+static bool auto_takes(const dnatok_bpe_t *t, const BpePlan &p)
+{
+    return t->auto_states != 0 && t->placement.load(std::memory_order_relaxed) == 0 &&
+           t->chunk_core.load(std::memory_order_relaxed) == 0 && p.ext <= 2048 && p.ext % 8 == 0;
+}
+
 // The launches of one encode call; p lies inside a scratch buffer that holds p.total_bytes.
 static int bpe_encode_launch(const dnatok_bpe_t *t, const uint8_t *bytes, const int64_t *offsets, int64_t n_rows,
                              int64_t max_len, int64_t total, const BpePlan &p, int32_t *tok_tmp, int32_t *lengths, hipStream_t s,
@@ -2525,6 +2541,7 @@ static int bpe_encode_launch(const dnatok_bpe_t *t, const uint8_t *bytes, const 
     BpeArgs a{t->tab, t->byte_to_sym, t->out_remap, t->shift, t->mul1, t->mul2, t->n_merges, t->ltab, t->lmul1, t->lmul2,
               t->first, char_lut, char_ids, char_mask};
     a.placement = t->placement.load(std::memory_order_relaxed);
+    const bool automaton = padded ? padded->by_automaton != 0 : auto_takes(t, p);
     if (padded) {
         a.pad_ids = padded->pad_ids; a.pad_mask = padded->pad_mask; a.pad_remap = padded->pad_remap;
         a.pad_elem = padded->pad_elem; a.pad_left = padded->pad_left;
@@ -2549,10 +2566,7 @@ static int bpe_encode_launch(const dnatok_bpe_t *t, const uint8_t *bytes, const 
     // get a launch of their own.  The two launches cannot both carry the longest row up the one
     // tree: it is taken from the lengths afterwards.
     const bool split = work_len > 512 && n_rows >= 1024 && total / n_rows <= 384 && p.ext / 4 <= 512;
-    // The automaton takes what it can: every row of at most 2,048 bytes, and chunks of the shipped sizes.
-    // (The switches of the tests and measurements select the merge engine, whose they are.)
-    const bool automaton = t->auto_states != 0 && a.placement == 0 && p.ext <= 2048 && p.ext % 8 == 0 && (!long_rows || chunking) &&
-                           t->chunk_core.load(std::memory_order_relaxed) == 0;
+    // (a table that has an automaton is monotone: its long rows are cut into chunks)
     int32_t *const longest_after = split && a.max_tree && !automaton ? a.longest : nullptr;
     if (split && !automaton) {
         a.in_order = 0;
@@ -2573,9 +2587,6 @@ static int bpe_encode_launch(const dnatok_bpe_t *t, const uint8_t *bytes, const 
     if (rc) return rc;
     if (long_rows) {
         if (chunking) {
-            // (the narrow automaton hands back the numbers of states instead of symbols)
-            BpeArgs ga = a;
-            if (automaton && !t->auto_wide) ga.out_remap = t->auto_id;
             int64_t g = p.max_mc < 4096 ? p.max_mc : 4096;
             if (2 * p.overlap <= kSeamMaskSpan) {                          // a wave per seam, the search on ballots
                 int64_t gs = (p.max_mc + 3) / 4;
@@ -2587,14 +2598,31 @@ static int bpe_encode_launch(const dnatok_bpe_t *t, const uint8_t *bytes, const 
                 bpe_seam_kernel<256><<<(int)(g < 1 ? 1 : g), 256, 0, s>>>(offsets, p);
             }
             DNATOK_HIP_TRY(hipGetLastError());
+            if (automaton) {
+                // (narrow: the chunks' tokens are the numbers of states instead of symbols)
+                const int32_t *const id = t->auto_wide ? a.out_remap : t->auto_id;
+                const int64_t chunk_groups = p.max_mc < 448 ? p.max_mc : 448;
+                const int grid = (int)(p.n_slabs + chunk_groups);
+                const int count_longest = a.pad_ids && a.longest && n_rows <= kAutoListRows ? 1 : 0;
+                if (a.pad_ids)
+                    bpe_auto_join_kernel<true><<<grid, 1024, 0, s>>>(a, id, bytes, offsets, n_rows, max_len, p, count_longest, tok_tmp, lengths);
+                else
+                    bpe_auto_join_kernel<false><<<grid, 1024, 0, s>>>(a, id, bytes, offsets, n_rows, max_len, p, 0, tok_tmp, lengths);
+                DNATOK_HIP_TRY(hipGetLastError());
+                if (a.pad_ids && a.longest && !count_longest) {
+                    bpe_longest_kernel<<<1, 1024, 0, s>>>(lengths, n_rows, a.longest);
+                    DNATOK_HIP_TRY(hipGetLastError());
+                }
+                return DNATOK_OK;
+            }
             if (p.max_mc >= kSeamWaveFrom) {
                 int64_t gs = (p.max_mc + 3) / 4;
                 if (p.ext <= kGatherExt && p.ext % 8 == 0)
-                    bpe_gather_wave_kernel<<<(int)(gs > 4096 ? 4096 : gs), 256, 0, s>>>(ga, offsets, p, tok_tmp, lengths);
+                    bpe_gather_wave_kernel<<<(int)(gs > 4096 ? 4096 : gs), 256, 0, s>>>(a, offsets, p, tok_tmp, lengths);
                 else
-                    bpe_gather_kernel<64><<<(int)(gs > 4096 ? 4096 : gs), 256, 0, s>>>(ga, offsets, p, tok_tmp, lengths);
+                    bpe_gather_kernel<64><<<(int)(gs > 4096 ? 4096 : gs), 256, 0, s>>>(a, offsets, p, tok_tmp, lengths);
             } else {
-                bpe_gather_kernel<256><<<(int)(g < 1 ? 1 : g), 256, 0, s>>>(ga, offsets, p, tok_tmp, lengths);
+                bpe_gather_kernel<256><<<(int)(g < 1 ? 1 : g), 256, 0, s>>>(a, offsets, p, tok_tmp, lengths);
             }
             DNATOK_HIP_TRY(hipGetLastError());
         }
@@ -2694,10 +2722,13 @@ extern "C" int dnatok_bpe_encode_padded_as(const dnatok_bpe_t *t, const uint8_t 
                    "%s: scratch holds %zu bytes, %zu needed", who, scratch_bytes, need.total_bytes);
     DNATOK_REQUIRE(((uintptr_t)scratch & 255) == 0, DNATOK_E_INVALID, "%s: scratch must be 256-byte aligned", who);
     const BpePlan p = make_plan(t, (uint8_t *)scratch, n_rows, max_len, total);
-    if (max_len > p.ext) {
-        // rows cut into chunks (or left to the whole-row kernel) are assembled in tok_tmp first
+    const bool long_rows = max_len > p.ext;
+    if (long_rows)
         DNATOK_REQUIRE(tok_tmp, DNATOK_E_INVALID,
                        "%s: a batch with a row of more than %d bytes needs tok_tmp (int32[total])", who, p.ext);
+    const bool automaton = auto_takes(t, p);
+    if (long_rows && !automaton) {
+        // rows cut into chunks (or left to the whole-row kernel) are assembled in tok_tmp first
         const int rc = bpe_encode_launch(t, bytes, offsets, n_rows, max_len, total, p, tok_tmp, lengths, s);
         if (rc) return rc;
         if (longest) {
@@ -2711,17 +2742,18 @@ extern "C" int dnatok_bpe_encode_padded_as(const dnatok_bpe_t *t, const uint8_t 
     pad.pad_ids = ids; pad.pad_mask = mask; pad.pad_remap = remap; pad.pad_stride = stride; pad.pad_id = pad_id;
     pad.pad_elem = id_bytes; pad.pad_left = pad_left ? 1 : 0;
     pad.longest = longest;
-    if (longest) {
+    pad.by_automaton = automaton ? 1 : 0;
+    if (longest && !long_rows) {
         std::lock_guard<std::mutex> hold(t->slot_lock);
         auto it = t->slot_of_stream.find(stream);
         if (it == t->slot_of_stream.end() && (int)t->slot_of_stream.size() < kMaxTreeSlots)
             it = t->slot_of_stream.emplace(stream, (int)t->slot_of_stream.size()).first;
         if (it != t->slot_of_stream.end()) pad.max_tree = t->max_trees + (size_t)it->second * kTreeWords;
     }
-    const int rc = bpe_encode_launch(t, bytes, offsets, n_rows, max_len, total, p, nullptr, lengths, s, nullptr, nullptr,
-                                     nullptr, &pad);
+    const int rc = bpe_encode_launch(t, bytes, offsets, n_rows, max_len, total, p, long_rows ? tok_tmp : nullptr, lengths, s,
+                                     nullptr, nullptr, nullptr, &pad);
     if (rc) return rc;
-    if (longest && !pad.max_tree) {
+    if (longest && !pad.max_tree && !long_rows) {
         bpe_longest_kernel<<<1, 1024, 0, s>>>(lengths, n_rows, longest);
         DNATOK_HIP_TRY(hipGetLastError());
     }

@@ -1143,6 +1143,36 @@ def test_bpe_automaton_at_the_edges_of_regions(bpe, longest, count):
         enc.set_chunk_geometry(0, 0)
 
 
+@pytest.mark.parametrize("count", [1, 64, 65, 256, 257])
+@pytest.mark.parametrize("pad_left,dtype", [(False, torch.int32), (True, torch.int64), (False, torch.int16)])
+def test_bpe_long_rows_padded_by_their_chunks(bpe, count, pad_left, dtype):
+    """Batches with rows that are cut into chunks, padded where the chunks are put together, with the
+    work list made by the kernel itself (up to 256 rows) and by a launch in front: rows of one chunk
+    more than whole, empty rows, rows without a seam (a tandem repeat longer than any shared stretch),
+    a stride that cuts rows off, and one that is no multiple of four."""
+    which, enc, bo = bpe
+    say(f"bpe{which} padded chunks, {count} rows, left {pad_left}, {dtype}")
+    rng = random.Random(count)
+    rnd = lambda n: "".join(rng.choices("ACGTN", weights=[24, 24, 24, 24, 1], k=n))
+    lens = [0, 1, 100, 2047, 2048, 2049, 3000, 5000]
+    seqs = [rnd(rng.choice(lens)) for _ in range(count)]
+    seqs[0] = rnd(6000)
+    if count > 2:
+        seqs[1] = rnd(300) + "AACCG" * 900 + rnd(300)
+        seqs[2] = "ACGTTG" * 700
+    b = util.batch_from_strings(seqs)
+    data, off = to_dev(b)
+    ref = bo.encode_batch(b.data, b.offsets)
+    for stride in (1600, 301):
+        ids, mask, lengths, longest = enc.encode_padded(data, off, int(b.lengths().max()), stride, 3, pad_left=pad_left, dtype=dtype)
+        torch.cuda.synchronize()
+        eids, emask = O.pad_rows(ref, 3, stride, pad_left=pad_left, dtype=np.int64)
+        np.testing.assert_array_equal(lengths.cpu().numpy(), [r.size for r in ref])
+        assert int(longest.item()) == max(r.size for r in ref)
+        np.testing.assert_array_equal(ids.cpu().numpy().astype(np.int64), eids)
+        np.testing.assert_array_equal(mask.cpu().numpy(), emask)
+
+
 @pytest.mark.parametrize("long_ones", ["up to 1 KB", "up to 2 KB", "cut into chunks"])
 def test_bpe_mostly_short_rows_with_some_long_ones(bpe, long_ones):
     """A batch of mostly short rows with a few long ones among them is split between two launches (the
