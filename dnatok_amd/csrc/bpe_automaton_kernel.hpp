@@ -47,8 +47,8 @@ struct AutoArgs {
     const int32_t *id;           // the same through the table's out_remap
     uint32_t other;              // the state behind a byte that is no letter; its successors are the row start's
     uint32_t letters;            // the letters by code (bits 1 and 2 of the byte)
-    int32_t lanes, rows;         // lanes per row, rows per wave (lanes * rows <= 64)
-    int32_t n_groups;            // whole rows: n_rows / rows, rounded up (chunks: the work list says)
+    int32_t rows;                // (whole rows) rows of an item, at most 64
+    int32_t n_groups;            // (whole rows) n_rows / rows, rounded up (chunks: the work list says)
     int32_t window;              // tokens a wave has room for on their way out
     int32_t list_here;           // (chunks) the kernel makes the work list itself: at most kAutoListRows rows
     int32_t *zero;               // (chunks) a word to be cleared for the kernels behind this one, or null
@@ -130,20 +130,21 @@ __device__ __forceinline__ void auto_put(void *ids, int elem, int64_t at, int32_
     else reinterpret_cast<uint8_t *>(ids)[at] = (uint8_t)v;
 }
 
-// The rows [row0, row0 + rows) of the padded output, whose tokens lie in `staged`: row r's n_tok tokens
-// from `base` on, both known to lane r * G.  The rows are taken as one run of cells, four to a lane
-// (they start on such a boundary).
+// `rows` rows of the padded output, whose tokens lie in `staged`: lane first + r knows the number of the
+// r-th of them, and that its n_tok tokens lie from `base` on.  The rows are taken as one run of cells,
+// four to a lane (they start on such a boundary).
 template <int ELEM, typename Entry>
 __device__ __forceinline__ void auto_put_rows(const BpeArgs &a, const int32_t *id, const Entry *staged, int base, int n_tok,
-                                              int G, int rows, int64_t row0, int lane)
+                                              int first, int rows, int32_t row_id, int lane)
 {
     const int stride = (int)a.pad_stride, quads = stride >> 2;
     const int64_t n_steps = ((int64_t)rows * quads + 63) >> 6;
     int r = 0, c = lane;
     for (int64_t step = 0; step < n_steps; ++step, c += 64) {
         while (c >= quads && r < rows) { c -= quads; ++r; }
-        const int from = (r < rows ? r : 0) * G;
+        const int from = first + (r < rows ? r : 0);
         const int n = __shfl(n_tok, from), b = __shfl(base, from);
+        const int64_t row = __shfl(row_id, from);
         if (r < rows) {
             const int kept = n < stride ? n : stride;
             const int shift = a.pad_left ? stride - kept : 0;
@@ -163,7 +164,7 @@ __device__ __forceinline__ void auto_put_rows(const BpeArgs &a, const int32_t *i
                 for (int q = 0; q < 4; ++q)
                     if (live >> (8 * q) & 1u) v[q] = a.pad_remap[v[q]];
             }
-            const int64_t at = (row0 + r) * stride + 4 * c;
+            const int64_t at = row * stride + 4 * c;
             if (ELEM == 4) {
                 *reinterpret_cast<auto_i32x4 *>(reinterpret_cast<int32_t *>(a.pad_ids) + at) = auto_i32x4{v[0], v[1], v[2], v[3]};
             } else if (ELEM == 8) {
@@ -231,15 +232,11 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
     };
     auto number_of = [&](Entry e) -> uint32_t { return WIDE ? (uint32_t)e >> 10 : (uint32_t)e >> 2; };
 
-    const int G = t.lanes, R = t.rows;
-    const int r = lane / G, j = lane - r * G;              // the lane's row within the wave, and its region within the row
-    const int s = j * P;                                   // first byte of the region
-    const int lane0 = lane - j;                            // the row's first lane
-    const int cap = G * P;
+    constexpr int kRowMax = 64 * P;                        // the longest row that a wave takes
     // (list_here) chunk slots and single rows up to and including row 64 q + lane
     constexpr int kListWords = CHUNKS ? kAutoListRows / 64 : 1;
     int32_t slots_to[kListWords], singles_to[kListWords];
-    int32_t n_items = t.n_groups, n_mc = 0, n_single0 = 0, n_single1 = 0;
+    int32_t n_items = t.n_groups, n_mc = 0, n_single0 = 0, n_single1 = 0, n_single2 = 0;
     if (CHUNKS && t.list_here) {
         int64_t from[kListWords], to[kListWords];
 #pragma unroll
@@ -269,10 +266,11 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
             p.counts[3] = 0;
         }
     } else if (CHUNKS) {
-        n_items = p.counts[0];
         n_mc = p.counts[1];
         n_single0 = p.counts[4];
         n_single1 = p.counts[5];
+        n_single2 = p.counts[6];
+        n_items = n_mc + n_single0 + (n_single1 + 1) / 2 + (n_single2 + 3) / 4;
     }
     if (CHUNKS && t.zero && blockIdx.x == 0 && threadIdx.x == 0) *t.zero = 0;
     int32_t longest = 0;
@@ -280,7 +278,10 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
     for (int64_t item64 = (int64_t)wv * gridDim.x + blockIdx.x; item64 < n_items; item64 += (int64_t)gridDim.x * n_waves) {
         const int32_t item = (int32_t)item64;
         int32_t row = 0, k = 0, nc = 1;
-        bool have = true;
+        const int64_t item_row0 = (int64_t)item * t.rows;
+        int item_rows = CHUNKS ? 1 : (int)(n_rows - item_row0 < t.rows ? n_rows - item_row0 : t.rows);
+        const int32_t *list = nullptr;
+        int32_t list_at = 0;
         if (CHUNKS && t.list_here) {
             // the first row whose slots (or single rows) reach beyond the item
             const bool cut = item < n_mc;
@@ -303,40 +304,73 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
                 k = item - before;
                 nc = upto - before;
             }
+        } else if (CHUNKS && item < n_mc) {
+            const int4 rc = p.rec[item];
+            row = __builtin_amdgcn_readfirstlane(rc.x);
+            k = __builtin_amdgcn_readfirstlane(rc.y);
+            nc = __builtin_amdgcn_readfirstlane(rc.z);
         } else if (CHUNKS) {
-            if (item < n_mc) {
-                const int4 rc = p.rec[item];
-                row = rc.x; k = rc.y; nc = rc.z;
-            } else {
-                int32_t q = item - n_mc;
-                const int32_t *list = p.single[0];
-                if (q >= n_single0) {
-                    q -= n_single0; list = p.single[1];
-                    if (q >= n_single1) { q -= n_single1; list = p.single[2]; }
-                }
-                row = list[q];
+            // one single row of the longest class, two of the next, four of the shortest
+            int32_t q = item - n_mc, many = 0, of = n_single0;
+            list = p.single[0];
+            if (q >= n_single0) {
+                q -= n_single0; list = p.single[1]; many = 1; of = n_single1;
+                if (q >= (n_single1 + 1) / 2) { q -= (n_single1 + 1) / 2; list = p.single[2]; many = 2; of = n_single2; }
             }
-            row = __builtin_amdgcn_readfirstlane(row);
-            k = __builtin_amdgcn_readfirstlane(k);
-            nc = __builtin_amdgcn_readfirstlane(nc);
-        } else {
-            row = item * R + r;
-            have = r < R && row < n_rows;
-            if (!have) row = n_rows - 1;
+            list_at = q << many;
+            item_rows = of - list_at < 1 << many ? of - list_at : 1 << many;
         }
-        const int64_t start = offsets[row];
-        const int64_t len = offsets[row + 1] - start;
+        const bool chunk = CHUNKS && nc > 1;
+        // The item's whole rows, one per lane, with the lanes each of them needs (a region of P bytes to a lane)
+        // summed up; they are then taken in as few steps as their lanes fit the wave.
+        int32_t row_id = row;
+        int64_t row_at = 0, row_len = 0;
+        int lanes_to = 0, lanes_own = 0;
+        if (!chunk) {
+            if (lane < item_rows) {
+                if (!CHUNKS) row_id = (int32_t)(item_row0 + lane);
+                else if (list) row_id = list[list_at + lane];
+                row_at = offsets[row_id];
+                row_len = offsets[row_id + 1] - row_at;
+                lanes_own = row_len <= 0 || row_len > kRowMax ? 1 : ((int)row_len + P - 1) / P;
+            }
+            lanes_to = (int)wave_inclusive_sum_u32((uint32_t)lanes_own);
+        }
+        for (int first = 0; first < item_rows;) {          // (chunks: one step)
+        int m = 1, r = 0, lane0 = 0, G = 64;
+        bool have = true;
+        int64_t start, len;
+        if (chunk) {
+            start = offsets[row];
+            len = offsets[row + 1] - start;
+        } else {
+            // rows [first, first + m) of the item; r: the lane's row, lane0 and G: that row's lanes
+            const int lanes_before = first > 0 ? __builtin_amdgcn_readlane(lanes_to, first - 1) : 0;
+            const uint64_t in_step = __ballot(lane >= first && lane < item_rows && lanes_to - lanes_before <= 64);
+            m = (int)__builtin_popcountll(in_step);
+            r = first;
+            for (int i = first; i + 1 < first + m; ++i)
+                if (lane >= __builtin_amdgcn_readlane(lanes_to, i) - lanes_before) r = i + 1;
+            G = __shfl(lanes_own, r);
+            lane0 = __shfl(lanes_to, r) - lanes_before - G;
+            have = lane < lane0 + G;                       // (lanes behind the last row's have none)
+            start = ((int64_t)__shfl((int)(row_at >> 32), r) << 32) | (uint32_t)__shfl((int)(uint32_t)row_at, r);
+            len = ((int64_t)__shfl((int)(row_len >> 32), r) << 32) | (uint32_t)__shfl((int)(uint32_t)row_len, r);
+            row = __shfl(row_id, r);
+        }
+        const int j = lane - lane0;                        // the lane's region within the row
+        const int s = j * P;                               // its first byte
         int64_t e0 = 0, e1 = len;
-        if (CHUNKS && t.list_here && nc > 1 && lane == 0) {
+        if (chunk && t.list_here && lane == 0) {
             p.rec[item] = make_int4(row, k, nc, (int)len);
             if (k == 0) p.row_fail[row] = 0;
         }
-        if (CHUNKS && nc > 1) {
+        if (chunk) {
             e0 = (int64_t)k * p.core - p.overlap < 0 ? 0 : (int64_t)k * p.core - p.overlap;
             e1 = (int64_t)(k + 1) * p.core + p.overlap;
             if (e1 > len) e1 = len;
         }
-        const bool too_long = e1 - e0 > cap;
+        const bool too_long = e1 - e0 > kRowMax;           // (longer than the caller declared)
         const int n = have && !too_long && e1 > e0 ? (int)(e1 - e0) : 0;
         const uint8_t *const src = bytes + start + e0;
 
@@ -484,7 +518,6 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
         const uint32_t base = lane0 > 0 ? before_row : 0u;
         const uint32_t row_last = (uint32_t)__shfl((int)inc, lane0 + G - 1 < 64 ? lane0 + G - 1 : 63);
         const uint32_t n_tok = row_last - base;
-        const bool chunk = CHUNKS && nc > 1;
 
         // the region's tokens, last one first: f(number of the token's state -- behind the states: the byte,
         // where it is no letter --, position of its first byte in the region).  Four at a time: their
@@ -552,9 +585,17 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
                     *reinterpret_cast<uint4 *>(raw + i) = uint4{y[0] | y[1] << 16, y[2] | y[3] << 16, y[4] | y[5] << 16, y[6] | y[7] << 16};
             }
         } else {
-            if (j == 0 && have) {
-                lengths[row] = too_long ? -1 : (int32_t)n_tok;
-                longest = (int32_t)n_tok > longest ? (int32_t)n_tok : longest;
+            // the step's rows, one per lane again
+            int row_tok = 0, row_base = 0;
+            {
+                const int at = lanes_to - lanes_own - (first > 0 ? __builtin_amdgcn_readlane(lanes_to, first - 1) : 0);
+                const int from = lane >= first && lane < first + m ? at : 0;
+                row_tok = __shfl((int)n_tok, from);
+                row_base = __shfl((int)base, from);
+                if (lane >= first && lane < first + m) {
+                    lengths[row_id] = row_len > kRowMax ? -1 : row_tok;
+                    longest = row_tok > longest ? row_tok : longest;
+                }
             }
             // through LDS, where the wave's tokens fit its window (a token per four bytes always does)
             const bool fits = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63) <= (uint32_t)t.window;
@@ -564,15 +605,13 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
                 wave_phase();
             }
             if (PADDED) {
-                const int64_t row0 = CHUNKS ? (int64_t)row : (int64_t)item * R;
-                const int rows = CHUNKS ? 1 : (n_rows - row0 < R ? (int)(n_rows - row0) : R);
                 const int elem = a.pad_elem;
                 if (fits && (a.pad_stride & 3) == 0 && ((uintptr_t)a.pad_ids & (elem >= 4 ? 15 : 4 * elem - 1)) == 0 &&
                     ((uintptr_t)a.pad_mask & 3) == 0) {
-                    if (elem == 4) auto_put_rows<4>(a, t.id, staged, (int)base, (int)n_tok, G, rows, row0, lane);
-                    else if (elem == 8) auto_put_rows<8>(a, t.id, staged, (int)base, (int)n_tok, G, rows, row0, lane);
-                    else if (elem == 2) auto_put_rows<2>(a, t.id, staged, (int)base, (int)n_tok, G, rows, row0, lane);
-                    else auto_put_rows<1>(a, t.id, staged, (int)base, (int)n_tok, G, rows, row0, lane);
+                    if (elem == 4) auto_put_rows<4>(a, t.id, staged, row_base, row_tok, first, m, row_id, lane);
+                    else if (elem == 8) auto_put_rows<8>(a, t.id, staged, row_base, row_tok, first, m, row_id, lane);
+                    else if (elem == 2) auto_put_rows<2>(a, t.id, staged, row_base, row_tok, first, m, row_id, lane);
+                    else auto_put_rows<1>(a, t.id, staged, row_base, row_tok, first, m, row_id, lane);
                 } else {
                     // cell by cell: the lanes their own tokens, the row's lanes its padding and mask
                     const int64_t stride = a.pad_stride, at0 = (int64_t)row * stride;
@@ -597,7 +636,7 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
             } else {
                 int32_t *const out = tok_tmp + start;
                 if (fits) {                                // the row's own lanes write its run
-                    for (uint32_t c = j; c < n_tok; c += G) out[c] = t.id[staged[base + c]];
+                    for (uint32_t c = j; have && c < n_tok; c += G) out[c] = t.id[staged[base + c]];
                 } else {
                     uint32_t at = inc - base;
                     each_token([&](uint32_t v, int) { out[--at] = t.id[v]; });
@@ -628,7 +667,9 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
                 }
             }
         }
-        wave_phase();                                      // the wave's part of LDS is rewritten by its next item
+        wave_phase();                                      // the wave's part of LDS is rewritten by the next step
+        first += m;
+        }
     }
     if (PADDED && !CHUNKS && a.max_tree) {
         const uint32_t m = wave_max_u32((uint32_t)longest);

@@ -2415,6 +2415,17 @@ int launch_auto_as(const dnatok_bpe_t *t, const BpeArgs &a, AutoArgs aa, const u
     const int waves = Lds::waves(t->auto_states);
     aa.window = Lds::window(t->auto_states);
     static const int64_t resident = resident_workgroups(kern, 64 * kAutoMaxWaves, kAutoLdsBytes, 1);
+    if (!CHUNKS) {
+        // as many rows to an item as give every wave the same number of items, if that is more: a wave
+        // takes them in as few steps as they fit, and no wave starts an item when the others are done
+        // (100,000 reads, items of eight rows, 3.05 to a wave: 57.3 us; of 25 rows, one to a wave: 56.0 us; 16,384 rows of
+        // 1 KB 29.2 and 28.6 us)
+        const int64_t all = resident * waves, turns = (n_rows + 64 * all - 1) / (64 * all);
+        const int64_t even = (n_rows + turns * all - 1) / (turns * all);
+        if (even > aa.rows) aa.rows = (int32_t)even;
+        items = (n_rows + aa.rows - 1) / aa.rows;
+        aa.n_groups = (int32_t)items;
+    }
     int64_t grid = items < resident ? items : resident;
     if (a.max_tree && grid > kTreeRows) grid = kTreeRows;
     if (grid < 1) grid = 1;
@@ -2428,7 +2439,7 @@ template <bool WIDE>
 int run_auto(const dnatok_bpe_t *t, const BpeArgs &a, int chunking, const uint8_t *bytes, const int64_t *offsets,
              const BpePlan &p, int64_t n_rows, int64_t max_len, int64_t total, int32_t *tok_tmp, int32_t *lengths, hipStream_t s)
 {
-    AutoArgs aa{t->auto_next, t->auto_len, t->auto_sym, t->auto_id, t->auto_states, t->auto_letters, 64, 1, 0, 0, 0, nullptr, total};
+    AutoArgs aa{t->auto_next, t->auto_len, t->auto_sym, t->auto_id, t->auto_states, t->auto_letters, 1, 0, 0, 0, nullptr, total};
     if (chunking & 1) {
         aa.list_here = n_rows <= kAutoListRows ? 1 : 0;
         if (!aa.list_here) {
@@ -2444,21 +2455,25 @@ int run_auto(const dnatok_bpe_t *t, const BpeArgs &a, int chunking, const uint8_
     }
     // Regions of 32 bytes, of 16 when the batch is so small that its waves find a place at once either way
     // (a lane's walk is then half as long, and twice the lanes share it).
-    const int64_t len = max_len < 1 ? 1 : max_len;
-    const int64_t lanes16 = (len + 15) / 16;
-    const bool small = len <= 1024 && (n_rows + 64 / lanes16 - 1) / (64 / lanes16) <= 256 * kAutoMaxWaves;
-    aa.lanes = (int32_t)(small ? lanes16 : (len + 31) / 32);
-    aa.rows = 64 / aa.lanes;
-    const int64_t groups = (n_rows + aa.rows - 1) / aa.rows;
-    aa.n_groups = (int32_t)groups;
+    // An item is as many rows as fit a wave for certain, or as many as nearly always fit it by the rows'
+    // mean length, if that is more (an item that does not fit takes two steps).
+    const int64_t len = max_len < 1 ? 1 : (max_len > 2048 ? 2048 : max_len);
+    const auto rows_of = [&](int64_t region) {
+        const int64_t sure = 64 / ((len + region - 1) / region);
+        const int64_t mean = (total / n_rows) * 2 / region + 1;                // twice the lanes of a row, on average
+        const int64_t likely = 56 * 2 / (mean < 2 ? 2 : mean);
+        return sure > likely ? sure : (likely > 64 ? (int64_t)64 : likely);
+    };
+    const bool small = len <= 1024 && (n_rows + rows_of(16) - 1) / rows_of(16) <= 256 * kAutoMaxWaves;
+    aa.rows = (int32_t)rows_of(small ? 16 : 32);
     if (small) {
-        if (a.pad_ids) return launch_auto_as<WIDE, 16, false, false, true>(t, a, aa, bytes, offsets, p, n_rows, groups, tok_tmp, lengths, s);
-        if (a.char_ids) return launch_auto_as<WIDE, 16, false, true, false>(t, a, aa, bytes, offsets, p, n_rows, groups, tok_tmp, lengths, s);
-        return launch_auto_as<WIDE, 16, false, false, false>(t, a, aa, bytes, offsets, p, n_rows, groups, tok_tmp, lengths, s);
+        if (a.pad_ids) return launch_auto_as<WIDE, 16, false, false, true>(t, a, aa, bytes, offsets, p, n_rows, n_rows, tok_tmp, lengths, s);
+        if (a.char_ids) return launch_auto_as<WIDE, 16, false, true, false>(t, a, aa, bytes, offsets, p, n_rows, n_rows, tok_tmp, lengths, s);
+        return launch_auto_as<WIDE, 16, false, false, false>(t, a, aa, bytes, offsets, p, n_rows, n_rows, tok_tmp, lengths, s);
     }
-    if (a.pad_ids) return launch_auto_as<WIDE, 32, false, false, true>(t, a, aa, bytes, offsets, p, n_rows, groups, tok_tmp, lengths, s);
-    if (a.char_ids) return launch_auto_as<WIDE, 32, false, true, false>(t, a, aa, bytes, offsets, p, n_rows, groups, tok_tmp, lengths, s);
-    return launch_auto_as<WIDE, 32, false, false, false>(t, a, aa, bytes, offsets, p, n_rows, groups, tok_tmp, lengths, s);
+    if (a.pad_ids) return launch_auto_as<WIDE, 32, false, false, true>(t, a, aa, bytes, offsets, p, n_rows, n_rows, tok_tmp, lengths, s);
+    if (a.char_ids) return launch_auto_as<WIDE, 32, false, true, false>(t, a, aa, bytes, offsets, p, n_rows, n_rows, tok_tmp, lengths, s);
+    return launch_auto_as<WIDE, 32, false, false, false>(t, a, aa, bytes, offsets, p, n_rows, n_rows, tok_tmp, lengths, s);
 }
 
 // The work list (plan) is needed when rows are cut into chunks or left to the whole-row kernel,
