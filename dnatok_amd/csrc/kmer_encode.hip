@@ -28,6 +28,7 @@
 
 #include <limits.h>
 #include <string.h>
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <stdlib.h>
@@ -38,6 +39,7 @@ struct dnatok_kmer_table {
     int k;
     int64_t pow4, pow5;
     int32_t pad_id, missing_id;
+    int all_plain;           // every ACGT-only window has an id
     int chars_mode;          // every non-plain window expands to its own characters
     void *blob;              // one device allocation holding all tables
     int8_t *digit;           // [256]
@@ -81,6 +83,7 @@ struct KmerArgs {
     const int2 *entry;
     const int32_t *flat;
     int32_t pad_id, missing_id;
+    int32_t all_plain;                    // every window of plain bases has an id
 };
 
 constexpr int kKmerThreads = 256;         // kmer_team_kernel: four waves share a row
@@ -782,22 +785,37 @@ __global__ __launch_bounds__(kGroupThreads) void kmer_groups_kernel(
     __shared__ int32_t s_spell[256];
     __shared__ int32_t s_lut4[LUT4_LDS ? POW4 : 1];
     __shared__ uint32_t s_wave_max[kGroupThreads / 64];
+    // A group's next row is looked up while it works on the one before (the first while the tables are
+    // staged): its place and its bytes are a chain of two trips to memory, and a row is little else.
+    const int lane = threadIdx.x & 63, gl = lane & 15;
+    const int64_t group = ((int64_t)blockIdx.x * kGroupThreads + threadIdx.x) >> 4;
+    const int64_t n_groups = (int64_t)gridDim.x * (kGroupThreads / 16);
+    int64_t next_start = 0, next_end = 0, next_cell = 0, next_cell_end = 0;
+    auto look_up = [&](int64_t row) {
+        if (row >= n_rows) return;
+        next_start = offsets[row];
+        next_end = offsets[row + 1];
+        if (place.row_at) {
+            next_cell = place.row_at[row];
+            next_cell_end = place.row_at[row + 1];
+        }
+    };
+    look_up(group);
+    const int64_t total = offsets[n_rows];
+    // (a count needs no ids where every plain window has one)
+    const bool ids_needed = !(place.count_only && a.all_plain);
     for (int i = threadIdx.x; i < 256; i += kGroupThreads) {
         const int d = a.digit[i];
         s_single[i] = a.single[i];
         s_spell[i] = a.single[(int)"ACGTN"[d < 0 || d > 4 ? 4 : d]];
     }
-    if (LUT4_LDS)
+    if (LUT4_LDS && ids_needed)
         for (uint32_t i = threadIdx.x; i < POW4; i += kGroupThreads) s_lut4[i] = a.lut4r[i];
     __syncthreads();
 
-    const int lane = threadIdx.x & 63, gl = lane & 15;
     const int cap_all = t_cap > INT_MAX - 16 ? INT_MAX - 16 : (int)t_cap;
     const int fill_all = fill_to > cap_all ? cap_all : (int)fill_to;
-    const int64_t group = ((int64_t)blockIdx.x * kGroupThreads + threadIdx.x) >> 4;
-    const int64_t n_groups = (int64_t)gridDim.x * (kGroupThreads / 16);
     const unsigned long long slot_gen = mref.slot ? mref.slot[1] : 0ull;
-    const int64_t total = offsets[n_rows];
     uint32_t group_max = 0;
 
     // every group of the wave makes the same number of trips (a group without a row idles), so
@@ -806,8 +824,10 @@ __global__ __launch_bounds__(kGroupThreads) void kmer_groups_kernel(
     for (int64_t row0 = wave_first; row0 < n_rows; row0 += n_groups) {
         const int64_t row = row0 + (lane >> 4);
         bool have = row < n_rows;
-        const int64_t start = have ? offsets[row] : 0;
-        int len = have ? (int)(offsets[row + 1] - start) : 0;
+        const int64_t start = have ? next_start : 0;
+        int len = have ? (int)(next_end - next_start) : 0;
+        const int64_t cell_from = next_cell, cell_end = next_cell_end;
+        look_up(row + n_groups);
         if (place.row_class == 1 && len / K + len % K > kGroupsMaxUnits) {     // (kmer_rows_kernel's row)
             have = false;
             len = 0;
@@ -815,8 +835,8 @@ __global__ __launch_bounds__(kGroupThreads) void kmer_groups_kernel(
         const int full = len / K, tail = len - full * K;
         const int n_slots = full + (tail ? 1 : 0);                // windows, and one slot for the trailing characters
         // the row's cells: a stride apart, or (packed) where the rows before it end
-        const int64_t cell0 = !have ? 0 : place.row_at ? place.row_at[row] : row * t_cap;
-        const int cap = place.count_only || !have ? 0 : place.row_at ? (int)(place.row_at[row + 1] - cell0) : cap_all;
+        const int64_t cell0 = !have ? 0 : place.row_at ? cell_from : row * t_cap;
+        const int cap = place.count_only || !have ? 0 : place.row_at ? (int)(cell_end - cell0) : cap_all;
         const int fill = place.row_at || !have ? 0 : fill_all;
         int32_t *out = ids + cell0;
         uint8_t *mout = HAS_MASK ? mask + cell0 : nullptr;
@@ -873,7 +893,7 @@ __global__ __launch_bounds__(kGroupThreads) void kmer_groups_kernel(
                 const int bit = 2 * K * j;
                 const uint64_t two = ((uint64_t)str[(bit >> 5) + 1] << 32) | str[bit >> 5];
                 const uint32_t code = (uint32_t)(two >> (bit & 31)) & (POW4 - 1);
-                t[j] = LUT4_LDS ? s_lut4[code] : a.lut4r[code];
+                t[j] = !ids_needed ? 0 : LUT4_LDS ? s_lut4[code] : a.lut4r[code];
                 uint32_t hit = 0;
 #pragma unroll
                 for (int i = 0; i < K; ++i) {
@@ -1524,6 +1544,7 @@ extern "C" int dnatok_kmer_table_create(int k, const int8_t *digit_h, const int3
     uint8_t *b = (uint8_t *)blob;
     t->k = k; t->pow4 = pow4; t->pow5 = pow5; t->pad_id = pad_id; t->missing_id = missing_id;
     t->chars_mode = chars_mode; t->blob = blob;
+    t->all_plain = std::all_of(lut4.begin(), lut4.end(), [](int32_t id) { return id >= 0; }) ? 1 : 0;
     t->digit = (int8_t *)(b + o_digit);
     t->single = (int32_t *)(b + o_single);
     t->lut4 = (int32_t *)(b + o_lut4);
@@ -1575,7 +1596,7 @@ extern "C" int dnatok_kmer_encode_padded(const dnatok_kmer_t *t, const uint8_t *
     if (to_longest) fill_to = guess;
     if (n_rows == 0) return DNATOK_OK;
     hipStream_t s = (hipStream_t)stream;
-    KmerArgs a{t->digit, t->single, t->lut4, t->lut4r, t->fold, t->entry, t->flat, t->pad_id, t->missing_id};
+    KmerArgs a{t->digit, t->single, t->lut4, t->lut4r, t->fold, t->entry, t->flat, t->pad_id, t->missing_id, t->all_plain};
     MaxRef mref{nullptr, nullptr};
     if (to_longest) {
         std::lock_guard<std::mutex> hold(t->slot_lock);
@@ -1695,7 +1716,7 @@ static int launch_placed(const dnatok_kmer_t *t, int which, const uint8_t *bytes
                          int64_t t_cap, int64_t fill_to, int32_t *ids, uint8_t *mask, int32_t *lengths,
                          int32_t *status, int32_t *max_len, MaxRef mref, RowPlace place, hipStream_t s)
 {
-    KmerArgs a{t->digit, t->single, t->lut4, t->lut4r, t->fold, t->entry, t->flat, t->pad_id, t->missing_id};
+    KmerArgs a{t->digit, t->single, t->lut4, t->lut4r, t->fold, t->entry, t->flat, t->pad_id, t->missing_id, t->all_plain};
     if (which == 1) {
 #define PG2(KK, L, M)                                                                              \
     do {                                                                                          \
