@@ -772,6 +772,12 @@ __device__ __forceinline__ uint32_t row16_last(uint32_t v)
     return (uint32_t)__builtin_amdgcn_ds_bpermute(src << 2, (int)v);
 }
 
+// A lane's 4K bytes, at any address: the widest loads there are.
+template <int K>
+struct __attribute__((packed, aligned(1), may_alias)) LaneBytes {
+    uint32_t v[K];
+};
+
 template <int K, bool LUT4_LDS, bool HAS_MASK>
 __global__ __launch_bounds__(kGroupThreads) void kmer_groups_kernel(
     KmerArgs a, const uint8_t *__restrict__ bytes, const int64_t *__restrict__ offsets,
@@ -851,20 +857,21 @@ __global__ __launch_bounds__(kGroupThreads) void kmer_groups_kernel(
             // bytes) is read and ignored, what lies past the end of the batch is not read
             const int64_t pos = start + (int64_t)wb * K;
             uint32_t w[K];
+            if (wb < n_slots && pos + kLaneBytes <= total) {
+                const LaneBytes<K> all = *reinterpret_cast<const LaneBytes<K> *>(bytes + pos);
 #pragma unroll
-            for (int i = 0; i < K; ++i) {
-                const int64_t at = pos + 4 * i;
-                uint32_t v = 0;
-                if (wb < n_slots) {
-                    if (at + 4 <= total) {
-                        v = *reinterpret_cast<const u32_a1 *>(bytes + at);
-                    } else {
+                for (int i = 0; i < K; ++i) w[i] = all.v[i];
+            } else {
+#pragma unroll
+                for (int i = 0; i < K; ++i) {
+                    uint32_t v = 0;
+                    if (wb < n_slots) {
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
-                            if (at + e < total) v |= (uint32_t)bytes[at + e] << (8 * e);
+                            if (pos + 4 * i + e < total) v |= (uint32_t)bytes[pos + 4 * i + e] << (8 * e);
                     }
+                    w[i] = v;
                 }
-                w[i] = v;
             }
             // digits, codes and the bytes that are no base, as in kmer_rows_kernel<..., ARITH>
             uint32_t odd[K], c8[K];
