@@ -317,8 +317,8 @@ int dnatok_bpe_table_set_chunk_geometry(dnatok_bpe_t *t, int32_t core, int32_t o
 /* MEASUREMENT ONLY: where the merge table of the calls with this table object is kept (no
  * counterpart in the reference, whose kernel reads its hash table from global memory,
  * dnatok_bpe.cu:822-837).  A table of at most 8192 symbols and 4095 rules also has a compact form
- * of 48 KB.  mode 0 (default): every batch reads the table from global memory (L2), which measured
- * faster.  mode 1: a batch of rows of at most 1024 bytes, few enough for one row per resident
+ * of 48 KB.  mode 0 (default): the shipped choice (the automaton where the table has one; the merges
+ * read their table from global memory, L2).  mode 1: a batch of rows of at most 1024 bytes, few enough for one row per resident
  * workgroup with those 48 KB added to each, is encoded by workgroups that keep the compact form in
  * LDS.  mode 2: the compact form for every batch of rows of at most 1024 bytes that one launch
  * encodes whole.  Results are identical in all modes. */
