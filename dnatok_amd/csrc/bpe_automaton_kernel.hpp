@@ -89,6 +89,12 @@ struct AutoLds {
     }
 };
 
+// From this many bytes on, walked into the regions to the right, a lane looks for a repeat: twice what a walk takes
+// in other text, and behind it lies the longest period of the states in the common repeats (80 bytes).  (From 96
+// bytes on, rows with short repeats in them, 10 % of their bases, were 3 % slower, 28.8 -> 29.6 us for 1,024 of 1 KB
+// with the vocabulary of 32,000; from 128 on they are 3 % faster, 27.8 us.)
+constexpr int kRepeatsFrom = 128;
+
 // Up to this many rows a wave finds its item among the rows itself (their lengths are one load per 64
 // rows, beside each other) instead of in a list that a launch in front has made: 5 us per call, as long
 // as anything that a batch of a few rows waits for.
@@ -179,6 +185,99 @@ __device__ __forceinline__ void auto_put_rows(const BpeArgs &a, const int32_t *i
                     ((uint32_t)v[0] & 0xFFu) | (((uint32_t)v[1] & 0xFFu) << 8) | (((uint32_t)v[2] & 0xFFu) << 16) | ((uint32_t)v[3] << 24);
             }
             if (a.pad_mask) *reinterpret_cast<uint32_t *>(a.pad_mask + at) = live;
+        }
+    }
+}
+
+// Lanes that have gone on (`going`, with state e) through the regions up to lane + ahead - 1 without meeting
+// the state that was there: inside a tandem repeat the run from the row's start and a run that began inside
+// may differ in phase for as long as it lasts.  But where a run's state is the one it had d bytes before, and
+// the bytes from here on are those d bytes before them, its next states are those of d bytes before as well.
+// So the walkers' last states are compared with the states of their own run behind them, all distances at once,
+// the regions ahead whose bytes repeat at such a distance are counted, and their states copied by their own
+// lanes; the walk goes on behind them, as that of the lane `ahead` regions before.  A row of 2,048 bases that is
+// one repeat takes at most 136 steps of the automaton in a row instead of 2,048: 64 rows of 2,000 bases of A, AC, AAT,
+// AAAT or AACCG with the vocabulary of 32,000 155 - 171 -> 23 - 26 us (the merge engine: 65 - 105), of AAT with that
+// of 4,096 117 -> 18.5 us (36).  Rows that never come here are 0.2 - 1.7 % slower for the code in their way (16,384
+// rows of 1 KB 28.5 -> 29.0 us); as a function of its own, or with a second copy of the walk for it, 2 - 5 %.
+// A walker's run behind it is only its own where no other walker of the row has come by since: not those
+// with a walker less than `ahead` lanes to their left.
+template <int P, typename Entry>
+__device__ __forceinline__ void copy_repeats(Entry *state, const uint32_t (&codes)[P / 16], uint32_t flags, bool any_foreign, int cnt,
+                                             int cnt_ahead, int lane, int lane0, int lane_end, int ahead, Entry &e, bool &going)
+{
+    constexpr int kTries = 4, kLongest = 256;              // walkers per call, and distances of one of them; the longest distance
+    const int behind = ahead * P < kLongest ? ahead * P : kLongest;
+    const uint64_t mine = P == 32 ? (uint64_t)codes[P / 16 - 1] << 32 | codes[0] : codes[0];
+    int done = -1;
+#pragma unroll 1
+    for (int tries = 0; tries < kTries; ++tries) {
+        const uint64_t left = __ballot(going) & ((1ull << lane) - 1ull);
+        const int nearest = left ? 63 - __builtin_clzll(left) : -1;
+        const uint64_t eligible = __ballot(going && lane > done && (nearest < lane0 || lane - nearest >= ahead));
+        if (!eligible) break;
+        const int walker = __builtin_ctzll(eligible);
+        const int first = walker + ahead;                  // the region it is about to enter
+        const int row_end = __builtin_amdgcn_readlane(lane_end, walker);
+        const Entry now = (Entry)__builtin_amdgcn_readlane((int)e, walker);
+        int k = 0, d = 0, looked = 0;
+#pragma unroll 1
+        for (int d0 = 1; k == 0 && looked < kTries && d0 < behind; d0 += 64) {
+            const int back = d0 + lane;
+            bool same = false;
+            if (back < behind) {
+                const int pos = first * P - 1 - back;
+                same = state[(pos & (P - 1)) * 64 + pos / P] == now;
+            }
+            uint64_t at = __ballot(same);
+            while (at && k == 0 && looked < kTries) {
+                d = d0 + __builtin_ctzll(at);
+                at &= at - 1;
+                ++looked;
+                // the region's bytes against those d before them
+                const int regions = (d + P - 1) / P, o = regions * P - d;
+                const int from = lane - regions;
+                uint64_t lo = (uint32_t)__shfl((int)codes[0], from & 63), hi = (uint32_t)__shfl((int)codes[0], (from + 1) & 63);
+                if (P == 32) {
+                    lo |= (uint64_t)(uint32_t)__shfl((int)codes[P / 16 - 1], from & 63) << 32;
+                    hi |= (uint64_t)(uint32_t)__shfl((int)codes[P / 16 - 1], (from + 1) & 63) << 32;
+                }
+                const uint64_t text = o == 0 ? lo : lo >> (2 * o) | hi << (2 * (P - o));
+                bool repeats = (P == 32 ? text : text & 0xFFFFFFFFull) == mine;
+                if (any_foreign) {
+                    const uint64_t f = (uint64_t)(uint32_t)__shfl((int)flags, (from + 1) & 63) << P | (uint32_t)__shfl((int)flags, from & 63);
+                    repeats = repeats && (uint32_t)(f >> o & ((1ull << P) - 1ull)) == flags;
+                }
+                const uint64_t run = __ballot(repeats && lane >= first && lane < row_end && cnt == P) >> first;
+                k = __builtin_ctzll(~run);                 // (first > 0, so that bits of zeros were shifted in)
+            }
+        }
+        done = walker;
+        if (k == 0) continue;
+        if (lane >= first && lane < first + k) {
+            int t = (lane - first) * P;
+#pragma unroll 1
+            for (int i = 10; i >= 0; --i)                  // t % d (t < 64 P <= 2,048)
+                if (t >= d << i) t -= d << i;
+#pragma unroll 1
+            for (int i = 0; i < P; i += 4) {
+                Entry v[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int pos = first * P - d + t;     // (behind region `first`: nobody writes there now)
+                    v[q] = state[(pos & (P - 1)) * 64 + pos / P];
+                    t = t + 1 == d ? 0 : t + 1;
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q) state[(i + q) * 64 + lane] = v[q];
+            }
+        }
+        wave_phase();
+        done = walker + k;
+        if (lane >= walker && lane < done) going = false;
+        if (lane == done) {
+            going = first + k < row_end && cnt_ahead > 0;
+            e = state[(P - 1) * 64 + first + k - 1];
         }
     }
 }
@@ -430,6 +529,8 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
             going = going && j + ahead < G && cnt2 > 0;
             if (!__ballot(going)) break;
             wave_phase();
+            if (__builtin_expect(ahead >= kRepeatsFrom / P, 0))
+                copy_repeats<P>(state, codes, flags, any_foreign, cnt, cnt2, lane, lane0, lane0 + G, ahead, e, going);
             for (int i = 0; i < P; i += 4) {
                 if (going) {
                     Entry *const at = state + i * 64 + lane + ahead;

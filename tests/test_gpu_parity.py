@@ -1143,6 +1143,80 @@ def test_bpe_automaton_at_the_edges_of_regions(bpe, longest, count):
         enc.set_chunk_geometry(0, 0)
 
 
+def repeats(rng, n):
+    """``n`` bytes, mostly inside tandem repeats of units of 1 - 9 letters: a single one, several behind
+    each other (some twice, so that a state is met again in front of other text), broken by single
+    letters and by bytes that are no letters."""
+    parts, total = [], 0
+    while total < n:
+        kind = rng.randrange(8)
+        if kind < 5:
+            unit = "".join(rng.choices("ACGT", k=rng.choice([1, 1, 2, 3, 3, 4, 5, 6, 7, 9])))
+            part = unit * (rng.choice([40, 150, 400, n]) // len(unit) + 1)
+        elif kind == 5 and parts:
+            part = rng.choice(parts)
+        else:
+            part = "".join(rng.choices("ACGTN", k=rng.choice([1, 2, 30])))
+        parts.append(part[:n - total])
+        total += len(parts[-1])
+    return "".join(parts)
+
+
+@pytest.mark.parametrize("longest,count", [(300, 3000), (700, 40), (1024, 600), (1000, 20000), (2048, 300), (7000, 40)])
+def test_bpe_rows_of_tandem_repeats(bpe, longest, count):
+    """Rows that are nothing but tandem repeats, one and several rows to a wave, in regions of 16 and of
+    32 bytes and in chunks: states copied from a period before are those that a walk would give."""
+    which, enc, bo = bpe
+    say(f"bpe{which} tandem repeats, {count} rows of up to {longest}")
+    rng = random.Random(longest + count)
+    some = [repeats(rng, rng.choice([longest, longest - 1, longest // 2 + 3, rng.randint(1, longest)])) for _ in range(min(count, 600))]
+    some[0] = "AAT" * (longest // 3 + 1)
+    some[1] = "AACCG" * (longest // 5)
+    seqs = [some[i % len(some)] for i in range(count)]
+    b = util.batch_from_strings(some)
+    ref = bo.encode_batch(b.data, b.offsets)
+    got = bpe_rows(enc, util.batch_from_strings(seqs))
+    for i, r in enumerate(got):
+        np.testing.assert_array_equal(r, ref[i % len(some)], err_msg=f"row {i}: {some[i % len(some)][:80]}")
+
+
+def call_us(call, reps=20):
+    """Device time of a call, in microseconds: the best of five replays of a graph of ``reps`` of them."""
+    torch.cuda.synchronize()
+    side, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        call()
+        side.synchronize()
+        with torch.cuda.graph(g, stream=side):
+            for _ in range(reps):
+                call()
+        best = float("inf")
+        for _ in range(5):
+            t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            t0.record(side)
+            g.replay()
+            t1.record(side)
+            side.synchronize()
+            best = min(best, t0.elapsed_time(t1) * 1e3 / reps)
+    return best
+
+
+def test_bpe_repeats_are_not_walked_byte_by_byte(bpe):
+    """A row of 2,000 bases that is one repeat takes at most four times as long as a random one (a walk
+    over all of it took 10 times as long with either vocabulary)."""
+    which, enc, _ = bpe
+    rng = random.Random(1)
+    times = {}
+    for unit in ("random", "A", "AC", "AAT", "AAAT", "AACCG", "AACCGT"):
+        text = "".join(rng.choices("ACGT", k=2000)) if unit == "random" else (unit * 2000)[:2000]
+        b = util.batch_from_strings([text] * 64)
+        data, off = to_dev(b)
+        tok, lengths = enc.encode(data, off, 2000)
+        times[unit] = call_us(lambda: enc.encode(data, off, 2000, tok_tmp=tok, lengths=lengths))
+    say(f"bpe{which} repeats: " + ", ".join(f"{u} {t:.1f} us" for u, t in times.items()))
+    assert max(times.values()) < 4 * times["random"], times
+
+
 @pytest.mark.parametrize("count", [1, 64, 65, 256, 257])
 @pytest.mark.parametrize("pad_left,dtype", [(False, torch.int32), (True, torch.int64), (False, torch.int16)])
 def test_bpe_long_rows_padded_by_their_chunks(bpe, count, pad_left, dtype):
