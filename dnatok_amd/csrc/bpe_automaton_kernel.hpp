@@ -100,6 +100,8 @@ constexpr int kRepeatsFrom = 128;
 // as anything that a batch of a few rows waits for.
 constexpr int kAutoListRows = 256;
 
+constexpr uint32_t kXcds = 8;                    // (workgroups go to them in turn)
+
 // Between two phases of a wave's work on its LDS: what a lane wrote before is what the others read after.
 __device__ __forceinline__ void wave_phase()
 {
@@ -370,6 +372,21 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
         n_single1 = p.counts[5];
         n_single2 = p.counts[6];
         n_items = n_mc + n_single0 + (n_single1 + 1) / 2 + (n_single2 + 3) / 4;
+    }
+    if (WIDE) {
+        // A call that follows other kernels finds the table in no L2, and its walks are chains of misses.  The waves that
+        // have no item read a word of a line of 128 bytes per lane, the states of the start first (the first twentieth
+        // of the 164,729 are every second step), so that the L2 of their XCD has it before the walks have come that far
+        // (behind a copy of 512 MB, vocabulary of 32,000: 1,024 rows of 1 KB 23.0 -> 19.4 us, 64 rows 24.9 -> 22.3, 32 of
+        // 100 kbp 45.6 -> 43.0; with the table in the L2 1 - 2 % slower).  More workgroups to read all of it: 64 rows
+        // of 1 KB 18.3 us, but 13.8 instead of 12.6 with the table in the L2.
+        const int32_t busy = n_items <= (int32_t)blockIdx.x ? 0 : (int32_t)((n_items - blockIdx.x + gridDim.x - 1) / gridDim.x);
+        if (wv >= busy) {
+            const uint32_t line = (blockIdx.x / kXcds * (n_waves - busy) + wv - busy) * 64 + lane;
+            uint32_t sum = 0;
+            if (32 * line < n_entries) sum = far_table[32 * line];
+            asm volatile("" : : "v"(sum));
+        }
     }
     if (CHUNKS && t.zero && blockIdx.x == 0 && threadIdx.x == 0) *t.zero = 0;
     int32_t longest = 0;

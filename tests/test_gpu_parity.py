@@ -1201,6 +1201,34 @@ def call_us(call, reps=20):
     return best
 
 
+def test_bpe_calls_behind_other_kernels():
+    """Calls whose tables other kernels have pushed out of the caches are no slower by the automaton than
+    by the merge engine (which a set chunk geometry selects), with a tenth for the measurement: 64 reads of
+    100 bp took 27 us against 23 while eight waves walked a table of 2.6 MB miss by miss."""
+    cfg = util.tokenizer_json("32000")
+    kv = bpe_vocab.KernelVocab(bpe_vocab.split_merges(cfg["model"]["merges"]))
+    enc = encoders.BpeEncoder(kv.pair_a, kv.pair_b, kv.new_id, len(kv))
+    src = torch.zeros(256 << 20, dtype=torch.uint8, device=DEV)
+    dst = torch.empty_like(src)
+    flush = lambda: torch.bitwise_not(src, out=dst)
+    rng = random.Random(2)
+    for rows, length in ((64, 100), (8, 200), (64, 1024)):
+        b = util.batch_from_strings(["".join(rng.choices("ACGT", k=length)) for _ in range(rows)])
+        data, off = to_dev(b)
+        out = enc.encode_padded(data, off, length, length // 4, 3)
+
+        def call():
+            flush()
+            enc.encode_padded(data, off, length, length // 4, 3, out=out)
+        times = []
+        for geometry in ((1792, 128), (0, 0)):
+            enc.set_chunk_geometry(*geometry)
+            enc.encode_padded(data, off, length, length // 4, 3, out=out)
+            times.append(call_us(call) - call_us(flush))
+        say(f"{rows} rows of {length} behind a copy: merge engine {times[0]:.1f} us, automaton {times[1]:.1f} us")
+        assert times[1] < 1.1 * times[0], (rows, length, times)
+
+
 def test_bpe_repeats_are_not_walked_byte_by_byte(bpe):
     """A row of 2,000 bases that is one repeat takes at most four times as long as a random one (a walk
     over all of it took 10 times as long with either vocabulary)."""
