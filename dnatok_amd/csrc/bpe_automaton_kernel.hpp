@@ -479,7 +479,10 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
         int64_t e0 = 0, e1 = len;
         if (chunk && t.list_here && lane == 0) {
             p.rec[item] = make_int4(row, k, nc, (int)len);
-            if (k == 0) p.row_fail[row] = 0;
+            if (k == 0) {
+                p.row_fail[row] = 0;
+                p.mc_off[row] = item;
+            }
         }
         if (chunk) {
             e0 = (int64_t)k * p.core - p.overlap < 0 ? 0 : (int64_t)k * p.core - p.overlap;
@@ -801,13 +804,62 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
     }
 }
 
+// A row of many chunks: the tokens of its chunks up to and including each, into the fourth word of their counts.
+// The join kernel would otherwise add up, for every chunk, the chunks of its row (padded: all of them, else those in
+// front of it), as many reads as the row has chunks squared.  Vocabulary of 4,096, padded: one row of 200 Mbp 16.6 ->
+// 0.76 ms (the merge engine 6.1 ms), of 4 Mbp 54.4 -> 43.7 us, of 2 Mbp (1,117 chunks) 32.2 -> 30.6, four of 2 Mbp 58.0 ->
+// 57.2; not padded: 200 Mbp 4.35 -> 0.67 ms, 4 Mbp (2,233 chunks) 39.1 -> 37.6, four of 2 Mbp 50.2 -> 53.6.  A workgroup
+// looks at kScanRows rows and takes those with as many chunks one after the other, a chunk per thread and step.
+__host__ __device__ constexpr int scan_from_chunks(bool padded) { return padded ? 1024 : 2048; }
+constexpr int kScanRows = 16;
+
+__global__ __launch_bounds__(1024) void bpe_row_scan_kernel(const int64_t *__restrict__ offsets, int64_t n_rows, int from_chunks, BpePlan p)
+{
+    __shared__ uint32_t sums[2][16];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int64_t row = (int64_t)blockIdx.x * kScanRows + lane;
+    int32_t chunks = 0, first = 0;
+    if (lane < kScanRows && row < n_rows) {
+        const int64_t len = offsets[row + 1] - offsets[row];
+        chunks = len > p.ext ? (int32_t)((len + p.core - 1) / p.core) : 0;
+        if (chunks >= from_chunks) first = p.mc_off[row];
+    }
+    int bank = 0;
+    for (uint64_t todo = __ballot(chunks >= from_chunks); todo; todo &= todo - 1) {
+        const int at = __builtin_ctzll(todo);              // (the same row in all waves)
+        const int32_t nc = __builtin_amdgcn_readlane(chunks, at), m0 = __builtin_amdgcn_readlane(first, at);
+        uint32_t before = 0;
+        for (int64_t k0 = 0; k0 < nc; k0 += 1024, bank ^= 1) {
+            const int64_t k = k0 + threadIdx.x;
+            int32_t *const cnt = p.cnt + 4 * ((size_t)m0 + (size_t)k);
+            uint32_t c = 0;
+            if (k < nc) {
+                const int4 part = *reinterpret_cast<const int4 *>(cnt);
+                c = (uint32_t)(part.x + (k > 0 ? part.y : 0) + (k + 1 < nc ? part.z : 0));
+            }
+            const uint32_t inc = wave_inclusive_sum_u32(c);
+            if (lane == 63) sums[bank][wv] = inc;
+            __syncthreads();                               // (the other bank is read by nobody any more)
+            uint32_t to = before + inc;
+#pragma unroll
+            for (int w = 0; w < 16; ++w) {
+                const uint32_t v = sums[bank][w];
+                if (w < wv) to += v;
+                before += v;
+            }
+            if (k < nc) cnt[3] = (int32_t)to;
+        }
+    }
+}
+
 // The rows behind the seam kernel: the chunks' tokens put together, a wave per chunk (the chunk is held as in
 // bpe_gather_wave_kernel), and the rows that have no seam redone whole.  The two are independent, so they
 // share a launch: the first n_slabs workgroups take the rows to be redone (nearly always none), the others
 // the chunks.  PADDED: a row goes straight to its cells of a.pad_ids, its padding shared out among its
 // chunks; then this launch stands for three (gather, whole rows, padding: 32 rows of 100 kbp, 6.5 + 4.5 +
-// 5.3 us).  count_longest: *a.longest (cleared by the kernel in front) becomes the longest row.
-template <bool PADDED>
+// 5.3 us).  count_longest: *a.longest (cleared by the kernel in front) becomes the longest row.  SCANNED: the
+// row scan kernel has run.
+template <bool PADDED, bool SCANNED>
 __global__ __launch_bounds__(1024) void bpe_auto_join_kernel(
     BpeArgs a, const int32_t *__restrict__ id, const uint8_t *__restrict__ bytes, const int64_t *__restrict__ offsets, int64_t n_rows,
     int64_t max_len, BpePlan p, int count_longest, int32_t *__restrict__ tok_tmp, int32_t *__restrict__ lengths)
@@ -889,14 +941,22 @@ __global__ __launch_bounds__(1024) void bpe_auto_join_kernel(
         const int32_t seam_r = k + 1 < nc ? p.seam[m] : 0;
         const int32_t failed = p.row_fail[row];
         const int64_t row_at = offsets[row];
-        uint32_t before = 0, behind = 0;
-        for (int32_t j = lane; j < (PADDED ? nc : k); j += 64) {
-            const int4 part = *reinterpret_cast<const int4 *>(p.cnt + 4 * (size_t)(m - k + j));   // {unshared, after left seam, before right seam, -}
-            const uint32_t c = (uint32_t)(part.x + (j > 0 ? part.y : 0) + (j + 1 < nc ? part.z : 0));
-            if (j < k) before += c; else behind += c;
+        // tokens of the row's chunks in front of this one, and (PADDED) of the whole row
+        uint32_t base, n_tok = 0;
+        if (SCANNED && nc >= scan_from_chunks(PADDED)) {
+            base = k > 0 ? (uint32_t)p.cnt[4 * ((size_t)m - 1) + 3] : 0u;
+            if (PADDED) n_tok = (uint32_t)p.cnt[4 * ((size_t)m - k + nc - 1) + 3];
+        } else {
+            uint32_t before = 0, behind = 0;
+            for (int32_t j = lane; j < (PADDED ? nc : k); j += 64) {
+                const int4 part = *reinterpret_cast<const int4 *>(p.cnt + 4 * (size_t)(m - k + j));   // {unshared, after left seam, before right seam, -}
+                const uint32_t c = (uint32_t)(part.x + (j > 0 ? part.y : 0) + (j + 1 < nc ? part.z : 0));
+                if (j < k) before += c; else behind += c;
+            }
+            base = (uint32_t)__builtin_amdgcn_readlane((int)wave_inclusive_sum_u32(before), 63);
+            if (PADDED) n_tok = base + (uint32_t)__builtin_amdgcn_readlane((int)wave_inclusive_sum_u32(behind), 63);
         }
         if (failed) continue;                              // (the same for the whole wave)
-        const uint32_t base = (uint32_t)__builtin_amdgcn_readlane((int)wave_inclusive_sum_u32(before), 63);
         const int64_t lo = k > 0 ? (int64_t)seam_l : 0, hi = k + 1 < nc ? (int64_t)seam_r : len;
         // which of the lane's positions lie in [lo, hi) and start a token
         const int64_t p0 = e0 + lane * 32;
@@ -927,7 +987,6 @@ __global__ __launch_bounds__(1024) void bpe_auto_join_kernel(
             for (uint32_t t = lane; t < total; t += 64) out[t] = id ? id[compact[t]] : (int32_t)compact[t];
             if (lane == 0 && k + 1 == nc) lengths[row] = (int32_t)(base + total);
         } else {
-            const uint32_t n_tok = base + (uint32_t)__builtin_amdgcn_readlane((int)wave_inclusive_sum_u32(behind), 63);
             const int64_t stride = a.pad_stride, at0 = (int64_t)row * stride;
             const int64_t kept = (int64_t)n_tok < stride ? (int64_t)n_tok : stride, shift = a.pad_left ? stride - kept : 0;
             const int64_t put = kept - (int64_t)base < (int64_t)total ? kept - (int64_t)base : (int64_t)total;

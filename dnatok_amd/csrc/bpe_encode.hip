@@ -2623,10 +2623,15 @@ static int bpe_encode_launch(const dnatok_bpe_t *t, const uint8_t *bytes, const 
                 const int64_t chunk_groups = p.max_mc < 448 ? p.max_mc : 448;
                 const int grid = (int)(p.n_slabs + chunk_groups);
                 const int count_longest = a.pad_ids && a.longest && n_rows <= kAutoListRows ? 1 : 0;
-                if (a.pad_ids)
-                    bpe_auto_join_kernel<true><<<grid, 1024, 0, s>>>(a, id, bytes, offsets, n_rows, max_len, p, count_longest, tok_tmp, lengths);
-                else
-                    bpe_auto_join_kernel<false><<<grid, 1024, 0, s>>>(a, id, bytes, offsets, n_rows, max_len, p, 0, tok_tmp, lengths);
+                const int scan_from = scan_from_chunks(a.pad_ids != nullptr);
+                const bool scanned = (max_len + p.core - 1) / p.core >= scan_from;
+                if (scanned) {
+                    bpe_row_scan_kernel<<<(int)((n_rows + kScanRows - 1) / kScanRows), 1024, 0, s>>>(offsets, n_rows, scan_from, p);
+                    DNATOK_HIP_TRY(hipGetLastError());
+                }
+                const auto join = a.pad_ids ? (scanned ? bpe_auto_join_kernel<true, true> : bpe_auto_join_kernel<true, false>)
+                                            : (scanned ? bpe_auto_join_kernel<false, true> : bpe_auto_join_kernel<false, false>);
+                join<<<grid, 1024, 0, s>>>(a, id, bytes, offsets, n_rows, max_len, p, count_longest, tok_tmp, lengths);
                 DNATOK_HIP_TRY(hipGetLastError());
                 if (a.pad_ids && a.longest && !count_longest) {
                     bpe_longest_kernel<<<1, 1024, 0, s>>>(lengths, n_rows, a.longest);

@@ -1201,6 +1201,60 @@ def call_us(call, reps=20):
     return best
 
 
+@pytest.mark.parametrize("others", [2, 300])
+def test_bpe_rows_of_a_thousand_chunks(bpe, others):
+    """Rows of so many chunks that their counts are scanned by a launch of their own, beside short rows
+    (with up to 256 rows and with more: the chunks' places come from the kernel or from the work list),
+    rows just below that, and one that is redone whole: plain, padded, and padded with a stride that
+    cuts rows off."""
+    which, enc, bo = bpe
+    say(f"bpe{which} rows of a thousand chunks, {others} others")
+    rng = np.random.default_rng(others)
+    rnd = lambda n: np.frombuffer(b"ACGT", dtype=np.uint8)[rng.integers(0, 4, n)].tobytes().decode()
+    seqs = [rnd(2_000_000), rnd(100), rnd(1792 * 1023), "", rnd(4_000_000), rnd(1792 * 1024 - 5)]
+    seqs += [rnd(int(n)) for n in rng.integers(0, 5000, others)]
+    seqs[6] = rnd(2000) + "AACCT" * 800 + rnd(500)
+    b = util.batch_from_strings(seqs)
+    ref = bo.encode_batch(b.data, b.offsets)
+    for i, r in enumerate(bpe_rows(enc, b)):
+        np.testing.assert_array_equal(r, ref[i], err_msg=f"row {i}")
+    data, off = to_dev(b)
+    most = max(r.size for r in ref)
+    for stride, pad_left in ([(most + 3, False), (most - 100_000, True)] if others < 10 else []) + [(2000, False), (1501, True)]:
+        ids, mask, lengths, longest = enc.encode_padded(data, off, 4_000_000, stride, 7, pad_left=pad_left)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(lengths.cpu().numpy(), [r.size for r in ref])
+        assert int(longest.item()) == most
+        eids, emask = O.pad_rows(ref, 7, stride, pad_left=pad_left, dtype=np.int32)
+        np.testing.assert_array_equal(ids.cpu().numpy(), eids)
+        np.testing.assert_array_equal(mask.cpu().numpy(), emask)
+
+
+def test_bpe_a_chromosome_in_one_row():
+    """A row of 64 million bases is padded in no more time by the automaton than by the merge engine
+    (which a set chunk geometry selects): 1.6 ms against 1.4 while every chunk added up the counts of
+    all of the row's 35,715 chunks.  Both give the same tokens."""
+    cfg = util.tokenizer_json("4096")
+    kv = bpe_vocab.KernelVocab(bpe_vocab.split_merges(cfg["model"]["merges"]))
+    enc = encoders.BpeEncoder(kv.pair_a, kv.pair_b, kv.new_id, len(kv))
+    n, stride = 64_000_000, 20_000_000
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(3)
+    data = torch.tensor(list(b"ACGT"), dtype=torch.uint8, device=DEV)[torch.randint(0, 4, (n,), generator=gen, device=DEV)]
+    off = torch.tensor([0, n], dtype=torch.int64, device=DEV)
+    tok = torch.empty(n, dtype=torch.int32, device=DEV)
+    times, results = [], []
+    for geometry in ((1792, 128), (0, 0)):
+        enc.set_chunk_geometry(*geometry)
+        out = enc.encode_padded(data, off, n, stride, 3, tok_tmp=tok)
+        results.append(out)
+        times.append(call_us(lambda: enc.encode_padded(data, off, n, stride, 3, tok_tmp=tok, out=out), 2))
+    say(f"a row of 64 Mbp, padded: merge engine {times[0]:.0f} us, automaton {times[1]:.0f} us")
+    for x, y in zip(*results):
+        assert torch.equal(x, y)
+    assert times[1] < times[0], times
+
+
 def test_bpe_calls_behind_other_kernels():
     """Calls whose tables other kernels have pushed out of the caches are no slower by the automaton than
     by the merge engine (which a set chunk geometry selects), with a tenth for the measurement: 64 reads of
