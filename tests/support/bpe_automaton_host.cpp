@@ -2,15 +2,19 @@
 #include "../../dnatok_amd/csrc/bpe_automaton.hpp"
 
 extern "C" void *automaton_create(const int32_t *byte_to_sym, const int32_t *a, const int32_t *b, const int32_t *product,
-                                  const uint8_t *in_effect, int32_t n_merges, int32_t n_symbols)
+                                  const uint8_t *in_effect, int32_t n_merges, int32_t n_symbols,
+                                  int64_t max_states)
 {
     dnatok::BpeAutomaton *fa = new dnatok::BpeAutomaton();
-    if (dnatok::build_bpe_automaton(byte_to_sym, a, b, product, in_effect, n_merges, n_symbols, fa)) return fa;
+    if (dnatok::build_bpe_automaton(byte_to_sym, a, b, product, in_effect, n_merges, n_symbols, fa,
+                                    max_states ? (size_t)max_states : dnatok::kAutoMaxStates)) return fa;
     delete fa;
     return nullptr;
 }
 
 extern "C" void automaton_destroy(void *h) { delete (dnatok::BpeAutomaton *)h; }
+
+extern "C" int64_t automaton_max_states() { return (int64_t)dnatok::kAutoMaxStates; }
 
 extern "C" int64_t automaton_states(const void *h) { return ((const dnatok::BpeAutomaton *)h)->n_states; }
 

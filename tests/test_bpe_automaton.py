@@ -23,18 +23,19 @@ def lib(tmp_path_factory):
     so = ctypes.CDLL(path)
     so.automaton_create.restype = ctypes.c_void_p
     so.automaton_states.restype = ctypes.c_int64
+    so.automaton_max_states.restype = ctypes.c_int64
     so.automaton_encode.restype = ctypes.c_int64
     return so
 
 
 class Automaton:
-    def __init__(self, lib, pair_a, pair_b, new_id, n_symbols):
+    def __init__(self, lib, pair_a, pair_b, new_id, n_symbols, max_states=0):
         self.lib, self.b2s = lib, np.arange(256, dtype=np.int32)
         a, b, p = (np.ascontiguousarray(x, dtype=np.int32) for x in (pair_a, pair_b, new_id))
         last = {(int(x), int(y)): i for i, (x, y) in enumerate(zip(a, b))}
         eff = np.array([last[(int(x), int(y))] == i for i, (x, y) in enumerate(zip(a, b))], dtype=np.uint8)
         self.h = lib.automaton_create(O._p(self.b2s), O._p(a), O._p(b), O._p(p), O._p(eff), ctypes.c_int32(a.size),
-                                      ctypes.c_int32(n_symbols))
+                                      ctypes.c_int32(n_symbols), ctypes.c_int64(max_states))
 
     def encode(self, row):
         row = np.ascontiguousarray(row, dtype=np.uint8)
@@ -122,3 +123,13 @@ def test_tables_without_an_automaton(lib):
     assert make(doubled[:7]) and not make(doubled)
     b2 = Automaton(lib, [65, 67], [67, 71], [256, 256], 257)         # one symbol for two texts
     assert not b2.h
+
+
+def test_limit_of_states(lib):
+    """As many states as the limit allows are built, one more is not (the shipped limit is the one the
+    kernels were measured to)."""
+    bo = util.bpe_oracle("4096")
+    tables = (bo.pair_a, bo.pair_b, bo.new_id, len(bo.vocab))
+    n = lib.automaton_states(ctypes.c_void_p(Automaton(lib, *tables).h))
+    assert lib.automaton_max_states() == 1 << 19
+    assert Automaton(lib, *tables, max_states=n).h and not Automaton(lib, *tables, max_states=n - 1).h
