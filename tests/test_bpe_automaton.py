@@ -130,6 +130,7 @@ def test_limit_of_states(lib):
     kernels were measured to)."""
     bo = util.bpe_oracle("4096")
     tables = (bo.pair_a, bo.pair_b, bo.new_id, len(bo.vocab))
-    n = lib.automaton_states(ctypes.c_void_p(Automaton(lib, *tables).h))
+    fa = Automaton(lib, *tables)
+    n = lib.automaton_states(ctypes.c_void_p(fa.h))
     assert lib.automaton_max_states() == 1 << 19
     assert Automaton(lib, *tables, max_states=n).h and not Automaton(lib, *tables, max_states=n - 1).h
