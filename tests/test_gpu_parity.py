@@ -731,14 +731,19 @@ def test_kmer_missing_windows_without_expansion(kmer_kernel_choice):
 
 # ------------------------------------------------------------------- BPE
 
-@pytest.fixture(scope="module", params=["4096", "32000"])
+@pytest.fixture(scope="module", params=["4096", "32000", "4096-merges"])
 def bpe(request):
-    which = request.param
+    """The trained vocabularies, which run on the automaton in its narrow (transitions in LDS) and its
+    wide form, and one that runs on the merge engine: a rule between two further bytes, which no row
+    of these tests has, is enough for a table to have no automaton."""
+    which, _, merges = request.param.partition("-")
     cfg = util.tokenizer_json(which)
+    if merges:
+        cfg = {**cfg, "model": {**cfg["model"], "merges": list(cfg["model"]["merges"]) + [["#", "%"]]}}
     kv = bpe_vocab.KernelVocab(bpe_vocab.split_merges(cfg["model"]["merges"]))
     remap = kv.remap_to(cfg["model"]["vocab"], cfg["model"]["vocab"]["[UNK]"])
     enc = encoders.BpeEncoder(kv.pair_a, kv.pair_b, kv.new_id, len(kv), out_remap=remap)
-    return which, enc, util.bpe_oracle(which)
+    return which, enc, O.bpe_oracle_from_tokenizer_json(cfg) if merges else util.bpe_oracle(which)
 
 
 def bpe_rows(enc, b: wl.Batch):
@@ -952,10 +957,11 @@ def check_padded(enc, bo, seqs, stride, *, remap_h=None, want_mask=True, want_lo
 
 def test_bpe_padded_in_one_pass(bpe):
     """dnatok_bpe_encode_padded: ids, mask, lengths and the longest row as dnatok_bpe_encode followed by
-    dnatok_pad_rows give them, on every route: one row per team, more rows than teams (the work
-    list), every LDS capacity, rows cut by a stride that is too small, empty rows and an empty
-    batch, a second id map or none, a mask or none, and batches with rows long enough to be cut into
-    chunks (assembled in the token buffer first)."""
+    dnatok_pad_rows give them, on every route of the automaton and of the merge engine (whose routes
+    the sizes are chosen by): one row per team, more rows than teams (the work list), every LDS
+    capacity, rows cut by a stride that is too small, empty rows and an empty batch, a second id map
+    or none, a mask or none, and batches with rows long enough to be cut into chunks (which the merge
+    engine assembles in the token buffer first, the automaton's chunks are put together in place)."""
     which, enc, bo = bpe
     say(f"bpe{which} padded in one pass")
     rng = random.Random(5)
@@ -981,7 +987,7 @@ def test_bpe_padded_in_one_pass(bpe):
     # several calls in a row on one stream share the tree that carries the longest row; a smaller batch after a larger one
     check_padded(enc, bo, many[:1500], 256, ref=ref[:1500])
     check_padded(enc, bo, many[:3], 256, ref=ref[:3])
-    # rows that are cut into chunks, or redone by the whole-row kernel: through the token buffer
+    # rows that are cut into chunks, or redone whole
     long_rows = wl.config5_ragged(40, seed=12).strings() + ["", rnd(5000), "A" * 9000, rnd(20_001)]
     ref = check_padded(enc, bo, long_rows, 6000, remap_h=remap_h)
     check_padded(enc, bo, long_rows, 300, ref=ref)
@@ -991,8 +997,9 @@ def test_bpe_padded_in_one_pass(bpe):
 @pytest.mark.parametrize("pad_left", [False, True])
 def test_bpe_padded_in_every_layout(bpe, dtype, pad_left):
     """dnatok_bpe_encode_padded_as: the engine's launch writes the final tensor -- any id width, the
-    padding on either side -- for rows it takes whole (every team shape, one row per team and a work
-    list) and, through the token buffer, for rows that are cut into chunks.  Expected: the oracle's
+    padding on either side -- for rows it takes whole (the merge engine: every team shape, one row per
+    team and a work list) and for rows that are cut into chunks (the merge engine: through the token
+    buffer).  Expected: the oracle's
     rows padded by the oracle's pad_rows with the same options (a row with more tokens than the
     stride keeps its first ones on either side)."""
     which, enc, bo = bpe
@@ -1027,7 +1034,7 @@ def test_bpe_padded_in_every_layout(bpe, dtype, pad_left):
 
 
 def test_bpe_padded_on_two_streams_and_in_a_graph(bpe):
-    """Every stream has its own tree; replays of a captured call give the eager result each time,
+    """Every stream has its own tree for the longest row; replays of a captured call give the eager result each time,
     with eager calls (which use the same tree) in between."""
     which, enc, bo = bpe
     say(f"bpe{which} padded: streams and graph")
@@ -1065,9 +1072,9 @@ def test_bpe_padded_on_two_streams_and_in_a_graph(bpe):
 
 
 def test_bpe_more_rows_of_about_one_length_than_teams(bpe):
-    """A batch of more rows than resident teams whose rows are about equally long is dealt in the
-    rows' given order, without the sorted work list: tokens as the oracle's, through the plain call
-    and through the one that pads."""
+    """A batch of more rows than the merge engine has resident teams whose rows are about equally long is
+    dealt in the rows' given order, without the sorted work list: tokens as the oracle's, through the
+    plain call and through the one that pads."""
     which, enc, bo = bpe
     say(f"bpe{which} rows of one length, dealt in order")
     rng = random.Random(23)
@@ -1081,8 +1088,9 @@ def test_bpe_more_rows_of_about_one_length_than_teams(bpe):
 
 @pytest.mark.parametrize("longest", [250, 380, 500])
 def test_bpe_many_short_rows_a_wave_each(bpe, longest):
-    """Batches whose rows are at most 256 / 384 / 512 bytes long go to teams of one wave (four rows to a
-    workgroup), more rows than teams through several work counters: every row as the oracle has it,
+    """Batches whose rows are at most 256 / 384 / 512 bytes long go, in the merge engine, to teams of one
+    wave (four rows to a workgroup), more rows than teams through several work counters, and several to
+    a wave's lanes in the automaton: every row as the oracle has it,
     through the plain call, the one that pads, and the one that also writes the single-character ids;
     a few rows only, empty rows, rows of one length (dealt in order) and ragged ones."""
     which, enc, bo = bpe
@@ -1331,8 +1339,9 @@ def test_bpe_long_rows_padded_by_their_chunks(bpe, count, pad_left, dtype):
 
 @pytest.mark.parametrize("long_ones", ["up to 1 KB", "up to 2 KB", "cut into chunks"])
 def test_bpe_mostly_short_rows_with_some_long_ones(bpe, long_ones):
-    """A batch of mostly short rows with a few long ones among them is split between two launches (the
-    shortest class of the work list to teams of one wave, the rest to 256-thread teams): every row as
+    """A batch of mostly short rows with a few long ones among them is split by the merge engine between
+    two launches (the shortest class of the work list to teams of one wave, the rest to 256-thread
+    teams), and packed into items by the rows' mean length by the automaton: every row as
     the oracle has it, through the plain call, the one that pads (whose longest row then comes from
     the lengths) and the one that also writes the single-character ids."""
     which, enc, bo = bpe
@@ -1394,8 +1403,9 @@ def test_bpe_rows_without_a_seam_fall_back_to_the_whole_row_kernel(bpe):
 
 def test_bpe_long_runs_of_equal_pairs(bpe):
     """Rows in which every pair has the rank of its neighbour for thousands of positions (a
-    homopolymer, a tandem repeat after its first merges): the left chain of a candidate would be
-    as long as the run, so such rounds decide by a scan over the positions instead of walking.
+    homopolymer, a tandem repeat after its first merges): in the merge engine the left chain of a
+    candidate would be as long as the run, so such rounds decide by a scan over the positions instead
+    of walking.
     100 kbp rows go through chunks, seams and, where no seam is accepted, the whole-row kernel."""
     which, enc, bo = bpe
     say(f"bpe{which} long runs of equal pairs")
@@ -1412,8 +1422,8 @@ def test_bpe_long_runs_of_equal_pairs(bpe):
 
 @pytest.mark.parametrize("core,overlap", [(256, 32), (512, 96), (300, 35), (700, 160)])
 def test_bpe_small_chunks_many_seams_and_fallbacks(bpe, core, overlap):
-    """The chunk / seam / gather / whole-row-fallback machinery with chunks far smaller than the
-    shipped ones: a few thousand ragged, random and tandem-repeat rows per vocabulary go through tens
+    """The chunk / seam / gather / whole-row-fallback machinery of the merge engine (a set geometry
+    selects it) with chunks far smaller than the shipped ones: a few thousand ragged, random and tandem-repeat rows per vocabulary go through tens
     of thousands of seams, many of which find no position and send their row to the whole-row
     kernel.  Every row is compared with the oracle.  (300, 35): a chunk of 370 symbols is no whole
     number of 16-byte loads, which takes the gather's general form instead of the one that holds
@@ -1450,8 +1460,9 @@ def test_bpe_small_chunks_many_seams_and_fallbacks(bpe, core, overlap):
 
 def test_bpe_compact_table_in_lds_gives_the_same_tokens():
     """The 4096 vocabulary has a compact form that workgroups keep in LDS for batches of short rows
-    that leave the room (not the default: it measured slower).  Same tokens as with the table in
-    global memory and as the oracle: a batch small enough for one row per resident workgroup, and the C3
+    that leave the room (a choice of the merge engine, not the default: it measured slower).  Same tokens
+    as with the table in global memory (the merge engine without the compact form: a set chunk geometry,
+    the shipped one, selects it), as the automaton's and as the oracle: a batch small enough for one row per resident workgroup, and the C3
     batch with the compact form forced."""
     from dnatok_amd import _lib
     say("bpe4096 compact table in LDS")
@@ -1473,8 +1484,9 @@ def test_bpe_compact_table_in_lds_gives_the_same_tokens():
     split = util.batch_from_strings(split_seqs)
     want_split = [np.asarray(r) for r in bo.encode_batch(split.data, split.offsets)]
     try:
-        for mode in (0, 1, 2):
-            enc.set_table_placement(mode)
+        for mode in ("automaton", "global memory", 1, 2):
+            enc.set_chunk_geometry(*((1792, 128) if mode == "global memory" else (0, 0)))
+            enc.set_table_placement(mode if mode in (1, 2) else 0)
             for s, r, e in zip(seqs, bpe_rows(enc, small), want):
                 np.testing.assert_array_equal(r, e, err_msg=f"mode {mode}: {s[:20]}")
             util.check_against_golden("C3_bpe4096", bpe_rows(enc, wl.config3_bpe4096()))
