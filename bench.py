@@ -296,8 +296,8 @@ class KmerPadded(Workload):
 
 
 class BpePadded(Workload):
-    """C3 / C4: BPE encode, remap, pad to the longest row, mask.  Rows that the engine takes whole
-    (C3) are padded by the engine itself while it writes them out (dnatok_bpe_encode_padded), the
+    """C3 / C4: BPE encode, remap, pad to the longest row, mask.  Rows that are encoded whole
+    (C3) are padded by the same launch while it writes them out (dnatok_bpe_encode_padded), the
     rows as far apart as the stream's width guess says (encoders.WidthGuess, fed by the set-up
     call); rows that are cut into chunks (C4) are assembled first and padded by a launch of its own."""
 
@@ -335,7 +335,7 @@ class BpePadded(Workload):
                         torch.empty((self.n_rows, length), dtype=torch.uint8, device="cuda"),
                         torch.empty(1, dtype=torch.int32, device="cuda"))
         self.bases = host.size
-        self.kernel = "bpe_lds_kernel" if length <= 4096 else "bpe_long_kernel"
+        self.kernel = "bpe_auto_kernel"
         self.name = (f"{'C3' if which == '4096' else 'C4'} BPE vocab-{which}, {rows}x{length} bp batches, "
                      f"{n_batches} distinct batch(es) per call, pad to longest row")
         self.one_pass = False
@@ -447,7 +447,7 @@ class RaggedBoth(Workload):
         self.cids = torch.empty(total, dtype=torch.int32, device="cuda")
         self.cmask = torch.empty(total, dtype=torch.uint8, device="cuda")
         self.bases = total
-        self.kernel = "bpe_lds_kernel"
+        self.kernel = "bpe_auto_kernel"
         self.name = (f"C5 ragged, {n_batches} x 4096 sequences ({total / 1e6:.1f} Mbp) per call: BPE vocab-4096 + char in one pass over the bytes, "
                      f"packed ids/offsets/masks")
         self.step()
@@ -1044,8 +1044,9 @@ PHASE_NAMES = ["initial_pairs", "round_minimum", "collect_candidates", "decide",
 
 
 def bpe_phase_cycles_extra():
-    """Where the teams of the BPE engine spend their cycles, phase by phase, on the three BPE
-    configurations: from the build of the library with the phase clocks compiled in
+    """Where the teams of the BPE merge engine spend their cycles, phase by phase, on the three BPE
+    configurations (whose vocabularies the product encodes by automaton; this build has none, so that its
+    tables run on the merges, as tables without an automaton do): from the build of the library with the phase clocks compiled in
     (libdnatok_hip_phases.so, which this process loads in place of the product library: run with
     --only-extra bpe_phase_cycles, nothing else in the line is then the product's).  The shares are
     what thread 0 of each team saw, barriers counted with the phase they end."""
@@ -1076,11 +1077,12 @@ def bpe_phase_cycles_extra():
 
 
 def merge_table_placement_extra():
-    """The BPE merge table of the 4096 vocabulary in global memory (L2; the default) against its compact
-    48 KB form kept in LDS by every workgroup (`dnatok_bpe_table_set_placement`), on batches of 1 KB rows:
-    512 rows (one per workgroup resident with the table in LDS) and the C3 batch of 1024 rows (two rounds
-    of workgroups with the table in LDS).  Tokens compared between the placements and, for C3, with the
-    golden vectors."""
+    """The merge engine with the merge table of the 4096 vocabulary in global memory (L2; a set chunk
+    geometry, the shipped one, selects the engine) against its compact 48 KB form kept in LDS by every
+    workgroup (`dnatok_bpe_table_set_placement`), on batches of 1 KB rows: 512 rows (one per workgroup
+    resident with the table in LDS) and the C3 batch of 1024 rows (two rounds of workgroups with the table
+    in LDS); beside them the automaton, which these batches get when nothing is set.  Tokens compared
+    between the three and, for C3, with the golden vectors."""
     import torch
     from dnatok_amd import _lib, bpe_vocab, encoders
     from tests.golden import check as util
@@ -1099,8 +1101,9 @@ def merge_table_placement_extra():
             tok = torch.empty(b.total, dtype=torch.int32, device="cuda")
             lengths = torch.empty(rows, dtype=torch.int32, device="cuda")
             seen = {}
-            for name, mode in (("global_memory", 0), ("lds", 2)):
+            for name, mode, geometry in (("automaton", 0, (0, 0)), ("global_memory", 0, (1792, 128)), ("lds", 2, (0, 0))):
                 place(mode)
+                enc.set_chunk_geometry(*geometry)
                 enc.encode(data, off, 1024, tok_tmp=tok, lengths=lengths)
                 torch.cuda.synchronize()
                 ln = lengths.cpu().numpy()
@@ -1112,11 +1115,13 @@ def merge_table_placement_extra():
                         enc.encode(data, off, 1024, tok_tmp=tok, lengths=lengths)
                 _, dm = time_steps(W(), 20, 3)
                 out[f"{rows}_rows_{name}_us"] = dm * 1e3
-            same_rows(seen["lds"], seen["global_memory"], f"merge table placement, {rows} rows")
+            for name in ("global_memory", "automaton"):
+                same_rows(seen["lds"], seen[name], f"merge table placement, {rows} rows, {name}")
             if rows == 1024:
                 util.check_against_golden("C3_bpe4096", seen["lds"])
     finally:
         place(0)
+        enc.set_chunk_geometry(0, 0)
     return out
 
 

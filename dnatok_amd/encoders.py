@@ -444,7 +444,7 @@ class KmerEncoder:
 
 
 class BpeEncoder:
-    """BPE merge engine + packer (C ABI: dnatok_bpe_*, dnatok_pack_ragged, dnatok_pad_rows)."""
+    """BPE by automaton or merge engine, and the packer (C ABI: dnatok_bpe_*, dnatok_pack_ragged, dnatok_pad_rows)."""
 
     def __init__(self, pair_a, pair_b, new_id, n_symbols: int, byte_to_id=None, out_remap=None):
         self.pair_a = np.ascontiguousarray(pair_a, dtype=np.int32)
@@ -504,8 +504,8 @@ class BpeEncoder:
         ``longest[1]`` (their maximum; None with ``want_longest=False`` or in ``out``: the caller takes it
         from the lengths), all on the device.  A row with more tokens than ``stride``
         keeps its first ``stride``: compare ``longest`` with it.  ``out`` = (ids, mask, lengths,
-        longest) reuses caller buffers.  Rows above ``padded_direct_max()`` bytes go through a token
-        buffer (``tok_tmp``, allocated here when not given)."""
+        longest) reuses caller buffers.  Rows above ``padded_direct_max()`` bytes need a token buffer
+        to work in (``tok_tmp``, allocated here when not given)."""
         _require_cuda(data, torch.uint8, "data")
         _require_cuda(offsets, torch.int64, "offsets")
         n_rows = offsets.numel() - 1
@@ -540,13 +540,15 @@ class BpeEncoder:
 
     def set_chunk_geometry(self, core: int, overlap: int) -> None:
         """Test hook (``dnatok_bpe_table_set_chunk_geometry``): this encoder's calls cut long rows
-        into chunks of ``core`` bytes extended by ``overlap`` on both sides; (0, 0) = shipped."""
+        into chunks of ``core`` bytes extended by ``overlap`` on both sides, and run on the merge engine
+        whatever their lengths (the shipped 1792 and 128 included); (0, 0) = the shipped choice."""
         _lib.check(_lib.lib().dnatok_bpe_table_set_chunk_geometry(self._h, int(core), int(overlap)),
                    "dnatok_bpe_table_set_chunk_geometry")
 
     def set_table_placement(self, mode: int) -> None:
-        """Measurement hook (``dnatok_bpe_table_set_placement``): 0 = merge table in global memory
-        (default), 1 / 2 = its compact form in LDS where the batch allows."""
+        """Measurement hook (``dnatok_bpe_table_set_placement``): 0 = the shipped choice (the automaton
+        where the table has one, else the merge table in global memory), 1 / 2 = the merge engine, with
+        the compact form of its table in LDS where the batch allows."""
         _lib.check(_lib.lib().dnatok_bpe_table_set_placement(self._h, int(mode)), "dnatok_bpe_table_set_placement")
 
     def encode_with_chars(self, data: torch.Tensor, offsets: torch.Tensor, max_len: int, char_lut: torch.Tensor, *,

@@ -209,8 +209,9 @@ int dnatok_kmer_encode_packed(const dnatok_kmer_t *t, const uint8_t *bytes, cons
  * (src/gputok_bpe_backend.py:451-466, 581).  n_symbols <= 65535, n_merges <= 65534.
  * A table whose rules are in order (no rule's product is used by a lower-ranked rule) and name at
  * most four bytes is also turned into a finite automaton here, which its calls then run on (a
- * vocabulary of 4,096 tokens: 6 ms, of 32,000: about 140 ms and 7 MB of device memory); any other
- * table's calls run the merges.  The results are the same. */
+ * vocabulary of 4,096 tokens: 6 ms and 0.14 MB of device memory, of 32,000: about 140 ms and 3.8 MB,
+ * of 60,000: 300 to 450 ms and 6 to 11 MB); any other table's calls run the merges.  The results are the
+ * same. */
 int  dnatok_bpe_table_create(const int32_t *byte_to_id_h, const int32_t *pair_a_h,
                              const int32_t *pair_b_h, const int32_t *new_id_h, int32_t n_merges,
                              int32_t n_symbols, const int32_t *out_remap_h, dnatok_bpe_t **out);
@@ -310,18 +311,20 @@ int dnatok_bpe_encode_static(const dnatok_bpe_t *t, const uint8_t *bytes, const 
  * longer than core + 2 * overlap bytes with: chunks of `core` bytes, extended by `overlap` bytes on
  * both sides, joined at seams inside the overlaps.  The shipped geometry is (1792, 128); (0, 0)
  * restores it.  Tests pass small chunks so that rows of a few kilobytes go through thousands of
- * seams and whole-row fallbacks.  Results never depend on the geometry.  The setting belongs to the
- * table object; a call reads it once when it starts (size the scratch buffer after setting it). */
+ * seams and whole-row fallbacks.  Any set geometry, the shipped one included, also selects the merge
+ * engine for a table that has an automaton.  Results never depend on the geometry.  The setting belongs
+ * to the table object; a call reads it once when it starts (size the scratch buffer after setting it). */
 int dnatok_bpe_table_set_chunk_geometry(dnatok_bpe_t *t, int32_t core, int32_t overlap);
 
 /* MEASUREMENT ONLY: where the merge table of the calls with this table object is kept (no
  * counterpart in the reference, whose kernel reads its hash table from global memory,
  * dnatok_bpe.cu:822-837).  A table of at most 8192 symbols and 4095 rules also has a compact form
  * of 48 KB.  mode 0 (default): the shipped choice (the automaton where the table has one; the merges
- * read their table from global memory, L2).  mode 1: a batch of rows of at most 1024 bytes, few enough for one row per resident
- * workgroup with those 48 KB added to each, is encoded by workgroups that keep the compact form in
- * LDS.  mode 2: the compact form for every batch of rows of at most 1024 bytes that one launch
- * encodes whole.  Results are identical in all modes. */
+ * read their table from global memory, L2).  Modes 1 and 2 select the merge engine.  mode 1: a batch of
+ * rows of at most 1024 bytes, few enough for one row per resident workgroup with those 48 KB added to
+ * each, is encoded by workgroups that keep the compact form in LDS.  mode 2: the compact form for every
+ * batch of rows of at most 1024 bytes that one launch encodes whole.  Results are identical in all
+ * modes. */
 int dnatok_bpe_table_set_placement(dnatok_bpe_t *t, int32_t mode);
 
 /* ---------------------------------------------------------------------------------------
