@@ -33,9 +33,9 @@
 // 1 KB 54.7 -> 29.2 us, 100,000 reads 123 -> 57 us.  (That includes the walk into the next region four bytes
 // at a time, comparing the last of the four, and the padded rows of a wave written as one run of cells.)
 //
-// Per call, the merge engine -> the automaton: 1,024 rows of 1 KB 29.4 -> 11.7 us, 16,384 of them 236.5 ->
-// 29.2 us, 100,000 reads of 100 - 300 bp (int64 rows) 349 -> 57 us, 4,096 ragged reads of 12 Mbp 253.5 ->
-// 83.9 us (all with the vocabulary of 4,096), 32 rows of 100 kbp (32,000) 143.8 -> 74.3 us.
+// Per call, the merge engine -> the automaton: 1,024 rows of 1 KB 29.4 -> 11.6 us, 16,384 of them 236.5 ->
+// 29.1 us, 100,000 reads of 100 - 300 bp (int64 rows) 349 -> 56.5 us, 4,096 ragged reads of 12 Mbp 253.5 ->
+// 80.2 us (all with the vocabulary of 4,096), 32 rows of 100 kbp (32,000) 143.8 -> 60.5 us.
 #pragma once
 
 namespace dnatok {
