@@ -2416,17 +2416,17 @@ int launch_auto_as(const dnatok_bpe_t *t, const BpeArgs &a, AutoArgs aa, const u
     aa.window = Lds::window(t->auto_states);
     static const int64_t resident = resident_workgroups(kern, 64 * kAutoMaxWaves, kAutoLdsBytes, 1);
     if (!CHUNKS) {
-        // as many rows to an item as give every wave the same number of items, if that is more: a wave
-        // takes them in as few steps as they fit, and no wave starts an item when the others are done
-        // (100,000 reads, items of eight rows, 3.05 to a wave: 57.3 us; of 25 rows, one to a wave: 56.0 us; 16,384 rows of
-        // 1 KB 29.2 and 28.6 us)
+        // An item: as many rows as surely fit a wave (aa.rows), spread over the CUs when there are fewer than that; or as
+        // many as give every wave one item, up to 64, if that is more: a wave takes them in as few steps as they fit,
+        // and none starts an item when the others are done.  (Vocabulary of 4,096, as many rows as surely fit / as many
+        // as give every wave its share: 4,000 rows of 200 bases 12.7 / 13.8 us, 18,000 16.9 / 18.1, 100,000 reads 57.3 /
+        // 56.0; 64 reads of 100 bases by 8 workgroups / by 64: 11.1 / 10.3 us, with the vocabulary of 32,000 12.1 / 11.3,
+        // its table in no L2 26.3 / 22.5.  As many rows as fit by their mean length, 20,000 reads of 100 - 300 bases:
+        // 23.1 us, their share 18.7: a wave whose rows do not fit takes two steps.)
         const int64_t all = resident * waves, turns = (n_rows + 64 * all - 1) / (64 * all);
-        const int64_t even = (n_rows + turns * all - 1) / (turns * all);
-        if (even > aa.rows) aa.rows = (int32_t)even;
-        // a batch that is smaller than that, its walks in global memory: a wave on as many CUs as there are rows (64 reads of
-        // 100 bp, vocabulary of 32,000: 12.1 -> 11.3 us, with the table in no L2 26.3 -> 22.5 us; the narrow form is left as
-        // it is: each of its workgroups brings the table into LDS)
-        if (WIDE && n_rows < resident * aa.rows) aa.rows = (int32_t)((n_rows + resident - 1) / resident);
+        const int64_t share = (n_rows + turns * all - 1) / (turns * all), spread = (n_rows + resident - 1) / resident;
+        if (aa.rows > spread) aa.rows = (int32_t)spread;
+        if (aa.rows < share) aa.rows = (int32_t)share;
         items = (n_rows + aa.rows - 1) / aa.rows;
         aa.n_groups = (int32_t)items;
     }
@@ -2457,19 +2457,16 @@ int run_auto(const dnatok_bpe_t *t, const BpeArgs &a, int chunking, const uint8_
         if (a.char_ids) return launch_auto_as<WIDE, 32, true, true, false>(t, a, aa, bytes, offsets, p, n_rows, p.max_items, tok_tmp, lengths, s);
         return launch_auto_as<WIDE, 32, true, false, false>(t, a, aa, bytes, offsets, p, n_rows, p.max_items, tok_tmp, lengths, s);
     }
-    // Regions of 32 bytes, of 16 when the batch is so small that its waves find a place at once either way
-    // (a lane's walk is then half as long, and twice the lanes share it).
-    // An item is as many rows as fit a wave for certain, or as many as nearly always fit it by the rows'
-    // mean length, if that is more (an item that does not fit takes two steps).
+    // Regions of 32 bytes, of 16 where a wave for every row or few rows then finds a place at once: their lanes' walks
+    // are half as long.  A wave's share of the rows has to fit its 64 lanes, surely or, by the rows' mean length, nearly
+    // always.  (Vocabulary of 4,096, regions of 16 / 32: 256 rows of 1 KB 11.6 / 13.5 us, 4,096 15.8 / 17.6, 4,400, two
+    // to some waves, 20.7 / 16.9; 16,000 rows of 200 bases, four to a wave, 52 lanes, 16.1 / 16.7, 18,000 21.9 / 16.7; reads
+    // of 100 - 300 bases, 12,000, 39 lanes on average, 15.8 / 17.8, 16,000, 52 lanes, 20.1 / 18.3.)
     const int64_t len = max_len < 1 ? 1 : (max_len > 2048 ? 2048 : max_len);
-    const auto rows_of = [&](int64_t region) {
-        const int64_t sure = 64 / ((len + region - 1) / region);
-        const int64_t mean = (total / n_rows) * 2 / region + 1;                // twice the lanes of a row, on average
-        const int64_t likely = 56 * 2 / (mean < 2 ? 2 : mean);
-        return sure > likely ? sure : (likely > 64 ? (int64_t)64 : likely);
-    };
-    const bool small = len <= 1024 && (n_rows + rows_of(16) - 1) / rows_of(16) <= 256 * kAutoMaxWaves;
-    aa.rows = (int32_t)rows_of(small ? 16 : 32);
+    const int64_t share = (n_rows + 256 * kAutoMaxWaves - 1) / (256 * kAutoMaxWaves);
+    const int64_t twice_lanes = (total / n_rows) * 2 / 16 + 1;                 // of a row of mean length, regions of 16
+    const bool small = len <= 1024 && (share * ((len + 15) / 16) <= 64 || share * twice_lanes <= 2 * 48);
+    aa.rows = (int32_t)(64 / (small ? (len + 15) / 16 : (len + 31) / 32));
     if (small) {
         if (a.pad_ids) return launch_auto_as<WIDE, 16, false, false, true>(t, a, aa, bytes, offsets, p, n_rows, n_rows, tok_tmp, lengths, s);
         if (a.char_ids) return launch_auto_as<WIDE, 16, false, true, false>(t, a, aa, bytes, offsets, p, n_rows, n_rows, tok_tmp, lengths, s);
@@ -2620,6 +2617,8 @@ static int bpe_encode_launch(const dnatok_bpe_t *t, const uint8_t *bytes, const 
             if (automaton) {
                 // (narrow: the chunks' tokens are the numbers of states instead of symbols)
                 const int32_t *const id = t->auto_wide ? a.out_remap : t->auto_id;
+                // (workgroups of sixteen chunks at a time, beside those for rows that are redone: at most 448; 32 rows of 100 kbp
+                // 26.4 us, with 192 26.9, with 1,024 31.3; eight rows of 4 Mbp 206, 234 and 240)
                 const int64_t chunk_groups = p.max_mc < 448 ? p.max_mc : 448;
                 const int grid = (int)(p.n_slabs + chunk_groups);
                 const int count_longest = a.pad_ids && a.longest && n_rows <= kAutoListRows ? 1 : 0;
