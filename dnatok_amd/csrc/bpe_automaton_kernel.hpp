@@ -453,343 +453,343 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
             lanes_to = (int)wave_inclusive_sum_u32((uint32_t)lanes_own);
         }
         for (int first = 0; first < item_rows;) {          // (chunks: one step)
-        int m = 1, r = 0, lane0 = 0, G = 64;
-        bool have = true;
-        int64_t start, len;
-        if (chunk) {
-            start = offsets[row];
-            len = offsets[row + 1] - start;
-        } else {
-            // rows [first, first + m) of the item; r: the lane's row, lane0 and G: that row's lanes
-            const int lanes_before = first > 0 ? __builtin_amdgcn_readlane(lanes_to, first - 1) : 0;
-            const uint64_t in_step = __ballot(lane >= first && lane < item_rows && lanes_to - lanes_before <= 64);
-            m = (int)__builtin_popcountll(in_step);
-            r = first;
-            for (int i = first; i + 1 < first + m; ++i)
-                if (lane >= __builtin_amdgcn_readlane(lanes_to, i) - lanes_before) r = i + 1;
-            G = __shfl(lanes_own, r);
-            lane0 = __shfl(lanes_to, r) - lanes_before - G;
-            have = lane < lane0 + G;                       // (lanes behind the last row's have none)
-            start = ((int64_t)__shfl((int)(row_at >> 32), r) << 32) | (uint32_t)__shfl((int)(uint32_t)row_at, r);
-            len = ((int64_t)__shfl((int)(row_len >> 32), r) << 32) | (uint32_t)__shfl((int)(uint32_t)row_len, r);
-            row = __shfl(row_id, r);
-        }
-        const int j = lane - lane0;                        // the lane's region within the row
-        const int s = j * P;                               // its first byte
-        int64_t e0 = 0, e1 = len;
-        if (chunk && t.list_here && lane == 0) {
-            p.rec[item] = make_int4(row, k, nc, (int)len);
-            if (k == 0) {
-                p.row_fail[row] = 0;
-                p.mc_off[row] = item;
+            int m = 1, r = 0, lane0 = 0, G = 64;
+            bool have = true;
+            int64_t start, len;
+            if (chunk) {
+                start = offsets[row];
+                len = offsets[row + 1] - start;
+            } else {
+                // rows [first, first + m) of the item; r: the lane's row, lane0 and G: that row's lanes
+                const int lanes_before = first > 0 ? __builtin_amdgcn_readlane(lanes_to, first - 1) : 0;
+                const uint64_t in_step = __ballot(lane >= first && lane < item_rows && lanes_to - lanes_before <= 64);
+                m = (int)__builtin_popcountll(in_step);
+                r = first;
+                for (int i = first; i + 1 < first + m; ++i)
+                    if (lane >= __builtin_amdgcn_readlane(lanes_to, i) - lanes_before) r = i + 1;
+                G = __shfl(lanes_own, r);
+                lane0 = __shfl(lanes_to, r) - lanes_before - G;
+                have = lane < lane0 + G;                       // (lanes behind the last row's have none)
+                start = ((int64_t)__shfl((int)(row_at >> 32), r) << 32) | (uint32_t)__shfl((int)(uint32_t)row_at, r);
+                len = ((int64_t)__shfl((int)(row_len >> 32), r) << 32) | (uint32_t)__shfl((int)(uint32_t)row_len, r);
+                row = __shfl(row_id, r);
             }
-        }
-        if (chunk) {
-            e0 = (int64_t)k * p.core - p.overlap < 0 ? 0 : (int64_t)k * p.core - p.overlap;
-            e1 = (int64_t)(k + 1) * p.core + p.overlap;
-            if (e1 > len) e1 = len;
-        }
-        const bool too_long = e1 - e0 > kRowMax;           // (longer than the caller declared)
-        const int n = have && !too_long && e1 > e0 ? (int)(e1 - e0) : 0;
-        const uint8_t *const src = bytes + start + e0;
-
-        // the region's bytes as codes; cnt: how many of its P positions the row has
-        const int cnt = n - s < 0 ? 0 : (n - s < P ? n - s : P);
-        uint32_t codes[P / 16], flags = 0;
-#pragma unroll
-        for (int q = 0; q < P / 16; ++q) {
-            auto_u32x4_a1 w = {0, 0, 0, 0};
-            if (cnt > 16 * q) {
-                const uint8_t *const at = src + s + 16 * q;
-                if (start + e0 + s + 16 * q + 16 <= t.total) {       // (bytes behind the row's end are read, but not behind the batch's)
-                    w = *reinterpret_cast<const auto_u32x4_a1 *>(at);
-                } else {
-                    uint8_t b[16];
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) b[i] = 16 * q + i < cnt ? at[i] : (uint8_t)0;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        w[i] = (uint32_t)b[4 * i] | ((uint32_t)b[4 * i + 1] << 8) | ((uint32_t)b[4 * i + 2] << 16) | ((uint32_t)b[4 * i + 3] << 24);
+            const int j = lane - lane0;                        // the lane's region within the row
+            const int s = j * P;                               // its first byte
+            int64_t e0 = 0, e1 = len;
+            if (chunk && t.list_here && lane == 0) {
+                p.rec[item] = make_int4(row, k, nc, (int)len);
+                if (k == 0) {
+                    p.row_fail[row] = 0;
+                    p.mc_off[row] = item;
                 }
             }
-            uint32_t foreign;
-            codes[q] = letter_codes16(w, t.letters, foreign);
-            flags |= foreign << (16 * q);
-        }
-        flags &= cnt >= 32 ? ~0u : (1u << cnt) - 1u;                 // (of the positions the row has)
-        const bool any_foreign = __ballot(flags != 0) != 0;
+            if (chunk) {
+                e0 = (int64_t)k * p.core - p.overlap < 0 ? 0 : (int64_t)k * p.core - p.overlap;
+                e1 = (int64_t)(k + 1) * p.core + p.overlap;
+                if (e1 > len) e1 = len;
+            }
+            const bool too_long = e1 - e0 > kRowMax;           // (longer than the caller declared)
+            const int n = have && !too_long && e1 > e0 ? (int)(e1 - e0) : 0;
+            const uint8_t *const src = bytes + start + e0;
 
-        // forward over the own region
-        Entry e = 0;
-        if (any_foreign) {
+            // the region's bytes as codes; cnt: how many of its P positions the row has
+            const int cnt = n - s < 0 ? 0 : (n - s < P ? n - s : P);
+            uint32_t codes[P / 16], flags = 0;
 #pragma unroll
-            for (int i = 0; i < P; ++i) {
-                e = step(e, (codes[i / 16] >> (2 * (i % 16))) & 3u);
-                if (flags >> i & 1u) e = other;
-                state[i * 64 + lane] = e;
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < P; ++i) {
-                e = step(e, (codes[i / 16] >> (2 * (i % 16))) & 3u);
-                state[i * 64 + lane] = e;
-            }
-        }
-        // and on into the regions to the right until the states are the same, four bytes at a time: once
-        // equal they stay equal, so the last of the four tells, and writing equal ones again does no
-        // harm (nor does a state behind the row's end, which nothing reads)
-        bool going = cnt == P;
-        for (int ahead = 1;; ++ahead) {
-            const int from = (lane + ahead) & 63;
-            uint32_t word = 0, next_word = 0, f2 = 0;
-            word = (uint32_t)__shfl((int)codes[0], from);
-            if (P == 32) next_word = (uint32_t)__shfl((int)codes[P / 16 - 1], from);
-            if (any_foreign) f2 = (uint32_t)__shfl((int)flags, from);
-            const int cnt2 = __shfl(cnt, from);
-            going = going && j + ahead < G && cnt2 > 0;
-            if (!__ballot(going)) break;
-            wave_phase();
-            if (__builtin_expect(ahead >= kRepeatsFrom / P, 0))
-                copy_repeats<P>(state, codes, flags, any_foreign, cnt, cnt2, lane, lane0, lane0 + G, ahead, e, going);
-            for (int i = 0; i < P; i += 4) {
-                if (going) {
-                    Entry *const at = state + i * 64 + lane + ahead;
-                    const Entry there = at[3 * 64];
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        e = step(e, (word >> (2 * q)) & 3u);
-                        if (any_foreign && (f2 >> q & 1u)) e = other;
-                        at[q * 64] = e;
-                    }
-                    going = e != there;
-                }
-                if (!__ballot(going)) break;
-                word >>= 8;
-                f2 >>= 4;
-                if (P == 32 && i == 12) word = next_word;
-            }
-        }
-        wave_phase();
-
-        // backward: token starts of the region as bits, first from the region's own end
-        auto state_at = [&](int pos) -> Entry { return state[(pos & (P - 1)) * 64 + lane0 + pos / P]; };
-        uint32_t starts = 0;
-        int entry = s + cnt, entry_end = s + cnt;          // where the walk comes into the region from the right (see border) ...
-        int border = s + cnt;                              // ... and where it leaves it: at s, or where the token begins that reaches over s;
-        int border_end = s + cnt;                          // that token's end (s itself, if none reaches over)
-        if (cnt == 0) border = border_end = n;
-        {
-            int pos = s + cnt;
-            while (pos > s) {
-                border_end = pos;
-                pos -= length_of(state[(pos - 1 - s) * 64 + lane]);
-                if (pos >= s) starts |= 1u << (pos - s);
-            }
-            if (cnt > 0) border = pos;                     // (an empty region: the row ends to its left)
-            if (cnt > 0 && pos == s) border_end = s;
-        }
-        const bool has_right = cnt > 0 && j + 1 < G && lane < 63;
-        int right_end;                                     // end of the token that reaches over the region's end
-        for (;;) {
-            const int told = __shfl(border, (lane + 1) & 63), told_end = __shfl(border_end, (lane + 1) & 63);
-            right_end = has_right ? told_end : s + cnt;
-            const bool moved = has_right && (told != entry || told_end != entry_end);
-            if (moved) { entry = told; entry_end = told_end; }
-            if (moved && told < s) {                       // one token from left of the region to right of it
-                starts = 0;
-                border = told;
-                border_end = told_end;
-            } else if (moved) {
-                uint32_t fresh = 0;
-                int pos = told, end = told_end;
-                for (;;) {
-                    if (pos - s < cnt) {
-                        const uint32_t bit = 1u << (pos - s);
-                        if (starts & bit) {                // from here on it is the walk made before
-                            fresh |= starts & (bit | (bit - 1u));
-                            break;
-                        }
-                        fresh |= bit;
-                    }
-                    if (pos > s) {
-                        end = pos;
-                        pos -= length_of(state[(pos - 1 - s) * 64 + lane]);
+            for (int q = 0; q < P / 16; ++q) {
+                auto_u32x4_a1 w = {0, 0, 0, 0};
+                if (cnt > 16 * q) {
+                    const uint8_t *const at = src + s + 16 * q;
+                    if (start + e0 + s + 16 * q + 16 <= t.total) {       // (bytes behind the row's end are read, but not behind the batch's)
+                        w = *reinterpret_cast<const auto_u32x4_a1 *>(at);
                     } else {
-                        end = s;
-                    }
-                    if (pos <= s) {
-                        if (pos == s) {
-                            fresh |= 1u;
-                            end = s;
-                        }
-                        border = pos;
-                        border_end = end;
-                        break;
+                        uint8_t b[16];
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) b[i] = 16 * q + i < cnt ? at[i] : (uint8_t)0;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            w[i] = (uint32_t)b[4 * i] | ((uint32_t)b[4 * i + 1] << 8) | ((uint32_t)b[4 * i + 2] << 16) | ((uint32_t)b[4 * i + 3] << 24);
                     }
                 }
-                starts = fresh;
+                uint32_t foreign;
+                codes[q] = letter_codes16(w, t.letters, foreign);
+                flags |= foreign << (16 * q);
             }
-            if (!__ballot(moved)) break;
-        }
+            flags &= cnt >= 32 ? ~0u : (1u << cnt) - 1u;                 // (of the positions the row has)
+            const bool any_foreign = __ballot(flags != 0) != 0;
 
-        // every token's number among the wave's
-        const uint32_t mine = (uint32_t)__builtin_popcount(starts);
-        const uint32_t inc = wave_inclusive_sum_u32(mine);
-        const uint32_t before_row = (uint32_t)__shfl((int)inc, lane0 > 0 ? lane0 - 1 : 0);
-        const uint32_t base = lane0 > 0 ? before_row : 0u;
-        const uint32_t row_last = (uint32_t)__shfl((int)inc, lane0 + G - 1 < 64 ? lane0 + G - 1 : 63);
-        const uint32_t n_tok = row_last - base;
-
-        // the region's tokens, last one first: f(number of the token's state -- behind the states: the byte,
-        // where it is no letter --, position of its first byte in the region).  Four at a time: their
-        // states are read together.
-        auto each_token = [&](auto f) {
-            uint32_t left = starts;
-            int end = right_end;
-            while (left) {
-                int b[4], last[4];
-                bool is[4];
-                uint32_t v[4];
+            // forward over the own region
+            Entry e = 0;
+            if (any_foreign) {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    is[q] = left != 0;
-                    b[q] = is[q] ? 31 - __builtin_clz(left) : 0;
-                    last[q] = is[q] ? end - 1 : s;
-                    left &= ~(1u << b[q]);
-                    end = s + b[q];
-                }
-#pragma unroll
-                for (int q = 0; q < 4; ++q) v[q] = number_of(state_at(last[q]));
-                if (any_foreign) {
-#pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        if (is[q] && v[q] == t.other) v[q] = t.other + 1 + src[last[q]];
-                }
-                if (WIDE && chunk) {
-#pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        if (is[q]) v[q] = t.sym[v[q]];
-                }
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    if (is[q]) f(v[q], b[q]);
-            }
-        };
-
-        if (chunk) {
-            // The state's number (wide: the symbol) at every start, kNone elsewhere, and how many start
-            // where no neighbour reaches.  A token's number goes to the place of its first byte, whose state
-            // no token needs (it is inside one, unless the token is that byte alone).
-            each_token([&](uint32_t v, int b) { state[b * 64 + lane] = (Entry)v; });
-            int64_t mid_lo = k > 0 ? (int64_t)k * p.core + p.overlap : 0;
-            if (mid_lo > len) mid_lo = len;
-            const int64_t mid_hi = k + 1 < nc ? (int64_t)(k + 1) * p.core - p.overlap : len;
-            uint32_t in_mid = starts;
-            const int lo = (int)(mid_lo - e0) - s, hi = (int)(mid_hi - e0) - s;
-            if (lo > 0) in_mid &= lo >= 32 ? 0u : ~0u << lo;
-            if (hi < 32) in_mid &= hi <= 0 ? 0u : ~0u >> (32 - hi);
-            const uint32_t live = wave_inclusive_sum_u32((uint32_t)__builtin_popcount(in_mid));
-            if (lane == 63) p.cnt[4 * (size_t)item] = (int32_t)live;
-            uint16_t *const raw = p.chunk_sym + (size_t)item * p.ext + s;
-#pragma unroll
-            for (int i = 0; i < P; i += 8) {
-                uint32_t y[8];
-#pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    y[q] = kNone;
-                    if (starts >> (i + q) & 1u) {
-                        const uint32_t v = state[(i + q) * 64 + lane];
-                        y[q] = v;
-                    }
-                }
-                if (i < cnt)                               // (a slot is whole vectors: what lies behind the chunk's end is kNone)
-                    *reinterpret_cast<uint4 *>(raw + i) = uint4{y[0] | y[1] << 16, y[2] | y[3] << 16, y[4] | y[5] << 16, y[6] | y[7] << 16};
-            }
-        } else {
-            // the step's rows, one per lane again
-            int row_tok = 0, row_base = 0;
-            {
-                const int at = lanes_to - lanes_own - (first > 0 ? __builtin_amdgcn_readlane(lanes_to, first - 1) : 0);
-                const int from = lane >= first && lane < first + m ? at : 0;
-                row_tok = __shfl((int)n_tok, from);
-                row_base = __shfl((int)base, from);
-                if (lane >= first && lane < first + m) {
-                    lengths[row_id] = row_len > kRowMax ? -1 : row_tok;
-                    longest = row_tok > longest ? row_tok : longest;
-                }
-            }
-            // through LDS, where the wave's tokens fit its window (a token per four bytes always does)
-            const bool fits = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63) <= (uint32_t)t.window;
-            if (fits) {
-                uint32_t at = inc;
-                each_token([&](uint32_t v, int) { staged[--at] = (Entry)v; });
-                wave_phase();
-            }
-            if (PADDED) {
-                const int elem = a.pad_elem;
-                if (fits && (a.pad_stride & 3) == 0 && ((uintptr_t)a.pad_ids & (elem >= 4 ? 15 : 4 * elem - 1)) == 0 &&
-                    ((uintptr_t)a.pad_mask & 3) == 0) {
-                    if (elem == 4) auto_put_rows<4>(a, t.id, staged, row_base, row_tok, first, m, row_id, lane);
-                    else if (elem == 8) auto_put_rows<8>(a, t.id, staged, row_base, row_tok, first, m, row_id, lane);
-                    else if (elem == 2) auto_put_rows<2>(a, t.id, staged, row_base, row_tok, first, m, row_id, lane);
-                    else auto_put_rows<1>(a, t.id, staged, row_base, row_tok, first, m, row_id, lane);
-                } else {
-                    // cell by cell: the lanes their own tokens, the row's lanes its padding and mask
-                    const int64_t stride = a.pad_stride, at0 = (int64_t)row * stride;
-                    const int kept = (int64_t)n_tok < stride ? (int)n_tok : (int)stride;
-                    const int64_t shift = a.pad_left ? stride - kept : 0;
-                    int at = (int)(inc - base);
-                    each_token([&](uint32_t v, int) {
-                        --at;
-                        if (at < kept) {
-                            const int32_t x = t.id[v];
-                            auto_put(a.pad_ids, elem, at0 + shift + at, a.pad_remap ? a.pad_remap[x] : x);
-                        }
-                    });
-                    if (have) {
-                        for (int64_t c = j; c < stride; c += G) {
-                            const bool token = c >= shift && c < shift + kept;
-                            if (!token) auto_put(a.pad_ids, elem, at0 + c, a.pad_id);
-                            if (a.pad_mask) a.pad_mask[at0 + c] = token ? 1 : 0;
-                        }
-                    }
+                for (int i = 0; i < P; ++i) {
+                    e = step(e, (codes[i / 16] >> (2 * (i % 16))) & 3u);
+                    if (flags >> i & 1u) e = other;
+                    state[i * 64 + lane] = e;
                 }
             } else {
-                int32_t *const out = tok_tmp + start;
-                if (fits) {                                // the row's own lanes write its run
-                    for (uint32_t c = j; have && c < n_tok; c += G) out[c] = t.id[staged[base + c]];
-                } else {
-                    uint32_t at = inc - base;
-                    each_token([&](uint32_t v, int) { out[--at] = t.id[v]; });
+#pragma unroll
+                for (int i = 0; i < P; ++i) {
+                    e = step(e, (codes[i / 16] >> (2 * (i % 16))) & 3u);
+                    state[i * 64 + lane] = e;
                 }
             }
-        }
-        if (CHARS) {
-            // the single-character ids of the item's bytes (a chunk: those of its core), by the row's lanes
-            int64_t lo = 0, hi = have ? len : 0;
-            if (chunk) {
-                lo = (int64_t)k * p.core;
-                hi = (int64_t)(k + 1) * p.core < len ? (int64_t)(k + 1) * p.core : len;
-            }
-            const int64_t g0 = start + lo, g1 = start + hi;
-            const bool quads = ((uintptr_t)a.char_ids & 15) == 0 && ((uintptr_t)a.char_mask & 3) == 0;
-            for (int64_t g = (g0 & ~(int64_t)3) + 4 * j; g < g1; g += 4 * G) {
-                if (quads && g >= g0 && g + 4 <= g1) {
-                    const uint32_t w = *reinterpret_cast<const auto_u32_a1 *>(bytes + g);
-                    const auto_i32x4 v = {s_lut[w & 255u], s_lut[w >> 8 & 255u], s_lut[w >> 16 & 255u], s_lut[w >> 24]};
-                    __builtin_nontemporal_store(v, reinterpret_cast<auto_i32x4 *>(a.char_ids + g));
-                    if (a.char_mask) __builtin_nontemporal_store(0x01010101u, reinterpret_cast<uint32_t *>(a.char_mask + g));
-                } else {
-                    for (int q = 0; q < 4; ++q)
-                        if (g + q >= g0 && g + q < g1) {
-                            a.char_ids[g + q] = s_lut[bytes[g + q]];
-                            if (a.char_mask) a.char_mask[g + q] = 1;
+            // and on into the regions to the right until the states are the same, four bytes at a time: once
+            // equal they stay equal, so the last of the four tells, and writing equal ones again does no
+            // harm (nor does a state behind the row's end, which nothing reads)
+            bool going = cnt == P;
+            for (int ahead = 1;; ++ahead) {
+                const int from = (lane + ahead) & 63;
+                uint32_t word = 0, next_word = 0, f2 = 0;
+                word = (uint32_t)__shfl((int)codes[0], from);
+                if (P == 32) next_word = (uint32_t)__shfl((int)codes[P / 16 - 1], from);
+                if (any_foreign) f2 = (uint32_t)__shfl((int)flags, from);
+                const int cnt2 = __shfl(cnt, from);
+                going = going && j + ahead < G && cnt2 > 0;
+                if (!__ballot(going)) break;
+                wave_phase();
+                if (__builtin_expect(ahead >= kRepeatsFrom / P, 0))
+                    copy_repeats<P>(state, codes, flags, any_foreign, cnt, cnt2, lane, lane0, lane0 + G, ahead, e, going);
+                for (int i = 0; i < P; i += 4) {
+                    if (going) {
+                        Entry *const at = state + i * 64 + lane + ahead;
+                        const Entry there = at[3 * 64];
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            e = step(e, (word >> (2 * q)) & 3u);
+                            if (any_foreign && (f2 >> q & 1u)) e = other;
+                            at[q * 64] = e;
                         }
+                        going = e != there;
+                    }
+                    if (!__ballot(going)) break;
+                    word >>= 8;
+                    f2 >>= 4;
+                    if (P == 32 && i == 12) word = next_word;
                 }
             }
-        }
-        wave_phase();                                      // the wave's part of LDS is rewritten by the next step
-        first += m;
+            wave_phase();
+
+            // backward: token starts of the region as bits, first from the region's own end
+            auto state_at = [&](int pos) -> Entry { return state[(pos & (P - 1)) * 64 + lane0 + pos / P]; };
+            uint32_t starts = 0;
+            int entry = s + cnt, entry_end = s + cnt;          // where the walk comes into the region from the right (see border) ...
+            int border = s + cnt;                              // ... and where it leaves it: at s, or where the token begins that reaches over s;
+            int border_end = s + cnt;                          // that token's end (s itself, if none reaches over)
+            if (cnt == 0) border = border_end = n;
+            {
+                int pos = s + cnt;
+                while (pos > s) {
+                    border_end = pos;
+                    pos -= length_of(state[(pos - 1 - s) * 64 + lane]);
+                    if (pos >= s) starts |= 1u << (pos - s);
+                }
+                if (cnt > 0) border = pos;                     // (an empty region: the row ends to its left)
+                if (cnt > 0 && pos == s) border_end = s;
+            }
+            const bool has_right = cnt > 0 && j + 1 < G && lane < 63;
+            int right_end;                                     // end of the token that reaches over the region's end
+            for (;;) {
+                const int told = __shfl(border, (lane + 1) & 63), told_end = __shfl(border_end, (lane + 1) & 63);
+                right_end = has_right ? told_end : s + cnt;
+                const bool moved = has_right && (told != entry || told_end != entry_end);
+                if (moved) { entry = told; entry_end = told_end; }
+                if (moved && told < s) {                       // one token from left of the region to right of it
+                    starts = 0;
+                    border = told;
+                    border_end = told_end;
+                } else if (moved) {
+                    uint32_t fresh = 0;
+                    int pos = told, end = told_end;
+                    for (;;) {
+                        if (pos - s < cnt) {
+                            const uint32_t bit = 1u << (pos - s);
+                            if (starts & bit) {                // from here on it is the walk made before
+                                fresh |= starts & (bit | (bit - 1u));
+                                break;
+                            }
+                            fresh |= bit;
+                        }
+                        if (pos > s) {
+                            end = pos;
+                            pos -= length_of(state[(pos - 1 - s) * 64 + lane]);
+                        } else {
+                            end = s;
+                        }
+                        if (pos <= s) {
+                            if (pos == s) {
+                                fresh |= 1u;
+                                end = s;
+                            }
+                            border = pos;
+                            border_end = end;
+                            break;
+                        }
+                    }
+                    starts = fresh;
+                }
+                if (!__ballot(moved)) break;
+            }
+
+            // every token's number among the wave's
+            const uint32_t mine = (uint32_t)__builtin_popcount(starts);
+            const uint32_t inc = wave_inclusive_sum_u32(mine);
+            const uint32_t before_row = (uint32_t)__shfl((int)inc, lane0 > 0 ? lane0 - 1 : 0);
+            const uint32_t base = lane0 > 0 ? before_row : 0u;
+            const uint32_t row_last = (uint32_t)__shfl((int)inc, lane0 + G - 1 < 64 ? lane0 + G - 1 : 63);
+            const uint32_t n_tok = row_last - base;
+
+            // the region's tokens, last one first: f(number of the token's state -- behind the states: the byte,
+            // where it is no letter --, position of its first byte in the region).  Four at a time: their
+            // states are read together.
+            auto each_token = [&](auto f) {
+                uint32_t left = starts;
+                int end = right_end;
+                while (left) {
+                    int b[4], last[4];
+                    bool is[4];
+                    uint32_t v[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        is[q] = left != 0;
+                        b[q] = is[q] ? 31 - __builtin_clz(left) : 0;
+                        last[q] = is[q] ? end - 1 : s;
+                        left &= ~(1u << b[q]);
+                        end = s + b[q];
+                    }
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) v[q] = number_of(state_at(last[q]));
+                    if (any_foreign) {
+#pragma unroll
+                        for (int q = 0; q < 4; ++q)
+                            if (is[q] && v[q] == t.other) v[q] = t.other + 1 + src[last[q]];
+                    }
+                    if (WIDE && chunk) {
+#pragma unroll
+                        for (int q = 0; q < 4; ++q)
+                            if (is[q]) v[q] = t.sym[v[q]];
+                    }
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        if (is[q]) f(v[q], b[q]);
+                }
+            };
+
+            if (chunk) {
+                // The state's number (wide: the symbol) at every start, kNone elsewhere, and how many start
+                // where no neighbour reaches.  A token's number goes to the place of its first byte, whose state
+                // no token needs (it is inside one, unless the token is that byte alone).
+                each_token([&](uint32_t v, int b) { state[b * 64 + lane] = (Entry)v; });
+                int64_t mid_lo = k > 0 ? (int64_t)k * p.core + p.overlap : 0;
+                if (mid_lo > len) mid_lo = len;
+                const int64_t mid_hi = k + 1 < nc ? (int64_t)(k + 1) * p.core - p.overlap : len;
+                uint32_t in_mid = starts;
+                const int lo = (int)(mid_lo - e0) - s, hi = (int)(mid_hi - e0) - s;
+                if (lo > 0) in_mid &= lo >= 32 ? 0u : ~0u << lo;
+                if (hi < 32) in_mid &= hi <= 0 ? 0u : ~0u >> (32 - hi);
+                const uint32_t live = wave_inclusive_sum_u32((uint32_t)__builtin_popcount(in_mid));
+                if (lane == 63) p.cnt[4 * (size_t)item] = (int32_t)live;
+                uint16_t *const raw = p.chunk_sym + (size_t)item * p.ext + s;
+#pragma unroll
+                for (int i = 0; i < P; i += 8) {
+                    uint32_t y[8];
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) {
+                        y[q] = kNone;
+                        if (starts >> (i + q) & 1u) {
+                            const uint32_t v = state[(i + q) * 64 + lane];
+                            y[q] = v;
+                        }
+                    }
+                    if (i < cnt)                               // (a slot is whole vectors: what lies behind the chunk's end is kNone)
+                        *reinterpret_cast<uint4 *>(raw + i) = uint4{y[0] | y[1] << 16, y[2] | y[3] << 16, y[4] | y[5] << 16, y[6] | y[7] << 16};
+                }
+            } else {
+                // the step's rows, one per lane again
+                int row_tok = 0, row_base = 0;
+                {
+                    const int at = lanes_to - lanes_own - (first > 0 ? __builtin_amdgcn_readlane(lanes_to, first - 1) : 0);
+                    const int from = lane >= first && lane < first + m ? at : 0;
+                    row_tok = __shfl((int)n_tok, from);
+                    row_base = __shfl((int)base, from);
+                    if (lane >= first && lane < first + m) {
+                        lengths[row_id] = row_len > kRowMax ? -1 : row_tok;
+                        longest = row_tok > longest ? row_tok : longest;
+                    }
+                }
+                // through LDS, where the wave's tokens fit its window (a token per four bytes always does)
+                const bool fits = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63) <= (uint32_t)t.window;
+                if (fits) {
+                    uint32_t at = inc;
+                    each_token([&](uint32_t v, int) { staged[--at] = (Entry)v; });
+                    wave_phase();
+                }
+                if (PADDED) {
+                    const int elem = a.pad_elem;
+                    if (fits && (a.pad_stride & 3) == 0 && ((uintptr_t)a.pad_ids & (elem >= 4 ? 15 : 4 * elem - 1)) == 0 &&
+                        ((uintptr_t)a.pad_mask & 3) == 0) {
+                        if (elem == 4) auto_put_rows<4>(a, t.id, staged, row_base, row_tok, first, m, row_id, lane);
+                        else if (elem == 8) auto_put_rows<8>(a, t.id, staged, row_base, row_tok, first, m, row_id, lane);
+                        else if (elem == 2) auto_put_rows<2>(a, t.id, staged, row_base, row_tok, first, m, row_id, lane);
+                        else auto_put_rows<1>(a, t.id, staged, row_base, row_tok, first, m, row_id, lane);
+                    } else {
+                        // cell by cell: the lanes their own tokens, the row's lanes its padding and mask
+                        const int64_t stride = a.pad_stride, at0 = (int64_t)row * stride;
+                        const int kept = (int64_t)n_tok < stride ? (int)n_tok : (int)stride;
+                        const int64_t shift = a.pad_left ? stride - kept : 0;
+                        int at = (int)(inc - base);
+                        each_token([&](uint32_t v, int) {
+                            --at;
+                            if (at < kept) {
+                                const int32_t x = t.id[v];
+                                auto_put(a.pad_ids, elem, at0 + shift + at, a.pad_remap ? a.pad_remap[x] : x);
+                            }
+                        });
+                        if (have) {
+                            for (int64_t c = j; c < stride; c += G) {
+                                const bool token = c >= shift && c < shift + kept;
+                                if (!token) auto_put(a.pad_ids, elem, at0 + c, a.pad_id);
+                                if (a.pad_mask) a.pad_mask[at0 + c] = token ? 1 : 0;
+                            }
+                        }
+                    }
+                } else {
+                    int32_t *const out = tok_tmp + start;
+                    if (fits) {                                // the row's own lanes write its run
+                        for (uint32_t c = j; have && c < n_tok; c += G) out[c] = t.id[staged[base + c]];
+                    } else {
+                        uint32_t at = inc - base;
+                        each_token([&](uint32_t v, int) { out[--at] = t.id[v]; });
+                    }
+                }
+            }
+            if (CHARS) {
+                // the single-character ids of the item's bytes (a chunk: those of its core), by the row's lanes
+                int64_t lo = 0, hi = have ? len : 0;
+                if (chunk) {
+                    lo = (int64_t)k * p.core;
+                    hi = (int64_t)(k + 1) * p.core < len ? (int64_t)(k + 1) * p.core : len;
+                }
+                const int64_t g0 = start + lo, g1 = start + hi;
+                const bool quads = ((uintptr_t)a.char_ids & 15) == 0 && ((uintptr_t)a.char_mask & 3) == 0;
+                for (int64_t g = (g0 & ~(int64_t)3) + 4 * j; g < g1; g += 4 * G) {
+                    if (quads && g >= g0 && g + 4 <= g1) {
+                        const uint32_t w = *reinterpret_cast<const auto_u32_a1 *>(bytes + g);
+                        const auto_i32x4 v = {s_lut[w & 255u], s_lut[w >> 8 & 255u], s_lut[w >> 16 & 255u], s_lut[w >> 24]};
+                        __builtin_nontemporal_store(v, reinterpret_cast<auto_i32x4 *>(a.char_ids + g));
+                        if (a.char_mask) __builtin_nontemporal_store(0x01010101u, reinterpret_cast<uint32_t *>(a.char_mask + g));
+                    } else {
+                        for (int q = 0; q < 4; ++q)
+                            if (g + q >= g0 && g + q < g1) {
+                                a.char_ids[g + q] = s_lut[bytes[g + q]];
+                                if (a.char_mask) a.char_mask[g + q] = 1;
+                            }
+                    }
+                }
+            }
+            wave_phase();                                      // the wave's part of LDS is rewritten by the next step
+            first += m;
         }
     }
     if (PADDED && !CHUNKS && a.max_tree) {
