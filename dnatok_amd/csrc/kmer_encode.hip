@@ -1826,10 +1826,10 @@ extern "C" int dnatok_kmer_encode_padded_sized(const dnatok_kmer_t *t, const uin
             mref.slot = t->max_slots + (size_t)it->second * kMaxSlotStride;
             mref.tree = t->max_trees + (size_t)it->second * kTreeWords;
         }
-        if (!mref.slot) {
-            kmer_init_kernel<<<1, 1, 0, s>>>(max_len);
-            DNATOK_HIP_TRY(hipGetLastError());
-        }
+    }
+    if (!mref.slot && max_len) {
+        kmer_init_kernel<<<1, 1, 0, s>>>(max_len);
+        DNATOK_HIP_TRY(hipGetLastError());
     }
     int rc = launch_placed(t, 1, bytes, offsets, n_rows, t_cap, fill_to, ids, mask, lengths, status, max_len, mref,
                            RowPlace{nullptr, 1, 0}, s);
