@@ -69,3 +69,44 @@ def test_kmer_fixed_width_reports_the_longest_row(enc, form):
         enc.encode_padded(data, off, cap, fill_to=fill_to, out=out)
         torch.cuda.synchronize()
         check_fixed(out, rows, status, cap, fill_to)
+
+
+@pytest.mark.parametrize("form", ["few", "reads", "rows"])
+def test_kmer_fixed_width_call_replayed_from_a_graph(enc, form):
+    """A captured call keeps to its own buffers: its replays on two streams at once, with eager calls on the
+    stream it was captured on in between, all report their own longest row."""
+    print(f"kmer fixed width from a graph {form}", flush=True)
+    n, (lo, hi), cap = FIXED[form]
+    made = [batch(np.random.default_rng(seed).integers(lo, hi + 1, size=n), seed) for seed in (11, 12, 13)]
+    room = max(b.data.size for b, _, _ in made)
+    side, graphs = torch.cuda.Stream(), []
+    for _ in range(2):
+        data, off = torch.zeros(room, dtype=torch.uint8, device=DEV), torch.zeros(n + 1, dtype=torch.int64, device=DEV)
+        out = fixed_width_out(n, cap)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            enc.encode_padded(data, off, cap, fill_to=cap, out=out)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=side):
+            enc.encode_padded(data, off, cap, fill_to=cap, out=out)
+        graphs.append((g, data, off, out))
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    eager_in, eager_out = on_gpu(made[2][0]), fixed_width_out(n, cap)
+    for first in (0, 1, 0):
+        for q, (g, data, off, out) in enumerate(graphs):
+            b = made[(first + q) % 2][0]
+            data[:b.data.size].copy_(torch.from_numpy(b.data))
+            off.copy_(torch.from_numpy(b.offsets))
+            out[4].fill_(1 << 29)
+        torch.cuda.synchronize()
+        for q, (g, *_) in enumerate(graphs):
+            with torch.cuda.stream(streams[q]):
+                g.replay()
+        with torch.cuda.stream(side):
+            enc.encode_padded(*eager_in, cap, fill_to=cap, out=eager_out)
+        torch.cuda.synchronize()
+        for q, (_, _, _, out) in enumerate(graphs):
+            _, rows, status = made[(first + q) % 2]
+            check_fixed(out, rows, status, cap, cap)
+        check_fixed(eager_out, made[2][1], made[2][2], cap, cap)
