@@ -65,6 +65,9 @@ struct dnatok_kmer_table {
     // Batches of up to this many rows are encoded by kmer_team_kernel (a workgroup per row); -1: as
     // many rows as workgroups of that kernel fit the chip at once.  (dnatok_kmer_table_set_team_rows)
     std::atomic<int> team_rows{-1};
+    // Packed calls: trips without an answer until a workgroup counts a tile before its own itself; -1: the
+    // shipped number.  (dnatok_kmer_table_set_packed_polls)
+    std::atomic<int> packed_polls{-1};
 };
 
 constexpr int kMaxSlots = 64;
@@ -83,7 +86,6 @@ struct KmerArgs {
     const int2 *entry;
     const int32_t *flat;
     int32_t pad_id, missing_id;
-    int32_t all_plain;                    // every window of plain bases has an id
 };
 
 constexpr int kKmerThreads = 256;         // kmer_team_kernel: four waves share a row
@@ -137,9 +139,9 @@ struct RowPlace {
     // packed output: row b's cells are ids[row_at[b] .. row_at[b + 1]) (and the same cells of the
     // mask), no padding; null: row b's cells start at ids[b * t_cap]
     const int64_t *row_at;
-    // 0: every row; 1: the rows of at most kGroupsMaxUnits units; 2: the other rows (a batch of
-    // mostly short rows with some long ones is split between kmer_groups_kernel and kmer_rows_kernel)
-    int32_t row_class;
+    // the rows of more than kGroupsMaxUnits units alone (a padded batch of mostly short rows with some long
+    // ones is split between kmer_groups_kernel and kmer_rows_kernel)
+    int32_t long_rows_only;
     // the rows' lengths are all that is written (the first pass of a packed encode)
     int32_t count_only;
 };
@@ -236,7 +238,7 @@ __global__ __launch_bounds__(kRowsThreads) void kmer_rows_kernel(
     // Which rows the wave takes: every n_waves-th row; of a batch that is split by row class, the
     // long rows of every n_waves-th block of 64 rows -- the lanes look at a row each, so that the
     // short rows, which are nearly all of such a batch, cost a wave one load per 64 of them.
-    const bool long_rows_only = PLACED && place.row_class == 2;
+    const bool long_rows_only = PLACED && place.long_rows_only;
     int64_t cursor = long_rows_only ? wave * 64 : wave;
     uint64_t pending = 0;                                // (long_rows_only) rows of the block at `cursor` still to do
     auto next_row = [&]() -> int64_t {
@@ -778,15 +780,122 @@ struct __attribute__((packed, aligned(1), may_alias)) LaneBytes {
     uint32_t v[K];
 };
 
+// The 4K bytes at `pos`, a word at a time; what lies past the row's end (the next rows' bytes) is read and
+// ignored, what lies past the end of the batch is not read.
+template <int K>
+__device__ __forceinline__ void load_lane(const uint8_t *__restrict__ bytes, int64_t pos, int64_t total, bool wanted, uint32_t (&w)[K])
+{
+    if (wanted && pos + kUnitsPerLane * K <= total) {
+        const LaneBytes<K> all = *reinterpret_cast<const LaneBytes<K> *>(bytes + pos);
+#pragma unroll
+        for (int i = 0; i < K; ++i) w[i] = all.v[i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+            uint32_t v = 0;
+            if (wanted) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (pos + 4 * i + e < total) v |= (uint32_t)bytes[pos + 4 * i + e] << (8 * e);
+            }
+            w[i] = v;
+        }
+    }
+}
+
+// What a window of a lane is, where it is no plain window with an id.
+constexpr int32_t kSpelled = -1, kNothing = -2;
+
+// The codes of the lane's four windows (lut4r's index), and of the first `n_win` of them, those the row has, which
+// hold a byte that is no base (bit j: window j); foreign: one of these holds a byte that is not even N.  Digits by
+// arithmetic, as in kmer_rows_kernel<..., ARITH>.  (A word's four digits are gathered by one dot product with 1, 4,
+// 16, 64: as shifts the compiler makes it a 32-bit multiplication, which takes four times as long.)
+template <int K>
+__device__ __forceinline__ uint32_t lane_codes(const uint32_t (&w)[K], int n_win, uint32_t fold, uint32_t (&code)[kUnitsPerLane], bool &foreign)
+{
+    constexpr uint32_t POW4 = 1u << (2 * K);
+    uint32_t odd[K], c2[K];                              // bytes that are no base; twice the word's four digits
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        const uint32_t d = w[i] & 0x06060606u;
+        odd[i] = (w[i] ^ __builtin_amdgcn_perm(0x00470054u, 0x00430041u, d)) & fold;
+        c2[i] = __builtin_amdgcn_udot4(d, 0x40100401u, 0u, false);
+    }
+    uint32_t str[(K + 3) / 4 + 1];
+#pragma unroll
+    for (int q = 0; q < (K + 3) / 4 + 1; ++q) {
+        uint32_t v = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (4 * q + e < K) v |= e == 0 ? c2[4 * q] >> 1 : c2[4 * q + e] << (8 * e - 1);
+        str[q] = v;
+    }
+    uint32_t hits = 0;
+#pragma unroll
+    for (int j = 0; j < kUnitsPerLane; ++j) {
+        const int bit = 2 * K * j;
+        const uint64_t two = ((uint64_t)str[(bit >> 5) + 1] << 32) | str[bit >> 5];
+        code[j] = (uint32_t)(two >> (bit & 31)) & (POW4 - 1);
+        uint32_t hit = 0;
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+            const int bi = j * K + i;
+            hit |= odd[bi >> 2] & (0xFFu << (8 * (bi & 3)));
+        }
+        hits |= hit ? 1u << j : 0u;
+    }
+    hits &= (1u << n_win) - 1u;
+    foreign = false;
+    if (hits) {
+        uint32_t f = 0;
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+            const uint32_t sel = (w[i] >> 1) & 0x07070707u;               // A 0, C 1, T 2, G 3, N 7
+            const int nb = n_win * K - 4 * i;
+            const uint32_t m = nb >= 4 ? 0xFFFFFFFFu : (nb <= 0 ? 0u : ((1u << (8 * nb)) - 1u));
+            f |= (w[i] ^ __builtin_amdgcn_perm(0x4E000000u, 0x47544341u, sel)) & m;
+        }
+        foreign = (f & fold) != 0;
+    }
+    return hits;
+}
+
+// The lane's windows, `n_win` of them: the plain ones' ids in t, the number of tokens of all of them returned, for
+// tables that spell every window without an id by its characters.  No branch between the four look-ups: they
+// are one trip to the table.
+template <int K>
+__device__ __forceinline__ uint32_t lane_windows(const uint32_t (&w)[K], int n_win, uint32_t fold, const int32_t *lut,
+                                                 int32_t (&t)[kUnitsPerLane], bool &foreign)
+{
+    uint32_t code[kUnitsPerLane];
+    const uint32_t hits = lane_codes<K>(w, n_win, fold, code, foreign);
+    int32_t id[kUnitsPerLane];
+#pragma unroll
+    for (int j = 0; j < kUnitsPerLane; ++j) id[j] = lut[code[j]];
+    uint32_t spelled = 0;
+#pragma unroll
+    for (int j = 0; j < kUnitsPerLane; ++j) {
+        t[j] = j >= n_win ? kNothing : (hits >> j & 1u) ? kSpelled : id[j] < 0 ? kSpelled : id[j];
+        spelled += t[j] == kSpelled ? 1u : 0u;
+    }
+    return (uint32_t)n_win + (K - 1) * spelled;
+}
+
+// How many of a lane's four windows, the first of which is the row's `first`, the row has.
+__device__ __forceinline__ int windows_here(int full, int first)
+{
+    const int n = full - first;
+    return n < 0 ? 0 : n > kUnitsPerLane ? kUnitsPerLane : n;
+}
+
 template <int K, bool LUT4_LDS, bool HAS_MASK>
 __global__ __launch_bounds__(kGroupThreads) void kmer_groups_kernel(
     KmerArgs a, const uint8_t *__restrict__ bytes, const int64_t *__restrict__ offsets,
     int64_t n_rows, int64_t t_cap, int64_t fill_to, int32_t *__restrict__ ids,
     uint8_t *__restrict__ mask, int32_t *__restrict__ lengths, int32_t *__restrict__ status,
-    int32_t *__restrict__ max_len, MaxRef mref, int publish, RowPlace place)
+    int32_t *__restrict__ max_len, MaxRef mref, int publish, int short_rows_only)
 {
     constexpr uint32_t POW4 = 1u << (2 * K);
-    constexpr int kLaneBytes = kUnitsPerLane * K;                 // bytes of a lane's four windows
     __shared__ int32_t s_single[256];
     __shared__ int32_t s_spell[256];
     __shared__ int32_t s_lut4[LUT4_LDS ? POW4 : 1];
@@ -796,26 +905,20 @@ __global__ __launch_bounds__(kGroupThreads) void kmer_groups_kernel(
     const int lane = threadIdx.x & 63, gl = lane & 15;
     const int64_t group = ((int64_t)blockIdx.x * kGroupThreads + threadIdx.x) >> 4;
     const int64_t n_groups = (int64_t)gridDim.x * (kGroupThreads / 16);
-    int64_t next_start = 0, next_end = 0, next_cell = 0, next_cell_end = 0;
+    int64_t next_start = 0, next_end = 0;
     auto look_up = [&](int64_t row) {
         if (row >= n_rows) return;
         next_start = offsets[row];
         next_end = offsets[row + 1];
-        if (place.row_at) {
-            next_cell = place.row_at[row];
-            next_cell_end = place.row_at[row + 1];
-        }
     };
     look_up(group);
     const int64_t total = offsets[n_rows];
-    // (a count needs no ids where every plain window has one)
-    const bool ids_needed = !(place.count_only && a.all_plain);
     for (int i = threadIdx.x; i < 256; i += kGroupThreads) {
         const int d = a.digit[i];
         s_single[i] = a.single[i];
         s_spell[i] = a.single[(int)"ACGTN"[d < 0 || d > 4 ? 4 : d]];
     }
-    if (LUT4_LDS && ids_needed)
+    if (LUT4_LDS)
         for (uint32_t i = threadIdx.x; i < POW4; i += kGroupThreads) s_lut4[i] = a.lut4r[i];
     __syncthreads();
 
@@ -832,138 +935,60 @@ __global__ __launch_bounds__(kGroupThreads) void kmer_groups_kernel(
         bool have = row < n_rows;
         const int64_t start = have ? next_start : 0;
         int len = have ? (int)(next_end - next_start) : 0;
-        const int64_t cell_from = next_cell, cell_end = next_cell_end;
         look_up(row + n_groups);
-        if (place.row_class == 1 && len / K + len % K > kGroupsMaxUnits) {     // (kmer_rows_kernel's row)
+        if (short_rows_only && len / K + len % K > kGroupsMaxUnits) {          // (kmer_rows_kernel's row)
             have = false;
             len = 0;
         }
         const int full = len / K, tail = len - full * K;
-        const int n_slots = full + (tail ? 1 : 0);                // windows, and one slot for the trailing characters
-        // the row's cells: a stride apart, or (packed) where the rows before it end
-        const int64_t cell0 = !have ? 0 : place.row_at ? cell_from : row * t_cap;
-        const int cap = place.count_only || !have ? 0 : place.row_at ? (int)(cell_end - cell0) : cap_all;
-        const int fill = place.row_at || !have ? 0 : fill_all;
+        const int64_t cell0 = have ? row * t_cap : 0;
+        const int cap = have ? cap_all : 0;
+        const int fill = have ? fill_all : 0;
         int32_t *out = ids + cell0;
         uint8_t *mout = HAS_MASK ? mask + cell0 : nullptr;
         int running = 0;
         bool foreign_seen = false;
+        // (the trailing characters are the row's last tokens: a lane each, requested here and stored at its end)
+        const uint8_t tail_byte = gl < tail ? bytes[start + full * K + gl] : (uint8_t)0;
 
-        const int steps = (n_slots + 63) >> 6;
+        const int steps = (full + 63) >> 6;
         const int wave_steps = (int)wave_max_u32((uint32_t)steps);        // (wave-uniform loop: the loads are wave-wide)
         for (int st = 0; st < wave_steps; ++st) {
             const int wb = st * 64 + gl * kUnitsPerLane;          // the lane's first window
-            // the lane's 4K bytes, a word at a time; what lies past the row's end (the next rows'
-            // bytes) is read and ignored, what lies past the end of the batch is not read
             const int64_t pos = start + (int64_t)wb * K;
             uint32_t w[K];
-            if (wb < n_slots && pos + kLaneBytes <= total) {
-                const LaneBytes<K> all = *reinterpret_cast<const LaneBytes<K> *>(bytes + pos);
-#pragma unroll
-                for (int i = 0; i < K; ++i) w[i] = all.v[i];
-            } else {
-#pragma unroll
-                for (int i = 0; i < K; ++i) {
-                    uint32_t v = 0;
-                    if (wb < n_slots) {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            if (pos + 4 * i + e < total) v |= (uint32_t)bytes[pos + 4 * i + e] << (8 * e);
-                    }
-                    w[i] = v;
-                }
-            }
-            // digits, codes and the bytes that are no base, as in kmer_rows_kernel<..., ARITH>
-            uint32_t odd[K], c8[K];
-#pragma unroll
-            for (int i = 0; i < K; ++i) {
-                const uint32_t d = w[i] & 0x06060606u;
-                odd[i] = (w[i] ^ __builtin_amdgcn_perm(0x00470054u, 0x00430041u, d)) & a.fold;
-                const uint32_t x1 = (d << 6) | d, x2 = (x1 << 12) | x1;
-                c8[i] = (x2 >> 19) & 255u;
-            }
-            uint32_t str[(K + 3) / 4 + 1];
-#pragma unroll
-            for (int q = 0; q < (K + 3) / 4 + 1; ++q) {
-                uint32_t v = 0;
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (4 * q + e < K) v |= c8[4 * q + e] << (8 * e);
-                str[q] = v;
-            }
-            // per slot: its token count, and for a plain window its id
+            load_lane<K>(bytes, pos, total, wb < full, w);
             int32_t t[kUnitsPerLane];
-            uint32_t cnt[kUnitsPerLane], lane_cnt = 0;
-            bool spelled_any = false;
-#pragma unroll
-            for (int j = 0; j < kUnitsPerLane; ++j) {
-                const int bit = 2 * K * j;
-                const uint64_t two = ((uint64_t)str[(bit >> 5) + 1] << 32) | str[bit >> 5];
-                const uint32_t code = (uint32_t)(two >> (bit & 31)) & (POW4 - 1);
-                t[j] = !ids_needed ? 0 : LUT4_LDS ? s_lut4[code] : a.lut4r[code];
-                uint32_t hit = 0;
-#pragma unroll
-                for (int i = 0; i < K; ++i) {
-                    const int bi = j * K + i;
-                    hit |= odd[bi >> 2] & (0xFFu << (8 * (bi & 3)));
-                }
-                const int slot = wb + j;
-                uint32_t c = 0;
-                if (slot < full) {
-                    c = (hit == 0 && t[j] >= 0) ? 1u : (uint32_t)K;
-                    if (c != 1u) { t[j] = -1; spelled_any = true; }
-                } else if (slot == full && tail) {
-                    c = (uint32_t)tail;
-                    t[j] = -2;                                     // the trailing characters
-                }
-                cnt[j] = c;
-                lane_cnt += c;
-            }
-            // a byte of a window (not of the trailing characters) that is neither a base nor N: the
-            // row is flagged
-            if (spelled_any) {
-                const int in_windows = full - wb < kUnitsPerLane ? (full - wb) * K : kLaneBytes;     // bytes of whole windows
-                uint32_t f = 0;
-#pragma unroll
-                for (int i = 0; i < K; ++i) {
-                    const uint32_t sel = (w[i] >> 1) & 0x07070707u;               // A 0, C 1, T 2, G 3, N 7
-                    const int nb = in_windows - 4 * i;
-                    const uint32_t m = nb >= 4 ? 0xFFFFFFFFu : (nb <= 0 ? 0u : ((1u << (8 * nb)) - 1u));
-                    f |= (w[i] ^ __builtin_amdgcn_perm(0x4E000000u, 0x47544341u, sel)) & m;
-                }
-                if (f & a.fold) foreign_seen = true;
-            }
+            bool foreign;
+            const uint32_t lane_cnt = lane_windows<K>(w, windows_here(full, wb), a.fold, LUT4_LDS ? s_lut4 : a.lut4r, t, foreign);
+            foreign_seen = foreign_seen || foreign;
             const uint32_t inc = row16_inclusive_sum(lane_cnt);
             const uint32_t step_total = row16_last(inc);
             uint32_t s = (uint32_t)running + inc - lane_cnt;      // cell of the lane's first token
 
             auto byte_of = [&](int bi) -> uint32_t { return (w[bi >> 2] >> (8 * (bi & 3))) & 255u; };
-            if (lane_cnt == kUnitsPerLane && cnt[0] == 1 && cnt[1] == 1 && cnt[2] == 1 && cnt[3] == 1 &&
-                (t[0] | t[1] | t[2] | t[3]) >= 0 && (int)s + 4 <= cap && ((reinterpret_cast<uintptr_t>(out + s) & 15) == 0)) {
+            if ((t[0] | t[1] | t[2] | t[3]) >= 0 && (int)s + 4 <= cap && ((reinterpret_cast<uintptr_t>(out + s) & 15) == 0)) {
                 const int4v x = {t[0], t[1], t[2], t[3]};
                 __builtin_nontemporal_store(x, reinterpret_cast<int4v *>(out + s));
             } else if (lane_cnt) {
 #pragma unroll
                 for (int j = 0; j < kUnitsPerLane; ++j) {
-                    if (cnt[j] == 0) continue;
                     if (t[j] >= 0) {
                         if ((int)s < cap) out[s] = t[j];
                         s += 1;
-                    } else if (t[j] == -1) {
+                    } else if (t[j] == kSpelled) {
 #pragma unroll
                         for (int i = 0; i < K; ++i)
                             if ((int)s + i < cap) out[s + i] = s_spell[byte_of(j * K + i)];
                         s += K;
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < K - 1; ++i)
-                            if (i < tail && (int)s + i < cap) out[s + i] = s_single[byte_of(j * K + i)];
-                        s += (uint32_t)tail;
                     }
                 }
             }
             running += (int)step_total;
         }
+
+        if (gl < tail && running + gl < cap) out[running + gl] = s_single[tail_byte];
+        running += tail;
 
         // the row's end: mask, padding, length and status, by the row's 16 lanes
         const int stored = running < cap ? running : cap;
@@ -1444,6 +1469,8 @@ int launch_pad_to_max(int32_t *ids, uint8_t *mask, const int32_t *lengths, int64
 
 }  // namespace dnatok
 
+#include "kmer_packed.hpp"
+
 using namespace dnatok;
 
 extern "C" int dnatok_kmer_table_create(int k, const int8_t *digit_h, const int32_t *kmer_lut_h,
@@ -1574,6 +1601,14 @@ extern "C" int dnatok_kmer_table_set_team_rows(dnatok_kmer_t *t, int32_t max_row
     return DNATOK_OK;
 }
 
+extern "C" int dnatok_kmer_table_set_packed_polls(dnatok_kmer_t *t, int32_t polls)
+{
+    DNATOK_REQUIRE(t, DNATOK_E_INVALID, "dnatok_kmer_table_set_packed_polls: null table");
+    DNATOK_REQUIRE(polls >= -1, DNATOK_E_INVALID, "dnatok_kmer_table_set_packed_polls: -1 (automatic) or a number of trips");
+    t->packed_polls.store(polls, std::memory_order_relaxed);
+    return DNATOK_OK;
+}
+
 extern "C" void dnatok_kmer_table_destroy(dnatok_kmer_t *t)
 {
     if (!t) return;
@@ -1623,7 +1658,7 @@ extern "C" int dnatok_kmer_encode_padded(const dnatok_kmer_t *t, const uint8_t *
     if (to_longest) fill_to = guess;
     if (n_rows == 0) return DNATOK_OK;
     hipStream_t s = (hipStream_t)stream;
-    KmerArgs a{t->digit, t->single, t->lut4, t->lut4r, t->fold, t->entry, t->flat, t->pad_id, t->missing_id, t->all_plain};
+    KmerArgs a{t->digit, t->single, t->lut4, t->lut4r, t->fold, t->entry, t->flat, t->pad_id, t->missing_id};
     // A fixed width has no padding pass that would need the maximum, so the kernel itself reports it as well,
     // up the stream's tree, where that fits (16-bit fields): without the launch that clears max_len for the
     // atomics 256 rows of 6,000 bases take 8.8 instead of 12.0 us per call, 65,536 of them 163.6 instead of 171.9.
@@ -1666,7 +1701,7 @@ extern "C" int dnatok_kmer_encode_padded(const dnatok_kmer_t *t, const uint8_t *
         const int publish = by_itself(grid);                                                      \
         kmer_groups_kernel<KK, L, M><<<(int)grid, kGroupThreads, 0, s>>>(                         \
             a, bytes, offsets, n_rows, t_cap, width(), ids, mask, lengths, status, max_len, mref, \
-            publish, RowPlace{nullptr, 0, 0});                                                    \
+            publish, 0);                                                                          \
     } while (0)
 #define GROUPS(KK, L)                                                                             \
     do {                                                                                          \
@@ -1739,40 +1774,47 @@ int launch_scan_lengths(const int32_t *lengths, int64_t n_rows, int64_t *out_off
                         size_t scratch_bytes, hipStream_t s);   // pack.hip
 }
 
-// One launch of kmer_rows_kernel<..., PLACED> (which = 0) or kmer_groups_kernel (which = 1) with a
-// RowPlace.  The longest row, where asked for, goes to mref.slot / max_len by atomicMax (no tree:
-// two launches may share one call).
-static int launch_placed(const dnatok_kmer_t *t, int which, const uint8_t *bytes, const int64_t *offsets, int64_t n_rows,
-                         int64_t t_cap, int64_t fill_to, int32_t *ids, uint8_t *mask, int32_t *lengths,
-                         int32_t *status, int32_t *max_len, MaxRef mref, RowPlace place, hipStream_t s)
+// The rows of at most kGroupsMaxUnits units, by kmer_groups_kernel.  The longest row, where asked for, goes to
+// mref.slot / max_len by atomicMax (no tree: two launches share a call).
+static int launch_short_rows(const dnatok_kmer_t *t, const uint8_t *bytes, const int64_t *offsets, int64_t n_rows,
+                             int64_t t_cap, int64_t fill_to, int32_t *ids, uint8_t *mask, int32_t *lengths,
+                             int32_t *status, int32_t *max_len, MaxRef mref, hipStream_t s)
 {
-    KmerArgs a{t->digit, t->single, t->lut4, t->lut4r, t->fold, t->entry, t->flat, t->pad_id, t->missing_id, t->all_plain};
-    if (which == 1) {
+    KmerArgs a{t->digit, t->single, t->lut4, t->lut4r, t->fold, t->entry, t->flat, t->pad_id, t->missing_id};
 #define PG2(KK, L, M)                                                                              \
     do {                                                                                          \
         static const int resident = resident_workgroups(kmer_groups_kernel<KK, L, M>, kGroupThreads, 0, 8); \
         int64_t grid = (n_rows + kGroupThreads / 16 - 1) / (kGroupThreads / 16);                  \
         if (grid > resident) grid = resident;                                                     \
         kmer_groups_kernel<KK, L, M><<<(int)grid, kGroupThreads, 0, s>>>(                         \
-            a, bytes, offsets, n_rows, t_cap, fill_to, ids, mask, lengths, status, max_len, mref, 0, place); \
+            a, bytes, offsets, n_rows, t_cap, fill_to, ids, mask, lengths, status, max_len, mref, 0, 1); \
     } while (0)
 #define PG(KK, L)                                                                                 \
     do {                                                                                          \
         if (mask) PG2(KK, L, true); else PG2(KK, L, false);                                       \
     } while (0)
-        switch (t->k) {
-            case 2: PG(2, true); break;
-            case 3: PG(3, true); break;
-            case 4: PG(4, true); break;
-            case 5: PG(5, true); break;
-            case 6: PG(6, true); break;
-            case 7: PG(7, false); break;
-            default: PG(8, false); break;
-        }
+    switch (t->k) {
+        case 2: PG(2, true); break;
+        case 3: PG(3, true); break;
+        case 4: PG(4, true); break;
+        case 5: PG(5, true); break;
+        case 6: PG(6, true); break;
+        case 7: PG(7, false); break;
+        default: PG(8, false); break;
+    }
 #undef PG
 #undef PG2
-    } else {
-        const int64_t want = (n_rows + kRowsThreads / 64 - 1) / (kRowsThreads / 64);
+    DNATOK_HIP_TRY(hipGetLastError());
+    return DNATOK_OK;
+}
+
+// One launch of kmer_rows_kernel<..., PLACED> with a RowPlace; the longest row as above.
+static int launch_placed(const dnatok_kmer_t *t, const uint8_t *bytes, const int64_t *offsets, int64_t n_rows,
+                         int64_t t_cap, int64_t fill_to, int32_t *ids, uint8_t *mask, int32_t *lengths,
+                         int32_t *status, int32_t *max_len, MaxRef mref, RowPlace place, hipStream_t s)
+{
+    KmerArgs a{t->digit, t->single, t->lut4, t->lut4r, t->fold, t->entry, t->flat, t->pad_id, t->missing_id};
+    const int64_t want = (n_rows + kRowsThreads / 64 - 1) / (kRowsThreads / 64);
 #define PR4(KK, L, C, M, AR)                                                                      \
     do {                                                                                          \
         static const int resident = resident_workgroups(kmer_rows_kernel<KK, L, C, M, AR, true>, kRowsThreads, 0, 2); \
@@ -1792,20 +1834,19 @@ static int launch_placed(const dnatok_kmer_t *t, int which, const uint8_t *bytes
     do {                                                                                          \
         if (t->chars_mode) PR2(KK, L, true); else PR2(KK, L, false);                              \
     } while (0)
-        switch (t->k) {
-            case 2: PR(2, true); break;
-            case 3: PR(3, true); break;
-            case 4: PR(4, true); break;
-            case 5: PR(5, true); break;
-            case 6: PR(6, true); break;
-            case 7: PR(7, false); break;
-            default: PR(8, false); break;
-        }
+    switch (t->k) {
+        case 2: PR(2, true); break;
+        case 3: PR(3, true); break;
+        case 4: PR(4, true); break;
+        case 5: PR(5, true); break;
+        case 6: PR(6, true); break;
+        case 7: PR(7, false); break;
+        default: PR(8, false); break;
+    }
 #undef PR
 #undef PR2
 #undef PR3
 #undef PR4
-    }
     DNATOK_HIP_TRY(hipGetLastError());
     return DNATOK_OK;
 }
@@ -1844,13 +1885,43 @@ extern "C" int dnatok_kmer_encode_padded_sized(const dnatok_kmer_t *t, const uin
         kmer_init_kernel<<<1, 1, 0, s>>>(max_len);
         DNATOK_HIP_TRY(hipGetLastError());
     }
-    int rc = launch_placed(t, 1, bytes, offsets, n_rows, t_cap, fill_to, ids, mask, lengths, status, max_len, mref,
-                           RowPlace{nullptr, 1, 0}, s);
+    int rc = launch_short_rows(t, bytes, offsets, n_rows, t_cap, fill_to, ids, mask, lengths, status, max_len, mref, s);
     if (rc) return rc;
-    rc = launch_placed(t, 0, bytes, offsets, n_rows, t_cap, fill_to, ids, mask, lengths, status, max_len, mref,
-                       RowPlace{nullptr, 2, 0}, s);
+    rc = launch_placed(t, bytes, offsets, n_rows, t_cap, fill_to, ids, mask, lengths, status, max_len, mref,
+                       RowPlace{nullptr, 1, 0}, s);
     if (rc) return rc;
     if (to_longest) return launch_pad(ids, mask, lengths, n_rows, t_cap, max_len, t->pad_id, (int32_t)guess, mref, s);
+    return DNATOK_OK;
+}
+
+// Packed rows of a batch that split_by_row_class() says is one of mostly short rows.
+static int launch_packed_rows(const dnatok_kmer_t *t, const uint8_t *bytes, const int64_t *offsets, int64_t n_rows,
+                              int32_t *ids, int64_t *out_offsets, uint8_t *mask, int32_t *lengths, int32_t *status, hipStream_t s)
+{
+    const KmerArgs a{t->digit, t->single, t->lut4, t->lut4r, t->fold, t->entry, t->flat, t->pad_id, t->missing_id};
+    // a tile per workgroup, as small as lets the whole batch be under way at once (30,000 reads in 469 tiles of 64 rows
+    // 16.4 us, 24,000 in 750 of 32 17.2)
+    constexpr int kAtOnce = 256 * kPackedPerCu;
+    int64_t held = (n_rows + (int64_t)kAtOnce * kPackedGroups - 1) / ((int64_t)kAtOnce * kPackedGroups);
+    if (held > kPackedHeld) held = kPackedHeld;
+    const int tile_rows = (int)held * kPackedGroups;
+    const int64_t n_tiles = (n_rows + tile_rows - 1) / tile_rows;
+    const int asked = t->packed_polls.load(std::memory_order_relaxed), polls = asked < 0 ? kPackedPolls : asked;
+    kmer_open_tiles_kernel<<<(int)((n_tiles + 255) / 256), 256, 0, s>>>(out_offsets, n_rows, tile_rows, n_tiles);
+#define PT(KK, L)                                                                                 \
+    kmer_packed_kernel<KK, L><<<(int)n_tiles, kPackedThreads, 0, s>>>(                            \
+        a, t->all_plain, bytes, offsets, n_rows, tile_rows, polls, ids, out_offsets, mask, lengths, status)
+    switch (t->k) {
+        case 2: PT(2, true); break;
+        case 3: PT(3, true); break;
+        case 4: PT(4, true); break;
+        case 5: PT(5, true); break;
+        case 6: PT(6, true); break;
+        case 7: PT(7, false); break;
+        default: PT(8, false); break;
+    }
+#undef PT
+    DNATOK_HIP_TRY(hipGetLastError());
     return DNATOK_OK;
 }
 
@@ -1862,29 +1933,19 @@ extern "C" int dnatok_kmer_encode_packed(const dnatok_kmer_t *t, const uint8_t *
     DNATOK_REQUIRE(n_rows >= 0 && total >= 0, DNATOK_E_INVALID, "dnatok_kmer_encode_packed: negative size");
     DNATOK_REQUIRE(ids_out || total == 0, DNATOK_E_INVALID, "dnatok_kmer_encode_packed: null ids_out");
     hipStream_t s = (hipStream_t)stream;
-    const bool split = split_by_row_class(t, n_rows, total);
+    if (split_by_row_class(t, n_rows, total))
+        return launch_packed_rows(t, bytes, offsets, n_rows, ids_out, out_offsets, mask_out, lengths, status, s);
+    // other batches in two passes of a wave per row: every row's token count, then where every row starts, ...
     const MaxRef none{nullptr, nullptr};
-    // first pass: every row's token count (nothing else is written), then where every row starts
     if (n_rows > 0) {
-        int rc;
-        if (split) {
-            rc = launch_placed(t, 1, bytes, offsets, n_rows, 0, 0, nullptr, nullptr, lengths, nullptr, nullptr, none,
-                               RowPlace{nullptr, 1, 1}, s);
-            if (rc) return rc;
-        }
-        rc = launch_placed(t, 0, bytes, offsets, n_rows, 0, 0, nullptr, nullptr, lengths, nullptr, nullptr, none,
-                           RowPlace{nullptr, split ? 2 : 0, 1}, s);
+        const int rc = launch_placed(t, bytes, offsets, n_rows, 0, 0, nullptr, nullptr, lengths, nullptr, nullptr, none,
+                                     RowPlace{nullptr, 0, 1}, s);
         if (rc) return rc;
     }
     // (ids_out is not written yet: its first bytes, when 8-byte aligned, are the scan's spare room)
-    int rc = launch_scan_lengths(lengths, n_rows, out_offsets, ids_out, (size_t)total * 4, s);
+    const int rc = launch_scan_lengths(lengths, n_rows, out_offsets, ids_out, (size_t)total * 4, s);
     if (rc || n_rows == 0) return rc;
-    // second pass: the tokens, each row behind the one before it
-    if (split) {
-        rc = launch_placed(t, 1, bytes, offsets, n_rows, 0, 0, ids_out, mask_out, lengths, status, nullptr, none,
-                           RowPlace{out_offsets, 1, 0}, s);
-        if (rc) return rc;
-    }
-    return launch_placed(t, 0, bytes, offsets, n_rows, 0, 0, ids_out, mask_out, lengths, status, nullptr, none,
-                         RowPlace{out_offsets, split ? 2 : 0, 0}, s);
+    // ... and the tokens, each row behind the one before it
+    return launch_placed(t, bytes, offsets, n_rows, 0, 0, ids_out, mask_out, lengths, status, nullptr, none,
+                         RowPlace{out_offsets, 0, 0}, s);
 }

@@ -391,6 +391,11 @@ class KmerEncoder:
         ``max_rows`` rows get a workgroup per row, larger ones a wave per row; -1 = automatic."""
         _lib.check(_lib.lib().dnatok_kmer_table_set_team_rows(self._h, int(max_rows)), "dnatok_kmer_table_set_team_rows")
 
+    def set_packed_polls(self, polls: int) -> None:
+        """Test hook (``dnatok_kmer_table_set_packed_polls``): 0 = a workgroup of a packed call counts whatever
+        has no sum yet itself, -1 = it waits for a while first."""
+        _lib.check(_lib.lib().dnatok_kmer_table_set_packed_polls(self._h, int(polls)), "dnatok_kmer_table_set_packed_polls")
+
     def encode_padded(self, data: torch.Tensor, offsets: torch.Tensor, t_cap: int, *,
                       fill_to: int = 0, width_guess: int = 0, want_mask: bool = True, out=None):
         """Returns (ids[B, t_cap], mask, lengths[B], status[B], max_len[1]); with fill_to = 0 the

@@ -152,6 +152,11 @@ void dnatok_kmer_table_destroy(dnatok_kmer_t *t);
  * when it starts. */
 int dnatok_kmer_table_set_team_rows(dnatok_kmer_t *t, int32_t max_rows);
 
+/* Test switch of packed calls (dnatok_kmer_encode_packed): after how many looks at a part of the batch
+ * that has no sum yet a workgroup counts that part itself; -1 (default) = the library's number, 0 = at
+ * once.  Results are identical. */
+int dnatok_kmer_table_set_packed_polls(dnatok_kmer_t *t, int32_t polls);
+
 /* ids int32[n_rows, t_cap], mask uint8[n_rows, t_cap] (NULL allowed): t_cap is the row stride.
  * lengths int32[n_rows] receives each row's token count (also when it exceeds t_cap),
  * status int32[n_rows] the DNATOK_ROW_* bits (NULL allowed), max_len int32[1] the largest
@@ -187,8 +192,9 @@ int dnatok_kmer_encode_padded_sized(const dnatok_kmer_t *t, const uint8_t *bytes
  * 100-300 bp beside a few rows of 20 kbp): ids_out int32[sum of lengths] holds the rows' tokens
  * back to back, out_offsets int64[n_rows + 1] their boundaries, mask_out uint8 (NULL allowed) is
  * one per token, lengths / status as above.  ids_out and mask_out have room for `total` cells (a row
- * never has more tokens than bytes).  Two passes over the bytes: the rows' token counts, their
- * prefix sum, then the tokens; no padding is written and nothing returns to the host.  The k-mer
+ * never has more tokens than bytes).  A batch of mostly short rows is read once (the workgroups
+ * tell each other their sums through out_offsets), any other in two passes, the rows' token counts and
+ * their prefix sum, then the tokens; no padding is written and nothing returns to the host.  The k-mer
  * counterpart of dnatok_pack_ragged; the reference has no packed k-mer output (its rows go through
  * _pad_id_list, src/dna_tokenizer.py:1878-1894). */
 int dnatok_kmer_encode_packed(const dnatok_kmer_t *t, const uint8_t *bytes, const int64_t *offsets,

@@ -110,3 +110,136 @@ def test_kmer_fixed_width_call_replayed_from_a_graph(enc, form):
             _, rows, status = made[(first + q) % 2]
             check_fixed(out, rows, status, cap, cap)
         check_fixed(eager_out, made[2][1], made[2][2], cap, cap)
+
+
+def check_packed(out, rows, status, total):
+    ids, out_off, mask, lengths, st = out
+    want = np.concatenate([[0], np.cumsum([r.size for r in rows])])
+    np.testing.assert_array_equal(out_off.cpu().numpy(), want)
+    np.testing.assert_array_equal(lengths.cpu().numpy(), [r.size for r in rows])
+    np.testing.assert_array_equal(st.cpu().numpy() & 7, status)
+    n = int(want[-1])
+    np.testing.assert_array_equal(ids[:n].cpu().numpy(), np.concatenate(rows))
+    assert bool((ids[n:] == -7).all())
+    if mask is not None:
+        assert bool((mask[:n] == 1).all()) and bool((mask[n:] == 9).all())
+
+
+def packed_out(n, total, shift=0):
+    # (nothing of an earlier content may count: the offsets' cells look like offsets)
+    ids = torch.full((total + shift,), -7, dtype=torch.int32, device=DEV)[shift:]
+    mask = torch.full((total + shift,), 9, dtype=torch.uint8, device=DEV)[shift:]
+    return (ids, torch.full((n + 1,), 77, dtype=torch.int64, device=DEV), mask,
+            torch.full((n,), -7, dtype=torch.int32, device=DEV), torch.full((n,), -7, dtype=torch.int32, device=DEV))
+
+
+def packed_lens(n, seed, most=300):
+    """Reads with rows of no byte, of less than a window, at the borders between the rows that are read once
+    (up to 389 bytes), those walked by sixteen lanes (773) and the others, and of several steps of a wave, anywhere
+    among them."""
+    rng = np.random.default_rng(seed)
+    lens = rng.integers(0, most + 1, size=n)
+    for v in (0, 1, 5, 6, 383, 384, 385, 389, 390, 768, 773, 774, 1536, 1537, 2304, 2311, 9001):
+        lens[rng.integers(0, n)] = v
+    return lens
+
+
+@pytest.mark.parametrize("n,polls", [(n, -1) for n in (1, 31, 32, 33, 127, 129, 2500, 24577, 25000, 49153, 70001, 98304 + 129, 123000, 160001)] +
+                         [(n, 0) for n in (1, 33, 513, 2500, 24577, 25000, 49153)])
+def test_kmer_packed_reads(enc, n, polls):
+    """Batches of fewer and of more tiles than the chip holds (and than a wave looks back on in one trip), of
+    tiles of 32 to 192 rows; the tiles' sums waited for, and counted by whoever finds one missing."""
+    print(f"kmer packed n={n} polls={polls}", flush=True)
+    lens = packed_lens(n, n, 300 if n < 50000 else 60)
+    if n == 1:
+        lens[:] = 300
+    b, rows, status = batch(lens, n + 1, n_rate=0.004)
+    data, off = on_gpu(b)
+    enc.set_packed_polls(polls)
+    try:
+        for shift in (0, 1, 3):
+            out = packed_out(n, b.data.size, shift)
+            enc.encode_packed(data, off, want_mask=True, out=out)
+            torch.cuda.synchronize()
+            check_packed(out, rows, status, b.data.size)
+        out = packed_out(n, b.data.size)
+        enc.encode_packed(data, off, out=(out[0], out[1], None, out[3], out[4]))
+        torch.cuda.synchronize()
+        check_packed((out[0], out[1], None, out[3], out[4]), rows, status, b.data.size)
+    finally:
+        enc.set_packed_polls(-1)
+
+
+@pytest.mark.parametrize("k", [2, 3, 4, 5, 7, 8])
+def test_kmer_packed_reads_of_other_k(k):
+    print(f"kmer packed k={k}", flush=True)
+    vocab = hf.kmer_vocab(k)
+    t = kmer_tables.tables_from_vocab(vocab, k, 0)
+    e = encoders.KmerEncoder(k, t.digit, t.kmer_lut, t.single, pad_id=1, missing_id=0, exp_off=t.exp_off, exp_len=t.exp_len, exp_flat=t.exp_flat)
+    rng = np.random.default_rng(k)
+    lens = rng.integers(0, 301, size=3000)
+    lens[7:14] = 65 * k - 1, 65 * k, 129 * k - 1, 129 * k, 256 * k, 256 * k + 1, 384 * k + 5
+    lens[2999] = 64 * k
+    b = util.batch_from_strings(["".join(rng.choice(list("ACGTNx"), p=[.247, .247, .247, .247, .008, .004], size=n)) for n in lens])
+    rows, status = O.kmer_encode(O.kmer_tables_from_vocab(vocab, k, 0), b.data, b.offsets)
+    out = packed_out(len(lens), b.data.size)
+    e.encode_packed(*on_gpu(b), want_mask=True, out=out)
+    torch.cuda.synchronize()
+    check_packed(out, rows, status, b.data.size)
+
+
+def test_kmer_packed_reads_replayed_from_a_graph(enc):
+    print("kmer packed from a graph", flush=True)
+    n = 9000
+    made = [batch(packed_lens(n, seed), seed, n_rate=0.004) for seed in (21, 22)]
+    room = max(b.data.size for b, _, _ in made)
+    data, off = torch.zeros(room, dtype=torch.uint8, device=DEV), torch.zeros(n + 1, dtype=torch.int64, device=DEV)
+    out = packed_out(n, room)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        enc.encode_packed(data, off, want_mask=True, out=out)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        enc.encode_packed(data, off, want_mask=True, out=out)
+    for which in (0, 1, 1, 0):
+        b, rows, status = made[which]
+        data[:b.data.size].copy_(torch.from_numpy(b.data))
+        off.copy_(torch.from_numpy(b.offsets))
+        out[0].fill_(-7), out[2].fill_(9)
+        g.replay()
+        torch.cuda.synchronize()
+        check_packed(out, rows, status, room)
+
+
+def test_kmer_packed_reads_full_of_n(enc):
+    """More spelled windows than a tile's list has room for, in some tiles; in others none."""
+    print("kmer packed, many N", flush=True)
+    rng = np.random.default_rng(5)
+    rows = []
+    for i in range(1200):
+        p = [.1, .1, .1, .1, .6] if 300 <= i < 500 else [.25, .25, .25, .25, 0] if i < 800 else [.24, .24, .24, .24, .04]
+        rows.append("".join(rng.choice(list("ACGTN"), p=p, size=int(rng.integers(0, 390)))))
+    b = util.batch_from_strings(rows)
+    want, status = O.kmer_encode(O.kmer_tables_from_vocab(hf.kmer_vocab(K), K, 0), b.data, b.offsets)
+    out = packed_out(len(rows), b.data.size)
+    enc.encode_packed(*on_gpu(b), want_mask=True, out=out)
+    torch.cuda.synchronize()
+    check_packed(out, want, status, b.data.size)
+
+
+def test_kmer_packed_reads_of_a_table_with_gaps():
+    """Plain windows without an id are spelled as well."""
+    print("kmer packed, table with gaps", flush=True)
+    vocab = {w: i for w, i in hf.kmer_vocab(K).items() if not (len(w) == K and w.startswith("CG"))}
+    t = kmer_tables.tables_from_vocab(vocab, K, 0)
+    e = encoders.KmerEncoder(K, t.digit, t.kmer_lut, t.single, pad_id=1, missing_id=0, exp_off=t.exp_off, exp_len=t.exp_len, exp_flat=t.exp_flat)
+    rng = np.random.default_rng(6)
+    b = util.batch_from_strings(["".join(rng.choice(list("ACGTN"), p=[.248, .248, .248, .248, .008], size=n)) for n in packed_lens(3000, 7)])
+    want, status = O.kmer_encode(O.kmer_tables_from_vocab(vocab, K, 0), b.data, b.offsets)
+    assert any((r < 0).any() for r in want) is False
+    out = packed_out(3000, b.data.size)
+    e.encode_packed(*on_gpu(b), want_mask=True, out=out)
+    torch.cuda.synchronize()
+    check_packed(out, want, status, b.data.size)
