@@ -33,9 +33,15 @@
 // 1 KB 54.7 -> 29.2 us, 100,000 reads 123 -> 57 us.  (That includes the walk into the next region four bytes
 // at a time, comparing the last of the four, and the padded rows of a wave written as one run of cells.)
 //
-// Per call, the merge engine -> the automaton: 1,024 rows of 1 KB 29.4 -> 11.6 us, 16,384 of them 236.5 ->
-// 29.1 us, 100,000 reads of 100 - 300 bp (int64 rows) 349 -> 56.5 us, 4,096 ragged reads of 12 Mbp 253.5 ->
-// 80.2 us (all with the vocabulary of 4,096), 32 rows of 100 kbp (32,000) 143.8 -> 60.5 us.
+// Per call, the merge engine -> the automaton: 1,024 rows of 1 KB 29.4 -> 11.7 us, 16,384 of them 236.5 ->
+// 26.9 us, 100,000 reads of 100 - 300 bp (int64 rows) 349 -> 51 us, 4,096 ragged reads of 12 Mbp 253.5 ->
+// 79 us (all with the vocabulary of 4,096), 32 rows of 100 kbp (32,000) 143.8 -> 59.6 us.
+//
+// Beside the chains of dependent reads vector issue is what a full chip runs out of (three fifths of the time), so the
+// steps of the chains are as few instructions as they can be: an entry and a code are the next entry's address in one
+// (32-bit entries on their way, the table at the start of LDS), a word's codes are gathered by one dot product, which
+// bytes are no letters is looked at where there are any, and the walk backwards notes the ends of tokens: 16,384 rows of
+// 1 KB 1,144 -> 933 vector instructions per step.
 #pragma once
 
 namespace dnatok {
@@ -48,7 +54,9 @@ struct AutoArgs {
     uint32_t other;              // the state behind a byte that is no letter; its successors are the row start's
     uint32_t letters;            // the letters by code (bits 1 and 2 of the byte)
     int32_t rows;                // (whole rows) rows of an item, at most 64
-    int32_t n_groups;            // (whole rows) n_rows / rows, rounded up (chunks: the work list says)
+    int32_t n_groups;            // (whole rows) items (chunks: the work list says)
+    int64_t bytes_each;          // (whole rows) 0, or: an item is the rows that start in its share of the batch's bytes
+    float rows_per_byte;         // ... and this is n_rows / total
     int32_t window;              // tokens a wave has room for on their way out
     int32_t list_here;           // (chunks) the kernel makes the work list itself: at most kAutoListRows rows
     int32_t *zero;               // (chunks) a word to be cleared for the kernels behind this one, or null
@@ -58,7 +66,8 @@ struct AutoArgs {
 // Waves of a workgroup, which has a CU to itself: as many as the LDS holds, at most sixteen (four per SIMD).
 constexpr int kAutoMaxWaves = 16;
 constexpr uint32_t kAutoNarrowStates = 10400;    // the most the narrow form has LDS for, beside the waves' share
-constexpr size_t kAutoLdsBytes = 163840 - 1152;  // what a workgroup may take: the CU's, less the static arrays (1,088 bytes)
+constexpr size_t kAutoLdsBytes = 163840;         // a CU's
+constexpr size_t kAutoLdsAside = 1152;           // of it, for what is neither table nor a wave's (the longest rows, or the characters' ids)
 
 typedef uint32_t auto_u32_a1 __attribute__((aligned(1), may_alias));
 typedef uint32_t auto_u32x4_a1 __attribute__((ext_vector_type(4), aligned(1), may_alias));
@@ -75,17 +84,17 @@ struct AutoLds {
     }
     static int waves(uint32_t n_states)
     {
-        const size_t w = (kAutoLdsBytes - table_bytes(n_states)) / (state_bytes + least_window * sizeof(Entry));
+        const size_t w = (kAutoLdsBytes - kAutoLdsAside - table_bytes(n_states)) / (state_bytes + least_window * sizeof(Entry));
         return w > (size_t)kAutoMaxWaves ? kAutoMaxWaves : (int)w;
     }
     static int window(uint32_t n_states)
     {
-        const size_t w = ((kAutoLdsBytes - table_bytes(n_states)) / waves(n_states) - state_bytes) / sizeof(Entry) & ~(size_t)7;
+        const size_t w = ((kAutoLdsBytes - kAutoLdsAside - table_bytes(n_states)) / waves(n_states) - state_bytes) / sizeof(Entry) & ~(size_t)7;
         return w > (size_t)(64 * P) ? 64 * P : (int)w;
     }
     static size_t bytes(uint32_t n_states)
     {
-        return table_bytes(n_states) + waves(n_states) * (state_bytes + window(n_states) * sizeof(Entry));
+        return table_bytes(n_states) + waves(n_states) * (state_bytes + window(n_states) * sizeof(Entry)) + kAutoLdsAside;
     }
 };
 
@@ -102,6 +111,14 @@ constexpr int kAutoListRows = 256;
 
 constexpr uint32_t kXcds = 8;                    // (workgroups go to them in turn)
 
+// 16 bits at an address of LDS (a kernel's dynamic array begins at 0 where it has no other)
+__device__ __forceinline__ uint32_t lds_u16(uint32_t at)
+{
+    uint32_t v = *reinterpret_cast<const __attribute__((address_space(3))) uint16_t *>(at);
+    asm("" : "+v"(v));                                  // (else the compiler forgets that the read has cleared the upper half)
+    return v;
+}
+
 // Between two phases of a wave's work on its LDS: what a lane wrote before is what the others read after.
 __device__ __forceinline__ void wave_phase()
 {
@@ -109,24 +126,33 @@ __device__ __forceinline__ void wave_phase()
     __builtin_amdgcn_wave_barrier();
 }
 
-// Codes of the 16 bytes of w (two bits each, the first byte lowest) and the bytes that are no letters.
-__device__ __forceinline__ uint32_t letter_codes16(const auto_u32x4_a1 w, uint32_t letters, uint32_t &foreign)
+// Codes of the 16 bytes of w (two bits each, the first byte lowest: a word's four by one dot product with 1, 4, 16,
+// 64); differs: has a bit wherever a byte is no letter.
+__device__ __forceinline__ uint32_t letter_codes16(const auto_u32x4_a1 w, uint32_t letters, uint32_t &differs)
 {
-    uint32_t codes = 0, bad = 0;
+    uint32_t codes = 0;
+    differs = 0;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         const uint32_t sel = (w[q] >> 1) & 0x03030303u;
-        const uint32_t back = __builtin_amdgcn_perm(letters, letters, sel);
-        const uint32_t two = sel | (sel >> 6);
-        codes |= ((two | (two >> 12)) & 0xFFu) << (8 * q);
-        // the high bit of every byte that differs, then four bits together
-        const uint32_t d = back ^ w[q];
-        const uint32_t hi = ((d & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | d;
-        const uint32_t f = (hi >> 7) & 0x01010101u;
-        bad |= ((f | (f >> 7) | (f >> 14) | (f >> 21)) & 0xFu) << (4 * q);
+        differs |= __builtin_amdgcn_perm(letters, letters, sel) ^ w[q];
+        codes |= __builtin_amdgcn_udot4(sel, 0x40100401u, 0u, false) << (8 * q);
     }
-    foreign = bad;
     return codes;
+}
+
+// Which of the 16 bytes of w are no letters.
+__device__ __forceinline__ uint32_t foreign16(const auto_u32x4_a1 w, uint32_t letters)
+{
+    uint32_t bad = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const uint32_t d = __builtin_amdgcn_perm(letters, letters, (w[q] >> 1) & 0x03030303u) ^ w[q];
+        // the high bit of every byte that differs, then four bits together
+        const uint32_t hi = ((d & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | d;
+        bad |= __builtin_amdgcn_udot4((hi >> 7) & 0x01010101u, 0x08040201u, 0u, false) << (4 * q);
+    }
+    return bad;
 }
 
 // One id, in the padded output's own integer width.
@@ -206,7 +232,7 @@ __device__ __forceinline__ void auto_put_rows(const BpeArgs &a, const int32_t *i
 // with a walker less than `ahead` lanes to their left.
 template <int P, typename Entry>
 __device__ __forceinline__ void copy_repeats(Entry *state, const uint32_t (&codes)[P / 16], uint32_t flags, bool any_foreign, int cnt,
-                                             int cnt_ahead, int lane, int lane0, int lane_end, int ahead, Entry &e, bool &going)
+                                             int cnt_ahead, int lane, int lane0, int lane_end, int ahead, uint32_t &e, bool &going)
 {
     constexpr int kTries = 4, kLongest = 256;              // walkers per call, and distances of one of them; the longest distance
     const int behind = ahead * P < kLongest ? ahead * P : kLongest;
@@ -221,7 +247,7 @@ __device__ __forceinline__ void copy_repeats(Entry *state, const uint32_t (&code
         const int walker = __builtin_ctzll(eligible);
         const int first = walker + ahead;                  // the region it is about to enter
         const int row_end = __builtin_amdgcn_readlane(lane_end, walker);
-        const Entry now = (Entry)__builtin_amdgcn_readlane((int)e, walker);
+        const uint32_t now = (uint32_t)__builtin_amdgcn_readlane((int)e, walker);
         int k = 0, d = 0, looked = 0;
 #pragma unroll 1
         for (int d0 = 1; k == 0 && looked < kTries && d0 < behind; d0 += 64) {
@@ -295,45 +321,37 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
     typedef typename AutoLds<WIDE, P>::Entry Entry;
     static_assert(P == 16 || P == 32, "a region's token starts are the bits of one word");
     static_assert(!CHUNKS || P == 32, "a chunk of 2,048 bytes is a wave");
+    // (all of it in one array, the table at its start: an entry and a code are then the next entry's address with one
+    // instruction between two reads of the chain)
     extern __shared__ __align__(16) uint8_t smem[];
-    __shared__ int32_t s_longest[PADDED ? kAutoMaxWaves : 1];
-    __shared__ int32_t s_lut[CHARS ? 256 : 1];
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int n_waves = (int)blockDim.x >> 6;
     const uint32_t n_entries = 4 * (t.other + 1);
     uint32_t table_bytes = 0;
-    if (!WIDE) {
-        // the transition table and the token lengths, 16 bytes per thread and step
-        const uint32_t tab16 = (n_entries * 2 + 15) / 16, len16 = (t.other + 1 + 15) / 16;
-        const uint4 *const src = reinterpret_cast<const uint4 *>(t.next);
-        uint4 *const dst = reinterpret_cast<uint4 *>(smem);
-        for (uint32_t i = threadIdx.x; i < tab16; i += blockDim.x) dst[i] = src[i];
-        const uint4 *const src_len = reinterpret_cast<const uint4 *>(t.len);
-        for (uint32_t i = threadIdx.x; i < len16; i += blockDim.x) dst[tab16 + i] = src_len[i];
-        table_bytes = 16 * (tab16 + len16);
-    }
-    if (CHARS)
-        for (int i = threadIdx.x; i < 256; i += blockDim.x) s_lut[i] = a.char_lut[i];
-    const uint16_t *const table = reinterpret_cast<const uint16_t *>(smem);
-    const uint8_t *const len_of = smem + (size_t)((n_entries * 2 + 15) / 16) * 16;
+    const uint32_t tab16 = (n_entries * 2 + 15) / 16, len16 = (t.other + 1 + 15) / 16;
+    if (!WIDE) table_bytes = 16 * (tab16 + len16);
+    int32_t *const s_longest = reinterpret_cast<int32_t *>(smem + table_bytes + (size_t)n_waves * (64 * P + t.window) * sizeof(Entry));    // [n_waves]
+    int32_t *const s_lut = s_longest;                                                                                                     // [256]
+    static_assert(!(PADDED && CHARS), "the two share their place");
+    const uint8_t *const len_of = smem + (size_t)tab16 * 16;
     const uint32_t *const far_table = reinterpret_cast<const uint32_t *>(t.next);
     Entry *const state = reinterpret_cast<Entry *>(smem + table_bytes) + (size_t)wv * (64 * P + t.window);   // [P][64]
     Entry *const staged = state + 64 * P;                                                                    // [t.window]
-    const Entry other = WIDE ? (Entry)((t.other * 4) << 8 | 1u) : (Entry)(t.other * 4);
-    __syncthreads();
+    const uint32_t other = WIDE ? (t.other * 4) << 8 | 1u : t.other * 4;
 
-    auto step = [&](Entry e, uint32_t code) -> Entry {
-        if (WIDE) return (Entry)far_table[((uint32_t)e >> 8) + code];
-        return (Entry)table[(uint32_t)e + code];
+    // (an entry on its way is 32 bits wide, also where one in LDS is 16: as 16 bits every step would clear the others)
+    auto step = [&](uint32_t e, uint32_t code) -> uint32_t { return WIDE ? far_table[(e >> 8) + code] : lds_u16(2 * (e + code)); };
+    // the same, or `other` if bit `at` of `flags` is set
+    auto step_or = [&](uint32_t e, uint32_t code, uint32_t flags, int at) -> uint32_t {
+        const uint32_t is = (uint32_t)((int32_t)(flags << (31 - at)) >> 31);
+        return (step(e, code) & ~is) | (other & is);
     };
-    auto length_of = [&](Entry e) -> int {
-        if (WIDE) return (int)((uint32_t)e & 0xFFu);
-        return (int)len_of[(uint32_t)e >> 2];
-    };
-    auto number_of = [&](Entry e) -> uint32_t { return WIDE ? (uint32_t)e >> 10 : (uint32_t)e >> 2; };
+    auto length_of = [&](uint32_t e) -> int { return WIDE ? (int)(e & 0xFFu) : (int)len_of[e >> 2]; };
+    auto number_of = [&](uint32_t e) -> uint32_t { return WIDE ? e >> 10 : e >> 2; };
 
     constexpr int kRowMax = 64 * P;                        // the longest row that a wave takes
+    constexpr bool kShares = !CHUNKS && P == 32;           // (items by bytes: batches of several steps per wave)
     // (list_here) chunk slots and single rows up to and including row 64 q + lane
     constexpr int kListWords = CHUNKS ? kAutoListRows / 64 : 1;
     int32_t slots_to[kListWords], singles_to[kListWords];
@@ -390,14 +408,68 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
     }
     if (CHUNKS && t.zero && blockIdx.x == 0 && threadIdx.x == 0) *t.zero = 0;
     int32_t longest = 0;
-    // (neighbouring items go to different CUs, so that a small batch spreads over the chip)
-    for (int64_t item64 = (int64_t)wv * gridDim.x + blockIdx.x; item64 < n_items; item64 += (int64_t)gridDim.x * n_waves) {
-        const int32_t item = (int32_t)item64;
-        int32_t row = 0, k = 0, nc = 1;
-        const int64_t item_row0 = (int64_t)item * t.rows;
-        int item_rows = CHUNKS ? 1 : (int)(n_rows - item_row0 < t.rows ? n_rows - item_row0 : t.rows);
+    // What a wave knows of its item: a chunk (of row `row`, the k-th of nc), or whole rows, one per lane [first, last),
+    // with the lanes each of them needs (a region of P bytes to a lane) summed up; they are then taken in as few steps
+    // as their lanes fit the wave.
+    int32_t item = 0, row_id = 0, k = 0, nc = 1;
+    int64_t row_at = 0, row_len = 0;
+    int first = 0, last = 0, lanes_to = 0, lanes_own = 0;
+    bool chunk = false, more = false;                      // more: (shares of bytes) rows of the item behind lane 63
+    auto sum_lanes = [&]() {
+        lanes_own = 0;
+        if (lane >= first && lane < last) lanes_own = row_len <= 0 || row_len > kRowMax ? 1 : ((int)row_len + P - 1) / P;
+        lanes_to = (int)wave_inclusive_sum_u32((uint32_t)lanes_own);
+    };
+    // Rows from row `row_base` on, one per lane: those that start in [from, to) are the item's.
+    auto take_rows = [&](int32_t row_base, int64_t from, int64_t to) {
+        row_id = row_base + lane;
+        const int32_t at = row_id < n_rows ? row_id : n_rows, behind = row_id + 1 < n_rows ? row_id + 1 : n_rows;
+        row_at = offsets[at];
+        row_len = offsets[behind] - row_at;
+        first = (int)__builtin_popcountll(__ballot(row_id < n_rows && row_at < from));
+        last = (int)__builtin_popcountll(__ballot(row_id < n_rows && row_at < to));
+        more = last == 64 && row_base + 64 < n_rows;
+        sum_lanes();
+    };
+    auto share_from = [&](int64_t i) -> int64_t { return i == 0 ? INT64_MIN : i >= t.n_groups ? INT64_MAX : i * t.bytes_each; };
+    auto take_item = [&](int64_t item64) {
+        item = (int32_t)item64;
+        k = 0;
+        nc = 1;
+        if (kShares && t.bytes_each) {
+            // The rows are looked for where the rows' mean length puts them: 64 rows from a few before that place on
+            // (rows of one length are there), and 64 rows eight rows apart around it, in one trip; in the next trip
+            // those are taken that the latter point to, or, if the place is not even among them, after a search through all.
+            const int64_t from = share_from(item64), to = share_from(item64 + 1);
+            const int32_t guess = item64 == 0 ? 0 : (int32_t)((float)from * t.rows_per_byte);
+            const int32_t near = guess < 8 ? 0 : guess - 8, apart8 = guess + 8 * (lane - 32);
+            const int32_t look = apart8 < 0 ? 0 : apart8 > n_rows ? n_rows : apart8;
+            const int64_t probe = offsets[look];
+            take_rows(near, from, to);
+            if ((near > 0 && first == 0) || (first == 64 && near + 64 < n_rows)) {
+                const int n_below = (int)__builtin_popcountll(__ballot(probe < from));
+                int32_t below = n_below > 0 ? __builtin_amdgcn_readlane(look, n_below - 1) : 0;      // starts below `from`, or is row 0
+                if ((n_below == 0 && guess - 256 > 0) || (n_below == 64 && guess + 248 < n_rows)) {
+                    int32_t lo = 0, hi = n_rows;
+                    while (hi - lo > 8) {
+                        const int32_t apart = (hi - lo + 63) >> 6;
+                        const int64_t here = (int64_t)lo + (int64_t)lane * apart;
+                        const int n = (int)__builtin_popcountll(__ballot(here < hi && offsets[here < hi ? here : hi] < from));
+                        const int32_t up = n > 0 ? lo + (n - 1) * apart : lo;
+                        hi = n > 0 ? (hi - up < apart ? hi : up + apart) : lo;
+                        lo = up;
+                    }
+                    below = lo;
+                }
+                take_rows(below, from, to);
+            }
+            return;
+        }
+        int32_t row = 0;
         const int32_t *list = nullptr;
         int32_t list_at = 0;
+        const int64_t item_row0 = (int64_t)item * t.rows;
+        int item_rows = CHUNKS ? 1 : (int)(n_rows - item_row0 < t.rows ? n_rows - item_row0 : t.rows);
         if (CHUNKS && t.list_here) {
             // the first row whose slots (or single rows) reach beyond the item
             const bool cut = item < n_mc;
@@ -436,47 +508,138 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
             list_at = q << many;
             item_rows = of - list_at < 1 << many ? of - list_at : 1 << many;
         }
-        const bool chunk = CHUNKS && nc > 1;
-        // The item's whole rows, one per lane, with the lanes each of them needs (a region of P bytes to a lane)
-        // summed up; they are then taken in as few steps as their lanes fit the wave.
-        int32_t row_id = row;
-        int64_t row_at = 0, row_len = 0;
-        int lanes_to = 0, lanes_own = 0;
-        if (!chunk) {
-            if (lane < item_rows) {
-                if (!CHUNKS) row_id = (int32_t)(item_row0 + lane);
-                else if (list) row_id = list[list_at + lane];
-                row_at = offsets[row_id];
-                row_len = offsets[row_id + 1] - row_at;
-                lanes_own = row_len <= 0 || row_len > kRowMax ? 1 : ((int)row_len + P - 1) / P;
-            }
-            lanes_to = (int)wave_inclusive_sum_u32((uint32_t)lanes_own);
+        chunk = CHUNKS && nc > 1;
+        first = 0;
+        last = item_rows;
+        row_id = row;
+        row_at = 0;
+        row_len = 0;
+        if (chunk || lane < item_rows) {
+            if (!CHUNKS) row_id = (int32_t)(item_row0 + lane);
+            else if (list) row_id = list[list_at + lane];
+            row_at = offsets[row_id];
+            row_len = offsets[row_id + 1] - row_at;
         }
-        for (int first = 0; first < item_rows;) {          // (chunks: one step)
-            int m = 1, r = 0, lane0 = 0, G = 64;
-            bool have = true;
-            int64_t start, len;
-            if (chunk) {
-                start = offsets[row];
-                len = offsets[row + 1] - start;
-            } else {
-                // rows [first, first + m) of the item; r: the lane's row, lane0 and G: that row's lanes
-                const int lanes_before = first > 0 ? __builtin_amdgcn_readlane(lanes_to, first - 1) : 0;
-                const uint64_t in_step = __ballot(lane >= first && lane < item_rows && lanes_to - lanes_before <= 64);
-                m = (int)__builtin_popcountll(in_step);
-                r = first;
-                for (int i = first; i + 1 < first + m; ++i)
-                    if (lane >= __builtin_amdgcn_readlane(lanes_to, i) - lanes_before) r = i + 1;
-                G = __shfl(lanes_own, r);
-                lane0 = __shfl(lanes_to, r) - lanes_before - G;
-                have = lane < lane0 + G;                       // (lanes behind the last row's have none)
-                start = ((int64_t)__shfl((int)(row_at >> 32), r) << 32) | (uint32_t)__shfl((int)(uint32_t)row_at, r);
-                len = ((int64_t)__shfl((int)(row_len >> 32), r) << 32) | (uint32_t)__shfl((int)(uint32_t)row_len, r);
-                row = __shfl(row_id, r);
+        if (!chunk) sum_lanes();
+    };
+
+    // A step: rows [first, first + m) of the item, or the chunk, and what a lane has of it: the row r, that row's lanes
+    // lane0 to lane0 + G, and the bytes of its region, [from, from + n) of the batch being what the row (or chunk) has.
+    struct Step {
+        int m, lane0, G, n;
+        bool have;
+        int32_t row;
+        int64_t start, len, e0, e1;
+    };
+    auto place = [&]() -> Step {
+        Step st;
+        st.m = 1;
+        st.lane0 = 0;
+        st.G = 64;
+        st.have = true;
+        if (chunk) {
+            st.row = row_id;
+            st.start = row_at;
+            st.len = row_len;
+            st.e0 = (int64_t)k * p.core - p.overlap < 0 ? 0 : (int64_t)k * p.core - p.overlap;
+            st.e1 = (int64_t)(k + 1) * p.core + p.overlap;
+            if (st.e1 > st.len) st.e1 = st.len;
+        } else {
+            const int lanes_before = first > 0 ? __builtin_amdgcn_readlane(lanes_to, first - 1) : 0;
+            const uint64_t in_step = __ballot(lane >= first && lane < last && lanes_to - lanes_before <= 64);
+            st.m = (int)__builtin_popcountll(in_step);
+            int r = first;
+            for (int i = first; i + 1 < first + st.m; ++i)
+                if (lane >= __builtin_amdgcn_readlane(lanes_to, i) - lanes_before) r = i + 1;
+            st.G = __shfl(lanes_own, r);
+            st.lane0 = __shfl(lanes_to, r) - lanes_before - st.G;
+            st.have = lane < st.lane0 + st.G;                  // (lanes behind the last row's have none)
+            st.start = ((int64_t)__shfl((int)(row_at >> 32), r) << 32) | (uint32_t)__shfl((int)(uint32_t)row_at, r);
+            st.len = ((int64_t)__shfl((int)(row_len >> 32), r) << 32) | (uint32_t)__shfl((int)(uint32_t)row_len, r);
+            st.row = __shfl(row_id, r);
+            st.e0 = 0;
+            st.e1 = st.len;
+        }
+        const bool too_long = st.e1 - st.e0 > kRowMax;         // (longer than the caller declared)
+        st.n = st.have && !too_long && st.e1 > st.e0 ? (int)(st.e1 - st.e0) : 0;
+        return st;
+    };
+    auto fetch = [&](const Step &st, auto_u32x4_a1 (&w)[P / 16]) {
+        const int s = (lane - st.lane0) * P, cnt = st.n - s;
+        const int64_t from = st.start + st.e0 + s;
+#pragma unroll
+        for (int q = 0; q < P / 16; ++q) {
+            w[q] = auto_u32x4_a1{t.letters, t.letters, t.letters, t.letters};
+            if (cnt > 16 * q) {
+                const uint8_t *const at = bytes + from + 16 * q;
+                if (from + 16 * q + 16 <= t.total) {           // (bytes behind the row's end are read, but not behind the batch's)
+                    w[q] = *reinterpret_cast<const auto_u32x4_a1 *>(at);
+                } else {
+                    uint8_t b[16];
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) b[i] = 16 * q + i < cnt ? at[i] : (uint8_t)0;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        w[q][i] = (uint32_t)b[4 * i] | ((uint32_t)b[4 * i + 1] << 8) | ((uint32_t)b[4 * i + 2] << 16) | ((uint32_t)b[4 * i + 3] << 24);
+                }
             }
+        }
+    };
+
+    // Whether the first bytes are requested while the tables are staged, and those of an item's next step while a step is
+    // worked on.  (Two more copies of the code that does it: forms that stage nothing, or whose waves rarely take more
+    // than one step, are 2 - 5 % slower with them.)
+    constexpr bool kAhead = !WIDE && P == 32;
+    // (neighbouring items go to different CUs, so that a small batch spreads over the chip)
+    int64_t item64 = (int64_t)wv * gridDim.x + blockIdx.x;
+    Step next{};
+    auto_u32x4_a1 ahead_bytes[P / 16];
+    // the tables (the transitions and the token lengths), 16 bytes per thread and step
+    constexpr int kTablePieces = 6;
+    uint4 piece[kAhead ? kTablePieces : 1];
+    auto table_piece = [&](uint32_t i) {
+        return i < tab16 ? reinterpret_cast<const uint4 *>(t.next)[i] : reinterpret_cast<const uint4 *>(t.len)[i - tab16];
+    };
+    uint4 *const table_to = reinterpret_cast<uint4 *>(smem);
+    if (kAhead) {
+#pragma unroll
+        for (int q = 0; q < kTablePieces; ++q) {
+            const uint32_t i = threadIdx.x + q * blockDim.x;
+            if (i < tab16 + len16) piece[q] = table_piece(i);
+        }
+        if (item64 < n_items) {
+            take_item(item64);
+            if (first < last) {
+                next = place();
+                fetch(next, ahead_bytes);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < kTablePieces; ++q) {
+            const uint32_t i = threadIdx.x + q * blockDim.x;
+            if (i < tab16 + len16) table_to[i] = piece[q];
+        }
+        for (uint32_t i = threadIdx.x + kTablePieces * blockDim.x; i < tab16 + len16; i += blockDim.x) table_to[i] = table_piece(i);
+    } else {
+        if (!WIDE) {
+            const uint4 *const src = reinterpret_cast<const uint4 *>(t.next), *const src_len = reinterpret_cast<const uint4 *>(t.len);
+            for (uint32_t i = threadIdx.x; i < tab16; i += blockDim.x) table_to[i] = src[i];
+            for (uint32_t i = threadIdx.x; i < len16; i += blockDim.x) table_to[tab16 + i] = src_len[i];
+        }
+        item64 -= (int64_t)gridDim.x * n_waves;            // (the loop below begins with the item)
+    }
+    if (CHARS)
+        for (int i = threadIdx.x; i < 256; i += blockDim.x) s_lut[i] = a.char_lut[i];
+    if (!WIDE || CHARS) __syncthreads();
+    while (item64 < n_items) {
+        while (first < last) {                             // (chunks: one step)
+            const Step now = next;
+            const int m = now.m, lane0 = now.lane0, G = now.G, n = now.n;
+            const bool have = now.have;
+            const int32_t row = now.row;
+            const int64_t start = now.start, len = now.len, e0 = now.e0;
             const int j = lane - lane0;                        // the lane's region within the row
             const int s = j * P;                               // its first byte
-            int64_t e0 = 0, e1 = len;
             if (chunk && t.list_here && lane == 0) {
                 p.rec[item] = make_int4(row, k, nc, (int)len);
                 if (k == 0) {
@@ -484,13 +647,6 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
                     p.mc_off[row] = item;
                 }
             }
-            if (chunk) {
-                e0 = (int64_t)k * p.core - p.overlap < 0 ? 0 : (int64_t)k * p.core - p.overlap;
-                e1 = (int64_t)(k + 1) * p.core + p.overlap;
-                if (e1 > len) e1 = len;
-            }
-            const bool too_long = e1 - e0 > kRowMax;           // (longer than the caller declared)
-            const int n = have && !too_long && e1 > e0 ? (int)(e1 - e0) : 0;
             const uint8_t *const src = bytes + start + e0;
 
             // the region's bytes as codes; cnt: how many of its P positions the row has
@@ -498,41 +654,33 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
             uint32_t codes[P / 16], flags = 0;
 #pragma unroll
             for (int q = 0; q < P / 16; ++q) {
-                auto_u32x4_a1 w = {0, 0, 0, 0};
-                if (cnt > 16 * q) {
-                    const uint8_t *const at = src + s + 16 * q;
-                    if (start + e0 + s + 16 * q + 16 <= t.total) {       // (bytes behind the row's end are read, but not behind the batch's)
-                        w = *reinterpret_cast<const auto_u32x4_a1 *>(at);
-                    } else {
-                        uint8_t b[16];
-#pragma unroll
-                        for (int i = 0; i < 16; ++i) b[i] = 16 * q + i < cnt ? at[i] : (uint8_t)0;
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            w[i] = (uint32_t)b[4 * i] | ((uint32_t)b[4 * i + 1] << 8) | ((uint32_t)b[4 * i + 2] << 16) | ((uint32_t)b[4 * i + 3] << 24);
-                    }
-                }
-                uint32_t foreign;
-                codes[q] = letter_codes16(w, t.letters, foreign);
-                flags |= foreign << (16 * q);
+                uint32_t differs;
+                codes[q] = letter_codes16(ahead_bytes[q], t.letters, differs);
+                if (__ballot(differs != 0)) flags |= foreign16(ahead_bytes[q], t.letters) << (16 * q);      // (few rows hold any)
+            }
+            // the item's next step begins where this one ends
+            const int from = first;
+            first += m;
+            if (kAhead && !chunk && first < last) {
+                next = place();
+                fetch(next, ahead_bytes);
             }
             flags &= cnt >= 32 ? ~0u : (1u << cnt) - 1u;                 // (of the positions the row has)
             const bool any_foreign = __ballot(flags != 0) != 0;
 
             // forward over the own region
-            Entry e = 0;
+            uint32_t e = 0;
             if (any_foreign) {
 #pragma unroll
                 for (int i = 0; i < P; ++i) {
-                    e = step(e, (codes[i / 16] >> (2 * (i % 16))) & 3u);
-                    if (flags >> i & 1u) e = other;
-                    state[i * 64 + lane] = e;
+                    e = step_or(e, (codes[i / 16] >> (2 * (i % 16))) & 3u, flags, i);
+                    state[i * 64 + lane] = (Entry)e;
                 }
             } else {
 #pragma unroll
                 for (int i = 0; i < P; ++i) {
                     e = step(e, (codes[i / 16] >> (2 * (i % 16))) & 3u);
-                    state[i * 64 + lane] = e;
+                    state[i * 64 + lane] = (Entry)e;
                 }
             }
             // and on into the regions to the right until the states are the same, four bytes at a time: once
@@ -554,12 +702,11 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
                 for (int i = 0; i < P; i += 4) {
                     if (going) {
                         Entry *const at = state + i * 64 + lane + ahead;
-                        const Entry there = at[3 * 64];
+                        const uint32_t there = at[3 * 64];
 #pragma unroll
                         for (int q = 0; q < 4; ++q) {
-                            e = step(e, (word >> (2 * q)) & 3u);
-                            if (any_foreign && (f2 >> q & 1u)) e = other;
-                            at[q * 64] = e;
+                            e = step_or(e, (word >> (2 * q)) & 3u, f2, q);
+                            at[q * 64] = (Entry)e;
                         }
                         going = e != there;
                     }
@@ -572,21 +719,21 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
             wave_phase();
 
             // backward: token starts of the region as bits, first from the region's own end
-            auto state_at = [&](int pos) -> Entry { return state[(pos & (P - 1)) * 64 + lane0 + pos / P]; };
-            uint32_t starts = 0;
+            uint32_t ends = 0;                                 // bit x: a token ends behind the region's byte x
             int entry = s + cnt, entry_end = s + cnt;          // where the walk comes into the region from the right (see border) ...
             int border = s + cnt;                              // ... and where it leaves it: at s, or where the token begins that reaches over s;
             int border_end = s + cnt;                          // that token's end (s itself, if none reaches over)
-            if (cnt == 0) border = border_end = n;
-            {
-                int pos = s + cnt;
-                while (pos > s) {
-                    border_end = pos;
-                    pos -= length_of(state[(pos - 1 - s) * 64 + lane]);
-                    if (pos >= s) starts |= 1u << (pos - s);
-                }
-                if (cnt > 0) border = pos;                     // (an empty region: the row ends to its left)
-                if (cnt > 0 && pos == s) border_end = s;
+            const auto token_length = [&](int x) -> int { return length_of(state[x * 64 + lane]); };      // of the token that ends behind byte x
+            if (cnt == 0) {                                    // (an empty region: the row ends to its left)
+                border = border_end = n;
+            } else {
+                int x = cnt - 1;
+                do {
+                    ends |= 1u << x;
+                    x -= token_length(x);
+                } while (x >= 0);
+                border = s + x + 1;
+                border_end = x == -1 ? s : s + __builtin_ctz(ends) + 1;
             }
             const bool has_right = cnt > 0 && j + 1 < G && lane < 63;
             int right_end;                                     // end of the token that reaches over the region's end
@@ -594,43 +741,32 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
                 const int told = __shfl(border, (lane + 1) & 63), told_end = __shfl(border_end, (lane + 1) & 63);
                 right_end = has_right ? told_end : s + cnt;
                 const bool moved = has_right && (told != entry || told_end != entry_end);
-                if (moved) { entry = told; entry_end = told_end; }
-                if (moved && told < s) {                       // one token from left of the region to right of it
-                    starts = 0;
-                    border = told;
-                    border_end = told_end;
-                } else if (moved) {
+                if (!__ballot(moved)) break;
+                if (moved) {
+                    entry = told;
+                    entry_end = told_end;
                     uint32_t fresh = 0;
-                    int pos = told, end = told_end;
-                    for (;;) {
-                        if (pos - s < cnt) {
-                            const uint32_t bit = 1u << (pos - s);
-                            if (starts & bit) {                // from here on it is the walk made before
-                                fresh |= starts & (bit | (bit - 1u));
-                                break;
-                            }
-                            fresh |= bit;
+                    int x = told - 1 - s;
+                    if (x < -1) {                              // one token from left of the region to right of it
+                        border = told;
+                        border_end = told_end;
+                    } else {
+                        while (x >= 0 && !(ends >> x & 1u)) {
+                            fresh |= 1u << x;
+                            x -= token_length(x);
                         }
-                        if (pos > s) {
-                            end = pos;
-                            pos -= length_of(state[(pos - 1 - s) * 64 + lane]);
+                        if (x >= 0) {                          // from here on it is the walk made before
+                            fresh |= ends & ((2u << x) - 1u);
                         } else {
-                            end = s;
-                        }
-                        if (pos <= s) {
-                            if (pos == s) {
-                                fresh |= 1u;
-                                end = s;
-                            }
-                            border = pos;
-                            border_end = end;
-                            break;
+                            border = s + x + 1;
+                            border_end = x == -1 ? s : s + __builtin_ctz(fresh) + 1;
                         }
                     }
-                    starts = fresh;
+                    ends = fresh;
                 }
-                if (!__ballot(moved)) break;
             }
+            // token starts of the region: where one ends within it, and at s where none reaches over
+            const uint32_t starts = (ends << 1 | (border == s ? 1u : 0u)) & (cnt >= 32 ? ~0u : (1u << cnt) - 1u);
 
             // every token's number among the wave's
             const uint32_t mine = (uint32_t)__builtin_popcount(starts);
@@ -645,7 +781,7 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
             // states are read together.
             auto each_token = [&](auto f) {
                 uint32_t left = starts;
-                int end = right_end;
+                int x = right_end - s - 1;                     // the token's last byte, counted from the region's first
                 while (left) {
                     int b[4], last[4];
                     bool is[4];
@@ -653,17 +789,18 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
                         is[q] = left != 0;
-                        b[q] = is[q] ? 31 - __builtin_clz(left) : 0;
-                        last[q] = is[q] ? end - 1 : s;
+                        b[q] = 31 - __builtin_clz(left | 1u);
+                        last[q] = x;
                         left &= ~(1u << b[q]);
-                        end = s + b[q];
+                        x = b[q] - 1;
                     }
+                    // (where there is no token any more the place is that of byte -1 or of a byte of the region)
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) v[q] = number_of(state_at(last[q]));
+                    for (int q = 0; q < 4; ++q) v[q] = number_of(state[(last[q] & (P - 1)) * 64 + lane + (last[q] >> (P == 32 ? 5 : 4))]);
                     if (any_foreign) {
 #pragma unroll
                         for (int q = 0; q < 4; ++q)
-                            if (is[q] && v[q] == t.other) v[q] = t.other + 1 + src[last[q]];
+                            if (is[q] && v[q] == t.other) v[q] = t.other + 1 + src[s + last[q]];
                     }
                     if (WIDE && chunk) {
 #pragma unroll
@@ -709,11 +846,11 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
                 // the step's rows, one per lane again
                 int row_tok = 0, row_base = 0;
                 {
-                    const int at = lanes_to - lanes_own - (first > 0 ? __builtin_amdgcn_readlane(lanes_to, first - 1) : 0);
-                    const int from = lane >= first && lane < first + m ? at : 0;
-                    row_tok = __shfl((int)n_tok, from);
-                    row_base = __shfl((int)base, from);
-                    if (lane >= first && lane < first + m) {
+                    const int at = lanes_to - lanes_own - (from > 0 ? __builtin_amdgcn_readlane(lanes_to, from - 1) : 0);
+                    const int at0 = lane >= from && lane < from + m ? at : 0;
+                    row_tok = __shfl((int)n_tok, at0);
+                    row_base = __shfl((int)base, at0);
+                    if (lane >= from && lane < from + m) {
                         lengths[row_id] = row_len > kRowMax ? -1 : row_tok;
                         longest = row_tok > longest ? row_tok : longest;
                     }
@@ -729,10 +866,10 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
                     const int elem = a.pad_elem;
                     if (fits && (a.pad_stride & 3) == 0 && ((uintptr_t)a.pad_ids & (elem >= 4 ? 15 : 4 * elem - 1)) == 0 &&
                         ((uintptr_t)a.pad_mask & 3) == 0) {
-                        if (elem == 4) auto_put_rows<4>(a, t.id, staged, row_base, row_tok, first, m, row_id, lane);
-                        else if (elem == 8) auto_put_rows<8>(a, t.id, staged, row_base, row_tok, first, m, row_id, lane);
-                        else if (elem == 2) auto_put_rows<2>(a, t.id, staged, row_base, row_tok, first, m, row_id, lane);
-                        else auto_put_rows<1>(a, t.id, staged, row_base, row_tok, first, m, row_id, lane);
+                        if (elem == 4) auto_put_rows<4>(a, t.id, staged, row_base, row_tok, from, m, row_id, lane);
+                        else if (elem == 8) auto_put_rows<8>(a, t.id, staged, row_base, row_tok, from, m, row_id, lane);
+                        else if (elem == 2) auto_put_rows<2>(a, t.id, staged, row_base, row_tok, from, m, row_id, lane);
+                        else auto_put_rows<1>(a, t.id, staged, row_base, row_tok, from, m, row_id, lane);
                     } else {
                         // cell by cell: the lanes their own tokens, the row's lanes its padding and mask
                         const int64_t stride = a.pad_stride, at0 = (int64_t)row * stride;
@@ -789,7 +926,20 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
                 }
             }
             wave_phase();                                      // the wave's part of LDS is rewritten by the next step
-            first += m;
+            if (!kAhead) break;
+        }
+        if (!kAhead && first < last) {
+            // (rows of the item are left)
+        } else if (kShares && more) {
+            take_rows(row_id - lane + 64, INT64_MIN, share_from((int64_t)item + 1));
+        } else {
+            item64 += (int64_t)gridDim.x * n_waves;
+            if (item64 >= n_items) break;
+            take_item(item64);
+        }
+        if (first < last) {
+            next = place();
+            fetch(next, ahead_bytes);
         }
     }
     if (PADDED && !CHUNKS && a.max_tree) {

@@ -2401,7 +2401,7 @@ int launch_plan(int chunking, const int64_t *offsets, const BpePlan &p, int64_t 
 
 template <bool WIDE, int P, bool CHUNKS, bool CHARS, bool PADDED>
 int launch_auto_as(const dnatok_bpe_t *t, const BpeArgs &a, AutoArgs aa, const uint8_t *bytes, const int64_t *offsets,
-                   const BpePlan &p, int64_t n_rows, int64_t items, int32_t *tok_tmp, int32_t *lengths, hipStream_t s)
+                   const BpePlan &p, int64_t n_rows, int64_t max_len, int64_t total, int64_t items, int32_t *tok_tmp, int32_t *lengths, hipStream_t s)
 {
     typedef AutoLds<WIDE, P> Lds;
     auto kern = bpe_auto_kernel<WIDE, P, CHUNKS, CHARS, PADDED>;
@@ -2422,12 +2422,22 @@ int launch_auto_as(const dnatok_bpe_t *t, const BpeArgs &a, AutoArgs aa, const u
         // as give every wave its share: 4,000 rows of 200 bases 12.7 / 13.8 us, 18,000 16.9 / 18.1, 100,000 reads 57.3 /
         // 56.0; 64 reads of 100 bases by 8 workgroups / by 64: 11.1 / 10.3 us, with the vocabulary of 32,000 12.1 / 11.3,
         // its table in no L2 26.3 / 22.5.  As many rows as fit by their mean length, 20,000 reads of 100 - 300 bases:
-        // 23.1 us, their share 18.7: a wave whose rows do not fit takes two steps.)
+        // 23.1 us, their share 18.7: a wave whose rows do not fit takes two steps.)  Where that share is several steps of
+        // rows that are not all of one length, the waves get the rows of an equal share of the bytes instead: of 100,000
+        // reads of 100 - 300 bases, 25 to a wave, one wave in 25 had rows for a fourth step, and the call took the time of
+        // four (56.8 us, now 51.5; 60,000 reads 36.5 -> 31.7).  With shares of less than a step, half of the steps that
+        // held two rows hold one (4,000 rows of 20 - 2,048 bases, vocabulary of 32,000, 38.3 us by rows, 45.2 by bytes).
         const int64_t all = resident * waves, turns = (n_rows + 64 * all - 1) / (64 * all);
         const int64_t share = (n_rows + turns * all - 1) / (turns * all), spread = (n_rows + resident - 1) / resident;
         if (aa.rows > spread) aa.rows = (int32_t)spread;
-        if (aa.rows < share) aa.rows = (int32_t)share;
-        items = (n_rows + aa.rows - 1) / aa.rows;
+        if (P == 32 && aa.rows < share && total < n_rows * max_len && total > all * turns * 64 * P) {
+            items = turns * all;
+            aa.bytes_each = (total + items - 1) / items;
+            aa.rows_per_byte = (float)((double)n_rows / (double)total);
+        } else {
+            if (aa.rows < share) aa.rows = (int32_t)share;
+            items = (n_rows + aa.rows - 1) / aa.rows;
+        }
         aa.n_groups = (int32_t)items;
     }
     int64_t grid = items < resident ? items : resident;
@@ -2443,7 +2453,7 @@ template <bool WIDE>
 int run_auto(const dnatok_bpe_t *t, const BpeArgs &a, int chunking, const uint8_t *bytes, const int64_t *offsets,
              const BpePlan &p, int64_t n_rows, int64_t max_len, int64_t total, int32_t *tok_tmp, int32_t *lengths, hipStream_t s)
 {
-    AutoArgs aa{t->auto_next, t->auto_len, t->auto_sym, t->auto_id, t->auto_states, t->auto_letters, 1, 0, 0, 0, nullptr, total};
+    AutoArgs aa{t->auto_next, t->auto_len, t->auto_sym, t->auto_id, t->auto_states, t->auto_letters, 1, 0, 0, 0.0f, 0, 0, nullptr, total};
     if (chunking & 1) {
         aa.list_here = n_rows <= kAutoListRows ? 1 : 0;
         if (!aa.list_here) {
@@ -2452,10 +2462,10 @@ int run_auto(const dnatok_bpe_t *t, const BpeArgs &a, int chunking, const uint8_
         }
         if (a.pad_ids) {
             aa.zero = a.longest;                     // (see the join kernel)
-            return launch_auto_as<WIDE, 32, true, false, true>(t, a, aa, bytes, offsets, p, n_rows, p.max_items, tok_tmp, lengths, s);
+            return launch_auto_as<WIDE, 32, true, false, true>(t, a, aa, bytes, offsets, p, n_rows, max_len, total, p.max_items, tok_tmp, lengths, s);
         }
-        if (a.char_ids) return launch_auto_as<WIDE, 32, true, true, false>(t, a, aa, bytes, offsets, p, n_rows, p.max_items, tok_tmp, lengths, s);
-        return launch_auto_as<WIDE, 32, true, false, false>(t, a, aa, bytes, offsets, p, n_rows, p.max_items, tok_tmp, lengths, s);
+        if (a.char_ids) return launch_auto_as<WIDE, 32, true, true, false>(t, a, aa, bytes, offsets, p, n_rows, max_len, total, p.max_items, tok_tmp, lengths, s);
+        return launch_auto_as<WIDE, 32, true, false, false>(t, a, aa, bytes, offsets, p, n_rows, max_len, total, p.max_items, tok_tmp, lengths, s);
     }
     // Regions of 32 bytes, of 16 where a wave for every row or few rows then finds a place at once: their lanes' walks
     // are half as long.  A wave's share of the rows has to fit its 64 lanes, surely or, by the rows' mean length, nearly
@@ -2468,13 +2478,13 @@ int run_auto(const dnatok_bpe_t *t, const BpeArgs &a, int chunking, const uint8_
     const bool small = len <= 1024 && (share * ((len + 15) / 16) <= 64 || share * twice_lanes <= 2 * 48);
     aa.rows = (int32_t)(64 / (small ? (len + 15) / 16 : (len + 31) / 32));
     if (small) {
-        if (a.pad_ids) return launch_auto_as<WIDE, 16, false, false, true>(t, a, aa, bytes, offsets, p, n_rows, n_rows, tok_tmp, lengths, s);
-        if (a.char_ids) return launch_auto_as<WIDE, 16, false, true, false>(t, a, aa, bytes, offsets, p, n_rows, n_rows, tok_tmp, lengths, s);
-        return launch_auto_as<WIDE, 16, false, false, false>(t, a, aa, bytes, offsets, p, n_rows, n_rows, tok_tmp, lengths, s);
+        if (a.pad_ids) return launch_auto_as<WIDE, 16, false, false, true>(t, a, aa, bytes, offsets, p, n_rows, max_len, total, n_rows, tok_tmp, lengths, s);
+        if (a.char_ids) return launch_auto_as<WIDE, 16, false, true, false>(t, a, aa, bytes, offsets, p, n_rows, max_len, total, n_rows, tok_tmp, lengths, s);
+        return launch_auto_as<WIDE, 16, false, false, false>(t, a, aa, bytes, offsets, p, n_rows, max_len, total, n_rows, tok_tmp, lengths, s);
     }
-    if (a.pad_ids) return launch_auto_as<WIDE, 32, false, false, true>(t, a, aa, bytes, offsets, p, n_rows, n_rows, tok_tmp, lengths, s);
-    if (a.char_ids) return launch_auto_as<WIDE, 32, false, true, false>(t, a, aa, bytes, offsets, p, n_rows, n_rows, tok_tmp, lengths, s);
-    return launch_auto_as<WIDE, 32, false, false, false>(t, a, aa, bytes, offsets, p, n_rows, n_rows, tok_tmp, lengths, s);
+    if (a.pad_ids) return launch_auto_as<WIDE, 32, false, false, true>(t, a, aa, bytes, offsets, p, n_rows, max_len, total, n_rows, tok_tmp, lengths, s);
+    if (a.char_ids) return launch_auto_as<WIDE, 32, false, true, false>(t, a, aa, bytes, offsets, p, n_rows, max_len, total, n_rows, tok_tmp, lengths, s);
+    return launch_auto_as<WIDE, 32, false, false, false>(t, a, aa, bytes, offsets, p, n_rows, max_len, total, n_rows, tok_tmp, lengths, s);
 }
 
 // The work list (plan) is needed when rows are cut into chunks or left to the whole-row kernel,
