@@ -597,15 +597,32 @@ class DNATok:
         worst = t_cap
         if guess:
             t_cap = min(worst, guess + (-guess) % 128)
-        # lengths, status and the longest row share one allocation: one copy brings them to the host
-        meta = torch.empty(2 * n + 1, dtype=torch.int32, device=data.device)
+        # lengths, status, the longest row and the packer's two statistics share one allocation: one copy
+        # brings them to the host
+        meta = torch.empty(2 * n + 3, dtype=torch.int32, device=data.device)
 
         def run(cap: int, guess: int):
             out = (torch.empty((n, cap), dtype=torch.int32, device=data.device),
-                   torch.empty((n, cap), dtype=torch.uint8, device=data.device), meta[:n], meta[n:2 * n], meta[2 * n:])
+                   torch.empty((n, cap), dtype=torch.uint8, device=data.device), meta[:n], meta[n:2 * n], meta[2 * n:2 * n + 1])
             return self._kmer_enc.encode_padded(data, offsets, cap, fill_to=0, width_guess=guess, out=out)
 
-        ids, mask, lengths, status, longest = run(t_cap, guess)
+        def lay_out(ids, lengths):
+            cap = max(t_cap, int(min_width))
+            if pad_multiple > 1 and cap % pad_multiple:
+                cap += pad_multiple - cap % pad_multiple
+            row_at = torch.arange(0, n * t_cap, t_cap, dtype=torch.int64, device=ids.device)
+            return encoders.pad_rows_as(ids.view(-1), row_at, lengths, int(self.id_pad), cap, min_width=min_width,
+                                        pad_multiple=pad_multiple, pad_left=left, dtype=dtype, stats=meta[2 * n + 1:])
+
+        if plain:
+            ids, mask, lengths, status, longest = run(t_cap, guess)
+        else:
+            # The packer lays the rows out whatever comes of them, so it follows at once and the call has one wait; what
+            # the encoder writes is seen by the packer alone: no mask, and no padding up to the longest row.
+            tokens, _, lengths, _, _ = self._kmer_enc.encode_padded(
+                data, offsets, t_cap, fill_to=1, out=(torch.empty((n, t_cap), dtype=torch.int32, device=data.device), None,
+                                                      meta[:n], meta[n:2 * n], meta[2 * n:2 * n + 1]))
+            ids, mask, _ = lay_out(tokens, lengths)
         staged = None
         if host_ids and plain and guess:
             # the ids start their way down before the width is known (the rows lie only the guess
@@ -623,15 +640,11 @@ class DNATok:
                 width = int(meta_h[2 * n])
             self._kmer_widths.update(width)
             plain = width >= min_width
-        if not plain:
-            cap = max(t_cap, int(min_width))
-            if pad_multiple > 1 and cap % pad_multiple:
-                cap += pad_multiple - cap % pad_multiple
-            row_at = torch.arange(n, dtype=torch.int64, device=ids.device) * t_cap
-            ids, mask, stats = encoders.pad_rows_as(ids.view(-1), row_at, lengths, int(self.id_pad), cap,
-                                                    min_width=min_width, pad_multiple=pad_multiple, pad_left=left,
-                                                    dtype=dtype)
-            width = int(stats[1].item())
+            if not plain:
+                ids, mask, stats = lay_out(ids, lengths)
+                width = int(stats[1].item())
+        else:
+            width = int(meta_h[2 * n + 2])
         ids, mask = ids[:, :width], mask[:, :width]
         self._staged_host_ids = staged[:, :width] if staged is not None and plain else None
         bad = meta_h[n:2 * n]
