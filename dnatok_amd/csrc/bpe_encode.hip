@@ -2379,10 +2379,10 @@ int launch_lds_ltab(const BpeArgs &a, const uint8_t *bytes, const int64_t *offse
     return DNATOK_OK;
 }
 
-// The work list of rows that are cut into chunks, or are dealt by length.
-int launch_plan(int chunking, const int64_t *offsets, const BpePlan &p, int64_t n_rows, hipStream_t s)
+// The work list of rows that are cut into chunks, or are dealt by length; entries: with those of the chunks.
+int launch_plan(int chunking, const int64_t *offsets, const BpePlan &p, int64_t n_rows, bool entries, hipStream_t s)
 {
-    const int expand_here = chunking >> 1;
+    const int expand_here = entries ? chunking >> 1 : 0;
     if (n_rows >= kPlanTiledFrom) {
         const int tiles = (int)((n_rows + kPlanTile - 1) / kPlanTile);
         bpe_plan_kernel<1><<<tiles, 1024, 0, s>>>(offsets, n_rows, chunking & 1, 0, p);
@@ -2392,7 +2392,7 @@ int launch_plan(int chunking, const int64_t *offsets, const BpePlan &p, int64_t 
         bpe_plan_kernel<0><<<1, 1024, 0, s>>>(offsets, n_rows, chunking & 1, expand_here, p);
     }
     DNATOK_HIP_TRY(hipGetLastError());
-    if ((chunking & 1) && !expand_here) {
+    if ((chunking & 1) && entries && !expand_here) {
         bpe_expand_kernel<<<(int)((n_rows + 255) / 256), 256, 0, s>>>(offsets, n_rows, p);
         DNATOK_HIP_TRY(hipGetLastError());
     }
@@ -2453,11 +2453,12 @@ template <bool WIDE>
 int run_auto(const dnatok_bpe_t *t, const BpeArgs &a, int chunking, const uint8_t *bytes, const int64_t *offsets,
              const BpePlan &p, int64_t n_rows, int64_t max_len, int64_t total, int32_t *tok_tmp, int32_t *lengths, hipStream_t s)
 {
-    AutoArgs aa{t->auto_next, t->auto_len, t->auto_sym, t->auto_id, t->auto_states, t->auto_letters, 1, 0, 0, 0.0f, 0, 0, nullptr, total};
+    AutoArgs aa{t->auto_next, t->auto_len, t->auto_sym, t->auto_id, t->auto_states, t->auto_letters, 1, 0, 0, 0.0f, 0, 0, 0, nullptr, total};
     if (chunking & 1) {
         aa.list_here = n_rows <= kAutoListRows ? 1 : 0;
+        aa.entries_here = !aa.list_here && n_rows <= kAutoEntryRows ? 1 : 0;
         if (!aa.list_here) {
-            const int rc = launch_plan(chunking, offsets, p, n_rows, s);
+            const int rc = launch_plan(chunking, offsets, p, n_rows, !aa.entries_here, s);
             if (rc) return rc;
         }
         if (a.pad_ids) {
@@ -2512,7 +2513,7 @@ int run_lds_part(bool long_rows, int chunking, bool force_plan, const BpeArgs &a
             bpe_plan_in_order_kernel<<<1, 64, 0, s>>>((int32_t)n_rows, p);
             DNATOK_HIP_TRY(hipGetLastError());
         } else {
-            const int rc = launch_plan(chunking, offsets, p, n_rows, s);
+            const int rc = launch_plan(chunking, offsets, p, n_rows, true, s);
             if (rc) return rc;
         }
         if (chunking & 1) {
