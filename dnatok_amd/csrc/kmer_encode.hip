@@ -1662,8 +1662,7 @@ extern "C" int dnatok_kmer_encode_padded(const dnatok_kmer_t *t, const uint8_t *
     // A fixed width has no padding pass that would need the maximum, so the kernel itself reports it as well,
     // up the stream's tree, where that fits (16-bit fields): without the launch that clears max_len for the
     // atomics 256 rows of 6,000 bases take 8.8 instead of 12.0 us per call, 65,536 of them 163.6 instead of 171.9.
-    // Not under capture: a graph may be
-    // replayed on other streams than the one it was captured on, on several at once.
+    // Not under capture: a graph may be replayed on other streams than the one it was captured on, on several at once.
     MaxRef mref{nullptr, nullptr};
     if (to_longest || (max_len && t_cap < 0xFFFF && !stream_captures(s))) mref = max_ref_of(t, stream);
     const auto clear_max = [&]() {
