@@ -6,6 +6,7 @@
 #include <stdio.h>
 
 #include "../../include/dnatok_hip.h"
+#include "stream_slots.hpp"
 
 namespace dnatok {
 
@@ -46,6 +47,21 @@ inline int resident_workgroups(Kernel kernel, int block_threads, size_t dynamic_
         per_cu = fallback_per_cu;
     }
     return cus * per_cu;
+}
+
+// The slot of a call on stream `s` (see StreamSlots), or -1: none is left, what the stream is doing cannot be
+// told, or the handle is not one stream but each host thread's own.
+inline int table_slot(StreamSlots &slots, hipStream_t s)
+{
+    if (s == hipStreamPerThread) return -1;
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long capture = 0;
+    hipError_t e = hipStreamIsCapturing(s, &status);
+    if (e == hipSuccess && status == hipStreamCaptureStatusNone) return slots.of(s, 0);
+    if (e == hipSuccess) e = hipStreamGetCaptureInfo(s, &status, &capture);
+    if (e == hipSuccess && status == hipStreamCaptureStatusActive && capture != 0) return slots.of(s, capture);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return -1;
 }
 
 // ---- wave64 cross-lane primitives (DPP within rows of 16 lanes, readlane across rows) ----

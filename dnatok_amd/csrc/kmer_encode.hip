@@ -30,9 +30,7 @@
 #include <string.h>
 #include <algorithm>
 #include <atomic>
-#include <mutex>
 #include <stdlib.h>
-#include <unordered_map>
 #include <vector>
 
 struct dnatok_kmer_table {
@@ -50,18 +48,16 @@ struct dnatok_kmer_table {
     uint32_t fold;           // or lower case as well: fold = 0xDFDFDFDF, else 0xFFFFFFFF): digits by arithmetic
     int2 *entry;             // [5^k]  {id, 0} | {-len, offset into flat} | {INT_MIN, 0} = nothing known
     int32_t *flat;           // expansion lists
-    // Running maxima of pad-to-longest calls.  Every stream that encodes with this table gets a
-    // slot of its own (calls on one stream are ordered, calls on different streams may overlap and
-    // must not share one); a stream beyond the kMaxSlots-th is served without a slot, by a clearing
-    // launch on the caller's max_len.  A slot is two 64-bit words: the running maximum, tagged in
+    // Running maxima of the calls that report or pad to their longest row.  Calls that may be under way at once must
+    // not share one (StreamSlots); a call for which no slot is left is served without, by a clearing launch
+    // on the caller's max_len.  A slot is two 64-bit words: the running maximum, tagged in
     // its upper half with the slot's generation, and the generation itself, which the padding pass
     // of a call bumps when it is done with the maximum.  A maximum of a later call is therefore
     // larger than anything an earlier call left behind, and the slot never has to be cleared (a
     // launch saved per call; replays of a captured call stay exact).
     unsigned long long *max_slots;
     unsigned long long *max_trees;       // kTreeWords words per slot (see kmer_team_kernel)
-    mutable std::mutex slot_lock;
-    mutable std::unordered_map<void *, int> slot_of_stream;
+    mutable dnatok::StreamSlots slots;
     // Batches of up to this many rows are encoded by kmer_team_kernel (a workgroup per row); -1: as
     // many rows as workgroups of that kernel fit the chip at once.  (dnatok_kmer_table_set_team_rows)
     std::atomic<int> team_rows{-1};
@@ -70,7 +66,7 @@ struct dnatok_kmer_table {
     std::atomic<int> packed_polls{-1};
 };
 
-constexpr int kMaxSlots = 64;
+constexpr int kMaxSlots = dnatok::StreamSlots::kSlots;
 constexpr int kMaxSlotStride = 32;       // 64-bit words between two slots (one 256-byte line each)
 // A call whose kernel reports the maximum itself (kmer_team_kernel, publish) gathers it up a tree
 // of atomics (climb_max_tree): kTreeWords words per slot.
@@ -127,11 +123,11 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 __global__ void kmer_init_kernel(int32_t *max_len) { *max_len = 0; }
 
-// Where a pad-to-longest call keeps its running maximum: slot[0] = generation << 32 | maximum,
+// Where a call keeps its running maximum (a tree without a padding pass): slot[0] = generation << 32 | maximum,
 // slot[1] = generation.
 struct MaxRef {
     unsigned long long *slot;
-    unsigned long long *tree;      // kTreeWords words of the slot's stream, all zero between calls
+    unsigned long long *tree;      // kTreeWords words of the same slot, all zero between calls
 };
 
 // Where a launch puts its rows and which rows it takes.
@@ -1616,24 +1612,12 @@ extern "C" void dnatok_kmer_table_destroy(dnatok_kmer_t *t)
     delete t;
 }
 
-// Where calls on a stream keep their maximum (nulls, if the table has no slot left for the stream).
-static MaxRef max_ref_of(const dnatok_kmer_t *t, void *stream)
+// Where a call on the stream keeps its maximum (nulls: nowhere, max_len has to be cleared and takes it by atomics).
+static MaxRef max_ref_of(const dnatok_kmer_t *t, hipStream_t s)
 {
-    std::lock_guard<std::mutex> hold(t->slot_lock);
-    auto it = t->slot_of_stream.find(stream);
-    if (it == t->slot_of_stream.end() && (int)t->slot_of_stream.size() < kMaxSlots)
-        it = t->slot_of_stream.emplace(stream, (int)t->slot_of_stream.size()).first;
-    if (it == t->slot_of_stream.end()) return MaxRef{nullptr, nullptr};
-    return MaxRef{t->max_slots + (size_t)it->second * kMaxSlotStride, t->max_trees + (size_t)it->second * kTreeWords};
-}
-
-// (also where it cannot be told)
-static bool stream_captures(hipStream_t s)
-{
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
-    (void)hipGetLastError();
-    return true;
+    const int slot = table_slot(t->slots, s);
+    if (slot < 0) return MaxRef{nullptr, nullptr};
+    return MaxRef{t->max_slots + (size_t)slot * kMaxSlotStride, t->max_trees + (size_t)slot * kTreeWords};
 }
 
 extern "C" int dnatok_kmer_encode_padded(const dnatok_kmer_t *t, const uint8_t *bytes,
@@ -1660,11 +1644,10 @@ extern "C" int dnatok_kmer_encode_padded(const dnatok_kmer_t *t, const uint8_t *
     hipStream_t s = (hipStream_t)stream;
     KmerArgs a{t->digit, t->single, t->lut4, t->lut4r, t->fold, t->entry, t->flat, t->pad_id, t->missing_id};
     // A fixed width has no padding pass that would need the maximum, so the kernel itself reports it as well,
-    // up the stream's tree, where that fits (16-bit fields): without the launch that clears max_len for the
+    // up a tree, where that fits (16-bit fields): without the launch that clears max_len for the
     // atomics 256 rows of 6,000 bases take 8.8 instead of 12.0 us per call, 65,536 of them 163.6 instead of 171.9.
-    // Not under capture: a graph may be replayed on other streams than the one it was captured on, on several at once.
     MaxRef mref{nullptr, nullptr};
-    if (to_longest || (max_len && t_cap < 0xFFFF && !stream_captures(s))) mref = max_ref_of(t, stream);
+    if (to_longest || (max_len && t_cap < 0xFFFF)) mref = max_ref_of(t, s);
     const auto clear_max = [&]() {
         mref = MaxRef{nullptr, nullptr};
         if (max_len) kmer_init_kernel<<<1, 1, 0, s>>>(max_len);
@@ -1879,7 +1862,7 @@ extern "C" int dnatok_kmer_encode_padded_sized(const dnatok_kmer_t *t, const uin
     if (guess > t_cap) guess = t_cap;
     if (to_longest) fill_to = guess;
     hipStream_t s = (hipStream_t)stream;
-    const MaxRef mref = to_longest ? max_ref_of(t, stream) : MaxRef{nullptr, nullptr};
+    const MaxRef mref = to_longest ? max_ref_of(t, s) : MaxRef{nullptr, nullptr};
     if (!mref.slot && max_len) {
         kmer_init_kernel<<<1, 1, 0, s>>>(max_len);
         DNATOK_HIP_TRY(hipGetLastError());

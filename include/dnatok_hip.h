@@ -168,9 +168,12 @@ int dnatok_kmer_table_set_packed_polls(dnatok_kmer_t *t, int32_t polls);
  *              the width of the previous batch of a stream).  Rows are padded to the guess while
  *              they are written and only what is missing afterwards; a guess that is too small
  *              or too large costs time, never correctness (cells past max_len are unspecified).
- * Calls on one table may overlap on different streams (fill_to <= 0 keeps its running maximum in
- * a device word per stream); calls issued from several host threads are serialised only for the
- * moment that word is looked up. */
+ * Calls on one table may overlap on different streams, and with replays of captured calls on any stream:
+ * a call that reports or pads to its longest row finds it in device words of the table that belong to its
+ * stream, or to its stream within the graph that it was captured into (replays of one graph are ordered).
+ * The words are there for 64 streams and for 64 captures; calls beyond these, and those on hipStreamPerThread (one
+ * handle for many streams), do the same without them, by a launch or two more.  Calls issued from
+ * several host threads are serialised only for the moment the words are looked up. */
 int dnatok_kmer_encode_padded(const dnatok_kmer_t *t, const uint8_t *bytes, const int64_t *offsets,
                               int64_t n_rows, int64_t t_cap, int64_t fill_to,
                               int32_t *ids, uint8_t *mask, int32_t *lengths, int32_t *status,

@@ -1,4 +1,6 @@
 """k-mer calls whose launches depend on their arguments, against the CPU oracle.  Bit-exact."""
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -110,6 +112,91 @@ def test_kmer_fixed_width_call_replayed_from_a_graph(enc, form):
             _, rows, status = made[(first + q) % 2]
             check_fixed(out, rows, status, cap, cap)
         check_fixed(eager_out, made[2][1], made[2][2], cap, cap)
+
+
+def check_longest(out, rows, status):
+    ids, mask, lengths, st, longest = out
+    kept = [r[:ids.shape[1]] for r in rows]
+    width = max(r.size for r in kept)
+    assert int(longest.item()) == width
+    np.testing.assert_array_equal(lengths.cpu().numpy(), [r.size for r in rows])
+    np.testing.assert_array_equal(st.cpu().numpy() & 3, status & 3)
+    eids, emask = O.pad_rows(kept, 1, width)
+    np.testing.assert_array_equal(ids[:, :width].cpu().numpy(), eids)
+    np.testing.assert_array_equal(mask[:, :width].cpu().numpy(), emask)
+
+
+@pytest.mark.parametrize("form,guess", [("few", 600), ("reads", 300), ("rows", 900), ("rows", 0)])
+def test_kmer_graphs_padded_to_the_longest_row_beside_eager_calls(enc, form, guess):
+    """Captured calls that pad to their longest row (with a guess: reported by the kernel itself), replayed on other
+    streams than the one they were captured on, where eager calls of a fixed width and of the longest row are made
+    meanwhile: every call reports its own longest row, also in the rounds after."""
+    print(f"kmer padded to the longest row from graphs {form} guess={guess}", flush=True)
+    n, (lo, hi), cap = FIXED[form]
+    made = [batch(np.random.default_rng(seed).integers(lo, hi // (1 + seed % 2) + 1, size=n), seed) for seed in (31, 32, 33, 34)]
+    room = max(b.data.size for b, _, _ in made)
+    side, graphs = torch.cuda.Stream(), []
+    for _ in range(2):
+        data, off = torch.zeros(room, dtype=torch.uint8, device=DEV), torch.zeros(n + 1, dtype=torch.int64, device=DEV)
+        out = fixed_width_out(n, cap)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            enc.encode_padded(data, off, cap, width_guess=guess, out=out)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=side):
+            enc.encode_padded(data, off, cap, width_guess=guess, out=out)
+        graphs.append((g, data, off, out))
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    fixed_in, fixed = on_gpu(made[2][0]), fixed_width_out(n, cap)
+    eager_in, eager = on_gpu(made[3][0]), fixed_width_out(n, cap)
+    for first in (0, 1, 0, 1):
+        for q, (_, data, off, out) in enumerate(graphs):
+            b = made[(first + q) % 2][0]
+            data[:b.data.size].copy_(torch.from_numpy(b.data))
+            off.copy_(torch.from_numpy(b.offsets))
+            out[4].fill_(1 << 29)
+        torch.cuda.synchronize()
+        for _ in range(4):
+            for q, (g, *_) in enumerate(graphs):
+                with torch.cuda.stream(streams[q]):
+                    g.replay()
+            with torch.cuda.stream(side):
+                enc.encode_padded(*fixed_in, cap, fill_to=cap, out=fixed)
+                enc.encode_padded(*eager_in, cap, width_guess=guess, out=eager)
+        torch.cuda.synchronize()
+        for q, (_, _, _, out) in enumerate(graphs):
+            check_longest(out, *made[(first + q) % 2][1:])
+        check_fixed(fixed, made[2][1], made[2][2], cap, cap)
+        check_longest(eager, *made[3][1:])
+
+
+def test_kmer_calls_of_two_threads_on_their_own_default_streams(enc):
+    """hipStreamPerThread is one handle and a stream for every host thread: calls on it may overlap."""
+    print("kmer calls on hipStreamPerThread", flush=True)
+    n, (lo, hi), cap = FIXED["rows"]
+    made = [batch(np.random.default_rng(seed).integers(lo, hi // (1 + seed % 2) + 1, size=n), seed) for seed in (41, 42)]
+    per_thread = torch.cuda.ExternalStream(2)
+    inputs, outs, failed = [on_gpu(b) for b, _, _ in made], [fixed_width_out(n, cap) for _ in made], []
+    torch.cuda.synchronize()
+
+    def calls(q):
+        try:
+            with torch.cuda.stream(per_thread):
+                for fill_to in (cap, 0) * 10 + (cap,):
+                    enc.encode_padded(*inputs[q], cap, fill_to=fill_to, width_guess=900, out=outs[q])
+        except Exception as e:                           # (an assertion in a thread is not seen by pytest)
+            failed.append(e)
+
+    threads = [threading.Thread(target=calls, args=(q,)) for q in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not failed
+    for q in range(2):
+        check_fixed(outs[q], made[q][1], made[q][2], cap, cap)
 
 
 def check_packed(out, rows, status, total):
