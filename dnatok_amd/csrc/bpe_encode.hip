@@ -36,7 +36,6 @@
 #include <stdlib.h>
 #include <string.h>
 #include <atomic>
-#include <mutex>
 #include <new>
 #include <type_traits>
 #include <unordered_map>
@@ -62,19 +61,16 @@ struct dnatok_bpe_table {
     int32_t *auto_id;
     void *first;                 // dnatok::FirstPairs on the device, or nullptr (more bytes with rules than classes)
     // dnatok_bpe_encode_padded: the tree of atomics that carries a call's longest row
-    // (dnatok::publish_max), one per stream that encodes with this table (calls on one stream are
-    // ordered, calls on different streams may overlap); a stream beyond the kMaxTreeSlots-th gets
-    // its maximum from a launch over the lengths instead
+    // (dnatok::publish_max), of which calls that may be under way at once never share one
+    // (dnatok::StreamSlots); a call that there is none left for gets its maximum from a launch over
+    // the lengths instead
     unsigned long long *max_trees;
-    mutable std::mutex slot_lock;
-    mutable std::unordered_map<void *, int> slot_of_stream;
+    mutable dnatok::StreamSlots slots_of_calls;
     // Test and measurement switches of this table (dnatok_bpe_table_set_chunk_geometry,
     // dnatok_bpe_table_set_placement); 0 / 0 / 0 are the shipped choices.  A call reads them once,
     // when it starts.
     std::atomic<int> chunk_core{0}, chunk_overlap{0}, placement{0};
 };
-
-constexpr int kMaxTreeSlots = 64;
 
 namespace dnatok {
 
@@ -2184,7 +2180,7 @@ extern "C" int dnatok_bpe_table_create(const int32_t *byte_to_id_h, const int32_
     const size_t o_first = up(o_remap + (out_remap_h ? (size_t)n_symbols * 4 : 0));
     const size_t o_ltab = up(o_first + sizeof(FirstPairs));
     const size_t o_trees = up(o_ltab + ltab.size() * 4);
-    const size_t o_anext = up(o_trees + (size_t)kMaxTreeSlots * kTreeWords * 8);
+    const size_t o_anext = up(o_trees + (size_t)StreamSlots::kSlots * kTreeWords * 8);
     const size_t o_alen = up(o_anext + auto_n * 4 * (wide ? 4 : 2));
     const size_t o_asym = up(o_alen + auto_n);
     const size_t o_aid = up(o_asym + (auto_n ? auto_n + 256 : 0) * 2);
@@ -2778,11 +2774,8 @@ extern "C" int dnatok_bpe_encode_padded_as(const dnatok_bpe_t *t, const uint8_t 
     pad.longest = longest;
     pad.by_automaton = automaton ? 1 : 0;
     if (longest && !long_rows) {
-        std::lock_guard<std::mutex> hold(t->slot_lock);
-        auto it = t->slot_of_stream.find(stream);
-        if (it == t->slot_of_stream.end() && (int)t->slot_of_stream.size() < kMaxTreeSlots)
-            it = t->slot_of_stream.emplace(stream, (int)t->slot_of_stream.size()).first;
-        if (it != t->slot_of_stream.end()) pad.max_tree = t->max_trees + (size_t)it->second * kTreeWords;
+        const int slot = table_slot(t->slots_of_calls, s);
+        if (slot >= 0) pad.max_tree = t->max_trees + (size_t)slot * kTreeWords;
     }
     const int rc = bpe_encode_launch(t, bytes, offsets, n_rows, max_len, total, p, long_rows ? tok_tmp : nullptr, lengths, s,
                                      nullptr, nullptr, nullptr, &pad);

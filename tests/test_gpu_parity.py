@@ -1035,7 +1035,7 @@ def test_bpe_padded_in_every_layout(bpe, dtype, pad_left):
 
 def test_bpe_padded_on_two_streams_and_in_a_graph(bpe):
     """Every stream has its own tree for the longest row; replays of a captured call give the eager result each time,
-    with eager calls (which use the same tree) in between."""
+    with eager calls in between."""
     which, enc, bo = bpe
     say(f"bpe{which} padded: streams and graph")
     rng = random.Random(9)
@@ -1069,6 +1069,53 @@ def test_bpe_padded_on_two_streams_and_in_a_graph(bpe):
         for got, want in zip(out, eager):
             assert torch.equal(got, want)
         check_padded(enc, bo, seqs_b[:900], 160, ref=ref_b[:900])
+
+
+def test_bpe_padded_graph_beside_eager_calls_on_its_capture_stream(bpe):
+    """A captured call finds its longest row by itself, also while it is replayed on one stream and eager calls are
+    made on the one it was captured on."""
+    which, enc, bo = bpe
+    say(f"bpe{which} padded: a graph beside eager calls")
+    rng = random.Random(19)
+    rnd = lambda n: "".join(rng.choices("ACGT", k=n))
+    calls = []
+    for n, longest in ((700, 1000), (2500, 400)):
+        b = util.batch_from_strings([rnd(rng.randint(1, longest)) for _ in range(n)])
+        want = bo.encode_batch(b.data, b.offsets)
+        data, off = to_dev(b)
+        out = (torch.empty((n, 320), dtype=torch.int32, device=DEV), torch.empty((n, 320), dtype=torch.uint8, device=DEV),
+               torch.empty(n, dtype=torch.int32, device=DEV), torch.empty(1, dtype=torch.int32, device=DEV))
+        calls.append((data, off, longest, out, want))
+
+    def call(q):
+        data, off, longest, out, _ = calls[q]
+        enc.encode_padded(data, off, longest, 320, 0, out=out)
+
+    side, other, g = torch.cuda.Stream(), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        call(0)
+        torch.cuda.synchronize()
+        with torch.cuda.graph(g, stream=side):
+            call(0)
+    held, enc._scratch = enc._scratch, None              # (a work buffer of its own for calls that overlap the graph's)
+    for _ in range(4):
+        for _, _, _, out, _ in calls:
+            out[3].fill_(-1)
+        torch.cuda.synchronize()
+        for _ in range(4):
+            with torch.cuda.stream(other):
+                g.replay()
+            with torch.cuda.stream(side):
+                call(1)
+        torch.cuda.synchronize()
+        for _, _, _, out, want in calls:
+            assert int(out[3].item()) == max(r.size for r in want)
+            ids, mask = O.pad_rows([r[:320] for r in want], 0, 320)
+            np.testing.assert_array_equal(out[2].cpu().numpy(), [r.size for r in want])
+            np.testing.assert_array_equal(out[0].cpu().numpy(), ids)
+            np.testing.assert_array_equal(out[1].cpu().numpy(), mask)
+    del held
 
 
 def test_bpe_more_rows_of_about_one_length_than_teams(bpe):
