@@ -1964,6 +1964,7 @@ __global__ __launch_bounds__(256) void bpe_gather_wave_kernel(
 
 }  // namespace dnatok
 
+#include "bpe_shares.hpp"
 #include "bpe_automaton_kernel.hpp"
 
 namespace dnatok {
@@ -2423,18 +2424,19 @@ int launch_auto_as(const dnatok_bpe_t *t, const BpeArgs &a, AutoArgs aa, const u
         // reads of 100 - 300 bases, 25 to a wave, one wave in 25 had rows for a fourth step, and the call took the time of
         // four (56.8 us, now 51.5; 60,000 reads 36.5 -> 31.7).  With shares of less than a step, half of the steps that
         // held two rows hold one (4,000 rows of 20 - 2,048 bases, vocabulary of 32,000, 38.3 us by rows, 45.2 by bytes).
+        // (`total` is what the caller's buffer holds: the kernel looks at the bytes of the rows again.)
         const int64_t all = resident * waves, turns = (n_rows + 64 * all - 1) / (64 * all);
         const int64_t share = (n_rows + turns * all - 1) / (turns * all), spread = (n_rows + resident - 1) / resident;
         if (aa.rows > spread) aa.rows = (int32_t)spread;
         if (P == 32 && aa.rows < share && total < n_rows * max_len && total > all * turns * 64 * P) {
-            items = turns * all;
-            aa.bytes_each = (total + items - 1) / items;
-            aa.rows_per_byte = (float)((double)n_rows / (double)total);
-        } else {
-            if (aa.rows < share) aa.rows = (int32_t)share;
-            items = (n_rows + aa.rows - 1) / aa.rows;
+            aa.shares = (int32_t)(turns * all);
+            aa.share_above = all * turns * 64 * P;
+            aa.inv_shares = 1.0 / (double)aa.shares;
         }
+        if (aa.rows < share) aa.rows = (int32_t)share;
+        items = (n_rows + aa.rows - 1) / aa.rows;
         aa.n_groups = (int32_t)items;
+        if (aa.shares > items) items = aa.shares;
     }
     int64_t grid = items < resident ? items : resident;
     if (a.max_tree && grid > kTreeRows) grid = kTreeRows;
@@ -2449,7 +2451,7 @@ template <bool WIDE>
 int run_auto(const dnatok_bpe_t *t, const BpeArgs &a, int chunking, const uint8_t *bytes, const int64_t *offsets,
              const BpePlan &p, int64_t n_rows, int64_t max_len, int64_t total, int32_t *tok_tmp, int32_t *lengths, hipStream_t s)
 {
-    AutoArgs aa{t->auto_next, t->auto_len, t->auto_sym, t->auto_id, t->auto_states, t->auto_letters, 1, 0, 0, 0.0f, 0, 0, 0, nullptr, total};
+    AutoArgs aa{t->auto_next, t->auto_len, t->auto_sym, t->auto_id, t->auto_states, t->auto_letters, 1, 0, 0, 0, 0.0, 0, 0, 0, nullptr, total};
     if (chunking & 1) {
         aa.list_here = n_rows <= kAutoListRows ? 1 : 0;
         aa.entries_here = !aa.list_here && n_rows <= kAutoEntryRows ? 1 : 0;
