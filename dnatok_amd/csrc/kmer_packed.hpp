@@ -10,20 +10,28 @@
 // before its own: with every tile's word read by every later tile, 782 tiles cost more than they saved (the
 // words lie a line apart and are read past the L2: 100,000 reads 37.0 us, with blocks and larger tiles 28.3).
 //
+// (A scan in one pass whose parts look back at those in front of them is Merrill and Garland's decoupled look-back.)
+//
 // No workgroup depends on another one being on the chip: who finds a word open for too long counts the rows
-// behind it itself (their bytes say the same to everybody) and goes on.
+// behind it itself (their bytes say the same to everybody) and goes on.  It counts only tiles that have published no
+// sum of their own, and only until the word comes after all: one row that takes longer than all others would otherwise
+// have everybody behind it count the block that it is in (100,000 reads with a row of 200,000 bases in front of them
+// 518 us, now 40.6; that row behind them 171, now 45.8).
 //
 // A row of at most 64 windows (sixteen lanes, kUnitsPerLane windows to a lane) is read once: its windows' codes
 // stay in registers from the count to the output, and its few spelled windows in a list in LDS, so that the
 // output waits for no load behind its own stores.  Rows of up to twice that are walked by their sixteen lanes,
-// longer ones by a wave, once to count and once to write.
+// longer ones by a wave, from eight steps on by several, once to count and once to write.
 //
 // What bounds it: trips to memory in a row (the rows' places, their bytes in two batches, the sums, the tokens) with
 // the whole batch in flight at once (three workgroups to a CU at 80 registers; at four the compiler spills: 50,000
 // reads 29.8 instead of 22.9 us), and vector issue in the count.  Two passes of a launch each for short and for long
 // rows with two launches of a scan between them -> one launch behind the one that opens the tiles:
 // 100,000 reads of 100 - 300 bp 62.9 -> 28.3 us, 1,000 of them 22.4 -> 11.5, 300,000 139 -> 58, with 50 rows of
-// 2 - 20 kbp among 100,000 87.7 -> 41.6, 300 among 3,000 287 -> 31; 20,000 rows of 1,000 bp 42.9 -> 34.9.
+// 2 - 20 kbp among 100,000 87.7 -> 41.6, 300 among 3,000 287 -> 31; 20,000 rows of 1,000 bp 42.9 -> 34.9.  With long
+// rows shared among a workgroup's waves, on another box: 50 rows of 2 - 20 kbp among 100,000 reads 45.1 -> 30.9 us (the
+// two passes 80.9), those 50 in front and all sorted 557 -> 128 (642), a row of 1 Mbp in front 762 -> 128 (578), of
+// 5 Mbp 4,176 -> 634 (2,640), ten of 200 kbp 686 -> 283 (1,297).
 #pragma once
 
 namespace dnatok {
@@ -37,8 +45,17 @@ constexpr int kPackedPerCu = 3;                          // workgroups of a CU
 constexpr int kPackedList = 512;                         // windows spelled by characters that a tile notes for the output
 constexpr int kPackedBlock = 16;                         // tiles whose last one publishes the sum of all of them
 constexpr int kPackedPolls = 64;                         // trips without an answer until a tile is counted here
+constexpr int kPackedStep = 64 * kUnitsPerLane;          // windows of a wave's step in a long row;
+constexpr int kPackedParts = kPackedThreads / 64;        // of which there are as many parts, at most,
+constexpr int kPackedPart = 4 * kPackedStep;             // of as many windows, at least
 constexpr int64_t kTileOpen = INT64_MIN;
 constexpr int64_t kBlockSum = -((int64_t)1 << 62);       // minus a block's tokens: its last tile's word
+
+// a value that all lanes of the wave have, as a scalar (what comes out of LDS is not known to be one)
+__device__ __forceinline__ int64_t of_wave(int64_t v)
+{
+    return (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)v));
+}
 
 // the cell of out_offsets behind tile j's last row
 __device__ __forceinline__ int64_t tile_word(int64_t j, int64_t n_rows, int tile_rows)
@@ -78,8 +95,10 @@ __global__ __launch_bounds__(kPackedThreads, kPackedPerCu * kPackedThreads / 256
     __shared__ uint32_t s_len[kPackedRows];              // their tokens,
     __shared__ int64_t s_to[kPackedRows];                // of them and all rows before them in the tile
     __shared__ uint8_t s_foreign[kPackedRows];
+    __shared__ uint32_t s_part[kPackedRows][kPackedParts];   // tokens of a long row's parts
     __shared__ int64_t s_base, s_open;
-    __shared__ int s_open_tiles;
+    __shared__ int64_t s_word[kPackedBlock];
+    __shared__ int s_open_tiles, s_came;
     __shared__ unsigned long long s_sum;
     // spelled windows of the held rows: row | first token's place in it << 8, and the characters
     __shared__ uint32_t s_list_at[kPackedList], s_list_lo[kPackedList], s_list_hi[kPackedList];
@@ -101,8 +120,13 @@ __global__ __launch_bounds__(kPackedThreads, kPackedPerCu * kPackedThreads / 256
     if (LUT4_LDS)
         for (uint32_t i = threadIdx.x; i < POW4; i += kPackedThreads) s_lut4[i] = a.lut4r[i];
     const int32_t *const lut = LUT4_LDS ? s_lut4 : a.lut4r;
+    if (threadIdx.x < kPackedRows) {
+        s_len[threadIdx.x] = 0;
+        s_foreign[threadIdx.x] = 0;
+    }
     if (threadIdx.x == 0) {
         s_sum = 0;
+        s_came = 0;
         s_listed = 0;
     }
     __syncthreads();
@@ -111,7 +135,57 @@ __global__ __launch_bounds__(kPackedThreads, kPackedPerCu * kPackedThreads / 256
     const auto held = [](int len) { return len < 65 * K; };
     const auto middling = [](int len) { return len >= 65 * K && len < 129 * K; };
 
-    // count
+    // Windows [w0, w1) of the row at `at` by the whole wave: f(bytes, their windows, tokens in front of the lane's)
+    auto walk = [&](int64_t at, int w0, int w1, bool &foreign_seen, auto f) -> uint32_t {
+        uint32_t running = 0;
+        bool any = false;
+        for (int s0 = w0; s0 < w1; s0 += kPackedStep) {
+            const int first = s0 + lane * kUnitsPerLane;
+            uint32_t w[K];
+            load_lane<K>(bytes, at + (int64_t)first * K, total, first < w1, w);
+            int32_t slots[kUnitsPerLane];
+            bool foreign;
+            const uint32_t mine = lane_windows<K>(w, windows_here(w1, first), a.fold, lut, slots, foreign);
+            any = any || foreign;
+            const uint32_t inc = wave_inclusive_sum_u32(mine);
+            f(w, slots, running + inc - mine);
+            running += (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
+        }
+        foreign_seen = __ballot(any) != 0;
+        return running;
+    };
+    // The rows that are not held nor middling, in parts of which every wave takes its share: f(row, its start and length,
+    // the part and its windows [w0, w1))
+    auto each_long_part = [&](auto f) {
+        int turn = 0;
+#pragma unroll 1
+        for (int i0 = 0; i0 < rows; i0 += 64) {
+            const bool is = i0 + lane < rows && s_start[i0 + lane + 1] - s_start[i0 + lane] >= 129 * K;
+            for (uint64_t todo = __ballot(is); todo; todo &= todo - 1) {
+                const int i = i0 + __builtin_ctzll(todo);
+                const int64_t at = of_wave(s_start[i]);
+                const int n = (int)(of_wave(s_start[i + 1]) - at), full = n / K;
+                const int most = full / kPackedPart, parts = most < 1 ? 1 : most > kPackedParts ? kPackedParts : most;
+                const int each = ((full - 1) / parts / kPackedStep + 1) * kPackedStep;
+#pragma unroll 1
+                for (int part = 0; part < parts; ++part, ++turn) {
+                    if ((turn & (kPackedThreads / 64 - 1)) != wv) continue;
+                    const int w0 = part * each < full ? part * each : full;
+                    f(i, at, n, part, w0, full - w0 < each ? full : w0 + each);
+                }
+            }
+        }
+    };
+    // count (the long rows first, before the others' codes take the registers)
+    each_long_part([&](int i, int64_t at, int n, int part, int w0, int w1) {
+        bool foreign;
+        const uint32_t count = walk(at, w0, w1, foreign, [](const uint32_t (&)[K], const int32_t (&)[kUnitsPerLane], uint32_t) {});
+        if (lane == 0) {
+            s_part[i][part] = count;
+            atomicAdd(&s_len[i], count + (uint32_t)(part == 0 ? n % K : 0));
+            if (foreign) s_foreign[i] = 1;
+        }
+    });
     const int sets = tile_rows / kPackedGroups;          // rows of a group
     uint32_t codes[kPackedHeld][kUnitsPerLane / 2];      // of the lane's windows, two to a word
     uint8_t kinds[kPackedHeld];                          // which of them are spelled (four bits) | how many there are << 4
@@ -231,39 +305,6 @@ __global__ __launch_bounds__(kPackedThreads, kPackedPerCu * kPackedThreads / 256
             if (is) g(i, start, len, running + (uint32_t)(len % K), bad != 0);
         }
     };
-    // A row by the whole wave, 64 * kUnitsPerLane windows to a step: f(bytes, their windows, tokens in front of the lane's)
-    auto walk_row = [&](int64_t at, int n, bool &row_foreign, auto f) -> uint32_t {
-        const int full = n / K;
-        uint32_t running = 0;
-        bool any = false;
-        for (int s0 = 0; s0 < full; s0 += 64 * kUnitsPerLane) {
-            const int first = s0 + lane * kUnitsPerLane;
-            uint32_t w[K];
-            load_lane<K>(bytes, at + (int64_t)first * K, total, first < full, w);
-            int32_t slots[kUnitsPerLane];
-            bool foreign;
-            const uint32_t mine = lane_windows<K>(w, windows_here(full, first), a.fold, lut, slots, foreign);
-            any = any || foreign;
-            const uint32_t inc = wave_inclusive_sum_u32(mine);
-            f(w, slots, running + inc - mine);
-            running += (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
-        }
-        row_foreign = __ballot(any) != 0;
-        return running + (uint32_t)(n - full * K);
-    };
-    // the rows that are not held, a wave each
-    auto each_long_row = [&](auto f) {
-#pragma unroll 1
-        for (int i0 = 0; i0 < rows; i0 += 64) {
-            const bool is = i0 + lane < rows && s_start[i0 + lane + 1] - s_start[i0 + lane] >= 129 * K;
-            int turn = 0;
-            for (uint64_t todo = __ballot(is); todo; todo &= todo - 1, ++turn) {
-                if ((turn & (kPackedThreads / 64 - 1)) != wv) continue;
-                const int i = i0 + __builtin_ctzll(todo);
-                f(i, s_start[i], (int)(s_start[i + 1] - s_start[i]));
-            }
-        }
-    };
     each_middling_row([](int, const uint32_t (&)[K], const int32_t (&)[kUnitsPerLane], uint32_t) {},
                       [&](int i, int64_t, int, uint32_t count, bool foreign) {
                           if (gl == 0) {
@@ -271,14 +312,6 @@ __global__ __launch_bounds__(kPackedThreads, kPackedPerCu * kPackedThreads / 256
                               s_foreign[i] = foreign ? 1 : 0;
                           }
                       });
-    each_long_row([&](int i, int64_t at, int n) {
-        bool foreign;
-        const uint32_t count = walk_row(at, n, foreign, [](const uint32_t (&)[K], const int32_t (&)[kUnitsPerLane], uint32_t) {});
-        if (lane == 0) {
-            s_len[i] = count;
-            s_foreign[i] = foreign ? 1 : 0;
-        }
-    });
     __syncthreads();
 
     // A row's tokens and those of all rows before it in the tile; the tile's sum is published, and the sums in front of
@@ -376,23 +409,53 @@ __global__ __launch_bounds__(kPackedThreads, kPackedPerCu * kPackedThreads / 256
                 s_base = before;
                 if (open < 0) agent_store(out_offsets + tile_word(tile, n_rows, tile_rows), before + own);
             }
+            if (lane < open_tiles) s_word[lane] = agent_load(out_offsets + (open + lane + 1) * tile_rows);      // (never the batch's last tile)
         }
         __syncthreads();
-        const int64_t open = s_open;
+        const int64_t open = of_wave(s_open);
         if (open < 0) break;
-        // nobody has counted these tiles: their rows' tokens, a row to a wave
-        const int64_t open0 = open * tile_rows, open1 = (open + s_open_tiles) * tile_rows;      // (never the batch's last tile)
-        for (int64_t i = open0 + wv; i < open1; i += kPackedThreads / 64) {
-            const int64_t at = offsets[i];
-            bool foreign;
-            const uint32_t count = walk_row(at, (int)(offsets[i + 1] - at), foreign, [](const uint32_t (&)[K], const int32_t (&)[kUnitsPerLane], uint32_t) {});
-            if (lane == 0) atomicAdd(&s_sum, (unsigned long long)count);
+        // Nobody has published the sum of these tiles: the tokens of the rows of those whose own is not known either, a row
+        // to a wave, for as long as the word that is waited for does not come.
+        const int open_tiles = __builtin_amdgcn_readfirstlane(s_open_tiles);
+        int64_t *const awaited = out_offsets + (open + open_tiles) * tile_rows;
+        bool came = false;
+        for (int q = 0; q < open_tiles && !came; ++q) {
+            const int64_t word = of_wave(s_word[q]);
+            if (word < 0 && word > kBlockSum) {
+                if (threadIdx.x == 0) atomicAdd(&s_sum, (unsigned long long)(-1 - word));
+                continue;
+            }
+            for (int i = wv; i < tile_rows && !came; i += kPackedThreads / 64) {
+                const int64_t row = (open + q) * tile_rows + i, at = of_wave(offsets[row]);
+                const int n = (int)(of_wave(offsets[row + 1]) - at), full = n / K;
+                // (a byte at a time: the held rows' codes have the registers)
+                uint32_t count = lane == 0 ? (uint32_t)(n % K) : 0u;
+#pragma unroll 1
+                for (int w0 = 0; w0 < full && !came; w0 += 64) {
+                    came = __builtin_amdgcn_readfirstlane(agent_load(awaited) == kTileOpen ? 0 : 1) != 0;
+                    if (w0 + lane >= full) continue;
+                    uint32_t code = 0, odd = 0;
+#pragma unroll 1
+                    for (int b = 0; b < K; ++b) {
+                        const uint32_t v = bytes[at + (int64_t)(w0 + lane) * K + b], d = v >> 1 & 3u;
+                        odd |= (v ^ (0x47544341u >> (8 * d) & 255u)) & a.fold & 255u;
+                        code |= d << (2 * b);
+                    }
+                    count += odd || lut[code] < 0 ? K : 1;
+                }
+                count = wave_inclusive_sum_u32(count);
+                if (lane == 63) atomicAdd(&s_sum, (unsigned long long)count);
+            }
         }
+        if (came && lane == 0) s_came = 1;
         __syncthreads();
         if (threadIdx.x == 0) {
-            const int64_t word = s_open_tiles == 1 ? -1 - (int64_t)s_sum : kBlockSum - (int64_t)s_sum;
-            atomicCAS(reinterpret_cast<unsigned long long *>(out_offsets + open1), (unsigned long long)kTileOpen, (unsigned long long)word);
+            if (!s_came) {
+                const int64_t word = open_tiles == 1 ? -1 - (int64_t)s_sum : kBlockSum - (int64_t)s_sum;
+                atomicCAS(reinterpret_cast<unsigned long long *>(awaited), (unsigned long long)kTileOpen, (unsigned long long)word);
+            }
             s_sum = 0;
+            s_came = 0;
         }
     }
 
@@ -468,15 +531,19 @@ __global__ __launch_bounds__(kPackedThreads, kPackedPerCu * kPackedThreads / 256
             const int tail = len % K;
             if (gl < tail) (ids + base + s_to[i])[gl - tail] = s_single[bytes[start + len - tail + gl]];
         });
-    each_long_row([&](int i, int64_t start, int len) {
-        int32_t *const row = ids + base + s_to[i] - s_len[i];
+    each_long_part([&](int i, int64_t start, int len, int part, int w0, int w1) {
+        int32_t *const end = ids + base + of_wave(s_to[i]);
+        uint32_t before = 0;
+        for (int q = 0; q < part; ++q) before += s_part[i][q];
+        before = (uint32_t)__builtin_amdgcn_readfirstlane((int)before);
+        int32_t *const first = end - s_len[i] + before;
         bool foreign;
-        walk_row(start, len, foreign, [&](const uint32_t (&b)[K], const int32_t (&win)[kUnitsPerLane], uint32_t at) {
-            put_plain(row + at, win);
-            put_spelled(row + at, b, win);
+        walk(start, w0, w1, foreign, [&](const uint32_t (&b)[K], const int32_t (&win)[kUnitsPerLane], uint32_t at) {
+            put_plain(first + at, win);
+            put_spelled(first + at, b, win);
         });
         const int tail = len % K;
-        if (lane < tail) (ids + base + s_to[i])[lane - tail] = s_single[bytes[start + len - tail + lane]];
+        if (part == 0 && lane < tail) end[lane - tail] = s_single[bytes[start + len - tail + lane]];
     });
     if ((int)threadIdx.x < rows) {
         const int i = threadIdx.x;

@@ -275,6 +275,58 @@ def test_kmer_packed_reads_of_other_k(k):
     check_packed(out, rows, status, b.data.size)
 
 
+@pytest.mark.parametrize("k,polls", [(2, -1), (3, -1), (5, -1), (6, -1), (6, 0), (7, -1), (8, -1), (8, 0)])
+def test_kmer_packed_long_rows_in_parts(k, polls):
+    """Rows that several waves share, at the borders where a part more begins and where a part is empty, beside each
+    other and among reads; also counted by those that find a sum missing."""
+    print(f"kmer packed, long rows k={k} polls={polls}", flush=True)
+    vocab = hf.kmer_vocab(k)
+    t = kmer_tables.tables_from_vocab(vocab, k, 0)
+    e = encoders.KmerEncoder(k, t.digit, t.kmer_lut, t.single, pad_id=1, missing_id=0, exp_off=t.exp_off, exp_len=t.exp_len, exp_flat=t.exp_flat)
+    rng = np.random.default_rng(k)
+    n = 9000
+    lens = rng.integers(0, 40 * k, size=n)
+    windows = [1023, 1024, 1025, 2047, 2048, 2049, 2304, 3071, 3072, 6 * 1024 + 1, 7 * 1024, 8 * 1024 - 1, 8 * 1024, 8 * 1024 + 1, 9 * 1024, 40001]
+    long = [w * k + int(rng.integers(0, k)) for w in windows] + [2048 * k + k - 1]
+    lens[:5] = long[-5:]
+    lens[4000:4000 + len(long)] = long
+    lens[n - 1] = 2049 * k
+    text = rng.choice(np.frombuffer(b"ACGTNx", dtype=np.uint8), p=[.248, .248, .248, .248, .007, .001], size=int(lens.sum()))
+    at = int(lens[:4003].sum())
+    text[at:at + int(lens[4003])] = np.where(np.isin(text[at:at + int(lens[4003])], list(b"Nx")), ord("A"), text[at:at + int(lens[4003])])
+    offsets = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    rows, status = O.kmer_encode(O.kmer_tables_from_vocab(vocab, k, 0), text, offsets)
+    out = packed_out(n, text.size)
+    e.set_packed_polls(polls)
+    e.encode_packed(torch.from_numpy(text).to(DEV), torch.from_numpy(offsets).to(DEV), want_mask=True, out=out)
+    torch.cuda.synchronize()
+    check_packed(out, rows, status, text.size)
+
+
+def test_kmer_packed_reads_behind_a_long_row_wait_for_it(enc):
+    """A row that takes longer than all others costs about the same in front of them as behind them (three times as
+    much where everybody behind it counted the rows around it)."""
+    print("kmer packed, a long row in front", flush=True)
+    rng = np.random.default_rng(8)
+    reads = rng.integers(100, 301, size=100000)
+    took = []
+    for lens in (np.concatenate([[200000], reads]), np.concatenate([reads, [200000]])):
+        off = torch.from_numpy(np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)).to(DEV)
+        data = torch.from_numpy(rng.choice(np.frombuffer(b"ACGT", dtype=np.uint8), size=int(lens.sum()))).to(DEV)
+        out = packed_out(lens.size, int(lens.sum()))
+        least = float("inf")
+        for _ in range(8):
+            began, ended = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            began.record()
+            for _ in range(4):
+                enc.encode_packed(data, off, out=out)
+            ended.record()
+            torch.cuda.synchronize()
+            least = min(least, began.elapsed_time(ended))
+        took.append(least)
+    assert took[0] < 2 * took[1]
+
+
 def test_kmer_packed_reads_replayed_from_a_graph(enc):
     print("kmer packed from a graph", flush=True)
     n = 9000
