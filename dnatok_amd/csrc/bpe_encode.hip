@@ -2407,6 +2407,10 @@ int launch_auto_as(const dnatok_bpe_t *t, const BpeArgs &a, AutoArgs aa, const u
     if (!attr_set.load(std::memory_order_acquire)) {
         DNATOK_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)kAutoLdsBytes));
+        // (its table is read from address 0 of LDS on, where the dynamic array begins if there is no other: lds_u16)
+        hipFuncAttributes attr;
+        DNATOK_HIP_TRY(hipFuncGetAttributes(&attr, reinterpret_cast<const void *>(kern)));
+        DNATOK_REQUIRE(attr.sharedSizeBytes == 0, DNATOK_E_INVALID, "bpe_auto_kernel: LDS in front of its table");
         attr_set.store(true, std::memory_order_release);
     }
     const int waves = Lds::waves(t->auto_states);
