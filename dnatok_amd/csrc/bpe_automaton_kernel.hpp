@@ -60,7 +60,7 @@ struct AutoArgs {
     double inv_shares;           // 1 / shares
     int32_t window;              // tokens a wave has room for on their way out
     int32_t list_here;           // (chunks) the kernel makes the work list itself: at most kAutoListRows rows
-    int32_t entries_here;        // (chunks) the list says where a row's chunks begin, their entries are written here: at most kAutoEntryRows rows
+    int32_t entries_here;        // (chunks) the list says where a row's chunks begin, their entries are written here (auto_entries_here)
     int32_t *zero;               // (chunks) a word to be cleared for the kernels behind this one, or null
     int64_t total;               // bytes of the batch
 };
@@ -112,9 +112,18 @@ constexpr int kRepeatsFrom = 128;
 constexpr int kAutoListRows = 256;
 
 // Up to this many rows a wave finds its chunk's row among the rows' first chunks (two trips, where the list's entry is
-// one) and writes the entry for the kernels behind; with more, bpe_expand_kernel has written the entries.  (A launch less:
-// 500 rows of 5 kbp 30.9 -> 30.0 us, 4,096 ragged reads of 12 Mbp 79.5 -> 78.9.)
+// one) and writes the entry for the kernels behind; with more, bpe_expand_kernel has written the entries.  A launch less,
+// or the work list's kernel without that part: 2,000 rows of 5 kbp 53.5 -> 50.2 us, 900 of 20 kbp 77.2 -> 72.8, 2,500 of 4 kbp
+// 59.2 -> 53.6, 4,096 ragged reads of 12 Mbp 54.4 -> 53.9 (one call on its own).  The search is made for every chunk and its
+// trips grow with the rows, so a batch of many rows stays with the entries where a wave has a third chunk: 3,000 rows of
+// 5 kbp 65.8 us, searched for 67.0, 4,096 of them 75.7 / 76.7, 4,097 78.5 / 83.2, 16,384 241.7 / 253.2, 50,000 ragged 425.8 / 444.9.
 constexpr int kAutoEntryRows = 4096;
+constexpr int kAutoEntryManyRows = 2048;                   // from here on
+constexpr int kAutoEntryChunks = 7168;                     // as many chunks by the batch's bytes (about 8,192 with what the rows' ends leave), two to a wave
+inline bool auto_entries_here(int64_t n_rows, int64_t total, int64_t core)
+{
+    return n_rows > kAutoListRows && n_rows <= kAutoEntryRows && (n_rows <= kAutoEntryManyRows || total <= kAutoEntryChunks * core);
+}
 
 constexpr uint32_t kXcds = 8;                    // (workgroups go to them in turn)
 

@@ -2458,7 +2458,7 @@ int run_auto(const dnatok_bpe_t *t, const BpeArgs &a, int chunking, const uint8_
     AutoArgs aa{t->auto_next, t->auto_len, t->auto_sym, t->auto_id, t->auto_states, t->auto_letters, 1, 0, 0, 0, 0.0, 0, 0, 0, nullptr, total};
     if (chunking & 1) {
         aa.list_here = n_rows <= kAutoListRows ? 1 : 0;
-        aa.entries_here = !aa.list_here && n_rows <= kAutoEntryRows ? 1 : 0;
+        aa.entries_here = auto_entries_here(n_rows, total, p.core) ? 1 : 0;
         if (!aa.list_here) {
             const int rc = launch_plan(chunking, offsets, p, n_rows, !aa.entries_here, s);
             if (rc) return rc;

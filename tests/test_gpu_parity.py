@@ -1256,6 +1256,28 @@ def call_us(call, reps=20):
     return best
 
 
+@pytest.mark.parametrize("n,most", [(2048, 12400), (2049, 10000), (2049, 11500), (4096, 4900), (4096, 5600), (4097, 4900)])
+def test_bpe_chunks_found_by_the_kernel_or_in_the_list(bpe, n, most):
+    """Batches on both sides of the lines between chunks whose rows the kernel looks for and chunks whose entries a launch
+    in front has written (more than 2,048 rows of more than 7,168 chunks' bytes, or more than 4,096 rows), with rows that are no chunks
+    among them and at both ends."""
+    which, enc, bo = bpe
+    say(f"bpe{which} chunks of {n} rows of up to {most} bases")
+    rng = np.random.default_rng(n + most)
+    lens = rng.integers(most // 3, most + 1, size=n)
+    lens[rng.integers(0, n, size=n // 8)] = rng.integers(0, 2049, size=n // 8)
+    lens[0], lens[n - 1] = 0, 2048
+    offsets = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    host = rng.choice(np.frombuffer(b"ACGTN", dtype=np.uint8), p=[.25, .25, .25, .2498, .0002], size=int(offsets[-1]))
+    rows = bo.encode_batch(host, offsets)
+    want = np.array([r.size for r in rows])
+    tok, lengths = enc.encode(torch.from_numpy(host).to(DEV), torch.from_numpy(offsets).to(DEV), int(lens.max()))
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(lengths.cpu().numpy(), want)
+    at = np.repeat(offsets[:-1] - np.concatenate([[0], np.cumsum(want)[:-1]]), want) + np.arange(int(want.sum()))
+    np.testing.assert_array_equal(tok.cpu().numpy()[at], np.concatenate(rows))
+
+
 @pytest.mark.parametrize("others", [2, 300])
 def test_bpe_rows_of_a_thousand_chunks(bpe, others):
     """Rows of so many chunks that their counts are scanned by a launch of their own, beside short rows
