@@ -135,6 +135,21 @@ __global__ __launch_bounds__(kPackedThreads, kPackedPerCu * kPackedThreads / 256
     const auto held = [](int len) { return len < 65 * K; };
     const auto middling = [](int len) { return len >= 65 * K && len < 129 * K; };
 
+    // A lane's bytes.  (It reads on behind its row's end, but not behind the batch's: only the rows at its very end have to look.)
+    const bool roomy = s_start[rows] + kUnitsPerLane * K <= total;
+    auto lane_bytes = [&](int64_t pos, bool wanted, uint32_t (&w)[K]) {
+        if (roomy) {
+#pragma unroll
+            for (int q = 0; q < K; ++q) w[q] = 0;
+            if (wanted) {
+                const LaneBytes<K> all = *reinterpret_cast<const LaneBytes<K> *>(bytes + pos);
+#pragma unroll
+                for (int q = 0; q < K; ++q) w[q] = all.v[q];
+            }
+        } else {
+            load_lane<K>(bytes, pos, total, wanted, w);
+        }
+    };
     // Windows [w0, w1) of the row at `at` by the whole wave: f(bytes, their windows, tokens in front of the lane's)
     auto walk = [&](int64_t at, int w0, int w1, bool &foreign_seen, auto f) -> uint32_t {
         uint32_t running = 0;
@@ -142,7 +157,7 @@ __global__ __launch_bounds__(kPackedThreads, kPackedPerCu * kPackedThreads / 256
         for (int s0 = w0; s0 < w1; s0 += kPackedStep) {
             const int first = s0 + lane * kUnitsPerLane;
             uint32_t w[K];
-            load_lane<K>(bytes, at + (int64_t)first * K, total, first < w1, w);
+            lane_bytes(at + (int64_t)first * K, first < w1, w);
             int32_t slots[kUnitsPerLane];
             bool foreign;
             const uint32_t mine = lane_windows<K>(w, windows_here(w1, first), a.fold, lut, slots, foreign);
@@ -154,24 +169,40 @@ __global__ __launch_bounds__(kPackedThreads, kPackedPerCu * kPackedThreads / 256
         foreign_seen = __ballot(any) != 0;
         return running;
     };
-    // The rows that are not held nor middling, in parts of which every wave takes its share: f(row, its start and length,
-    // the part and its windows [w0, w1))
+    // The rows that are not held nor middling, of which every wave takes its share, those of several parts part by part:
+    // f(row, its start and length, the part and its windows [w0, w1)).  (A wave picks its rows out of all by
+    // their number: stepping over the others, a few scalar instructions each, took as long as four rows of its own.)
     auto each_long_part = [&](auto f) {
         int turn = 0;
 #pragma unroll 1
         for (int i0 = 0; i0 < rows; i0 += 64) {
-            const bool is = i0 + lane < rows && s_start[i0 + lane + 1] - s_start[i0 + lane] >= 129 * K;
-            for (uint64_t todo = __ballot(is); todo; todo &= todo - 1) {
-                const int i = i0 + __builtin_ctzll(todo);
-                const int64_t at = of_wave(s_start[i]);
-                const int n = (int)(of_wave(s_start[i + 1]) - at), full = n / K;
-                const int most = full / kPackedPart, parts = most < 1 ? 1 : most > kPackedParts ? kPackedParts : most;
+            int64_t start = 0;
+            int len = 0;
+            if (i0 + lane < rows) {
+                start = s_start[i0 + lane];
+                len = (int)(s_start[i0 + lane + 1] - start);
+            }
+            const bool in_parts = len / K >= 2 * kPackedPart, whole = len >= 129 * K && !in_parts;
+            const uint64_t wholes = __ballot(whole);
+            const int number = turn + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(wholes >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)wholes, 0u));
+            turn += (int)__builtin_popcountll(wholes);
+            const auto start_of = [&](int at) {
+                return (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(start >> 32), at) << 32 |
+                                 (uint32_t)__builtin_amdgcn_readlane((int)start, at));
+            };
+            for (uint64_t todo = __ballot(whole && (number & (kPackedThreads / 64 - 1)) == wv); todo; todo &= todo - 1) {
+                const int at = __builtin_ctzll(todo), n = __builtin_amdgcn_readlane(len, at);
+                f(i0 + at, start_of(at), n, 0, 0, n / K);
+            }
+            for (uint64_t todo = __ballot(in_parts); todo; todo &= todo - 1) {
+                const int at = __builtin_ctzll(todo), n = __builtin_amdgcn_readlane(len, at), full = n / K;
+                const int most = full / kPackedPart, parts = most > kPackedParts ? kPackedParts : most;
                 const int each = ((full - 1) / parts / kPackedStep + 1) * kPackedStep;
 #pragma unroll 1
                 for (int part = 0; part < parts; ++part, ++turn) {
                     if ((turn & (kPackedThreads / 64 - 1)) != wv) continue;
                     const int w0 = part * each < full ? part * each : full;
-                    f(i, at, n, part, w0, full - w0 < each ? full : w0 + each);
+                    f(i0 + at, start_of(at), n, part, w0, full - w0 < each ? full : w0 + each);
                 }
             }
         }
@@ -191,12 +222,10 @@ __global__ __launch_bounds__(kPackedThreads, kPackedPerCu * kPackedThreads / 256
     uint8_t kinds[kPackedHeld];                          // which of them are spelled (four bits) | how many there are << 4
     uint16_t from[kPackedHeld];                          // tokens of the row in front of the lane's
     uint8_t tail_byte[kPackedHeld];                      // a trailing character (lanes below the tail's length)
-    const bool roomy = s_start[rows] + kUnitsPerLane * K <= total;
 #pragma unroll
     for (int r0 = 0; r0 < kPackedHeld; r0 += kPackedBatch) {
         if (r0 >= sets) break;
-        // The bytes of a batch of rows first, so that they are one trip to memory.  (A lane reads on behind its row's
-        // end, but not behind the batch's: only the rows at its very end have to look.)
+        // The bytes of a batch of rows first, so that they are one trip to memory.
         uint32_t w[kPackedBatch][K];
 #pragma unroll
         for (int b = 0; b < kPackedBatch; ++b) {
@@ -205,17 +234,7 @@ __global__ __launch_bounds__(kPackedThreads, kPackedPerCu * kPackedThreads / 256
             const int len = i < rows ? (int)(s_start[i + 1] - start) : 0;
             const bool here = held(len) && gl * kUnitsPerLane * K + K <= len;
             const int64_t pos = start + gl * (kUnitsPerLane * K);
-            if (roomy) {
-#pragma unroll
-                for (int q = 0; q < K; ++q) w[b][q] = 0;
-                if (here) {
-                    const LaneBytes<K> all = *reinterpret_cast<const LaneBytes<K> *>(bytes + pos);
-#pragma unroll
-                    for (int q = 0; q < K; ++q) w[b][q] = all.v[q];
-                }
-            } else {
-                load_lane<K>(bytes, pos, total, here, w[b]);
-            }
+            lane_bytes(pos, here, w[b]);
             tail_byte[r] = 0;
             if (gl < len % K) tail_byte[r] = bytes[start + len - len % K + gl];
         }
@@ -292,7 +311,7 @@ __global__ __launch_bounds__(kPackedThreads, kPackedPerCu * kPackedThreads / 256
             for (int s0 = 0; s0 < 128; s0 += 64) {
                 const int first = s0 + gl * kUnitsPerLane;
                 uint32_t w[K];
-                load_lane<K>(bytes, start + (int64_t)first * K, total, first < full, w);
+                lane_bytes(start + (int64_t)first * K, first < full, w);
                 int32_t slots[kUnitsPerLane];
                 bool foreign;
                 const uint32_t mine = lane_windows<K>(w, windows_here(full, first), a.fold, lut, slots, foreign);
@@ -517,7 +536,7 @@ __global__ __launch_bounds__(kPackedThreads, kPackedPerCu * kPackedThreads / 256
             uint32_t b[K];
             int32_t win[kUnitsPerLane];
             windows_of(r, win);
-            load_lane<K>(bytes, s_start[i] + gl * (kUnitsPerLane * K), total, win[0] != kNothing, b);
+            lane_bytes(s_start[i] + gl * (kUnitsPerLane * K), win[0] != kNothing, b);
             put_spelled(ids + base + s_to[i] - s_len[i] + from[r], b, win);
         }
     }
@@ -537,13 +556,15 @@ __global__ __launch_bounds__(kPackedThreads, kPackedPerCu * kPackedThreads / 256
         for (int q = 0; q < part; ++q) before += s_part[i][q];
         before = (uint32_t)__builtin_amdgcn_readfirstlane((int)before);
         int32_t *const first = end - s_len[i] + before;
+        // (the trailing characters are requested in front of the walk: behind its stores they are another trip)
+        const int tail = part == 0 ? len % K : 0;
+        const uint8_t tail_at = lane < tail ? bytes[start + len - tail + lane] : (uint8_t)0;
         bool foreign;
         walk(start, w0, w1, foreign, [&](const uint32_t (&b)[K], const int32_t (&win)[kUnitsPerLane], uint32_t at) {
             put_plain(first + at, win);
             put_spelled(first + at, b, win);
         });
-        const int tail = len % K;
-        if (part == 0 && lane < tail) end[lane - tail] = s_single[bytes[start + len - tail + lane]];
+        if (lane < tail) end[lane - tail] = s_single[tail_at];
     });
     if ((int)threadIdx.x < rows) {
         const int i = threadIdx.x;
