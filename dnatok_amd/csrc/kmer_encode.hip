@@ -1756,8 +1756,10 @@ int launch_scan_lengths(const int32_t *lengths, int64_t n_rows, int64_t *out_off
                         size_t scratch_bytes, hipStream_t s);   // pack.hip
 }
 
-// The rows of at most kGroupsMaxUnits units, by kmer_groups_kernel.  The longest row, where asked for, goes to
-// mref.slot / max_len by atomicMax (no tree: two launches share a call).
+// The rows of at most kGroupsMaxUnits units, by kmer_groups_kernel.  The longest of them, where asked for, goes to max_len,
+// up mref.tree if there is one.  (Their waves are nearly all done at once, and then thousands of them find
+// max_len too small: 20,000 rows of 1,900 - 2,100 bases 62 us by atomicMax, 28.5 up the tree; of 1,000 - 3,000 with k = 8,
+// padded to the longest, 62 -> 42.4.)
 static int launch_short_rows(const dnatok_kmer_t *t, const uint8_t *bytes, const int64_t *offsets, int64_t n_rows,
                              int64_t t_cap, int64_t fill_to, int32_t *ids, uint8_t *mask, int32_t *lengths,
                              int32_t *status, int32_t *max_len, MaxRef mref, hipStream_t s)
@@ -1768,8 +1770,10 @@ static int launch_short_rows(const dnatok_kmer_t *t, const uint8_t *bytes, const
         static const int resident = resident_workgroups(kmer_groups_kernel<KK, L, M>, kGroupThreads, 0, 8); \
         int64_t grid = (n_rows + kGroupThreads / 16 - 1) / (kGroupThreads / 16);                  \
         if (grid > resident) grid = resident;                                                     \
+        if (grid > kTreeRows) grid = kTreeRows;                                                   \
         kmer_groups_kernel<KK, L, M><<<(int)grid, kGroupThreads, 0, s>>>(                         \
-            a, bytes, offsets, n_rows, t_cap, fill_to, ids, mask, lengths, status, max_len, mref, 0, 1); \
+            a, bytes, offsets, n_rows, t_cap, fill_to, ids, mask, lengths, status, max_len, MaxRef{nullptr, mref.tree}, \
+            mref.tree ? 1 : 0, 1);                                                                \
     } while (0)
 #define PG(KK, L)                                                                                 \
     do {                                                                                          \
@@ -1790,7 +1794,8 @@ static int launch_short_rows(const dnatok_kmer_t *t, const uint8_t *bytes, const
     return DNATOK_OK;
 }
 
-// One launch of kmer_rows_kernel<..., PLACED> with a RowPlace; the longest row as above.
+// One launch of kmer_rows_kernel<..., PLACED> with a RowPlace.  The longest row, where asked for, goes to mref.slot or
+// max_len by atomicMax.
 static int launch_placed(const dnatok_kmer_t *t, const uint8_t *bytes, const int64_t *offsets, int64_t n_rows,
                          int64_t t_cap, int64_t fill_to, int32_t *ids, uint8_t *mask, int32_t *lengths,
                          int32_t *status, int32_t *max_len, MaxRef mref, RowPlace place, hipStream_t s)
@@ -1862,17 +1867,18 @@ extern "C" int dnatok_kmer_encode_padded_sized(const dnatok_kmer_t *t, const uin
     if (guess > t_cap) guess = t_cap;
     if (to_longest) fill_to = guess;
     hipStream_t s = (hipStream_t)stream;
-    const MaxRef mref = to_longest ? max_ref_of(t, s) : MaxRef{nullptr, nullptr};
-    if (!mref.slot && max_len) {
+    // the first launch writes max_len (or it is cleared and takes the maximum by atomics), the second raises it
+    const MaxRef none{nullptr, nullptr}, mref = max_len ? max_ref_of(t, s) : none;
+    if (!mref.tree && max_len) {
         kmer_init_kernel<<<1, 1, 0, s>>>(max_len);
         DNATOK_HIP_TRY(hipGetLastError());
     }
     int rc = launch_short_rows(t, bytes, offsets, n_rows, t_cap, fill_to, ids, mask, lengths, status, max_len, mref, s);
     if (rc) return rc;
-    rc = launch_placed(t, bytes, offsets, n_rows, t_cap, fill_to, ids, mask, lengths, status, max_len, mref,
+    rc = launch_placed(t, bytes, offsets, n_rows, t_cap, fill_to, ids, mask, lengths, status, max_len, none,
                        RowPlace{nullptr, 1, 0}, s);
     if (rc) return rc;
-    if (to_longest) return launch_pad(ids, mask, lengths, n_rows, t_cap, max_len, t->pad_id, (int32_t)guess, mref, s);
+    if (to_longest) return launch_pad(ids, mask, lengths, n_rows, t_cap, max_len, t->pad_id, (int32_t)guess, none, s);
     return DNATOK_OK;
 }
 

@@ -73,6 +73,31 @@ def test_kmer_fixed_width_reports_the_longest_row(enc, form):
         check_fixed(out, rows, status, cap, fill_to)
 
 
+def test_kmer_longest_row_of_a_batch_split_by_class_costs_little(enc):
+    """Thousands of waves that are done at once do not raise the maximum one after the other (with it the call took
+    more than twice as long as without)."""
+    print("kmer longest row of a split batch", flush=True)
+    n, cap = 20000, 512
+    lens = np.random.default_rng(4).integers(1900, 2101, size=n)
+    b = batch(lens, 4)[0]
+    data, off = on_gpu(b)
+    out = fixed_width_out(n, cap)
+    took = []
+    for longest in (out[4], None):
+        least = float("inf")
+        for _ in range(8):
+            began, ended = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            began.record()
+            for _ in range(4):
+                enc.encode_padded(data, off, cap, fill_to=cap, out=(*out[:4], longest))
+            ended.record()
+            torch.cuda.synchronize()
+            least = min(least, began.elapsed_time(ended))
+        took.append(least)
+    assert int(out[4].item()) == min(cap, int(out[2].max().item()))
+    assert took[0] < 1.7 * took[1]
+
+
 @pytest.mark.parametrize("form", ["few", "reads", "rows"])
 def test_kmer_fixed_width_call_replayed_from_a_graph(enc, form):
     """A captured call keeps to its own buffers: its replays on two streams at once, with eager calls on the
