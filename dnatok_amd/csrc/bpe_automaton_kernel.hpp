@@ -55,9 +55,6 @@ struct AutoArgs {
     uint32_t letters;            // the letters by code (bits 1 and 2 of the byte)
     int32_t rows;                // (whole rows) rows of an item, at most 64
     int32_t n_groups;            // (whole rows) items (chunks: the work list says)
-    int32_t shares;              // (whole rows) 0, or: a batch of more than share_above bytes is dealt out in as many shares
-    int64_t share_above;         // of one cost (RowShares)
-    double inv_shares;           // 1 / shares
     int32_t window;              // tokens a wave has room for on their way out
     int32_t list_here;           // (chunks) the kernel makes the work list itself: at most kAutoListRows rows
     int32_t entries_here;        // (chunks) the list says where a row's chunks begin, their entries are written here (auto_entries_here)
@@ -367,9 +364,6 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
     auto number_of = [&](uint32_t e) -> uint32_t { return WIDE ? e >> 10 : e >> 2; };
 
     constexpr int kRowMax = 64 * P;                        // the longest row that a wave takes
-    constexpr bool kShares = !CHUNKS && P == 32;           // (items by their cost: batches of several steps per wave)
-    RowShares<P> shares{};
-    bool by_cost = false;
     // (list_here) chunk slots and single rows up to and including row 64 q + lane
     constexpr int kListWords = CHUNKS ? kAutoListRows / 64 : 1;
     int32_t slots_to[kListWords], singles_to[kListWords];
@@ -432,66 +426,16 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
     int32_t item = 0, row_id = 0, k = 0, nc = 1;
     int64_t row_at = 0, row_len = 0;
     int first = 0, last = 0, lanes_to = 0, lanes_own = 0;
-    bool chunk = false, more = false;                      // more: (shares) rows of the item behind lane 63
+    bool chunk = false;
     auto sum_lanes = [&]() {
         lanes_own = 0;
         if (lane >= first && lane < last) lanes_own = row_len <= 0 || row_len > kRowMax ? 1 : ((int)row_len + P - 1) / P;
         lanes_to = (int)wave_inclusive_sum_u32((uint32_t)lanes_own);
     };
-    // Rows from row `row_base` on, one per lane: those whose cost_to() is in [from, to) are the item's.
-    auto take_rows = [&](int32_t row_base, int64_t from, int64_t to) {
-        row_id = row_base + lane;
-        const int32_t at = row_id < n_rows ? row_id : n_rows, behind = row_id + 1 < n_rows ? row_id + 1 : n_rows;
-        row_at = offsets[at];
-        row_len = offsets[behind] - row_at;
-        const int64_t cost = shares.cost_to(row_id, row_at);
-        first = (int)__builtin_popcountll(__ballot(row_id < n_rows && cost < from));
-        last = (int)__builtin_popcountll(__ballot(row_id < n_rows && cost < to));
-        more = last == 64 && row_base + 64 < n_rows;
-        sum_lanes();
-    };
-    // (the batch's bytes are those of its rows: the caller's buffer may be larger)
-    auto start_shares = [&]() {
-        if (!kShares || !t.shares) return;
-        const int64_t begin = offsets[0], end = offsets[n_rows];
-        by_cost = end - begin > t.share_above;
-        if (!by_cost) return;
-        shares = RowShares<P>::of(begin, end, n_rows, t.shares, t.inv_shares);
-        n_items = t.shares;
-    };
     auto take_item = [&](int64_t item64) {
         item = (int32_t)item64;
         k = 0;
         nc = 1;
-        if (kShares && by_cost) {
-            // The rows are looked for where the rows' mean length puts them: 64 rows from a few before that place on
-            // (rows of one length are there), and 64 rows eight rows apart around it, in one trip; in the next trip
-            // those are taken that the latter point to, or, if the place is not even among them, after a search through all.
-            const int64_t from = shares.from(item64), to = shares.from(item64 + 1);
-            const int32_t guess = item64 == 0 ? 0 : shares.guess(item64);
-            const int32_t near = guess < 8 ? 0 : guess - 8, apart8 = guess + 8 * (lane - 32);
-            const int32_t look = apart8 < 0 ? 0 : apart8 > n_rows ? n_rows : apart8;
-            const int64_t probe = offsets[look];
-            take_rows(near, from, to);
-            if ((near > 0 && first == 0) || (first == 64 && near + 64 < n_rows)) {
-                const int n_below = (int)__builtin_popcountll(__ballot(shares.cost_to(look, probe) < from));
-                int32_t below = n_below > 0 ? __builtin_amdgcn_readlane(look, n_below - 1) : 0;      // starts below `from`, or is row 0
-                if ((n_below == 0 && guess - 256 > 0) || (n_below == 64 && guess + 248 < n_rows)) {
-                    int32_t lo = 0, hi = n_rows;
-                    while (hi - lo > 8) {
-                        const int32_t apart = (hi - lo + 63) >> 6;
-                        const int64_t here = (int64_t)lo + (int64_t)lane * apart;
-                        const int n = (int)__builtin_popcountll(__ballot(here < hi && shares.cost_to(here, offsets[here < hi ? here : hi]) < from));
-                        const int32_t up = n > 0 ? lo + (n - 1) * apart : lo;
-                        hi = n > 0 ? (hi - up < apart ? hi : up + apart) : lo;
-                        lo = up;
-                    }
-                    below = lo;
-                }
-                take_rows(below, from, to);
-            }
-            return;
-        }
         int32_t row = 0;
         const int32_t *list = nullptr;
         int32_t list_at = 0;
@@ -647,7 +591,6 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
             const uint32_t i = threadIdx.x + q * blockDim.x;
             if (i < tab16 + len16) piece[q] = table_piece(i);
         }
-        start_shares();
         if (item64 < n_items) {
             take_item(item64);
             if (first < last) {
@@ -667,7 +610,6 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
             for (uint32_t i = threadIdx.x; i < tab16; i += blockDim.x) table_to[i] = src[i];
             for (uint32_t i = threadIdx.x; i < len16; i += blockDim.x) table_to[tab16 + i] = src_len[i];
         }
-        start_shares();
         item64 -= (int64_t)gridDim.x * n_waves;            // (the loop below begins with the item)
     }
     if (CHARS)
@@ -972,8 +914,6 @@ __global__ __launch_bounds__(64 * kAutoMaxWaves) void bpe_auto_kernel(
         }
         if (!kAhead && first < last) {
             // (rows of the item are left)
-        } else if (kShares && more) {
-            take_rows(row_id - lane + 64, INT64_MIN, shares.from((int64_t)item + 1));
         } else {
             item64 += (int64_t)gridDim.x * n_waves;
             if (item64 >= n_items) break;

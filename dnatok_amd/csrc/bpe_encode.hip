@@ -1964,7 +1964,6 @@ __global__ __launch_bounds__(256) void bpe_gather_wave_kernel(
 
 }  // namespace dnatok
 
-#include "bpe_shares.hpp"
 #include "bpe_automaton_kernel.hpp"
 
 namespace dnatok {
@@ -2398,7 +2397,7 @@ int launch_plan(int chunking, const int64_t *offsets, const BpePlan &p, int64_t 
 
 template <bool WIDE, int P, bool CHUNKS, bool CHARS, bool PADDED>
 int launch_auto_as(const dnatok_bpe_t *t, const BpeArgs &a, AutoArgs aa, const uint8_t *bytes, const int64_t *offsets,
-                   const BpePlan &p, int64_t n_rows, int64_t max_len, int64_t total, int64_t items, int32_t *tok_tmp, int32_t *lengths, hipStream_t s)
+                   const BpePlan &p, int64_t n_rows, int64_t items, int32_t *tok_tmp, int32_t *lengths, hipStream_t s)
 {
     typedef AutoLds<WIDE, P> Lds;
     auto kern = bpe_auto_kernel<WIDE, P, CHUNKS, CHARS, PADDED>;
@@ -2423,24 +2422,18 @@ int launch_auto_as(const dnatok_bpe_t *t, const BpeArgs &a, AutoArgs aa, const u
         // as give every wave its share: 4,000 rows of 200 bases 12.7 / 13.8 us, 18,000 16.9 / 18.1, 100,000 reads 57.3 /
         // 56.0; 64 reads of 100 bases by 8 workgroups / by 64: 11.1 / 10.3 us, with the vocabulary of 32,000 12.1 / 11.3,
         // its table in no L2 26.3 / 22.5.  As many rows as fit by their mean length, 20,000 reads of 100 - 300 bases:
-        // 23.1 us, their share 18.7: a wave whose rows do not fit takes two steps.)  Where that share is several steps of
-        // rows that are not all of one length, the waves get the rows of an equal share of the bytes instead: of 100,000
-        // reads of 100 - 300 bases, 25 to a wave, one wave in 25 had rows for a fourth step, and the call took the time of
-        // four (56.8 us, now 51.5; 60,000 reads 36.5 -> 31.7).  With shares of less than a step, half of the steps that
-        // held two rows hold one (4,000 rows of 20 - 2,048 bases, vocabulary of 32,000, 38.3 us by rows, 45.2 by bytes).
-        // (`total` is what the caller's buffer holds: the kernel looks at the bytes of the rows again.)
+        // 23.1 us, their share 18.7: a wave whose rows do not fit takes two steps.)  Where a share is several steps of rows that
+        // are not all of one length, some waves have rows for a step more than the others.  Shares of one cost instead,
+        // the first row of each looked for by its place in the batch, are two trips to memory for every share and were slower
+        // but at 55,000 - 60,000 reads of 100 - 300 bases (31.2 us by cost, 33.2 by rows; 45,000 30.3 / 29.2, 80,000 39.4 / 38.2,
+        // 100,000 46.4 / 45.0, int64 47.9 / 45.5, 150,000 60.7 / 57.4; 200,000 rows of 30 - 60 bases 41.4 / 34.3; vocabulary of
+        // 32,000: 60,000 reads 98.4 / 108.5, 90,000 145.7 / 138.6, 100,000 157.4 / 157.5).
         const int64_t all = resident * waves, turns = (n_rows + 64 * all - 1) / (64 * all);
         const int64_t share = (n_rows + turns * all - 1) / (turns * all), spread = (n_rows + resident - 1) / resident;
         if (aa.rows > spread) aa.rows = (int32_t)spread;
-        if (P == 32 && aa.rows < share && total < n_rows * max_len && total > all * turns * 64 * P) {
-            aa.shares = (int32_t)(turns * all);
-            aa.share_above = all * turns * 64 * P;
-            aa.inv_shares = 1.0 / (double)aa.shares;
-        }
         if (aa.rows < share) aa.rows = (int32_t)share;
         items = (n_rows + aa.rows - 1) / aa.rows;
         aa.n_groups = (int32_t)items;
-        if (aa.shares > items) items = aa.shares;
     }
     int64_t grid = items < resident ? items : resident;
     if (a.max_tree && grid > kTreeRows) grid = kTreeRows;
@@ -2455,7 +2448,7 @@ template <bool WIDE>
 int run_auto(const dnatok_bpe_t *t, const BpeArgs &a, int chunking, const uint8_t *bytes, const int64_t *offsets,
              const BpePlan &p, int64_t n_rows, int64_t max_len, int64_t total, int32_t *tok_tmp, int32_t *lengths, hipStream_t s)
 {
-    AutoArgs aa{t->auto_next, t->auto_len, t->auto_sym, t->auto_id, t->auto_states, t->auto_letters, 1, 0, 0, 0, 0.0, 0, 0, 0, nullptr, total};
+    AutoArgs aa{t->auto_next, t->auto_len, t->auto_sym, t->auto_id, t->auto_states, t->auto_letters, 1, 0, 0, 0, 0, nullptr, total};
     if (chunking & 1) {
         aa.list_here = n_rows <= kAutoListRows ? 1 : 0;
         aa.entries_here = auto_entries_here(n_rows, total, p.core) ? 1 : 0;
@@ -2465,10 +2458,10 @@ int run_auto(const dnatok_bpe_t *t, const BpeArgs &a, int chunking, const uint8_
         }
         if (a.pad_ids) {
             aa.zero = a.longest;                     // (see the join kernel)
-            return launch_auto_as<WIDE, 32, true, false, true>(t, a, aa, bytes, offsets, p, n_rows, max_len, total, p.max_items, tok_tmp, lengths, s);
+            return launch_auto_as<WIDE, 32, true, false, true>(t, a, aa, bytes, offsets, p, n_rows, p.max_items, tok_tmp, lengths, s);
         }
-        if (a.char_ids) return launch_auto_as<WIDE, 32, true, true, false>(t, a, aa, bytes, offsets, p, n_rows, max_len, total, p.max_items, tok_tmp, lengths, s);
-        return launch_auto_as<WIDE, 32, true, false, false>(t, a, aa, bytes, offsets, p, n_rows, max_len, total, p.max_items, tok_tmp, lengths, s);
+        if (a.char_ids) return launch_auto_as<WIDE, 32, true, true, false>(t, a, aa, bytes, offsets, p, n_rows, p.max_items, tok_tmp, lengths, s);
+        return launch_auto_as<WIDE, 32, true, false, false>(t, a, aa, bytes, offsets, p, n_rows, p.max_items, tok_tmp, lengths, s);
     }
     // Regions of 32 bytes, of 16 where a wave for every row or few rows then finds a place at once: their lanes' walks
     // are half as long.  A wave's share of the rows has to fit its 64 lanes, surely or, by the rows' mean length, nearly
@@ -2481,13 +2474,13 @@ int run_auto(const dnatok_bpe_t *t, const BpeArgs &a, int chunking, const uint8_
     const bool small = len <= 1024 && (share * ((len + 15) / 16) <= 64 || share * twice_lanes <= 2 * 48);
     aa.rows = (int32_t)(64 / (small ? (len + 15) / 16 : (len + 31) / 32));
     if (small) {
-        if (a.pad_ids) return launch_auto_as<WIDE, 16, false, false, true>(t, a, aa, bytes, offsets, p, n_rows, max_len, total, n_rows, tok_tmp, lengths, s);
-        if (a.char_ids) return launch_auto_as<WIDE, 16, false, true, false>(t, a, aa, bytes, offsets, p, n_rows, max_len, total, n_rows, tok_tmp, lengths, s);
-        return launch_auto_as<WIDE, 16, false, false, false>(t, a, aa, bytes, offsets, p, n_rows, max_len, total, n_rows, tok_tmp, lengths, s);
+        if (a.pad_ids) return launch_auto_as<WIDE, 16, false, false, true>(t, a, aa, bytes, offsets, p, n_rows, n_rows, tok_tmp, lengths, s);
+        if (a.char_ids) return launch_auto_as<WIDE, 16, false, true, false>(t, a, aa, bytes, offsets, p, n_rows, n_rows, tok_tmp, lengths, s);
+        return launch_auto_as<WIDE, 16, false, false, false>(t, a, aa, bytes, offsets, p, n_rows, n_rows, tok_tmp, lengths, s);
     }
-    if (a.pad_ids) return launch_auto_as<WIDE, 32, false, false, true>(t, a, aa, bytes, offsets, p, n_rows, max_len, total, n_rows, tok_tmp, lengths, s);
-    if (a.char_ids) return launch_auto_as<WIDE, 32, false, true, false>(t, a, aa, bytes, offsets, p, n_rows, max_len, total, n_rows, tok_tmp, lengths, s);
-    return launch_auto_as<WIDE, 32, false, false, false>(t, a, aa, bytes, offsets, p, n_rows, max_len, total, n_rows, tok_tmp, lengths, s);
+    if (a.pad_ids) return launch_auto_as<WIDE, 32, false, false, true>(t, a, aa, bytes, offsets, p, n_rows, n_rows, tok_tmp, lengths, s);
+    if (a.char_ids) return launch_auto_as<WIDE, 32, false, true, false>(t, a, aa, bytes, offsets, p, n_rows, n_rows, tok_tmp, lengths, s);
+    return launch_auto_as<WIDE, 32, false, false, false>(t, a, aa, bytes, offsets, p, n_rows, n_rows, tok_tmp, lengths, s);
 }
 
 // The work list (plan) is needed when rows are cut into chunks or left to the whole-row kernel,
