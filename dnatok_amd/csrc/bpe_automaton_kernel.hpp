@@ -34,7 +34,7 @@
 // at a time, comparing the last of the four, and the padded rows of a wave written as one run of cells.)
 //
 // Per call, the merge engine -> the automaton: 1,024 rows of 1 KB 29.4 -> 11.7 us, 16,384 of them 236.5 ->
-// 26.9 us, 100,000 reads of 100 - 300 bp (int64 rows) 349 -> 51 us, 4,096 ragged reads of 12 Mbp 253.5 ->
+// 26.9 us, 100,000 reads of 100 - 300 bp (int64 rows) 349 -> 49.5 us, 4,096 ragged reads of 12 Mbp 253.5 ->
 // 79 us (all with the vocabulary of 4,096), 32 rows of 100 kbp (32,000) 143.8 -> 59.6 us.
 //
 // Beside the chains of dependent reads vector issue is what a full chip runs out of (three fifths of the time), so the
