@@ -29,7 +29,7 @@
 // rows with two launches of a scan between them -> one launch behind the one that opens the tiles:
 // 100,000 reads of 100 - 300 bp 62.9 -> 28.3 us, 1,000 of them 22.4 -> 11.5, 300,000 139 -> 58, with 50 rows of
 // 2 - 20 kbp among 100,000 87.7 -> 41.6, 300 among 3,000 287 -> 31; 20,000 rows of 1,000 bp 42.9 -> 34.9.  With long
-// rows shared among a workgroup's waves, on another box: 50 rows of 2 - 20 kbp among 100,000 reads 45.1 -> 31.2 us (the
+// rows shared among a workgroup's waves, on another card: 50 rows of 2 - 20 kbp among 100,000 reads 45.1 -> 31.2 us (the
 // two passes 80.9), those 50 in front and all sorted 557 -> 116 (642), a row of 1 Mbp in front 762 -> 128 (578), of
 // 5 Mbp 4,176 -> 621 (2,640), ten of 200 kbp 686 -> 280 (1,297); 50,000 rows of 800 - 1,000 bp 66 -> 59 (62).
 #pragma once
